@@ -2,11 +2,13 @@
 from __future__ import annotations
 
 import ctypes as C
+import importlib.util
 import os
 import subprocess
 
 CSRC = os.path.join(os.path.dirname(os.path.abspath(__file__)), "csrc")
 SO_PATH = os.path.join(CSRC, "libmi355x_wq.so")
+NATIVE_PATH = os.path.join(CSRC, "_wq_torch.so")
 
 KERNEL_AUTO, KERNEL_GEMV, KERNEL_GEMM, KERNEL_SKINNY = 0, 1, 2, 3
 ACT_NONE, ACT_RELU, ACT_SILU_MUL, ACT_GELU = 0, 1, 2, 3
@@ -126,6 +128,26 @@ def load() -> C.CDLL:
     L.mi355x_wq_module_set_workspace_rows.argtypes = [vp, i32]
     _lib = L
     return L
+
+
+_native = None
+
+
+def native():
+    """The tensor front end's native host path (csrc/wq_torch.cpp), bound to the library `load` has opened."""
+    global _native
+    if _native is not None:
+        return _native
+    L = load()
+    if not os.path.exists(NATIVE_PATH):
+        raise ImportError(f"{NATIVE_PATH} is missing: build it with `make -C {CSRC}` (or __graft_entry__.build())")
+    spec = importlib.util.spec_from_file_location("_wq_torch", NATIVE_PATH)
+    mod = importlib.util.module_from_spec(spec)
+    spec.loader.exec_module(mod)
+    mod.bind(*(C.cast(getattr(L, f), C.c_void_p).value for f in
+               ("mi355x_wq_matmul_fused_ex", "mi355x_wq_matmul_tiled_ex", "mi355x_wq_matmul_ws", "mi355x_wq_dequantize")))
+    _native = mod
+    return mod
 
 
 def last_error() -> str:

@@ -200,7 +200,15 @@ class SubgraphModule:
             return None
         cfunc = _PACKED_CFUNC(fn.value)
 
+        native, address, resource, init = _lib.native(), fn.value, res.value, name.startswith("__init_")
+
         def packed(*tensors):
+            if not init:  # device tensors, described and passed natively (None: something else among them)
+                done = native.packed_call(address, resource, tensors)
+                if done is not None:
+                    if not done:
+                        raise PackedError(_lib.last_error())
+                    return None
             targs = [_as_tensor_arg(t) for t in tensors]
             n = len(targs)
             values = (TVMValue * max(n, 1))()
@@ -210,7 +218,7 @@ class SubgraphModule:
                 codes[i] = K_TVM_NDARRAY_HANDLE
             if cfunc(C.addressof(values), codes, n, None, res) != 0:
                 raise PackedError(_lib.last_error())
-            if name.startswith("__init_"):
+            if init:
                 self._keep.extend(targs)
             return None
         return packed

@@ -34,6 +34,13 @@ def wq_matmul(x: torch.Tensor, wq: torch.Tensor, scales: torch.Tensor, bits: int
 
     ``workspace``: a device buffer from `wq_workspace` (zeroed once, then reusable by calls that do
     not overlap in time); lets the decode kernel split K across workgroups where that pays."""
+    # the native path takes the ordinary case; None = one it does not take, checked and reported (or served) below
+    y = _lib.native().matmul(x, wq, scales, bits, group, zero_point, out, kernel | (variant << 8), stream, bias,
+                             _lib.ACTIVATIONS.get(activation, -1), residual, tiled_n, workspace)
+    if y is not None:
+        if y is False:
+            raise _lib.WqError(_lib.last_error())
+        return y
     if workspace is not None:
         if kernel != 0 or variant != 0:
             raise ValueError("a workspace goes with the library's own kernel choice")
@@ -211,6 +218,11 @@ def wq_dequantize(wq: torch.Tensor, scales: torch.Tensor, bits: int, group: int,
                   zero_point: int | None = None, out: torch.Tensor | None = None,
                   stream=None) -> torch.Tensor:
     """wd[N,K] float16, bit-exact with the CPU path's `decode`."""
+    y = _lib.native().dequantize(wq, scales, bits, group, zero_point, out, stream)  # as in wq_matmul
+    if y is not None:
+        if y is False:
+            raise _lib.WqError(_lib.last_error())
+        return y
     L = _lib.load()
     wq = _as_u32_storage(wq)
     if not (wq.is_cuda and scales.is_cuda):
