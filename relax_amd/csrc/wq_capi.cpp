@@ -380,10 +380,15 @@ int matmul_any_layout(const mi355x_wq_desc* desc, const void* x, const void* wq_
   if (workspace != nullptr && family == MI355X_WQ_KERNEL_AUTO) {
     // a caller workspace allows the decode kernel's K split where it pays; everything else is as without
     if (!check_ptr(workspace, "workspace", 16)) return -1;
-    // (above 64 rows, where the plain call runs row slices of the register-activation kernel, that is the faster
-    // one -- 5120 x 5120 int8 at 192 rows: 26 us against 34 us split -- and the workspace stays unused)
-    const bool sliced = m > 64 && select_kernel(desc, m, tiled) == MI355X_WQ_KERNEL_SKINNY;
-    const int rc = sliced ? 0 : m <= 16 ? launch_gemv_split(p, workspace, workspace_bytes) : launch_gemm_split(p, workspace, workspace_bytes);
+    int rc = 0;
+    if (m <= 16) {
+      rc = launch_gemv_split(p, workspace, workspace_bytes);
+    } else if (gemm_stream_applicable(p)) {
+      const bool skinny = select_kernel(desc, m, tiled) == MI355X_WQ_KERNEL_SKINNY;
+      if (skinny || launch_gemm_streams(p)) rc = launch_gemm_stream_planned(p, workspace, workspace_bytes, skinny);
+    } else {
+      rc = launch_gemm_split(p, workspace, workspace_bytes);
+    }
     if (rc != 0) return rc < 0 ? -1 : 0;
   }
   if (library_scratch) {

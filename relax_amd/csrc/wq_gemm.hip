@@ -231,8 +231,21 @@ int launch_gemm_any(const Problem& p, int variant, bool direct_ok);
 
 }  // namespace
 
+// The streamed kernel wherever it applies (every tail fused); the others by explicit variant, up to 16 rows, for int8
+// groups of 16, short K, and for gelu onto its own residual buffer, which keeps the LDS-staged kernels.  Tile-major
+// weights and the gated tail are defined here for the direct-weight kernel's problems: K % 256 == 0, the standard group,
+// operands below 1 GiB.
+bool launch_gemm_streams(const Problem& p) {
+  const bool direct = p.k % 256 == 0 && p.group == (p.bits == 4 ? 32 : 128) && gemm_pipe_applicable(p);
+  return (direct || !(p.tiled || p.activation == kActGated)) && !(p.activation == kActGelu && p.residual == p.y);
+}
+
 int launch_gemm(const Problem& p, int variant) {
-  if (p.activation != kActGelu) return launch_gemm_any(p, variant, true);
+  if (variant == 0 && launch_gemm_streams(p)) {
+    const int rc = launch_gemm_stream_planned(p, nullptr, 0, false);
+    if (rc != 0) return rc < 0 ? -1 : 0;
+  }
+  if (p.activation != kActGelu || variant >= 31) return launch_gemm_any(p, variant, true);
   // gelu: fused by the LDS-staged kernels; behind the direct-weight kernel as a pass of its own -- unless the
   // residual is the output buffer itself, which the first pass would overwrite: then the fused kernels run.
   if (p.residual == p.y) {
@@ -283,6 +296,19 @@ int launch_gemm_any(const Problem& p, int variant, bool direct_ok) {
     set_error("gemm kernel: gelu with the residual in the output buffer is not available on the direct-weight kernel "
               "(tile-major weights, variants 21..29); pass the residual in a buffer of its own");
     return -1;
+  }
+  if (variant >= 31) {
+    if (!launch_gemm_stream(p, variant - 30, 1, nullptr)) {
+      set_error("gemm kernel: streamed variant %d does not apply to M=%lld N=%lld K=%lld group=%d", variant, (long long)p.m,
+                (long long)p.n, (long long)p.k, p.group);
+      return -1;
+    }
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) {
+      set_error("gemm kernel launch failed: %s", hipGetErrorString(e));
+      return -1;
+    }
+    return 0;
   }
   if (p.tiled) {
     // only the direct-weight kernel addresses the tile-major layout

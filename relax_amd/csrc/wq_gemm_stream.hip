@@ -1,0 +1,808 @@
+// MFMA GEMM whose operands stream through LDS: y[M,N] = x[M,K] @ dequant(Wq,S)^T, from 17 rows on.
+//
+// What bounds it: with 128 rows and more per tile the matrix pipes and, on random data, the board's power (the chip clocks
+// down); below that the vector instructions of the conversion (a weight is converted once per tile of rows: 8 per MFMA
+// at 64 rows, 4 at 128, 2 at 256; up to six per MFMA hide behind it, measured) and, for few tiles, start and end of a launch.
+//
+// A workgroup owns a TM*32 x CW*TN*32 output tile.  Activations, packed weights and scales go from memory straight into LDS
+// (buffer loads with the lds modifier: no registers, no stores), many stages ahead -- 60 to 110 KB in flight per CU,
+// which a register-staged pipeline had no room for.  Weights and scales are staged by macro steps of 128 - 256 k, so
+// that a request reads a row's whole 128-byte lines in either layout; activations by stages of 32 - 128 k.  K is an
+// index of both operands, so a lane's k of a slice are chosen to be one packed word (int4) or two (int8) of its column,
+// which it converts in registers to the float16 values of the CPU path, one slice ahead of the MFMAs that use them;
+// the A fragments come from LDS, read once per 32 * TN columns.  K groups (G): wavefronts that share columns take
+// different slices of every stage and add up at the end through LDS, in the order of the groups.
+//
+// Requests are sent by four wavefronts of their own (PROD = 4), so that a full address queue never holds up an MFMA; the
+// 256 x 256 tile, whose accumulators take half of the register file, sends them from its four wavefronts, spread over
+// the MFMAs.  Requests are counted, not tracked: every stage sends the same number (out of range once K is done), so
+// "stage t + 1 has landed" is a constant s_waitcnt and one workgroup barrier per stage.
+//
+// Rows past M, columns past N, k past K and groups past the row's end are out-of-range buffer offsets: LDS gets zeros.
+//
+// Measured against the kernels it takes over from (us, weights from memory): int4 4096 x 11008 at 37 / 128 / 512 rows 24.7 /
+// 34.8 / 69 -> 15.7 / 23.2 / 57, 12288 x 4096 at 64 / 256 rows 24.2 / 39.5 -> 17.0 / 32.3, int8 5120 x 13824 at 64 / 256
+// rows 38.7 / 78 -> 22 / 54, 15360 x 5120 at 256 rows 73 -> 48.5, 2048 rows 5 % (power).
+#include <algorithm>
+#include <atomic>
+#include <mutex>
+#include <type_traits>
+
+#include "wq_device.h"
+#include "wq_internal.h"
+
+namespace wq {
+
+namespace {
+constexpr int64_t kSplitMaxTiles = 4096;                   // arrival counters at the head of a workspace
+constexpr int64_t kSplitCounterBytes = kSplitMaxTiles * 4;  // (the same head as the other kernels' splits)
+constexpr uint32_t kStreamOob = 0x80000000u;
+
+template <int B, int E, class F>
+__device__ __forceinline__ void static_for_s(F&& f) {
+  if constexpr (B < E) {
+    f(std::integral_constant<int, B>{});
+    static_for_s<B + 1, E>(f);
+  }
+}
+
+// One request of 64 lanes from a buffer straight into LDS: lane l's 16 bytes land at lds + 16 l (its two bytes, zero
+// extended, at lds + 4 l); a lane whose offset is out of range writes zeros.  Written as assembly because the
+// compiler would order every LDS read behind every such request in flight; the kernel orders them itself.
+__device__ __forceinline__ void dma_b128(uint32_t lds, uint32_t voff, rsrc_t r, uint32_t soff) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds" ::"s"(lds), "v"(voff), "s"(r), "s"(soff) : "memory");
+}
+__device__ __forceinline__ void dma_u16(uint32_t lds, uint32_t voff, rsrc_t r, uint32_t soff) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_ushort %1, %2, %3 offen lds" ::"s"(lds), "v"(voff), "s"(r), "s"(soff) : "memory");
+}
+template <int N>
+__device__ __forceinline__ void wait_dma() {
+  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
+}
+}  // namespace
+
+template <int BITS, int TM, int TN, int CW, int G, int PROD, int KA, int KM, int NM>
+struct StreamShape {
+  static constexpr int kBM = TM * 32, kBN = CW * TN * 32, kWaves = CW * G, kThreads = (kWaves + PROD) * 64;
+  static constexpr int kIssuers = PROD > 0 ? PROD : kWaves;  // wavefronts that send requests
+  static constexpr int kKM = KM;                       // k per macro step: what weights and scales are staged by
+  static constexpr int kSPM = kKM / KA;                // activation stages per macro step
+  static constexpr int kKG = KA / G;                   // k of a stage that one wavefront multiplies
+  static constexpr int kSlices = kKG / 16;             // MFMA k slices of it
+  static constexpr int kARow = KA * 2;                 // bytes of an activation row per stage
+  static constexpr int kWRow = kKM * BITS / 8;         // packed bytes of a weight row per macro step
+  static constexpr int kSub = kKM / 32;                // scales of a row per macro step (one dword per 32 k)
+  static constexpr int kABytes = kBM * kARow, kWBytes = kBN * kWRow, kSBytes = kBN * kSub * 4;
+  static constexpr int kQA = kABytes / 1024, kQW = kWBytes / 1024, kQS = kSBytes / 256;  // requests
+  static constexpr int kNA = kQA / kIssuers;                                    // ... of one of them
+  static constexpr int kNW = (kQW + kIssuers - 1) / kIssuers;
+  static constexpr int kNS = (kQS + kIssuers - 1) / kIssuers;
+  static constexpr int kNWS = kNW + kNS;
+  static constexpr bool kDummy = kQW % kIssuers != 0 || kQS % kIssuers != 0;
+  static constexpr int kLdsMax = 160 * 1024 - (kDummy ? 1024 : 0);
+  static constexpr int kMacros = NM;                      // macro steps in the ring
+  static constexpr int kRoom = (kLdsMax - kMacros * (kWBytes + kSBytes)) / kABytes;
+  static constexpr int kStages = kRoom < 8 ? kRoom : 8;  // activation stages in the ring
+  static constexpr int kWBase = kStages * kABytes, kSBase = kWBase + kMacros * kWBytes, kDummyBase = kSBase + kMacros * kSBytes;
+  // end of the K loop: the G groups exchange partial sums, each finishing PG of the TM*4 row quads
+  static constexpr int kPG = TM * 4 / G;
+  static constexpr int kXPerTarget = (G - 1) * CW * kPG * TN * 1024;              // LDS bytes a target group receives
+  static constexpr int kTargets = G == 1 ? 1 : (160 * 1024 / kXPerTarget < G ? 160 * 1024 / kXPerTarget : G);  // per phase
+  static constexpr int kLds = std::max(kDummyBase + (kDummy ? 1024 : 0), kTargets * kXPerTarget);
+  static_assert(kQA % kIssuers == 0 && kSlices >= 1 && kStages >= 3 && TM * 4 % G == 0 && kSPM % 2 == 0 && CW * G % 4 == 0, "shape");
+
+  // Requests that may still be in flight at the top of stage t (of a macro step), where the activations of stage t + 1 and
+  // the weights of stage t + kAhead have to be there.  Stage u issues the activations of stage u + kStages - 1, and a macro
+  // step's first stage, before those, the weights of the macro step kMacros - 1 later.
+  static constexpr int kAhead = kSlices == 1 ? 2 : 1;
+  static constexpr int in_flight(int t) {
+    const int t0 = t + 4 * kSPM * kMacros;  // (any macro step of the steady state)
+    const int last_a = t0 + 2 - kStages;    // stage that issued the activations needed
+    const int need_macro = (t0 + kAhead) / kSPM, u_w = (need_macro - kMacros + 1) * kSPM;
+    int n = 0;
+    for (int u = t0 - 1; u > last_a; --u) {
+      n += kNA;
+      if (u == u_w) return n;
+      if (u % kSPM == 0) n += kNWS;
+    }
+    return n;
+  }
+};
+
+// LDS rows hold their 16-byte chunks XOR-swizzled with the row so that sixteen consecutive rows reading the same chunk cover all
+// 64 banks once.
+__device__ __forceinline__ int stream_swizzle(int row, int chunks) { return (row / (16 / chunks)) % chunks; }
+
+// The requests of one wavefront: request q of an operand fills 1 KB of its LDS area (64 dwords for scales).
+template <class C, int BITS, int TN, bool TILED>
+struct StreamRequests {
+  static constexpr int R = C::kIssuers;
+  uint32_t av[C::kNA], wv[C::kNW], sv[C::kNS];
+  int a_k, w_k, s_sub, me, k_end, group_log2;
+  uint32_t lds0;
+  rsrc_t rx, rw, rs;
+
+  // LDS row r of the weights and scales is column tile r / 32 % TN of column wave r / (32 TN), lane r % 32: a matrix row such
+  // that a lane ends up with TN adjacent outputs
+  __device__ __forceinline__ static int matrix_row(int r) { return r / (32 * TN) * (32 * TN) + TN * (r & 31) + (TN == 1 ? 0 : (r >> 5) % TN); }
+
+  __device__ __forceinline__ void init(int me_, int lane, int m0, int n0, int M, int N, int K, bool gated) {
+    me = me_;
+    const uint32_t row_bytes = (uint32_t)K * BITS / 8, groups_per_row = (uint32_t)K >> group_log2;
+    {
+      constexpr int CPR = C::kARow / 16, RPQ = 64 / CPR;  // chunks per row, rows per request
+      static_assert(R * RPQ % 16 == 0, "the swizzle term is the same for all requests of a lane");
+      const int r0 = me * RPQ + lane / CPR;
+      const int chunk = (lane % CPR) ^ stream_swizzle(r0, CPR);
+      a_k = chunk * 8;
+#pragma unroll
+      for (int i = 0; i < C::kNA; ++i) {
+        const int m = m0 + r0 + i * R * RPQ;
+        av[i] = m < M ? (uint32_t)m * (uint32_t)K * 2u + (uint32_t)chunk * 16u : kStreamOob;
+      }
+    }
+    {
+      constexpr int CPR = C::kWRow / 16, RPQ = 64 / CPR;
+      static_assert(R * RPQ % 16 == 0, "the swizzle term is the same for all requests of a lane");
+#pragma unroll
+      for (int i = 0; i < C::kNW; ++i) {
+        const int r = (me + i * R) * RPQ + lane / CPR;
+        const int c = (lane % CPR) ^ stream_swizzle(r, CPR);
+        const int n = n0 + matrix_row(r);
+        w_k = c * (128 / BITS);
+        if (r >= C::kBN || n >= N) {
+          wv[i] = kStreamOob;
+        } else if constexpr (TILED) {
+          // chunk c of row n: 128-byte super step s = c / 8, chunk cc = c % 8 of it at ((n/16 * nsuper + s) * 2 + cc%2) * 1024 +
+          // (cc/2 * 16 + n%16) * 16
+          const uint32_t nsuper = row_bytes / 128u, cc = (uint32_t)c & 7u;
+          wv[i] = ((((uint32_t)n >> 4) * nsuper + ((uint32_t)c >> 3)) * 2u + (cc & 1u)) * 1024u + ((cc >> 1) * 16u + ((uint32_t)n & 15u)) * 16u;
+        } else {
+          wv[i] = (uint32_t)(gated ? gated_physical_row(n, N) : n) * row_bytes + (uint32_t)c * 16u;
+        }
+      }
+    }
+    s_sub = lane % C::kSub;
+#pragma unroll
+    for (int i = 0; i < C::kNS; ++i) {
+      const int r = (me + i * R) * (64 / C::kSub) + lane / C::kSub;
+      const int n = n0 + matrix_row(r);
+      if (r >= C::kBN || n >= N) sv[i] = kStreamOob;
+      else if constexpr (TILED && BITS == 4) sv[i] = ((uint32_t)n >> 4) * (row_bytes / 128u) * 256u + (((uint32_t)s_sub >> 1) * 16u + ((uint32_t)n & 15u)) * 4u + ((uint32_t)s_sub & 1u) * 2u;
+      else if constexpr (TILED) sv[i] = ((((uint32_t)n >> 4) * (row_bytes / 128u) + ((uint32_t)s_sub >> 2)) * 16u + ((uint32_t)n & 15u)) * 2u;
+      else sv[i] = (uint32_t)(gated ? gated_physical_row(n, N) : n) * groups_per_row * 2u;
+    }
+  }
+
+  // request P of the activations from k0 on, into the stage at LDS offset `buf`; lanes past k_end read zeros
+  template <int P>
+  __device__ __forceinline__ void issue_a(int k0, uint32_t buf) const {
+    dma_b128(lds0 + buf + (uint32_t)(me + P * R) * 1024u, k0 + a_k < k_end ? av[P] : kStreamOob, rx, (uint32_t)k0 * 2u);
+  }
+  // request P of the weights and scales of the macro step from k0 on, into place `ring` of their rings
+  template <int P>
+  __device__ __forceinline__ void issue_ws(int k0, uint32_t ring) const {
+    if constexpr (P < C::kNW) {
+      const int q = me + P * R;
+      const bool mine = C::kQW % R == 0 || q < C::kQW;
+      const uint32_t byte = (uint32_t)k0 * BITS / 8u, off = TILED ? (byte >> 7) * 2048u + ((byte >> 5) & 3u) * 256u : byte;
+      dma_b128(lds0 + (mine ? C::kWBase + ring * C::kWBytes + (uint32_t)q * 1024u : (uint32_t)C::kDummyBase), k0 + w_k < k_end ? wv[P] : kStreamOob, rw, off);
+    } else {
+      constexpr int i = P - C::kNW;
+      const int q = me + i * R;
+      const bool mine = C::kQS % R == 0 || q < C::kQS;
+      uint32_t v = sv[i], off = 0;
+      if constexpr (TILED) off = BITS == 4 ? (uint32_t)k0 : (uint32_t)k0 / 4u;  // (256 bytes per 256 k, 32 per 128 k)
+      else v += (uint32_t)((k0 + s_sub * 32) >> group_log2) * 2u;
+      dma_u16(lds0 + (mine ? C::kSBase + ring * C::kSBytes + (uint32_t)q * 256u : (uint32_t)C::kDummyBase), k0 + s_sub * 32 < k_end ? v : kStreamOob, rs, off);
+    }
+  }
+  // What stages -(kStages - 1) .. -1 would have issued, in their order; weights due before that first.
+  template <int SPM, int KA, int KM>
+  __device__ __forceinline__ void prologue(int k_begin) const {
+    auto issue_macro = [&](auto mm) __attribute__((always_inline)) {
+      static_for_s<0, C::kNWS>([&](auto piece) __attribute__((always_inline)) { issue_ws<decltype(piece)::value>(k_begin + decltype(mm)::value * KM, decltype(mm)::value); });
+    };
+    static_for_s<0, C::kMacros - 1>([&](auto mm) __attribute__((always_inline)) {
+      if constexpr ((C::kMacros - 1 - decltype(mm)::value) * SPM > C::kStages - 1) issue_macro(mm);
+    });
+    static_for_s<0, C::kStages - 1>([&](auto p) __attribute__((always_inline)) {
+      constexpr int back = C::kStages - 1 - decltype(p)::value;  // stage -back
+      if constexpr (back % SPM == 0 && back / SPM <= C::kMacros - 1) issue_macro(std::integral_constant<int, C::kMacros - 1 - back / SPM>{});
+      static_for_s<0, C::kNA>([&](auto piece) __attribute__((always_inline)) { issue_a<decltype(piece)::value>(k_begin + decltype(p)::value * KA, decltype(p)::value * C::kABytes); });
+    });
+    wait_dma<C::in_flight(SPM - 1)>();
+  }
+};
+
+template <int BITS, int TM, int TN, int CW, int G, int PROD, int KA, int KM, int NM, bool TILED, bool KSPLIT>
+__global__ __launch_bounds__((CW * G + PROD) * 64, 1) void wq_gemm_stream_kernel(
+    const half_t* __restrict__ x, const uint32_t* __restrict__ wq, const half_t* __restrict__ scales, int M, int N, int K,
+    int shift_and_zero, int tiles_m, int tiles_n, int ksplit, half_t* y, const Epilogue ep, float* partials,
+    unsigned int* counters) {
+  using C = StreamShape<BITS, TM, TN, CW, G, PROD, KA, KM, NM>;
+  constexpr int BM = C::kBM, BN = C::kBN, WAVES = C::kWaves, SPM = C::kSPM, NS = C::kSlices;
+  const int group_log2 = shift_and_zero & 0xFF, zero_point = (shift_and_zero >> 8) & 0xFF;  // group = 1 << group_log2 >= 32
+  const bool gated = (shift_and_zero >> 16) & 1;
+  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+  const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) unsigned char*)smem;
+
+  // ---- which tile: workgroup ids go round the XCDs; give each XCD a contiguous range of the list (K windows, then
+  // panels of eight column tiles, rows of the panel) so that it shares activation blocks and weight tiles in its L2
+  const int S = KSPLIT ? ksplit : 1;
+  const int ntiles = tiles_m * tiles_n, nblocks = ntiles * S;
+  const int xcd = blockIdx.x & 7, per_xcd = nblocks >> 3, extra = nblocks & 7;
+  int lin = xcd * per_xcd + min(xcd, extra) + ((int)blockIdx.x >> 3);
+  const int ks = S > 1 ? lin / ntiles : 0;
+  const int tile_lin = lin - ks * ntiles;
+  constexpr int PANEL = 8;
+  const int full = tiles_n / PANEL, panel = min(tile_lin / (tiles_m * PANEL), full);
+  const int width = panel < full ? PANEL : tiles_n - full * PANEL;
+  const int rest = tile_lin - panel * tiles_m * PANEL;
+  const int m0 = rest / width * BM, n0 = (panel * PANEL + rest % width) * BN;
+
+  const int lane = threadIdx.x & 63, fr = lane & 31, fh = lane >> 5;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int grp = wave / CW, cw = wave % CW;
+
+  // macro steps [k_begin, k_end) / 256 of this workgroup; lanes past k_end read zeros
+  const int macros_all = (K + KM - 1) / KM, per_window = (macros_all + S - 1) / S;
+  const int k_begin = ks * per_window * KM, k_end = min(k_begin + per_window * KM, K);
+
+  using std::integral_constant;
+  StreamRequests<C, BITS, TN, TILED> req;
+  req.k_end = k_end;
+  req.group_log2 = group_log2;
+  req.lds0 = lds0;
+  req.rx = make_rsrc(x, (uint32_t)M * (uint32_t)K * 2u);
+  {
+    const uint32_t n_stored = TILED ? ((uint32_t)N + 15u) / 16u * 16u : (uint32_t)N;
+    req.rw = make_rsrc(wq, n_stored * ((uint32_t)K * BITS / 8));
+    req.rs = make_rsrc(scales, n_stored * ((uint32_t)K >> group_log2) * 2u);
+  }
+  if constexpr (PROD > 0) {
+    if (wave >= WAVES) {
+      // producer wavefronts: requests only
+      __builtin_amdgcn_s_setprio(2);
+      req.init(wave - WAVES, lane, m0, n0, M, N, K, gated);
+      req.template prologue<SPM, KA, KM>(k_begin);
+      __builtin_amdgcn_s_barrier();
+      asm volatile("" ::: "memory");
+      uint32_t abuf = (C::kStages - 1) * C::kABytes, ring = C::kMacros - 1;
+      for (int k0 = k_begin; k0 < k_end; k0 += KM) {
+        static_for_s<0, SPM>([&](auto tc) __attribute__((always_inline)) {
+          constexpr int t = decltype(tc)::value;
+          wait_dma<C::in_flight(t)>();
+          __builtin_amdgcn_s_barrier();
+          asm volatile("" ::: "memory");
+          if constexpr (t == 0) {
+            static_for_s<0, C::kNWS>([&](auto piece) __attribute__((always_inline)) { req.template issue_ws<decltype(piece)::value>(k0 + (C::kMacros - 1) * KM, ring); });
+            ring = ring + 1 == C::kMacros ? 0 : ring + 1;
+          }
+          static_for_s<0, C::kNA>([&](auto piece) __attribute__((always_inline)) { req.template issue_a<decltype(piece)::value>(k0 + (t + C::kStages - 1) * KA, abuf); });
+          abuf = abuf + C::kABytes == C::kStages * C::kABytes ? 0 : abuf + C::kABytes;
+        });
+      }
+      wait_dma<0>();
+      __builtin_amdgcn_s_barrier();
+      return;
+    }
+  } else {
+    req.init(wave, lane, m0, n0, M, N, K, gated);
+    req.template prologue<SPM, KA, KM>(k_begin);
+  }
+
+  // ---- LDS reads of this lane: KL contiguous k of a stage, from (grp * kKG + fh * KL) on ------------------------
+  constexpr int KL = C::kKG / 2, WB = KL * BITS / 8, WL = WB > 16 ? WB / 16 : 1, WORDS = WB / 4;
+  const int kl0 = grp * C::kKG + fh * KL;
+  uint32_t a_rd[NS], w_rd[SPM][WL], s_rd[SPM];
+#pragma unroll
+  for (int kk = 0; kk < NS; ++kk) a_rd[kk] = (uint32_t)fr * C::kARow + (uint32_t)(((kl0 / 8 + kk) ^ stream_swizzle(fr, C::kARow / 16)) << 4);
+  const int wrow = cw * TN * 32 + fr;  // + 32 j
+#pragma unroll
+  for (int t = 0; t < SPM; ++t) {
+#pragma unroll
+    for (int v = 0; v < WL; ++v) {
+      const int byte = (t * KA + kl0) * BITS / 8 + v * 16;
+      w_rd[t][v] = C::kWBase + (uint32_t)wrow * C::kWRow + (uint32_t)(((byte / 16) ^ stream_swizzle(wrow, C::kWRow / 16)) << 4) + (byte & 15);
+    }
+    s_rd[t] = C::kSBase + (uint32_t)(wrow * C::kSub + (t * KA + kl0) / 32) * 4u;
+  }
+
+  const Q4Consts qc = make_q4_consts(zero_point);
+  float16_t acc[TM][TN];
+#pragma unroll
+  for (int i = 0; i < TM; ++i)
+#pragma unroll
+    for (int j = 0; j < TN; ++j)
+#pragma unroll
+      for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.f;
+
+  struct Words {
+    uint32_t w[TN][WORDS];
+    half_t s[TN];
+  };
+  Words words[2];
+  auto read_words = [&](Words& d, uint32_t ring, auto tt) __attribute__((always_inline)) {
+    constexpr int t = decltype(tt)::value;
+    const unsigned char* const wb = smem + ring * C::kWBytes;
+    const unsigned char* const sb = smem + ring * C::kSBytes;
+#pragma unroll
+    for (int j = 0; j < TN; ++j) {
+      if constexpr (WB >= 16) {
+#pragma unroll
+        for (int v = 0; v < WL; ++v) {
+          const u32x4 q = *reinterpret_cast<const u32x4*>(wb + w_rd[t][v] + j * 32 * C::kWRow);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) d.w[j][v * 4 + e] = q[e];
+        }
+      } else if constexpr (WB == 8) {
+        const u32x2 q = *reinterpret_cast<const u32x2*>(wb + w_rd[t][0] + j * 32 * C::kWRow);
+        d.w[j][0] = q[0], d.w[j][1] = q[1];
+      } else {
+        d.w[j][0] = *reinterpret_cast<const uint32_t*>(wb + w_rd[t][0] + j * 32 * C::kWRow);
+      }
+      d.s[j] = *reinterpret_cast<const half_t*>(sb + s_rd[t] + j * 32 * C::kSub * 4);
+    }
+  };
+  // Weight pair PR (of four) of a lane's eight k of slice KK, column tile J, in two halves: integers with the float16
+  // exponent bits in place, then the exact subtraction and the one rounding of the product with the scale.
+  auto convert_front = [&](const Words& d, auto kk, auto jj, auto pp) __attribute__((always_inline)) -> uint32_t {
+    constexpr int KK = decltype(kk)::value, J = decltype(jj)::value, PR = decltype(pp)::value;
+    if constexpr (BITS == 4) {
+      const uint32_t t = __builtin_amdgcn_perm(0u, d.w[J][KK], 0x0c000c00u | PR | (PR << 16));
+      return (t & 0x00F0000Fu) | qc.magic;
+    } else {
+      return cvt_i8_lo<PR % 2 * 2>(d.w[J][2 * KK + PR / 2]);
+    }
+  };
+  auto convert_back = [&](const Words& d, uint32_t f, auto kk, auto jj, auto pp) __attribute__((always_inline)) -> uint32_t {
+    constexpr int KK = decltype(kk)::value, J = decltype(jj)::value, PR = decltype(pp)::value;
+    if constexpr (BITS == 4) return as_u32(__builtin_elementwise_fma(as_h2(f), qc.mix_mul, -qc.mix_sub) * bcast_h2(d.s[J]));
+    else return as_u32(as_h2(cvt_i8_hi<PR % 2 * 2 + 1>(f, d.w[J][2 * KK + PR / 2])) * bcast_h2(d.s[J]));
+  };
+  half8_t a[2][TM];
+  uint32_t b[2][TN][4];
+  constexpr int SLOTS = TM * TN, PAIRS = TN * 4;  // MFMAs and weight pairs of a slice
+
+  // ---- K loop (program order is issue order: sched_barrier after every MFMA).  Slice q is multiplied while the A fragments of slice q + 1 are read and its weights converted; packed
+  // words and scales are read a slice before their conversion begins.
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+  read_words(words[0], 0, integral_constant<int, 0>{});
+  if constexpr (NS == 1) read_words(words[1], 0, integral_constant<int, 1>{});
+#pragma unroll
+  for (int i = 0; i < TM; ++i) a[0][i] = *reinterpret_cast<const half8_t*>(smem + a_rd[0] + i * 32 * C::kARow);
+  static_for_s<0, PAIRS>([&](auto q) __attribute__((always_inline)) {
+    constexpr int j = decltype(q)::value / 4, pr = decltype(q)::value % 4;
+    integral_constant<int, 0> kk;
+    integral_constant<int, j> jj;
+    integral_constant<int, pr> pp;
+    b[0][j][pr] = convert_back(words[0], convert_front(words[0], kk, jj, pp), kk, jj, pp);
+  });
+  uint32_t abuf = 0, abuf_issue = (C::kStages - 1) * C::kABytes, ring = 0;
+  for (int k0 = k_begin; k0 < k_end; k0 += KM) {
+    const uint32_t ring_next = ring + 1 == C::kMacros ? 0 : ring + 1, ring_issue = ring == 0 ? C::kMacros - 1 : ring - 1;
+    static_for_s<0, SPM>([&](auto tc) __attribute__((always_inline)) {
+      constexpr int t = decltype(tc)::value;
+      const uint32_t abuf_next = abuf + C::kABytes == C::kStages * C::kABytes ? 0 : abuf + C::kABytes;
+      if constexpr (PROD == 0) wait_dma<C::in_flight(t)>();  // (otherwise the producers have waited)
+      __builtin_amdgcn_sched_barrier(0);
+      __builtin_amdgcn_s_barrier();
+      asm volatile("" ::: "memory");
+      static_for_s<0, NS>([&](auto kkc) __attribute__((always_inline)) {
+        constexpr int kk = decltype(kkc)::value, q = t * NS + kk;         // slice of the macro step
+        constexpr int t1 = (q + 1) / NS, kk1 = (q + 1) % NS;              // the next slice, being converted
+        constexpr int t2 = (q + 2) / NS, kk2 = (q + 2) % NS;              // the one after it
+        uint32_t front[PAIRS];
+        static_for_s<0, SLOTS>([&](auto sc) __attribute__((always_inline)) {
+          constexpr int s = decltype(sc)::value, i = s / TN, j = s % TN;
+          acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(
+              a[q & 1][i], __builtin_bit_cast(half8_t, *reinterpret_cast<const u32x4*>(b[q & 1][j])), acc[i][j], 0, 0, 0);
+          if constexpr (s < TM)
+            a[(q + 1) & 1][s] = *reinterpret_cast<const half8_t*>(smem + (kk1 == 0 ? abuf_next : abuf) + a_rd[kk1] + s * 32 * C::kARow);
+          if constexpr (s == 0 && kk2 == 0) read_words(words[t2 & 1], t2 >= SPM ? ring_next : ring, integral_constant<int, t2 % SPM>{});
+          if constexpr (PROD == 0) {
+            // requests of later stages, evenly over the slots: weights and scales first
+            constexpr int slot = kk * SLOTS + s, WS = t == 0 ? C::kNWS : 0, ALL = WS + C::kNA;
+            constexpr int P0 = slot * ALL / (NS * SLOTS), P1 = (slot + 1) * ALL / (NS * SLOTS);
+            static_for_s<P0, P1>([&](auto pc) __attribute__((always_inline)) {
+              constexpr int P = decltype(pc)::value;
+              if constexpr (P < WS) req.template issue_ws<P>(k0 + (C::kMacros - 1) * KM, ring_issue);
+              else req.template issue_a<P - WS>(k0 + (t + C::kStages - 1) * KA, abuf_issue);
+            });
+          }
+          constexpr int F0 = s * PAIRS / SLOTS, F1 = (s + 1) * PAIRS / SLOTS, B0 = s == 0 ? 0 : (s - 1) * PAIRS / SLOTS, B1 = s + 1 == SLOTS ? PAIRS : F0;
+          static_for_s<F0, F1>([&](auto qc_) __attribute__((always_inline)) {
+            constexpr int p = decltype(qc_)::value;
+            front[p] = convert_front(words[t1 & 1], integral_constant<int, kk1>{}, integral_constant<int, p / 4>{}, integral_constant<int, p % 4>{});
+          });
+          static_for_s<B0, B1>([&](auto qc_) __attribute__((always_inline)) {
+            constexpr int p = decltype(qc_)::value;
+            b[(q + 1) & 1][p / 4][p % 4] = convert_back(words[t1 & 1], front[p], integral_constant<int, kk1>{}, integral_constant<int, p / 4>{}, integral_constant<int, p % 4>{});
+          });
+          __builtin_amdgcn_sched_barrier(0);
+        });
+      });
+      abuf_issue = abuf;
+      abuf = abuf_next;
+    });
+    ring = ring_next;
+  }
+  if constexpr (PROD == 0) wait_dma<0>();
+  __builtin_amdgcn_s_barrier();  // the last requests (all out of range) have landed
+  asm volatile("" ::: "memory");
+
+  // ---- K groups: every group hands its partial sums of the other groups' row quads over through LDS ----------------
+  constexpr int PG = C::kPG;
+  float4_t fin[PG][TN];
+  auto part = [&](int pair, int j) __attribute__((always_inline)) {
+    const float16_t& c = acc[pair / 4][j];
+    const int v = pair % 4 * 4;
+    return float4_t{c[v], c[v + 1], c[v + 2], c[v + 3]};
+  };
+  if constexpr (G == 1) {
+#pragma unroll
+    for (int p = 0; p < PG; ++p)
+#pragma unroll
+      for (int j = 0; j < TN; ++j) fin[p][j] = part(p, j);
+  } else {
+    static_for_s<0, (G + C::kTargets - 1) / C::kTargets>([&](auto phase) __attribute__((always_inline)) {
+      constexpr int T0 = decltype(phase)::value * C::kTargets, T1 = T0 + C::kTargets < G ? T0 + C::kTargets : G;
+      __syncthreads();
+      static_for_s<T0, T1>([&](auto tt) __attribute__((always_inline)) {
+        constexpr int t = decltype(tt)::value;
+        if (grp != t) {
+          const int src = grp < t ? grp : grp - 1;
+          float4_t* const dst = reinterpret_cast<float4_t*>(smem) + (((t - T0) * (G - 1) + src) * CW + cw) * PG * TN * 64 + lane;
+#pragma unroll
+          for (int p = 0; p < PG; ++p)
+#pragma unroll
+            for (int j = 0; j < TN; ++j) dst[(p * TN + j) * 64] = part(t * PG + p, j);
+        }
+      });
+      __syncthreads();
+      static_for_s<T0, T1>([&](auto tt) __attribute__((always_inline)) {
+        constexpr int t = decltype(tt)::value;
+        if (grp == t) {
+          const float4_t* const sp = reinterpret_cast<const float4_t*>(smem) + ((t - T0) * (G - 1) * CW + cw) * PG * TN * 64 + lane;
+#pragma unroll
+          for (int p = 0; p < PG; ++p)
+#pragma unroll
+            for (int j = 0; j < TN; ++j) {
+              // (in the order of the groups, whichever of them adds: an output does not depend on its place in the tile)
+              float4_t f = t == 0 ? part(p, j) : sp[(p * TN + j) * 64];
+#pragma unroll
+              for (int g = 1; g < G; ++g) f += g == t ? part(t * PG + p, j) : sp[((g < t ? g : g - 1) * CW * PG * TN + p * TN + j) * 64];
+              fin[p][j] = f;
+            }
+        }
+      });
+    });
+  }
+
+  if constexpr (KSPLIT) {
+    // K split over workgroups: float32 partial tiles through the workspace, added in window order by the last to arrive.
+    // Partials and counters are only touched by accesses performed at the memory side of the L2s (sc1).
+    constexpr uint32_t kWaveBytes = PG * TN * 1024u;
+    const rsrc_t rp = make_rsrc(reinterpret_cast<char*>(partials) + (size_t)tile_lin * S * WAVES * kWaveBytes, (uint32_t)S * WAVES * kWaveBytes);
+#pragma unroll
+    for (int p = 0; p < PG; ++p)
+#pragma unroll
+      for (int j = 0; j < TN; ++j)
+        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, fin[p][j]), rp, (uint32_t)(ks * WAVES + wave) * kWaveBytes + (p * TN + j) * 1024u + lane * 16u, 0, 0x10);
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+    int* const last = reinterpret_cast<int*>(smem);
+    if (threadIdx.x == 0)
+      *last = __hip_atomic_fetch_add(&counters[tile_lin], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == (unsigned)(S - 1);
+    __syncthreads();
+    if (!*last) return;
+    if (threadIdx.x == 0) __hip_atomic_store(&counters[tile_lin], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+#pragma unroll
+    for (int p = 0; p < PG; ++p)
+#pragma unroll
+      for (int j = 0; j < TN; ++j) fin[p][j] = float4_t{0.f, 0.f, 0.f, 0.f};
+    constexpr int WIN = PG * TN <= 4 ? 4 : PG * TN <= 16 ? 2 : 1;  // windows in flight
+    for (int q = 0; q < S; q += WIN) {
+      u32x4 win[WIN][PG][TN];
+#pragma unroll
+      for (int w = 0; w < WIN; ++w)
+#pragma unroll
+        for (int p = 0; p < PG; ++p)
+#pragma unroll
+          for (int j = 0; j < TN; ++j)
+            win[w][p][j] = __builtin_amdgcn_raw_buffer_load_b128(rp, (q + w < S ? (uint32_t)((q + w) * WAVES + wave) * kWaveBytes : kStreamOob) + (p * TN + j) * 1024u + lane * 16u, 0, 0x10);
+#pragma unroll
+      for (int w = 0; w < WIN; ++w)
+#pragma unroll
+        for (int p = 0; p < PG; ++p)
+#pragma unroll
+          for (int j = 0; j < TN; ++j) fin[p][j] += __builtin_bit_cast(float4_t, win[w][p][j]);
+    }
+  }
+
+  // ---- epilogue: lane holds columns n .. n + TN - 1, rows 8 (pair % 4) + 4 fh + e of row block pair / 4.  The tail's shape
+  // is decided once; rows are addressed with 32-bit offsets from the first, rows past M go out of the buffer's range.
+  const int n = n0 + cw * TN * 32 + TN * fr;
+  const int pair0 = grp * PG;
+  auto row_in_tile = [&](int p, int e) __attribute__((always_inline)) { return ((pair0 + p) >> 2) * 32 + ((pair0 + p) & 3) * 8 + fh * 4 + e; };
+  if (gated) {
+    // columns 2 c (gate) and 2 c + 1 (up) of the interleaved order: in one lane, or (one column tile) in a lane and the next
+    const int rows = min(BM, M - m0), half_n = N >> 1;
+    const rsrc_t ry = make_rsrc(y + (size_t)m0 * half_n, (uint32_t)rows * (uint32_t)half_n * 2u);
+    const uint32_t col = (n & 1) == 0 && n + 1 < N ? (uint32_t)(n >> 1) * 2u : kStreamOob;
+#pragma unroll
+    for (int p = 0; p < PG; ++p)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const uint32_t r = (uint32_t)row_in_tile(p, e);
+        float up = fin[p][TN - 1][e];
+        if constexpr (TN == 1) up = __shfl_down(up, 1);
+        const half_t h = silu_mul((half_t)fin[p][0][e], (half_t)up);
+        __builtin_amdgcn_raw_buffer_store_b16(__builtin_bit_cast(uint16_t, h), ry, r < (uint32_t)rows && col != kStreamOob ? r * (uint32_t)half_n * 2u + col : kStreamOob, 0, 0);
+      }
+    return;
+  }
+  if (TN == 2 && pair_store_ok(ep, y, N)) {
+    const int rows = min(BM, M - m0);
+    const uint32_t bytes = (uint32_t)rows * (uint32_t)N * 2u, pitch = (uint32_t)N * 2u;
+    const uint32_t col = n < N ? (uint32_t)n * 2u : kStreamOob;
+    const uint32_t base = col + (uint32_t)row_in_tile(0, 0) * pitch;
+    auto offset = [&](int p, int e) __attribute__((always_inline)) {  // of row quad p, row e; p = 0, e = 0 is `base`
+      const int r = row_in_tile(p, e);
+      return r < rows ? base + (uint32_t)(r - row_in_tile(0, 0)) * pitch : kStreamOob;
+    };
+    // (in portions of four row quads, which keeps the registers of the loop's accumulators apart from the tail's)
+    constexpr int PC = PG < 4 ? PG : 4;
+    static_for_s<0, PG / PC>([&](auto portion) __attribute__((always_inline)) {
+      constexpr int p0 = decltype(portion)::value * PC;
+      half2_t h[PC][4];
+#pragma unroll
+      for (int p = 0; p < PC; ++p)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) h[p][e] = half2_t{(half_t)fin[p0 + p][0][e], (half_t)fin[p0 + p][TN - 1][e]};
+      if (ep.bias != nullptr) {
+        const half2_t b2 = as_h2(load_b32(make_rsrc(ep.bias, (uint32_t)N * 2u), col));
+#pragma unroll
+        for (int p = 0; p < PC; ++p)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) h[p][e] = h[p][e] + b2;
+      }
+      if (ep.activation == 1) {
+#pragma unroll
+        for (int p = 0; p < PC; ++p)
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+#pragma unroll
+            for (int c = 0; c < 2; ++c) h[p][e][c] = h[p][e][c] > (half_t)0 ? h[p][e][c] : (half_t)0;
+      }
+      if (__builtin_expect(ep.activation == kActGelu, 0)) {
+#pragma unroll
+        for (int p = 0; p < PC; ++p)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) h[p][e] = half2_t{gelu_f16(h[p][e][0]), gelu_f16(h[p][e][1])};
+      }
+      if (ep.residual != nullptr) {
+        const rsrc_t rr = make_rsrc(ep.residual + (size_t)m0 * N, bytes);
+        uint32_t res[PC][4];
+#pragma unroll
+        for (int p = 0; p < PC; ++p)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) res[p][e] = load_b32(rr, offset(p0 + p, e));
+#pragma unroll
+        for (int p = 0; p < PC; ++p)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) h[p][e] = h[p][e] + as_h2(res[p][e]);
+      }
+      const rsrc_t ry = make_rsrc(y + (size_t)m0 * N, bytes);
+#pragma unroll
+      for (int p = 0; p < PC; ++p)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) __builtin_amdgcn_raw_buffer_store_b32(as_u32(h[p][e]), ry, offset(p0 + p, e), 0, 0);
+      __builtin_amdgcn_sched_barrier(0);
+    });
+    return;
+  }
+#pragma unroll
+  for (int p = 0; p < PG; ++p)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const int m = m0 + row_in_tile(p, e);
+      if (m >= M) continue;
+#pragma unroll
+      for (int j = 0; j < TN; ++j)
+        if (n + j < N) store_out(ep, y, m, n + j, N, fin[p][j][e]);
+    }
+}
+
+namespace {
+
+template <int BITS, int TM, int TN, int CW, int G, int PROD, int KA, int KM, int NM, bool TILED, bool KSPLIT>
+bool launch_stream(const Problem& p, int ksplit, void* workspace) {
+  using C = StreamShape<BITS, TM, TN, CW, G, PROD, KA, KM, NM>;
+  const int tiles_m = (int)((p.m + C::kBM - 1) / C::kBM), tiles_n = (int)((p.n + C::kBN - 1) / C::kBN);
+  static std::atomic<bool> lds_ok[kMaxDevices];
+  const auto kernel = wq_gemm_stream_kernel<BITS, TM, TN, CW, G, PROD, KA, KM, NM, TILED, KSPLIT>;
+  if (!ensure_dynamic_lds((const void*)kernel, C::kLds, lds_ok)) return false;
+  int group_log2 = 0;
+  while ((1 << group_log2) < p.group) ++group_log2;
+  unsigned int* const counters = static_cast<unsigned int*>(workspace);
+  float* const partials = reinterpret_cast<float*>(static_cast<char*>(workspace) + kSplitCounterBytes);
+  hipLaunchKernelGGL(kernel, dim3(tiles_m * tiles_n * ksplit), dim3(C::kThreads), C::kLds, p.stream, (const half_t*)p.x,
+                     (const uint32_t*)p.wq, (const half_t*)p.scales, (int)p.m, (int)p.n, (int)p.k,
+                     group_log2 | (p.zero_point << 8) | (p.activation == kActGated ? 1 << 16 : 0), tiles_m, tiles_n, ksplit,
+                     (half_t*)p.y, Epilogue{(const half_t*)p.bias, (const half_t*)p.residual, p.activation}, partials, counters);
+  return true;
+}
+
+template <int BITS, int TM, int TN, int CW, int G, int PROD, int KA, int KM, int NM>
+bool launch_stream_any(const Problem& p, int ksplit, void* ws) {
+  if (ksplit > 1)
+    return p.tiled ? launch_stream<BITS, TM, TN, CW, G, PROD, KA, KM, NM, true, true>(p, ksplit, ws)
+                   : launch_stream<BITS, TM, TN, CW, G, PROD, KA, KM, NM, false, true>(p, ksplit, ws);
+  return p.tiled ? launch_stream<BITS, TM, TN, CW, G, PROD, KA, KM, NM, true, false>(p, 1, nullptr)
+                 : launch_stream<BITS, TM, TN, CW, G, PROD, KA, KM, NM, false, false>(p, 1, nullptr);
+}
+
+}  // namespace
+
+bool launch_gemm_stream(const Problem& p, int variant, int ksplit, void* workspace) {
+  if (!gemm_stream_applicable(p)) return false;
+#define WQ_STREAM(V, ...) \
+  case V: return p.bits == 4 ? launch_stream_any<4, __VA_ARGS__>(p, ksplit, workspace)
+#define WQ_STREAM8(...) launch_stream_any<8, __VA_ARGS__>(p, ksplit, workspace)
+  switch (variant) {
+    WQ_STREAM(kStream128x256, 4, 2, 4, 1, 4, 64, 256, 2) : WQ_STREAM8(4, 2, 4, 1, 4, 64, 128, 3);
+    WQ_STREAM(kStream128x128, 4, 2, 2, 2, 4, 64, 256, 2) : WQ_STREAM8(4, 2, 2, 2, 4, 64, 128, 3);
+    WQ_STREAM(kStream256x256, 8, 2, 4, 1, 0, 64, 128, 3) : WQ_STREAM8(8, 2, 4, 1, 0, 32, 128, 2);
+    WQ_STREAM(kStream64x128, 2, 2, 2, 4, 4, 128, 256, 3) : WQ_STREAM8(2, 2, 2, 4, 4, 128, 256, 2);
+    WQ_STREAM(kStream64x64, 2, 1, 2, 4, 4, 128, 256, 3) : WQ_STREAM8(2, 1, 2, 4, 4, 128, 256, 3);
+    default: return false;
+  }
+#undef WQ_STREAM
+#undef WQ_STREAM8
+}
+
+bool gemm_stream_applicable(const Problem& p) {
+  // groups of at least 32 (a lane's k of a stage share a scale); output rows of a tile within a 32-bit buffer
+  return p.group >= 32 && p.n <= (4 << 20);
+}
+
+namespace {
+
+// What a launch takes, in us: start + rounds of tiles * (tile start and end + K * (its loop alone on the chip + what a
+// full chip adds)), and with the K range split the exchange.  Fitted to 1,600 timings (both bit widths, M 20 - 512,
+// N 1024 - 22016, K 4096 - 13824, weights from memory, data random; 4 - 8 % rms); choosing by it costs 0.7 % against always
+// taking the fastest.
+struct StreamCost {
+  int variant, bm, bn;
+  float start, tile, loop, loaded, split, window, spread;
+};
+constexpr StreamCost kStreamCost4[] = {
+    {kStream128x256, 128, 256, 3.46f, 0.80f, 2.256f, 1.250f, 0.f, 0.f, 0.f},
+    {kStream128x128, 128, 128, 1.05f, 6.52f, 1.108f, 0.515f, 3.60f, 1.16f, 0.f},
+    {kStream256x256, 256, 256, 0.00f, 0.00f, 5.102f, 1.669f, 0.f, 0.f, 0.f},
+    {kStream64x128, 64, 128, 1.76f, 5.02f, 0.783f, 0.304f, 2.12f, 0.77f, 0.f},
+    {kStream64x64, 64, 64, 1.83f, 3.37f, 0.492f, 0.203f, 1.53f, 0.49f, 0.f},
+};
+constexpr StreamCost kStreamCost8[] = {
+    {kStream128x256, 128, 256, 0.00f, 0.00f, 3.595f, 0.949f, 0.f, 0.f, 0.f},
+    {kStream128x128, 128, 128, 0.09f, 5.01f, 1.416f, 0.603f, 4.62f, 1.03f, 0.f},
+    {kStream256x256, 256, 256, 0.00f, 0.00f, 3.810f, 4.601f, 0.f, 0.f, 0.f},
+    {kStream64x128, 64, 128, 2.18f, 2.61f, 1.280f, 0.343f, 2.86f, 0.64f, 0.95f},
+    {kStream64x64, 64, 64, 2.63f, 1.01f, 0.630f, 0.248f, 2.38f, 0.43f, 0.28f},
+};
+
+// The register-activation kernel in the same terms (M 20 - 128; 11 % rms): K * (rows + what columns beyond 4096 add).
+float skinny_cost(const Problem& p) {
+  if (p.m > kSkinnyMaxM) return 1e30f;
+  const int64_t slices = p.m > 64 ? (p.m + 63) / 64 : 1, blocks = ((p.m + 15) / 16 + slices - 1) / slices;
+  const float wide = std::max(1.0f, (float)(p.n * slices) / 4096.0f), macro = (float)p.k / 256.0f, rb = (float)blocks;
+  if (p.bits == 4) return 2.19f + macro * (0.041f + 0.127f * rb + (wide - 1.0f) * (0.153f + 0.031f * rb)) + 0.671f * wide;
+  return 1.59f + macro * (0.148f + 0.112f * rb + (wide - 1.0f) * 0.294f) + 0.835f * wide;
+}
+
+struct StreamPlan {
+  int variant = 0, split = 1;
+  float us = 1e30f;
+  int64_t bytes = 0;
+};
+
+StreamPlan plan_stream(const Problem& p, int64_t workspace_bytes) {
+  StreamPlan best;
+  const int64_t cu = cu_count(), macros = (p.k + 255) / 256;
+  for (const StreamCost& c : p.bits == 4 ? kStreamCost4 : kStreamCost8) {
+    const int64_t tiles = ((p.m + c.bm - 1) / c.bm) * ((p.n + c.bn - 1) / c.bn);
+    for (int64_t s = 1; s <= 8; ++s) {
+      // a window has at least two macro steps; windows that would be empty are dropped
+      const int64_t per = (macros + s - 1) / s;
+      const int64_t bytes = s > 1 ? kSplitCounterBytes + tiles * s * c.bm * c.bn * 4 : 0;
+      if (s > 1 && (c.split == 0.f || per < 2 || (s - 1) * per >= macros || tiles > kSplitMaxTiles || tiles * s > cu + cu / 8 || bytes > workspace_bytes)) continue;
+      const int64_t rounds = (tiles * s + cu - 1) / cu;
+      const float full = (float)(tiles * s) / (float)(rounds * cu);
+      float us = c.start + (float)rounds * (c.tile + (float)per * (c.loop + c.loaded * full));
+      if (s > 1) us += c.split + c.window * (float)s * full + c.spread * full;
+      if (us < best.us) best = StreamPlan{c.variant, (int)s, us, bytes};
+    }
+  }
+  return best;
+}
+
+// Workspaces of the library's own for calls that bring none (or one too small): a slot belongs to a stream -- whose
+// calls run one after the other -- and passes to another that asks for one when its owner has nothing left to do.
+// Without a free slot a call runs unsplit, as do calls under capture (a graph may be replayed beside anything) and calls
+// of more than 256 rows, which fill the chip without a split.  The memory is part of the code object (zero at load, as
+// the counters have to be): no call allocates.
+constexpr int kSlots = 8;
+constexpr int64_t kSlotBytes = kSplitCounterBytes + (20ll << 20);  // (the largest plan: 288 windows of 128 x 128 float32)
+__device__ unsigned char stream_slots[kSlots][kSlotBytes];
+
+void* library_slot(const Problem& p) {
+  if (p.m > 256 || p.stream == hipStreamPerThread) return nullptr;
+  struct Owners {
+    std::mutex mutex;
+    int used = 0;
+    hipStream_t stream[kSlots];
+    char* base = nullptr;
+  };
+  static Owners owners[kMaxDevices];
+  hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(p.stream, &status) != hipSuccess) {
+    (void)hipGetLastError();
+    return nullptr;
+  }
+  if (status != hipStreamCaptureStatusNone) return nullptr;
+  Owners& o = owners[current_device_slot()];
+  std::lock_guard<std::mutex> lock(o.mutex);
+  for (int i = 0; i < o.used; ++i)
+    if (o.stream[i] == p.stream) return o.base + i * kSlotBytes;
+  if (o.used == kSlots) {
+    for (int i = 0; i < kSlots; ++i) {  // (an owner that is being captured, was destroyed or is busy keeps its slot)
+      if (hipStreamIsCapturing(o.stream[i], &status) == hipSuccess && status == hipStreamCaptureStatusNone && hipStreamQuery(o.stream[i]) == hipSuccess) {
+        o.stream[i] = p.stream;
+        return o.base + i * kSlotBytes;
+      }
+      (void)hipGetLastError();
+    }
+    return nullptr;
+  }
+  if (o.base == nullptr) {
+    void* base = nullptr;
+    if (hipGetSymbolAddress(&base, HIP_SYMBOL(stream_slots)) != hipSuccess) {
+      (void)hipGetLastError();
+      return nullptr;
+    }
+    o.base = static_cast<char*>(base);
+  }
+  o.stream[o.used] = p.stream;
+  return o.base + o.used++ * kSlotBytes;
+}
+
+}  // namespace
+
+int64_t gemm_stream_workspace_bytes(const Problem& p) {
+  if (p.m <= 16 || !gemm_stream_applicable(p)) return 0;
+  return plan_stream(p, INT64_MAX).bytes;
+}
+
+int launch_gemm_stream_planned(const Problem& p, void* workspace, int64_t workspace_bytes, bool against_skinny) {
+  // (Up to 16 rows the decode kernel and the register-activation kernel read the weights faster.  With K below 1024 a launch
+  // is mostly start-up and the kernels are level -- 600 x 15323 x 512: 38.2 us there, 36.3 - 40.9 here -- so those stay.)
+  if (p.m <= 16 || p.k < 1024 || !gemm_stream_applicable(p)) return 0;
+  StreamPlan plan = plan_stream(p, p.m <= 256 ? std::max(workspace_bytes, kSlotBytes) : workspace_bytes);
+  if (plan.split > 1 && plan.bytes > workspace_bytes) {
+    workspace = library_slot(p);
+    if (workspace == nullptr) plan = plan_stream(p, 0);
+  }
+  if (plan.variant == 0 || (against_skinny && p.activation != kActGated && skinny_cost(p) < plan.us)) return 0;
+  if (!launch_gemm_stream(p, plan.variant, plan.split, workspace)) return -1;
+  const hipError_t e = hipGetLastError();
+  if (e != hipSuccess) {
+    set_error("gemm kernel (streamed operands) launch failed: %s", hipGetErrorString(e));
+    return -1;
+  }
+  return 1;
+}
+
+}  // namespace wq

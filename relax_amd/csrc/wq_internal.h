@@ -42,8 +42,17 @@ int64_t gemm_split_workspace_bytes(const Problem& p);
 int launch_gemm_split(const Problem& p, void* workspace, int64_t workspace_bytes);
 int launch_skinny(const Problem& p, int variant);
 int launch_gemm(const Problem& p, int variant);
+bool launch_gemm_streams(const Problem& p);  // whether the GEMM family's default may be the streamed kernel for `p`
 bool gemm_pipe_applicable(const Problem& p);  // K % 64 == 0, operands below 1 GiB
 bool launch_gemm_pipe(const Problem& p, int group_shift, int variant);
+// The streamed GEMM (wq_gemm_stream.hip): its tiles, an explicit launch, and the one its cost model picks -- the K range
+// split over workgroups where `workspace` has room for that and it pays.  `against_skinny`: not where the
+// register-activation kernel is the faster one.  1 launched, 0 not its problem, -1 failure.
+enum { kStream128x256 = 1, kStream128x128, kStream256x256, kStream64x128, kStream64x64 };
+bool gemm_stream_applicable(const Problem& p);
+bool launch_gemm_stream(const Problem& p, int variant, int ksplit, void* workspace);
+int launch_gemm_stream_planned(const Problem& p, void* workspace, int64_t workspace_bytes, bool against_skinny);
+int64_t gemm_stream_workspace_bytes(const Problem& p);  // what the plan would use, given any workspace
 bool launch_gemm_direct(const Problem& p, int group_shift, int variant);
 int launch_dequant(const Problem& p, void* wd);
 // canonical -> tile-major (forward) or back; p.wq / p.scales are the source, p.y is unused

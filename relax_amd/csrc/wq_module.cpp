@@ -420,6 +420,9 @@ bool bind_constants(mi355x_wq_module* m, const mi355x_dl_tensor* const* consts, 
       const int64_t b = mi355x_wq_workspace_bytes(&d, rows, tiled);
       if (b < 0) return false;
       if (b > need) need = b;
+      wq::Problem p{nullptr, nullptr, nullptr, nullptr, rows, d.n, d.k, d.bits, d.group, d.zero_point, nullptr};
+      p.activation = m->spec.activation;
+      if (wq::gemm_stream_workspace_bytes(p) > need) need = wq::gemm_stream_workspace_bytes(p);
     }
     if (need > 0) {
       if (!hip_ok(hipMalloc(&m->workspace, need), "hipMalloc")) return false;

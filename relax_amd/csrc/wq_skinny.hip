@@ -424,6 +424,10 @@ int launch_skinny(const Problem& p, int variant) {
     set_error("skinny kernel: M = %lld exceeds %lld", (long long)p.m, (long long)kSkinnyMaxM);
     return -1;
   }
+  if (variant == 0) {  // from 17 rows on the streamed GEMM where it is the faster one
+    const int rc = launch_gemm_stream_planned(p, nullptr, 0, true);
+    if (rc != 0) return rc < 0 ? -1 : 0;
+  }
   const int mt = (int)((std::min<int64_t>(p.m, skinny_slice_rows(p.m)) + 15) / 16);
   if (variant == 0) {
     // Measured on MI355X (q4f16, Llama-2-7B shapes, M = 4 .. 64): the number of workgroups is what
