@@ -8,6 +8,8 @@
 // exact tensors of the expected types, shapes and devices.  Anything else returns None without a side effect,
 // and the caller runs its Python path, which reports the error (or serves a case not covered here).
 // A return value of False is a call that the C ABI refused: its message is in mi355x_wq_last_error.
+// Tensor accessors throw for tensors without plain storage (sparse, nested, batched by a transform): no exception
+// leaves an entry, such a call is one not taken here.
 //
 // The C ABI is reached through addresses the Python side passes to bind() -- those of the library it has loaded --, so
 // this file links against nothing of the library.
@@ -230,11 +232,26 @@ PyObject* packed_call(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
   Py_RETURN_TRUE;
 }
 
+template <PyObject* (*F)(PyObject*, PyObject* const*, Py_ssize_t)>
+PyObject* guarded(PyObject* self, PyObject* const* a, Py_ssize_t nargs) {
+  try {
+    return F(self, a, nargs);
+  } catch (...) {
+    PyErr_Clear();
+    return none();
+  }
+}
+
+template <PyObject* (*F)(PyObject*, PyObject* const*, Py_ssize_t)>
+PyCFunction entry() {
+  return reinterpret_cast<PyCFunction>(reinterpret_cast<void*>(&guarded<F>));
+}
+
 PyMethodDef methods[] = {
     {"bind", bind, METH_VARARGS, nullptr},
-    {"matmul", reinterpret_cast<PyCFunction>(reinterpret_cast<void*>(matmul)), METH_FASTCALL, nullptr},
-    {"dequantize", reinterpret_cast<PyCFunction>(reinterpret_cast<void*>(dequantize)), METH_FASTCALL, nullptr},
-    {"packed_call", reinterpret_cast<PyCFunction>(reinterpret_cast<void*>(packed_call)), METH_FASTCALL, nullptr},
+    {"matmul", entry<matmul>(), METH_FASTCALL, nullptr},
+    {"dequantize", entry<dequantize>(), METH_FASTCALL, nullptr},
+    {"packed_call", entry<packed_call>(), METH_FASTCALL, nullptr},
     {nullptr, nullptr, 0, nullptr}};
 
 PyModuleDef module_def = {PyModuleDef_HEAD_INIT, "_wq_torch", "native host path of relax_amd", -1, methods, nullptr, nullptr, nullptr, nullptr};

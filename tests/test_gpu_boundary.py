@@ -333,3 +333,21 @@ def test_concurrent_callers_on_their_own_streams():
     assert not any(t.is_alive() for t in threads), "a caller thread did not finish"
     assert not errors, errors[:3]
     vm_harness.set_stream()
+
+
+@pytest.mark.parametrize("place", ["x", "wq", "scales", "bias", "residual", "workspace"])
+def test_sparse_tensors_are_refused_with_an_exception(place):
+    """The accessors that the native front end calls throw for these: a Python exception, never the process's end."""
+    import relax_amd
+
+    x, wq, s, g = O.make_case(1, 4, 64, 256, 4)
+    t = dict(x=_dev(x), wq=_dev(wq), scales=_dev(s), bias=torch.zeros(64, dtype=torch.float16, device="cuda"),
+             residual=torch.zeros((4, 64), dtype=torch.float16, device="cuda"),
+             workspace=torch.zeros((4, 4096), dtype=torch.uint8, device="cuda"))
+    t[place] = torch.sparse_coo_tensor(size=t[place].shape, dtype=t[place].dtype, device="cuda")
+    with pytest.raises(Exception):
+        relax_amd.wq_matmul(t["x"], t["wq"], t["scales"], 4, g, bias=t["bias"], residual=t["residual"], workspace=t["workspace"])
+    if place in ("wq", "scales"):
+        with pytest.raises(Exception):
+            relax_amd.wq_dequantize(t["wq"], t["scales"], 4, g)
+    torch.cuda.synchronize()
