@@ -174,10 +174,11 @@ struct StreamRequests {
     }
   }
 
-  // request P of the activations from k0 on, into the stage at LDS offset `buf`; lanes past k_end read zeros
+  // request P of the activations from k0 on, into the stage at LDS offset `buf`; lanes past k_end read zeros (a stage that is
+  // all past k_end without a scalar offset: the hardware compares the lane's offset with the buffer's size less that one)
   template <int P>
   __device__ __forceinline__ void issue_a(int k0, uint32_t buf) const {
-    dma_b128(lds0 + buf + (uint32_t)(me + P * R) * 1024u, k0 + a_k < k_end ? av[P] : kStreamOob, rx, (uint32_t)k0 * 2u);
+    dma_b128(lds0 + buf + (uint32_t)(me + P * R) * 1024u, k0 + a_k < k_end ? av[P] : kStreamOob, rx, k0 < k_end ? (uint32_t)k0 * 2u : 0u);
   }
   // request P of the weights and scales of the macro step from k0 on, into place `ring` of their rings
   template <int P>
@@ -185,14 +186,14 @@ struct StreamRequests {
     if constexpr (P < C::kNW) {
       const int q = me + P * R;
       const bool mine = C::kQW % R == 0 || q < C::kQW;
-      const uint32_t byte = (uint32_t)k0 * BITS / 8u, off = TILED ? (byte >> 7) * 2048u + ((byte >> 5) & 3u) * 256u : byte;
+      const uint32_t byte = k0 < k_end ? (uint32_t)k0 * BITS / 8u : 0u, off = TILED ? (byte >> 7) * 2048u + ((byte >> 5) & 3u) * 256u : byte;
       dma_b128(lds0 + (mine ? C::kWBase + ring * C::kWBytes + (uint32_t)q * 1024u : (uint32_t)C::kDummyBase), k0 + w_k < k_end ? wv[P] : kStreamOob, rw, off);
     } else {
       constexpr int i = P - C::kNW;
       const int q = me + i * R;
       const bool mine = C::kQS % R == 0 || q < C::kQS;
       uint32_t v = sv[i], off = 0;
-      if constexpr (TILED) off = BITS == 4 ? (uint32_t)k0 : (uint32_t)k0 / 4u;  // (256 bytes per 256 k, 32 per 128 k)
+      if constexpr (TILED) off = k0 >= k_end ? 0u : BITS == 4 ? (uint32_t)k0 : (uint32_t)k0 / 4u;  // (256 bytes per 256 k, 32 per 128 k)
       else v += (uint32_t)((k0 + s_sub * 32) >> group_log2) * 2u;
       dma_u16(lds0 + (mine ? C::kSBase + ring * C::kSBytes + (uint32_t)q * 256u : (uint32_t)C::kDummyBase), k0 + s_sub * 32 < k_end ? v : kStreamOob, rs, off);
     }
@@ -738,7 +739,9 @@ constexpr int kSlots = 8;
 constexpr int64_t kSlotBytes = kSplitCounterBytes + (20ll << 20);  // (the largest plan: 288 windows of 128 x 128 float32)
 __device__ unsigned char stream_slots[kSlots][kSlotBytes];
 
-void* library_slot(const Problem& p) {
+// The caller passes `lock` in and keeps it until its launch is in the stream: between the two the stream may look idle, and
+// another thread would take the slot over.
+void* library_slot(const Problem& p, std::unique_lock<std::mutex>* lock) {
   if (p.m > 256 || p.stream == hipStreamPerThread) return nullptr;
   struct Owners {
     std::mutex mutex;
@@ -754,7 +757,7 @@ void* library_slot(const Problem& p) {
   }
   if (status != hipStreamCaptureStatusNone) return nullptr;
   Owners& o = owners[current_device_slot()];
-  std::lock_guard<std::mutex> lock(o.mutex);
+  *lock = std::unique_lock<std::mutex>(o.mutex);
   for (int i = 0; i < o.used; ++i)
     if (o.stream[i] == p.stream) return o.base + i * kSlotBytes;
   if (o.used == kSlots) {
@@ -791,8 +794,9 @@ int launch_gemm_stream_planned(const Problem& p, void* workspace, int64_t worksp
   // is mostly start-up and the kernels are level -- 600 x 15323 x 512: 38.2 us there, 36.3 - 40.9 here -- so those stay.)
   if (p.m <= 16 || p.k < 1024 || !gemm_stream_applicable(p)) return 0;
   StreamPlan plan = plan_stream(p, p.m <= 256 ? std::max(workspace_bytes, kSlotBytes) : workspace_bytes);
+  std::unique_lock<std::mutex> slot_lock;
   if (plan.split > 1 && plan.bytes > workspace_bytes) {
-    workspace = library_slot(p);
+    workspace = library_slot(p, &slot_lock);
     if (workspace == nullptr) plan = plan_stream(p, 0);
   }
   if (plan.variant == 0 || (against_skinny && p.activation != kActGated && skinny_cost(p) < plan.us)) return 0;

@@ -83,3 +83,36 @@ def test_k_split_on_the_librarys_slots_on_a_workspace_and_under_capture(bits, m,
         first = out.clone() if first is None else first
         assert torch.equal(out, first)
     assert_close(first.cpu().numpy()[rows], want, ("captured", bits, m, n, k), ulp_fraction=0.005)
+
+
+def test_more_threads_and_streams_than_slots():
+    """Twelve streams, a thread each, for eight slots that pass from idle streams to others: every result is the split call's
+    or, without a slot, the unsplit one's."""
+    import threading
+
+    import relax_amd
+
+    x, wq, s, g = O.make_case(3, 40, 1000, 11008, 4)
+    dx, dw, ds = _dev(x), _dev(wq), _dev(s)
+    split = relax_amd.wq_matmul(dx, dw, ds, 4, g)
+    graph, unsplit = torch.cuda.CUDAGraph(), torch.empty_like(split)
+    with torch.cuda.graph(graph):
+        relax_amd.wq_matmul(dx, dw, ds, 4, g, out=unsplit)
+    graph.replay()
+    torch.cuda.synchronize()
+    outs = [[] for _ in range(12)]
+
+    def worker(mine):
+        stream = torch.cuda.Stream()
+        for burst in range(10):
+            for _ in range(3):
+                mine.append(relax_amd.wq_matmul(dx, dw, ds, 4, g, stream=stream, out=torch.empty_like(split)))
+            stream.synchronize()
+
+    threads = [threading.Thread(target=worker, args=(o,)) for o in outs]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    torch.cuda.synchronize()
+    assert all(torch.equal(y, split) or torch.equal(y, unsplit) for mine in outs for y in mine)
