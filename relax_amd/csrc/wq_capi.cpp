@@ -125,6 +125,7 @@ bool check_ptr(const void* p, const char* name, size_t align) {
 
 int select_kernel(const mi355x_wq_desc* d, int64_t m, bool tiled = false) {
   Problem p{nullptr, nullptr, nullptr, nullptr, m, d->n, d->k, d->bits, d->group, d->zero_point, nullptr};
+  p.tiled = tiled;
   if (gemv_applicable(p)) {
     // The GEMV kernel stages the activations in LDS, in K phases when they do not fit in one piece.
     const int64_t tiles = (d->n + 15) / 16;

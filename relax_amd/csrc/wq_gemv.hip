@@ -97,7 +97,10 @@ struct GemvKernArgs {
   unsigned int* counters;
 };
 
-template <int BITS, int WAVES, int D, int SPL, bool TILED, int XS, bool KSPLIT, bool PHASES>
+// ROUNDS: a workgroup has more tiles than its LDS has slots for.  The tiles are walked in rounds of half the slots (an even
+// number, so that a round ends with a trip of the stream); after a round one barrier, and the round's tiles are summed
+// and stored from one half of the slots while the next round fills the other, its first item already in flight.
+template <int BITS, int WAVES, int D, int SPL, bool TILED, int XS, bool KSPLIT, bool PHASES, bool ROUNDS>
 // PHASES: the launch walks K in more than one phase (activations beyond the LDS).  The host knows; as a template
 // flag it keeps the second phase description out of the build that runs the common launches, whose first memory
 // requests otherwise wait behind that bookkeeping (and behind the late kernel arguments, which the compiler
@@ -119,6 +122,7 @@ __global__ __launch_bounds__(WAVES * 64) __attribute__((amdgpu_waves_per_eu(2, 8
     int shift_and_zero_, int max_tiles_, int phase_chunks_, int ksplit_, int grid_, half_t* y_late, const Epilogue ep_late,
     float* partials_late, unsigned int* counters_late) {
   static_assert(!KSPLIT || !PHASES, "the cross-workgroup K split walks one window of K");
+  static_assert(!ROUNDS || (!KSPLIT && !PHASES && XS == 0), "rounds of tiles: all of K in one phase");
   static_assert(XS == 0 || XS == 1 || XS == 2 || XS == 3 || XS == 4 || XS == 8 || XS == 16, "staging mode");
   constexpr bool ROWS = XS >= 4;
   constexpr bool XPRE = PHASES && (XS == 4 || XS == 8);  // (up to eight rows) a phase's activations are requested a phase ahead
@@ -147,9 +151,10 @@ __global__ __launch_bounds__(WAVES * 64) __attribute__((amdgpu_waves_per_eu(2, 8
   const int M = M_, N = N_, K = K_;
 
   extern __shared__ __attribute__((aligned(16))) unsigned char wq_gemv_smem[];
-  // [max_tiles][WAVES][4][64] float partial tiles, then [M][lds_stride] staged activations
+  // [slot_tiles][WAVES][4][64] float partial tiles, then [M][lds_stride] staged activations
+  const int slot_tiles = ROUNDS ? ksplit_ : max_tiles_;
   float* slots = reinterpret_cast<float*>(wq_gemv_smem);
-  half_t* xs = reinterpret_cast<half_t*>(wq_gemv_smem + (size_t)max_tiles_ * WAVES * 1024);
+  half_t* xs = reinterpret_cast<half_t*>(wq_gemv_smem + (size_t)slot_tiles * WAVES * 1024);
 
   const uint32_t row_bytes = (uint32_t)K * BITS / 8;
   const int nchunks = K / CH;
@@ -298,8 +303,10 @@ __global__ __launch_bounds__(WAVES * 64) __attribute__((amdgpu_waves_per_eu(2, 8
   };
 
   // adds the finished partial tile to this wavefront's private slot and clears it
+  int ring = 0;  // ROUNDS: slot of the tile being summed (tiles are flushed in order)
   auto flush_tile = [&](int i, bool first_phase) {
-    float* s = slots + ((size_t)(i * WAVES + wave) * 4) * 64 + lane;
+    float* s = slots + ((size_t)((ROUNDS ? ring : i) * WAVES + wave) * 4) * 64 + lane;
+    if constexpr (ROUNDS) ring = ring + 1 == slot_tiles ? 0 : ring + 1;
 #pragma unroll
     for (int r = 0; r < 4; ++r) s[r * 64] = first_phase ? acc[r] : s[r * 64] + acc[r];
     acc = float4_t{0.f, 0.f, 0.f, 0.f};
@@ -366,6 +373,37 @@ __global__ __launch_bounds__(WAVES * 64) __attribute__((amdgpu_waves_per_eu(2, 8
   auto pin_late_arguments = [&]() {
     asm volatile("" ::"s"(y_), "s"(ep_.bias), "s"(ep_.residual), "s"(ep_.activation));
     if constexpr (KSPLIT) asm volatile("" ::"s"(partials_), "s"(counters_));
+  };
+
+  // adds up and stores tiles first .. first + count - 1 of this workgroup from the slots slot0 on
+  auto store_tiles = [&](int first, int count, int slot0) __attribute__((always_inline)) {
+    // (the plain store first and on its own: the tails' code -- erf, exp -- is then a block the common launch never
+    // enters, instead of four stretches it jumps over on a cold instruction cache)
+    const bool plain = !gated && ep_.bias == nullptr && ep_.residual == nullptr && ep_.activation == 0;
+    for (int idx = tid; idx < count * 256; idx += NT) {
+      const int i = idx >> 8, r = (idx >> 6) & 3, l = idx & 63;
+      const int m = 4 * (l >> 4) + r;
+      const int n = (tile0 + (first + i) * tstride) * tile_rows + (l & 15);
+      if (m < M && n < N && (l & 15) < tile_rows) {
+        const float* const part = slots + ((size_t)((slot0 + i) * WAVES) * 4 + r) * 64 + l;
+        float sum = 0.f;
+#pragma unroll
+        for (int w = 0; w < WAVES; ++w) sum += part[w * 256];
+        if (plain) {
+          y_[(size_t)m * N + n] = (half_t)sum;
+        } else if (gated) {
+          // adjacent columns of the tile hold a gate / up pair: the even lane also sums its neighbour's
+          if ((l & 1) == 0 && n + 1 < N) {
+            float up = 0.f;
+#pragma unroll
+            for (int w = 0; w < WAVES; ++w) up += part[w * 256 + 1];
+            store_gated(y_, m, n >> 1, N >> 1, sum, up);
+          }
+        } else {
+          store_out(ep_, y_, m, n, N, sum);
+        }
+      }
+    }
   };
 
   // One K phase: stage its activations, stream every tile of the workgroup over it.  The first phase
@@ -523,6 +561,7 @@ __global__ __launch_bounds__(WAVES * 64) __attribute__((amdgpu_waves_per_eu(2, 8
     const int items = my_tiles * c.cnt;
     int ci = first_tile(c), cs = 0;  // tile / step of the item being consumed
     int pi = ci, ps = 0;             // ... of the item being prefetched
+    auto stream = [&](const int items) __attribute__((always_inline)) {
     for (int j = 0; j < items; j += 2) {
       advance(c, pi, ps);
       load_super(b1, c, pi, ps);
@@ -553,6 +592,22 @@ __global__ __launch_bounds__(WAVES * 64) __attribute__((amdgpu_waves_per_eu(2, 8
       advance(c, ci, cs);
       __builtin_amdgcn_sched_barrier(0);
     }
+    };
+    if constexpr (ROUNDS) {
+      const int half = slot_tiles / 2;
+      int slot0 = 0;
+      for (int t0 = 0; t0 < my_tiles; t0 += half) {
+        const int count = min(half, my_tiles - t0);
+        stream(count * c.cnt);
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+        store_tiles(t0, count, slot0);
+        slot0 = slot0 == 0 ? half : 0;
+      }
+    } else {
+      stream(items);
+    }
     WQ_STAMP(4);
     // a wavefront without work in the first phase still owns slots that the epilogue sums
     if (ph == 0 && c.cnt == 0)
@@ -576,32 +631,7 @@ __global__ __launch_bounds__(WAVES * 64) __attribute__((amdgpu_waves_per_eu(2, 8
   __syncthreads();
   WQ_STAMP(6);
   if constexpr (!KSPLIT) {
-    // (the plain store first and on its own: the tails' code -- erf, exp -- is then a block the common launch never
-    // enters, instead of four stretches it jumps over on a cold instruction cache)
-    const bool plain = !gated && ep_.bias == nullptr && ep_.residual == nullptr && ep_.activation == 0;
-    for (int idx = tid; idx < my_tiles * 256; idx += NT) {
-      const int i = idx >> 8, r = (idx >> 6) & 3, l = idx & 63;
-      const int m = 4 * (l >> 4) + r;
-      const int n = (tile0 + i * tstride) * tile_rows + (l & 15);
-      if (m < M && n < N && (l & 15) < tile_rows) {
-        float sum = 0.f;
-#pragma unroll
-        for (int w = 0; w < WAVES; ++w) sum += slots[((size_t)(i * WAVES + w) * 4 + r) * 64 + l];
-        if (plain) {
-          y_[(size_t)m * N + n] = (half_t)sum;
-        } else if (gated) {
-          // adjacent columns of the tile hold a gate / up pair: the even lane also sums its neighbour's
-          if ((l & 1) == 0 && n + 1 < N) {
-            float up = 0.f;
-#pragma unroll
-            for (int w = 0; w < WAVES; ++w) up += slots[((size_t)(i * WAVES + w) * 4 + r) * 64 + l + 1];
-            store_gated(y_, m, n >> 1, N >> 1, sum, up);
-          }
-        } else {
-          store_out(ep_, y_, m, n, N, sum);
-        }
-      }
-    }
+    if constexpr (!ROUNDS) store_tiles(0, my_tiles, 0);
   } else {
     // K split over R workgroups: every workgroup writes its float32 partial tile (1 KB) to the
     // workspace and counts itself in; the one that finds R - 1 others counted adds the R partials in
@@ -655,7 +685,7 @@ __global__ __launch_bounds__(WAVES * 64) __attribute__((amdgpu_waves_per_eu(2, 8
   // (the plain builds do not use ksplit_: the measurement build's launcher passes a launch counter there)
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   WQ_STAMP(7);
-  if (!KSPLIT && lane == 0 && (int)blockIdx.x * WAVES + wave < kStampWaves) {
+  if (!KSPLIT && !ROUNDS && lane == 0 && (int)blockIdx.x * WAVES + wave < kStampWaves) {
     unsigned long long* t =
         g_gemv_stamps + ((size_t)(ksplit_ & (kStampLaunches - 1)) * kStampWaves + (size_t)blockIdx.x * WAVES + wave) * kStampPoints;
     for (int q = 0; q < kStampPoints; ++q) t[q] = stamps_[q];
@@ -717,10 +747,12 @@ bool make_plan(const Problem& p, int wgs_per_cu, Plan* out, int tile_rows = 0) {
   const int unit = 4 * D * WAVES;
   const int64_t max_k = (int64_t)(x_budget / (2 * (size_t)p.m)) - 8;
   int phase_chunks = (int)(max_k / ch) / unit * unit;
-  if (phase_chunks <= 0) return false;
   const int whole = (nchunks + 4 * D - 1) / (4 * D) * (4 * D);  // K as one phase, padded to a super step
-  if (phase_chunks >= whole) {
+  // (43008 x 6144 at 8 rows, whose 192 chunks fit but are no multiple of the unit: 33.5 us in phases, 30.3 in one)
+  if (max_k / ch >= whole) {
     phase_chunks = whole;
+  } else if (phase_chunks <= 0) {
+    return false;
   } else if (p.m > 2) {
     // K is walked in phases anyway: phases of equal length, and of at most one 16-byte vector per
     // thread and row where that costs at most one phase more, so that the staging takes the
@@ -740,6 +772,31 @@ bool make_plan(const Problem& p, int wgs_per_cu, Plan* out, int tile_rows = 0) {
   return out->lds_bytes <= budget;
 }
 
+// The plan of a ROUNDS launch: eight wavefronts, two-chunk super steps, 16-row tiles, all of K in one phase with at least one
+// super step per wavefront; `slots` = slots of both halves, as many as fit and at most 16.  (A round's items have to
+// be even in number for every wavefront: an even number of tiles, or an even number of super steps.)
+template <int BITS>
+bool make_rounds_plan(const Problem& p, int wgs_per_cu, Plan* out, int* slots) {
+  constexpr int ch = 128 / BITS, kUnit = 8;  // chunks per super step
+  const int64_t nsuper = p.k / (kUnit * ch);
+  if (p.k % (kUnit * ch) != 0 || nsuper < 8) return false;
+  const int tiles = (int)((p.n + 15) / 16);
+  const int64_t budget = (int64_t)std::min(kLdsPerWgMax, kLdsPerCu / (size_t)wgs_per_cu - 1024);
+  const int64_t x_bytes = p.m * (p.k + 8) * 2;
+  if (x_bytes > budget) return false;
+  int half = (int)std::min<int64_t>((budget - x_bytes) / (8 * 1024 * 2), 8);
+  if (nsuper % 16 != 0) half = half / 2 * 2;
+  if (half < 1) return false;
+  out->grid = std::min(tiles, cu_count() * wgs_per_cu);
+  out->max_tiles = (tiles + out->grid - 1) / out->grid;
+  out->tile_rows = 16;
+  out->phase_chunks = (int)(p.k / ch);
+  out->lds_stride = (int)p.k + 8;
+  out->lds_bytes = (size_t)(half * 2 * 8192 + x_bytes);
+  *slots = half * 2;
+  return true;
+}
+
 // Launch results of the helpers below: the variant does not fit the problem (try another),
 // the kernel was launched, or a runtime call failed (error already set).
 enum { kNotApplicable = 0, kLaunched = 1, kFailed = -1 };
@@ -757,7 +814,7 @@ inline int stamp_slot_or(int ksplit, bool split_build) {
   return ksplit;
 }
 
-template <int BITS, int WAVES, int D, int SPL, bool TILED = false, bool KSPLIT = false>
+template <int BITS, int WAVES, int D, int SPL, bool TILED = false, bool KSPLIT = false, bool ROUNDS = false>
 int launch_one(const Problem& p, int group_shift, const Plan& plan, int ksplit = 1, void* workspace = nullptr) {
   const Epilogue ep{(const half_t*)p.bias, (const half_t*)p.residual, p.activation};
   // workspace of the K split: kSplitMaxTiles arrival counters at a fixed place -- a workspace shared by
@@ -771,40 +828,44 @@ int launch_one(const Problem& p, int group_shift, const Plan& plan, int ksplit =
     constexpr int XS = decltype(xs)::value;
     constexpr bool PHASES = decltype(phases)::value;
     static std::atomic<bool> lds_ok[kMaxDevices];
-    if (!ensure_dynamic_lds((const void*)wq_gemv_kernel<BITS, WAVES, D, SPL, TILED, XS, KSPLIT, PHASES>, (int)kLdsPerWgMax,
+    if (!ensure_dynamic_lds((const void*)wq_gemv_kernel<BITS, WAVES, D, SPL, TILED, XS, KSPLIT, PHASES, ROUNDS>, (int)kLdsPerWgMax,
                             lds_ok))
       return kFailed;
-    hipLaunchKernelGGL((wq_gemv_kernel<BITS, WAVES, D, SPL, TILED, XS, KSPLIT, PHASES>), dim3(plan.grid), dim3(WAVES * 64),
+    hipLaunchKernelGGL((wq_gemv_kernel<BITS, WAVES, D, SPL, TILED, XS, KSPLIT, PHASES, ROUNDS>), dim3(plan.grid), dim3(WAVES * 64),
                        plan.lds_bytes, p.stream, (const half_t*)p.x, (const uint32_t*)p.wq, (const half_t*)p.scales,
                        (int)p.m, (int)p.n, (int)p.k,
                        group_shift | (p.zero_point << 8) | (p.activation == kActGated ? 1 << 16 : 0) | (plan.tile_rows << 20),
-                       plan.max_tiles, plan.phase_chunks, stamp_slot_or(ksplit, KSPLIT), plan.grid, (half_t*)p.y, ep,
+                       plan.max_tiles, plan.phase_chunks, stamp_slot_or(ksplit, KSPLIT || ROUNDS), plan.grid, (half_t*)p.y, ep,
                        partials, counters);
     return kLaunched;
   };
   using std::integral_constant;
-  constexpr int ch = 128 / BITS, NT = WAVES * 64;
-  const int phase_vectors = (plan.phase_chunks + 3) / 4 * 4 * ch / 8;  // 16-byte vectors per staged row
-  const bool flat = p.m <= 2 || phase_vectors > NT;
-  const bool phases = !KSPLIT && (int64_t)plan.phase_chunks * ch < p.k;
-  auto with_phases = [&](auto xs) -> int {
-    if constexpr (KSPLIT) return go(xs, std::false_type{});
-    else return phases ? go(xs, std::true_type{}) : go(xs, std::false_type{});
-  };
-  if (!flat) {
-    if (p.m <= 4) return with_phases(integral_constant<int, 4>{});
-    return p.m <= 8 ? with_phases(integral_constant<int, 8>{}) : with_phases(integral_constant<int, 16>{});
-  }
-  if constexpr (!KSPLIT && WAVES == 8) {
-    // (the default shapes only: every exact build is a kernel more)
-    const int64_t total = p.m * (int64_t)phase_vectors;
-    if (!phases && phase_vectors >= NT && total <= 3 * NT) {
-      if (total <= NT) return go(integral_constant<int, 1>{}, std::false_type{});
-      if (total <= 2 * NT) return go(integral_constant<int, 2>{}, std::false_type{});
-      return go(integral_constant<int, 3>{}, std::false_type{});
+  if constexpr (ROUNDS) {
+    return go(integral_constant<int, 0>{}, std::false_type{});
+  } else {
+    constexpr int ch = 128 / BITS, NT = WAVES * 64;
+    const int phase_vectors = (plan.phase_chunks + 3) / 4 * 4 * ch / 8;  // 16-byte vectors per staged row
+    const bool flat = p.m <= 2 || phase_vectors > NT;
+    const bool phases = !KSPLIT && (int64_t)plan.phase_chunks * ch < p.k;
+    auto with_phases = [&](auto xs) -> int {
+      if constexpr (KSPLIT) return go(xs, std::false_type{});
+      else return phases ? go(xs, std::true_type{}) : go(xs, std::false_type{});
+    };
+    if (!flat) {
+      if (p.m <= 4) return with_phases(integral_constant<int, 4>{});
+      return p.m <= 8 ? with_phases(integral_constant<int, 8>{}) : with_phases(integral_constant<int, 16>{});
     }
+    if constexpr (!KSPLIT && WAVES == 8) {
+      // (the default shapes only: every exact build is a kernel more)
+      const int64_t total = p.m * (int64_t)phase_vectors;
+      if (!phases && phase_vectors >= NT && total <= 3 * NT) {
+        if (total <= NT) return go(integral_constant<int, 1>{}, std::false_type{});
+        if (total <= 2 * NT) return go(integral_constant<int, 2>{}, std::false_type{});
+        return go(integral_constant<int, 3>{}, std::false_type{});
+      }
+    }
+    return with_phases(integral_constant<int, 0>{});
   }
-  return with_phases(integral_constant<int, 0>{});
 }
 
 // D chunks per lane need K to be a multiple of 4*D chunks, and the lane's D
@@ -829,7 +890,24 @@ int try_launch(const Problem& p, int group_shift, int wgs_per_cu, int tile_rows)
   return kNotApplicable;
 }
 
-// variant = 100 * rows-per-tile (0: the rule's choice, else 8 .. 16) + 10 * workgroups-per-CU + shape index
+template <int BITS>
+int try_rounds(const Problem& p, int gs, int wgs_per_cu) {
+  Plan plan;
+  int slots;
+  if (!make_rounds_plan<BITS>(p, wgs_per_cu, &plan, &slots)) return kNotApplicable;
+  if (p.tiled) {
+    if constexpr (BITS == 4) {
+      if (gs == 0) return launch_one<BITS, 8, 2, 2, true, false, true>(p, gs, plan, slots);
+    } else {
+      if (gs == 3) return launch_one<BITS, 8, 2, 1, true, false, true>(p, gs, plan, slots);
+    }
+    return kNotApplicable;
+  }
+  if (gs == 0) return launch_one<BITS, 8, 2, 2, false, false, true>(p, gs, plan, slots);
+  return launch_one<BITS, 8, 2, 1, false, false, true>(p, gs, plan, slots);
+}
+
+// variant = 100 * rows-per-tile (0: the rule's choice, else 8 .. 16) + 10 * workgroups-per-CU + shape index (9: rounds)
 template <int BITS>
 int dispatch(const Problem& p, int gs, int variant) {
   const int tr = variant / 100, wpc = variant % 100 / 10, shape = variant % 10;
@@ -844,6 +922,7 @@ int dispatch(const Problem& p, int gs, int variant) {
     case 6: return try_launch<BITS, 8, 4>(p, gs, wpc, tr);
     case 7: return try_launch<BITS, 16, 1>(p, gs, wpc, tr);
     case 8: return try_launch<BITS, 16, 2>(p, gs, wpc, tr);
+    case 9: return tr == 0 || tr == 16 ? try_rounds<BITS>(p, gs, wpc) : kNotApplicable;
     default: return kNotApplicable;
   }
 }
@@ -893,15 +972,37 @@ bool variant_has_plan(const Problem& p, int gs, int variant) {
 
 }  // namespace
 
-// M <= 16 and one of the default variants fits: with very many row tiles per workgroup (N in the
-// hundreds of thousands) the per-tile partial-sum slots outgrow LDS and the caller falls back to
-// the register-activation kernel.
+namespace {
+
+// Whether the default launch walks its tiles in rounds (one workgroup per CU; two are level or behind: 152064 x 4096 int4 at 3
+// rows 69.5 us against 65.2).  Canonical weights: where a slot for every tile does not fit -- the register-activation
+// kernel ran those (152064 x 4096 int4 at 1 / 3 / 8 / 16 rows 92 / 91 / 94 / 101 -> 70 / 65 / 72 / 83 us, 5.4 TB/s at 3 rows;
+// 152064 x 5120 int8 at 1 / 12 rows 182 / 197 -> 133 / 156) -- or would leave so little that K is walked in phases, from
+// 12 tiles per workgroup on (65536 x 4096 at 8 rows: int4 41.5 -> 32.9 us, int8 60.6 -> 51.5; with 7 - 11 tiles the
+// phases are level or ahead, 43008 x 6144 at 10 rows 33.9 against 34.6).  Tile-major weights: without a slot per tile up to
+// 12 rows (152064 x 4096 at 3 rows 66.9 -> 62.8 us; at 16 the register-activation kernel stays ahead, 72.5 against 75.0).
+template <int BITS>
+bool use_rounds(const Problem& p) {
+  Plan rounds, whole;
+  int slots;
+  if ((p.tiled && p.m > 12) || !make_rounds_plan<BITS>(p, 1, &rounds, &slots)) return false;
+  if (!make_plan<BITS, 8, 2>(p, 1, &whole)) return true;
+  return !p.tiled && (int64_t)whole.phase_chunks * (128 / BITS) < p.k && whole.max_tiles >= 12;
+}
+
+bool use_rounds_any(const Problem& p) { return p.bits == 4 ? use_rounds<4>(p) : use_rounds<8>(p); }
+
+}  // namespace
+
+// M <= 16 and one of the default variants fits.  (With very many row tiles per workgroup and K too short or too long
+// for rounds, the per-tile partial-sum slots outgrow LDS and the caller falls back to the register-activation kernel.)
 bool gemv_applicable(const Problem& p) {
   if (p.m < 1 || p.m > 16) return false;
   const int ch = 128 / p.bits;
   int ratio = p.group / ch, gs = 0;
   while ((1 << gs) < ratio) ++gs;
   if (ratio < 1 || (1 << gs) != ratio) return false;
+  if (use_rounds_any(p)) return true;
   const int* order = default_order(p);
   for (int q = 0; q < 4; ++q) {
     const int shape = order[q] % 10;
@@ -924,7 +1025,9 @@ int launch_gemv(const Problem& p, int variant) {
     return -1;
   }
   int ok = kNotApplicable;
-  if (variant == 0) {
+  if (variant == 0 && use_rounds_any(p)) {
+    ok = p.bits == 4 ? try_rounds<4>(p, gs, 1) : try_rounds<8>(p, gs, 1);
+  } else if (variant == 0) {
     const int* order = default_order(p);
     for (int q = 0; q < 4; ++q) {
       const int v = order[q];

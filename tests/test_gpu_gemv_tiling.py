@@ -129,3 +129,52 @@ def test_activation_staging_builds(bits, group, k, rows):
         torch.cuda.synchronize()
         want_f = ((y0.cpu().numpy() + bias.cpu().numpy()[None, :]).astype(np.float16) + np.float16(0.5)).astype(np.float16)
         assert np.array_equal(yf.cpu().numpy().view(np.int16), want_f.view(np.int16)), ("fused", bits, group, k, m)
+
+
+# More tiles than slots: rounds of one tile (16 rows of 4096), of two (12 of 5120) and of up to eight, with an even and an odd
+# number of super steps per wavefront (K = 4096 and 2048), super steps that do not divide evenly (1152 = 9 of 128) and a rest
+# of tiles in the last round; groups of several super steps' worth of chunks; the tails.
+@pytest.mark.parametrize("bits,m,n,k,group", [(4, 16, 5000, 4096, 32), (4, 12, 13001, 5120, 32), (4, 1, 37001, 2048, 32), (4, 3, 70002, 2048, 128),
+                                              (8, 5, 40000, 1152, 128), (8, 2, 33333, 1024, 64), (8, 8, 36900, 2048, 16), (4, 15, 4090, 4096, 32)])
+def test_more_tiles_than_slots(bits, m, n, k, group):
+    import relax_amd
+    from relax_amd import lib
+
+    x, wq, s, g = O.make_case(n + m, m, n, k, bits, group)
+    dx, dw, ds = _dev(x), _dev(wq), _dev(s)
+    want = c_oracle.wq_matmul(x, wq, s, bits, g, nthreads=16)
+    rng = np.random.default_rng(m)
+    bias, res = rng.standard_normal(n).astype(np.float16), rng.standard_normal((m, n)).astype(np.float16)
+    ran = 0
+    for variant in (19, 29):
+        kw = dict(kernel=lib.KERNEL_GEMV, variant=variant)
+        try:
+            y = relax_amd.wq_matmul(dx, dw, ds, bits, g, **kw)
+        except lib.WqError:
+            continue  # (two workgroups' activations and slots do not fit a CU)
+        torch.cuda.synchronize()
+        ran += 1
+        plain = y.cpu().numpy()
+        _close(plain, want, (variant, bits, m, n, k))
+        fused = relax_amd.wq_matmul(dx, dw, ds, bits, g, bias=_dev(bias), activation="relu", residual=_dev(res), **kw)
+        assert np.array_equal(fused.cpu().numpy().view(np.uint16), c_oracle.epilogue(plain, bias, "relu", res).view(np.uint16))
+        if n % 2 == 0:
+            gated = relax_amd.wq_matmul(dx, dw, ds, bits, g, activation="silu_mul", **kw).cpu().numpy()
+            off = gated.view(np.uint16) != c_oracle.epilogue(plain, activation="silu_mul").view(np.uint16)
+            assert off.sum() <= max(1, gated.size // 1000)
+        if group == (32 if bits == 4 else 128) and k % 256 == 0:
+            wt, st = relax_amd.wq_tile_weights(dw, ds, bits, g)
+            assert torch.equal(relax_amd.wq_matmul(dx, wt, st, bits, g, tiled_n=n, **kw).view(torch.int16), y.view(torch.int16)), "tile-major"
+    assert ran >= 1
+
+
+@pytest.mark.parametrize("bits,m,n,k", [(4, 3, 152064, 1024), (4, 9, 65536, 2048), (8, 8, 65536, 4096), (8, 16, 131072, 512)])
+def test_very_many_tiles_by_default_on_both_layouts(bits, m, n, k):
+    import relax_amd
+
+    x, wq, s, g = O.make_case(n, m, n, k, bits)
+    dx, dw, ds = _dev(x), _dev(wq), _dev(s)
+    want = c_oracle.wq_matmul(x, wq, s, bits, g, nthreads=16)
+    _close(relax_amd.wq_matmul(dx, dw, ds, bits, g).cpu().numpy(), want, (bits, m, n, k))
+    wt, st = relax_amd.wq_tile_weights(dw, ds, bits, g)
+    _close(relax_amd.wq_matmul(dx, wt, st, bits, g, tiled_n=n).cpu().numpy(), want, (bits, m, n, k, "tile-major"))
