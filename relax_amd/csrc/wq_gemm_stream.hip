@@ -23,6 +23,14 @@
 // Measured against the kernels it takes over from (us, weights from memory): int4 4096 x 11008 at 37 / 128 / 512 rows 24.7 /
 // 34.8 / 69 -> 15.7 / 23.2 / 57, 12288 x 4096 at 64 / 256 rows 24.2 / 39.5 -> 17.0 / 32.3, int8 5120 x 13824 at 64 / 256
 // rows 38.7 / 78 -> 22 / 54, 15360 x 5120 at 256 rows 73 -> 48.5, 2048 rows 5 % (power).
+//
+// Rings: what a tile has in flight decides below 128 rows.  int8 64 x 128 with 128-byte weight rows has 32 KB a macro step, and
+// two of them leave one ahead: with 64-byte rows, four macro steps and two K groups 15360 x 5120 at 128 rows 37.9 -> 35.2 us,
+// 27648 x 5120 at 99 71.7 -> 65.3, 5120 x 5120 at 256 29.5 -> 25.7.  int4 64 x 128 has enough in flight and gains from two K
+// groups instead of four (half of the exchange at the end): 12288 x 4096 at 37 rows 20.2 -> 18.7.  32-row tiles for up to 32
+// rows (half of the MFMAs and of the activation traffic; a remainder of up to 32 rows as well): int4 12288 x 4096 at 20 rows
+// 14.0 -> 11.8, 22016 x 4096 21.1 -> 17.8, int8 27648 x 5120 at 32 rows 41.5 -> 32.7 us.  Level or behind: deeper rings elsewhere,
+// reading fragments two slices ahead from LDS, one column wave, not requesting rows past M.
 #include <algorithm>
 #include <atomic>
 #include <mutex>
@@ -657,8 +665,10 @@ bool launch_gemm_stream(const Problem& p, int variant, int ksplit, void* workspa
     WQ_STREAM(kStream128x256, 4, 2, 4, 1, 4, 64, 256, 2) : WQ_STREAM8(4, 2, 4, 1, 4, 64, 128, 3);
     WQ_STREAM(kStream128x128, 4, 2, 2, 2, 4, 64, 256, 2) : WQ_STREAM8(4, 2, 2, 2, 4, 64, 128, 3);
     WQ_STREAM(kStream256x256, 8, 2, 4, 1, 0, 64, 128, 3) : WQ_STREAM8(8, 2, 4, 1, 0, 32, 128, 2);
-    WQ_STREAM(kStream64x128, 2, 2, 2, 4, 4, 128, 256, 3) : WQ_STREAM8(2, 2, 2, 4, 4, 128, 256, 2);
+    WQ_STREAM(kStream64x128, 2, 2, 2, 2, 4, 128, 256, 3) : WQ_STREAM8(2, 2, 2, 2, 4, 64, 128, 4);
     WQ_STREAM(kStream64x64, 2, 1, 2, 4, 4, 128, 256, 3) : WQ_STREAM8(2, 1, 2, 4, 4, 128, 256, 3);
+    WQ_STREAM(kStream32x64, 1, 1, 2, 4, 4, 128, 256, 3) : WQ_STREAM8(1, 1, 2, 4, 4, 128, 256, 3);
+    WQ_STREAM(kStream32x128, 1, 2, 2, 4, 4, 128, 256, 3) : WQ_STREAM8(1, 2, 2, 4, 4, 128, 256, 3);
     default: return false;
   }
 #undef WQ_STREAM
@@ -674,8 +684,8 @@ namespace {
 
 // What a launch takes, in us: start + rounds of tiles * (tile start and end + K * (its loop alone on the chip + what a
 // full chip adds)), and with the K range split the exchange.  Fitted to 1,600 timings (both bit widths, M 20 - 512,
-// N 1024 - 22016, K 4096 - 13824, weights from memory, data random; 4 - 8 % rms); choosing by it costs 0.7 % against always
-// taking the fastest.
+// N 1024 - 22016, K 4096 - 13824, weights from memory, data random; 4 - 8 % rms; the 32-row tiles and 64 x 128 to 60 more at
+// 17 - 128 rows, to about 10 %); choosing by it costs about 1 % against always taking the fastest.
 struct StreamCost {
   int variant, bm, bn;
   float start, tile, loop, loaded, split, window, spread;
@@ -684,22 +694,27 @@ constexpr StreamCost kStreamCost4[] = {
     {kStream128x256, 128, 256, 3.46f, 0.80f, 2.256f, 1.250f, 0.f, 0.f, 0.f},
     {kStream128x128, 128, 128, 1.05f, 6.52f, 1.108f, 0.515f, 3.60f, 1.16f, 0.f},
     {kStream256x256, 256, 256, 0.00f, 0.00f, 5.102f, 1.669f, 0.f, 0.f, 0.f},
-    {kStream64x128, 64, 128, 1.76f, 5.02f, 0.783f, 0.304f, 2.12f, 0.77f, 0.f},
+    {kStream64x128, 64, 128, 1.5f, 4.4f, 0.75f, 0.29f, 2.12f, 0.77f, 0.f},
     {kStream64x64, 64, 64, 1.83f, 3.37f, 0.492f, 0.203f, 1.53f, 0.49f, 0.f},
+    {kStream32x64, 32, 64, 0.5f, 4.2f, 0.44f, 0.12f, 1.53f, 0.25f, 0.f},
+    {kStream32x128, 32, 128, 0.5f, 4.2f, 0.78f, 0.22f, 1.53f, 0.49f, 0.f},
 };
 constexpr StreamCost kStreamCost8[] = {
     {kStream128x256, 128, 256, 0.00f, 0.00f, 3.595f, 0.949f, 0.f, 0.f, 0.f},
     {kStream128x128, 128, 128, 0.09f, 5.01f, 1.416f, 0.603f, 4.62f, 1.03f, 0.f},
     {kStream256x256, 256, 256, 0.00f, 0.00f, 3.810f, 4.601f, 0.f, 0.f, 0.f},
-    {kStream64x128, 64, 128, 2.18f, 2.61f, 1.280f, 0.343f, 2.86f, 0.64f, 0.95f},
+    {kStream64x128, 64, 128, 1.6f, 2.2f, 1.18f, 0.31f, 2.86f, 0.64f, 0.95f},
     {kStream64x64, 64, 64, 2.63f, 1.01f, 0.630f, 0.248f, 2.38f, 0.43f, 0.28f},
+    {kStream32x64, 32, 64, 0.8f, 3.0f, 0.52f, 0.25f, 2.38f, 0.22f, 0.28f},
+    {kStream32x128, 32, 128, 0.4f, 1.0f, 0.88f, 0.80f, 2.38f, 0.43f, 0.28f},
 };
 
 // The register-activation kernel in the same terms (M 20 - 128; 11 % rms): K * (rows + what columns beyond 4096 add).
 float skinny_cost(const Problem& p) {
   if (p.m > kSkinnyMaxM) return 1e30f;
   const int64_t slices = p.m > 64 ? (p.m + 63) / 64 : 1, blocks = ((p.m + 15) / 16 + slices - 1) / slices;
-  const float wide = std::max(1.0f, (float)(p.n * slices) / 4096.0f), macro = (float)p.k / 256.0f, rb = (float)blocks;
+  // (in halves: past 256 tiles a workgroup takes two -- int4 5120 x 5120 at 33 rows 15.0 us)
+  const float wide = std::max(1.0f, (float)((p.n * slices + 2047) / 2048) / 2.0f), macro = (float)p.k / 256.0f, rb = (float)blocks;
   if (p.bits == 4) return 2.19f + macro * (0.041f + 0.127f * rb + (wide - 1.0f) * (0.153f + 0.031f * rb)) + 0.671f * wide;
   return 1.59f + macro * (0.148f + 0.112f * rb + (wide - 1.0f) * 0.294f) + 0.835f * wide;
 }

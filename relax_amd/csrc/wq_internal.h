@@ -48,7 +48,7 @@ bool launch_gemm_pipe(const Problem& p, int group_shift, int variant);
 // The streamed GEMM (wq_gemm_stream.hip): its tiles, an explicit launch, and the one its cost model picks -- the K range
 // split over workgroups where `workspace` has room for that and it pays.  `against_skinny`: not where the
 // register-activation kernel is the faster one.  1 launched, 0 not its problem, -1 failure.
-enum { kStream128x256 = 1, kStream128x128, kStream256x256, kStream64x128, kStream64x64 };
+enum { kStream128x256 = 1, kStream128x128, kStream256x256, kStream64x128, kStream64x64, kStream32x64, kStream32x128 };
 bool gemm_stream_applicable(const Problem& p);
 bool launch_gemm_stream(const Problem& p, int variant, int ksplit, void* workspace);
 int launch_gemm_stream_planned(const Problem& p, void* workspace, int64_t workspace_bytes, bool against_skinny);

@@ -10,7 +10,7 @@ pytestmark = pytest.mark.gpu
 
 from tests.test_gpu_parity import _dev, _fused_operands, assert_close, assert_fused  # noqa: E402
 
-VARIANTS = [31, 32, 33, 34, 35]  # 128 x 256, 128 x 128, 256 x 256, 64 x 128, 64 x 64
+VARIANTS = [31, 32, 33, 34, 35, 36, 37]  # 128 x 256, 128 x 128, 256 x 256, 64 x 128, 64 x 64, 32 x 64, 32 x 128
 
 
 def run(x, wq, s, bits, g, variant, **kw):
