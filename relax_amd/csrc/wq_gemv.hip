@@ -994,15 +994,14 @@ bool use_rounds_any(const Problem& p) { return p.bits == 4 ? use_rounds<4>(p) : 
 
 }  // namespace
 
-// M <= 16 and one of the default variants fits.  (With very many row tiles per workgroup and K too short or too long
-// for rounds, the per-tile partial-sum slots outgrow LDS and the caller falls back to the register-activation kernel.)
+// M <= 16 and one of the default variants fits: with very many row tiles per workgroup (N in the hundreds of thousands) the
+// per-tile partial-sum slots outgrow LDS; the register-activation family then starts with launch_gemv_rounds.
 bool gemv_applicable(const Problem& p) {
   if (p.m < 1 || p.m > 16) return false;
   const int ch = 128 / p.bits;
   int ratio = p.group / ch, gs = 0;
   while ((1 << gs) < ratio) ++gs;
   if (ratio < 1 || (1 << gs) != ratio) return false;
-  if (use_rounds_any(p)) return true;
   const int* order = default_order(p);
   for (int q = 0; q < 4; ++q) {
     const int shape = order[q] % 10;
@@ -1025,7 +1024,7 @@ int launch_gemv(const Problem& p, int variant) {
     return -1;
   }
   int ok = kNotApplicable;
-  if (variant == 0 && use_rounds_any(p)) {
+  if (variant == 0 && gemv_applicable(p) && use_rounds_any(p)) {
     ok = p.bits == 4 ? try_rounds<4>(p, gs, 1) : try_rounds<8>(p, gs, 1);
   } else if (variant == 0) {
     const int* order = default_order(p);
@@ -1049,6 +1048,21 @@ int launch_gemv(const Problem& p, int variant) {
     return -1;
   }
   return 0;
+}
+
+int launch_gemv_rounds(const Problem& p) {
+  const int ch = 128 / p.bits;
+  int gs = 0;
+  while ((ch << gs) < p.group) ++gs;
+  if (p.m < 1 || p.m > 16 || !use_rounds_any(p)) return 0;
+  const int ok = p.bits == 4 ? try_rounds<4>(p, gs, 1) : try_rounds<8>(p, gs, 1);
+  if (ok != kLaunched) return ok;
+  const hipError_t e = hipGetLastError();
+  if (e != hipSuccess) {
+    set_error("gemv kernel (rounds) launch failed: %s", hipGetErrorString(e));
+    return -1;
+  }
+  return 1;
 }
 
 namespace {

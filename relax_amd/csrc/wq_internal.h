@@ -26,6 +26,8 @@ struct Problem {
 // (only reachable through mi355x_wq_matmul_ex; used by sweeps).
 int launch_gemv(const Problem& p, int variant);
 bool gemv_applicable(const Problem& p);  // M <= 16 and a default variant's LDS plan (slots + activations) fits
+// The decode kernel with its tiles in rounds, where the default takes that: 1 launched, 0 not its problem, -1 failure.
+int launch_gemv_rounds(const Problem& p);
 // Cross-workgroup K split of the decode kernel (M <= 16): bytes of caller workspace it needs for `p`
 // (0 = no split for this problem), and the launch (1 launched, 0 not applicable / workspace too small,
 // -1 failure).  The workspace holds float32 partial tiles and per-tile arrival counters; the counters

@@ -424,8 +424,8 @@ int launch_skinny(const Problem& p, int variant) {
     set_error("skinny kernel: M = %lld exceeds %lld", (long long)p.m, (long long)kSkinnyMaxM);
     return -1;
   }
-  if (variant == 0) {  // from 17 rows on the streamed GEMM where it is the faster one
-    const int rc = launch_gemm_stream_planned(p, nullptr, 0, true);
+  if (variant == 0) {  // from 17 rows on the streamed GEMM where it is the faster one, below the decode kernel's rounds
+    const int rc = p.m <= 16 ? launch_gemv_rounds(p) : launch_gemm_stream_planned(p, nullptr, 0, true);
     if (rc != 0) return rc < 0 ? -1 : 0;
   }
   const int mt = (int)((std::min<int64_t>(p.m, skinny_slice_rows(p.m)) + 15) / 16);
