@@ -1,5 +1,6 @@
 // Runtime module of one offloaded subgraph (include/mi355x_wq_module.h): constant binding at load
 // time, the call with the remaining arguments, and the binary form that survives export / load.
+#include <algorithm>
 #include <dlfcn.h>
 #include <hip/hip_runtime_api.h>
 
@@ -420,9 +421,10 @@ bool bind_constants(mi355x_wq_module* m, const mi355x_dl_tensor* const* consts, 
       const int64_t b = mi355x_wq_workspace_bytes(&d, rows, tiled);
       if (b < 0) return false;
       if (b > need) need = b;
+      if (rows != 17 && rows % 32 != 1) continue;  // (from 17 rows on the streamed kernel's plan is the same for 32 rows)
       wq::Problem p{nullptr, nullptr, nullptr, nullptr, rows, d.n, d.k, d.bits, d.group, d.zero_point, nullptr};
       p.activation = m->spec.activation;
-      if (wq::gemm_stream_workspace_bytes(p) > need) need = wq::gemm_stream_workspace_bytes(p);
+      need = std::max(need, wq::gemm_stream_workspace_bytes(p));
     }
     if (need > 0) {
       if (!hip_ok(hipMalloc(&m->workspace, need), "hipMalloc")) return false;
