@@ -33,7 +33,7 @@ MFMA_F16_PEAK_TFLOPS = 2500.0  # MI355X published dense fp16 MFMA rate
 GEMV_PROFILE = os.path.join(ROOT, "profiles", "gemv_decode_llama7b.md")
 GEMV_KERNEL_SOURCES = ("relax_amd/csrc/wq_gemv.hip", "relax_amd/csrc/wq_device.h")
 GEMM_PROFILE = os.path.join(ROOT, "profiles", "gemm_prefill_llama7b.md")
-GEMM_KERNEL_SOURCES = ("relax_amd/csrc/wq_gemm_direct.hip", "relax_amd/csrc/wq_device.h")
+GEMM_KERNEL_SOURCES = ("relax_amd/csrc/wq_gemm_stream.hip", "relax_amd/csrc/wq_device.h")
 PROBE_SO = os.path.join(ROOT, "relax_amd", "csrc", "libmi355x_probe.so")
 STAMPS_SO = os.path.join(ROOT, "relax_amd", "csrc", "libmi355x_wq_stamps.so")
 
@@ -662,7 +662,7 @@ def main() -> int:
                                    "peak": MFMA_F16_PEAK_TFLOPS, "unit": "TFLOP/s",
                                    "frac": round(tflops / MFMA_F16_PEAK_TFLOPS, 4),
                                    "traffic": measured_traffic(GEMM_PROFILE, GEMM_KERNEL_SOURCES),
-                                   "kernel": "wq::wq_gemm_direct_kernel"}
+                                   "kernel": "wq::wq_gemm_stream_kernel"}
         del wds, tiled_w
 
     # ---- fused residual add: O and down projections of every layer, batch 1 and 8 -------------
