@@ -386,7 +386,7 @@ int matmul_any_layout(const mi355x_wq_desc* desc, const void* x, const void* wq_
       rc = launch_gemv_split(p, workspace, workspace_bytes);
     } else if (gemm_stream_applicable(p)) {
       const bool skinny = select_kernel(desc, m, tiled) == MI355X_WQ_KERNEL_SKINNY;
-      if (skinny || launch_gemm_streams(p)) rc = launch_gemm_stream_planned(p, workspace, workspace_bytes, skinny);
+      if (skinny ? !skinny_keeps(p) : launch_gemm_streams(p)) rc = launch_gemm_stream_planned(p, workspace, workspace_bytes, skinny);
     } else {
       rc = launch_gemm_split(p, workspace, workspace_bytes);
     }

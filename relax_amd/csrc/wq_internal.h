@@ -43,6 +43,7 @@ int64_t gemv_static_scratch_bytes();
 int64_t gemm_split_workspace_bytes(const Problem& p);
 int launch_gemm_split(const Problem& p, void* workspace, int64_t workspace_bytes);
 int launch_skinny(const Problem& p, int variant);
+bool skinny_keeps(const Problem& p);  // a problem of the skinny family that the streamed kernel's cost model misjudges
 int launch_gemm(const Problem& p, int variant);
 bool launch_gemm_streams(const Problem& p);  // whether the GEMM family's default may be the streamed kernel for `p`
 bool gemm_pipe_applicable(const Problem& p);  // K % 64 == 0, operands below 1 GiB

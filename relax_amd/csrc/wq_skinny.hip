@@ -412,6 +412,11 @@ bool dispatch_variant(const Problem& p, int group_shift, int variant) {
 
 }  // namespace
 
+// int8 at 17 - 32 rows on the narrowest projections: the streamed kernel's K split costs more there than its model says
+// (2048 x 5632 at 17 / 32 rows 9.8 / 11.0 us here, 11.6 / 11.6 there, tile-major 9.3 / 10.3 against 12.0 / 12.2, 1024 x 8192
+// tile-major 11.2 / 12.3 against 12.7 / 12.9; on canonical weights that one is 11.8 / 13.8 here and 11.7 / 11.9 there).
+bool skinny_keeps(const Problem& p) { return p.bits == 8 && p.m > 16 && p.m <= 32 && p.n <= 2048 && (p.tiled || p.k < 8192); }
+
 int launch_skinny(const Problem& p, int variant) {
   const int ch = 128 / p.bits;
   int ratio = p.group / ch, group_shift = 0;
@@ -425,7 +430,7 @@ int launch_skinny(const Problem& p, int variant) {
     return -1;
   }
   if (variant == 0) {  // from 17 rows on the streamed GEMM where it is the faster one, below the decode kernel's rounds
-    const int rc = p.m <= 16 ? launch_gemv_rounds(p) : launch_gemm_stream_planned(p, nullptr, 0, true);
+    const int rc = p.m <= 16 ? launch_gemv_rounds(p) : skinny_keeps(p) ? 0 : launch_gemm_stream_planned(p, nullptr, 0, true);
     if (rc != 0) return rc < 0 ? -1 : 0;
   }
   const int mt = (int)((std::min<int64_t>(p.m, skinny_slice_rows(p.m)) + 15) / 16);
@@ -451,7 +456,9 @@ int launch_skinny(const Problem& p, int variant) {
     // and with several rounds of workgroups (a 152064 x 4096 vocabulary projection: 108 - 153 -> 91 - 102 us,
     // tile-major 75 - 106 -> 70 - 76).
     const bool staged = mt >= 2;
-    if (tiles <= 256) variant = staged ? (p.bits == 4 ? 26 : 21) : (p.bits == 8 || p.m >= 9) ? 26 : 1;
+    // (int8 on eight wavefronts too with up to 192 tiles or short K: 2048 x 2048 at 17 / 64 rows 5.16 / 7.68 -> 4.76 / 7.15 us,
+    // 4096 x 1024 4.06 / 5.84 -> 3.78 / 5.28, level at 3072 x 3072, behind at 4096 x 4096 up to 33 rows, 7.9 against 8.15)
+    if (tiles <= 256) variant = staged ? (p.bits == 4 || tiles <= 192 || p.k <= 2048 ? 26 : 21) : (p.bits == 8 || p.m >= 9) ? 26 : 1;
     // (one tile per workgroup is 1.5 - 1.8x slower here; int8 at up to 4 rows on tile-major weights:
     // eight wavefronts, 3 - 5 % ahead)
     else if (tiles <= 512) variant = (staged || p.m >= 9) ? 25 : ((p.bits == 4 || (p.tiled && p.m <= 4)) ? 5 : 2);
