@@ -236,6 +236,9 @@ int launch_gemm_any(const Problem& p, int variant, bool direct_ok);
 // weights and the gated tail are defined here for the direct-weight kernel's problems: K % 256 == 0, the standard group,
 // operands below 1 GiB.
 bool launch_gemm_streams(const Problem& p) {
+  // (short K and more than 256 rows: a launch is mostly the start and end of its tiles, which the other kernels do faster --
+  // int8 1906 x 2637 x 1152 25.4 us there, 33.8 here, int4 1049 x 5425 x 1088 27.9 / 32.2, int8 407 x 13173 x 1280 33.7 / 38.3)
+  if (p.m > 256 && p.k < 1536) return false;
   const bool direct = p.k % 256 == 0 && p.group == (p.bits == 4 ? 32 : 128) && gemm_pipe_applicable(p);
   return (direct || !(p.tiled || p.activation == kActGated)) && !(p.activation == kActGelu && p.residual == p.y);
 }
