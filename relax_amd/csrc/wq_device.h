@@ -154,12 +154,33 @@ struct Epilogue {
 constexpr int kActGated = 2;
 constexpr int kActGelu = 3;
 
+// erf of a float16 value, rounded to float16.  The tails are vector work behind a workgroup's last MFMA with nothing beside
+// it, and erff, which evaluates both of its branches for a wavefront whose values fall into either, is sixty instructions of
+// it (int4 1024 x 10000 x 4224, bias and gelu: 128.6 -> 112.2 us, 105 with the bias alone).  This is x * P(x^2) with the first coefficient split
+// in two, the coefficients by a linear program that keeps every float16 input inside the rounding interval of its result: for
+// each of the 65536 the same float16 value as erff's, which is the correctly rounded one.
+__device__ __forceinline__ half_t erf_f16(half_t h) {
+  const float x = fminf(fabsf((float)h), 2.6f);  // (erf rounds to 1 from 2.5957 on)
+  const float t = x * x;
+  float p = -0x1.13902ap-29f;
+  p = __builtin_fmaf(p, t, 0x1.c90658p-23f);
+  p = __builtin_fmaf(p, t, -0x1.8862bap-18f);
+  p = __builtin_fmaf(p, t, 0x1.5afc40p-14f);
+  p = __builtin_fmaf(p, t, -0x1.8cefbcp-11f);
+  p = __builtin_fmaf(p, t, 0x1.4cd49cp-8f);
+  p = __builtin_fmaf(p, t, -0x1.b66322p-6f);
+  p = __builtin_fmaf(p, t, 0x1.ce0d9cp-4f);
+  p = __builtin_fmaf(p, t, -0x1.81267cp-2f);
+  p = __builtin_fmaf(p, t, -0x1.0a295ep-24f);
+  return (half_t)__builtin_copysignf(__builtin_fmaf(x, 0x1.20dd76p+0f, x * p), (float)h);
+}
+
 // nn.gelu on a float16 value as its legalized form x * (0.5 + erf(x * sqrt(0.5)) * 0.5) runs on float16 tensors
 // (python/tvm/relax/transform/legalize_ops.py:495-503): every operation rounded once, the constants rounded
 // to float16 first, erf evaluated in float32 and rounded.
 __device__ __forceinline__ half_t gelu_f16(half_t h) {
   const half_t a = h * (half_t)0.70710678118654752440f;
-  const half_t e = (half_t)erff((float)a);
+  const half_t e = erf_f16(a);
   const half_t b = e * (half_t)0.5f;
   const half_t c = (half_t)0.5f + b;
   return h * c;
@@ -172,12 +193,14 @@ __device__ __forceinline__ half_t gelu_f16(half_t h) {
 __device__ __forceinline__ int gated_physical_row(int logical, int N) { return (logical >> 1) + ((logical & 1) ? (N >> 1) : 0); }
 
 // multiply(nn.silu(g), u) on float16 values, every operation rounded once as the CPU path executes them:
-// e = f16(exp(-g)) (evaluated in float32), d = f16(1 + e), s = f16(1 / d), t = f16(g * s), y = f16(t * u).
-// The float32 quotient is correctly rounded and its second rounding to float16 is innocuous.
+// e = f16(exp(-g)), d = f16(1 + e), s = f16(1 / d), t = f16(g * s), y = f16(t * u).
+// exp and the quotient in float32 by one hardware instruction each (exp2 of g * -log2(e), rcp): rounded to float16 they are,
+// for each of the 65536 values of g and of d, the same as expf's and the division's, which took 40 instructions more (int4
+// 2048 x 22016 x 4096: 362 -> 356 us).
 __device__ __forceinline__ half_t silu_mul(half_t g, half_t u) {
-  const half_t e = (half_t)expf(-(float)g);
+  const half_t e = (half_t)__builtin_amdgcn_exp2f((float)g * -1.4426950408889634f);
   const half_t d = (half_t)1 + e;
-  const half_t s = (half_t)(1.0f / (float)d);
+  const half_t s = (half_t)__builtin_amdgcn_rcpf((float)d);
   const half_t t = g * s;
   return t * u;
 }
