@@ -599,17 +599,42 @@ __global__ __launch_bounds__((CW * G + PROD) * 64, 1) void wq_gemm_stream_kernel
       }
     return;
   }
-  if (TN == 2 && pair_store_ok(ep, y, N)) {
-    const int rows = min(BM, M - m0);
-    const uint32_t bytes = (uint32_t)rows * (uint32_t)N * 2u, pitch = (uint32_t)N * 2u;
-    const uint32_t col = n < N ? (uint32_t)n * 2u : kStreamOob;
-    const uint32_t base = col + (uint32_t)row_in_tile(0, 0) * pitch;
-    auto offset = [&](int p, int e) __attribute__((always_inline)) {  // of row quad p, row e; p = 0, e = 0 is `base`
-      const int r = row_in_tile(p, e);
-      return r < rows ? base + (uint32_t)(r - row_in_tile(0, 0)) * pitch : kStreamOob;
-    };
-    // (in portions of four row quads, which keeps the registers of the loop's accumulators apart from the tail's)
-    constexpr int PC = PG < 4 ? PG : 4;
+  // (in portions of four row quads, which keeps the registers of the loop's accumulators apart from the tail's)
+  const int rows = min(BM, M - m0);
+  const uint32_t bytes = (uint32_t)rows * (uint32_t)N * 2u, pitch = (uint32_t)N * 2u;
+  const rsrc_t ry = make_rsrc(y + (size_t)m0 * N, bytes), rr = make_rsrc(ep.residual + (size_t)m0 * N, bytes), rb = make_rsrc(ep.bias, (uint32_t)N * 2u);
+  constexpr int PC = PG < 4 ? PG : 4;
+  const bool paired = TN == 2 && pair_store_ok(ep, y, N);
+  const uint32_t col = n < N ? (uint32_t)n * 2u : kStreamOob, col1 = TN == 2 && n + 1 < N ? col + 2u : kStreamOob;
+  const uint32_t base = (uint32_t)row_in_tile(0, 0) * pitch;
+  // of row quad p, row e, column offset c; p = 0, e = 0 is `base`
+  auto offset = [&](int p, int e, uint32_t c) __attribute__((always_inline)) {
+    const int r = row_in_tile(p, e);
+    return r < rows && c != kStreamOob ? base + (uint32_t)(r - row_in_tile(0, 0)) * pitch + c : kStreamOob;
+  };
+  auto tail = [&](half2_t (&h)[PC][4], half2_t b2) __attribute__((always_inline)) {
+    if (ep.bias != nullptr) {
+#pragma unroll
+      for (int p = 0; p < PC; ++p)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) h[p][e] = h[p][e] + b2;
+    }
+    if (ep.activation == 1) {
+#pragma unroll
+      for (int p = 0; p < PC; ++p)
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+#pragma unroll
+          for (int c = 0; c < 2; ++c) h[p][e][c] = h[p][e][c] > (half_t)0 ? h[p][e][c] : (half_t)0;
+    }
+    if (__builtin_expect(ep.activation == kActGelu, 0)) {
+#pragma unroll
+      for (int p = 0; p < PC; ++p)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) h[p][e] = half2_t{gelu_f16(h[p][e][0]), TN == 2 ? gelu_f16(h[p][e][1]) : (half_t)0};
+    }
+  };
+  if (paired) {
     static_for_s<0, PG / PC>([&](auto portion) __attribute__((always_inline)) {
       constexpr int p0 = decltype(portion)::value * PC;
       half2_t h[PC][4];
@@ -617,58 +642,82 @@ __global__ __launch_bounds__((CW * G + PROD) * 64, 1) void wq_gemm_stream_kernel
       for (int p = 0; p < PC; ++p)
 #pragma unroll
         for (int e = 0; e < 4; ++e) h[p][e] = half2_t{(half_t)fin[p0 + p][0][e], (half_t)fin[p0 + p][TN - 1][e]};
-      if (ep.bias != nullptr) {
-        const half2_t b2 = as_h2(load_b32(make_rsrc(ep.bias, (uint32_t)N * 2u), col));
-#pragma unroll
-        for (int p = 0; p < PC; ++p)
-#pragma unroll
-          for (int e = 0; e < 4; ++e) h[p][e] = h[p][e] + b2;
-      }
-      if (ep.activation == 1) {
-#pragma unroll
-        for (int p = 0; p < PC; ++p)
-#pragma unroll
-          for (int e = 0; e < 4; ++e)
-#pragma unroll
-            for (int c = 0; c < 2; ++c) h[p][e][c] = h[p][e][c] > (half_t)0 ? h[p][e][c] : (half_t)0;
-      }
-      if (__builtin_expect(ep.activation == kActGelu, 0)) {
-#pragma unroll
-        for (int p = 0; p < PC; ++p)
-#pragma unroll
-          for (int e = 0; e < 4; ++e) h[p][e] = half2_t{gelu_f16(h[p][e][0]), gelu_f16(h[p][e][1])};
-      }
+      tail(h, ep.bias != nullptr ? as_h2(load_b32(rb, col)) : half2_t{});
       if (ep.residual != nullptr) {
-        const rsrc_t rr = make_rsrc(ep.residual + (size_t)m0 * N, bytes);
         uint32_t res[PC][4];
 #pragma unroll
         for (int p = 0; p < PC; ++p)
 #pragma unroll
-          for (int e = 0; e < 4; ++e) res[p][e] = load_b32(rr, offset(p0 + p, e));
+          for (int e = 0; e < 4; ++e) res[p][e] = load_b32(rr, offset(p0 + p, e, col));
 #pragma unroll
         for (int p = 0; p < PC; ++p)
 #pragma unroll
           for (int e = 0; e < 4; ++e) h[p][e] = h[p][e] + as_h2(res[p][e]);
       }
-      const rsrc_t ry = make_rsrc(y + (size_t)m0 * N, bytes);
 #pragma unroll
       for (int p = 0; p < PC; ++p)
 #pragma unroll
-        for (int e = 0; e < 4; ++e) __builtin_amdgcn_raw_buffer_store_b32(as_u32(h[p][e]), ry, offset(p0 + p, e), 0, 0);
+        for (int e = 0; e < 4; ++e) __builtin_amdgcn_raw_buffer_store_b32(as_u32(h[p][e]), ry, offset(p0 + p, e, col), 0, 0);
       __builtin_amdgcn_sched_barrier(0);
     });
     return;
   }
+  // One column per lane, an odd N or operands that are only 2-byte aligned.  Bound by the latency of what an element asks for: bias
+  // and residual are requested for a portion at a time, and the tail's shape is not asked per element (int4 333 x 10001 x
+  // 4224: plain 41.2 -> 38.5 us, bias and gelu 51.7 -> 40.9, residual 51.4 -> 40.8; 64 x 64 tiles, 37 x 4096 x 11008 with a residual
+  // 18.0 -> 16.3).  Two columns: rows that begin on a 4-byte boundary (odd
+  // N: every second one) are stored in pairs all the same, the others in pairs of the second column and the next lane's first
+  // (what a half-wavefront's first and last lane have left over goes out as 2 bytes).
+  const bool odd_n = N & 1, shifted0 = (reinterpret_cast<uintptr_t>(y) >> 1 & 1) ^ (odd_n & m0 & 1);
+  static_for_s<0, PG / PC>([&](auto portion) __attribute__((always_inline)) {
+    constexpr int p0 = decltype(portion)::value * PC;
+    half2_t h[PC][4];
 #pragma unroll
-  for (int p = 0; p < PG; ++p)
+    for (int p = 0; p < PC; ++p)
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      const int m = m0 + row_in_tile(p, e);
-      if (m >= M) continue;
+      for (int e = 0; e < 4; ++e) h[p][e] = half2_t{(half_t)fin[p0 + p][0][e], (half_t)fin[p0 + p][TN - 1][e]};
+    auto two = [](uint32_t first, uint32_t second) __attribute__((always_inline)) { return as_h2(first | second << 16); };
+    tail(h, ep.bias != nullptr ? two(load_b16(rb, col), TN == 2 ? load_b16(rb, col1) : 0u) : half2_t{});
+    if (ep.residual != nullptr) {
+      uint32_t res[PC][4][TN];
 #pragma unroll
-      for (int j = 0; j < TN; ++j)
-        if (n + j < N) store_out(ep, y, m, n + j, N, fin[p][j][e]);
+      for (int p = 0; p < PC; ++p)
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+#pragma unroll
+          for (int j = 0; j < TN; ++j) res[p][e][j] = load_b16(rr, offset(p0 + p, e, j == 0 ? col : col1));
+#pragma unroll
+      for (int p = 0; p < PC; ++p)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) h[p][e] = h[p][e] + two(res[p][e][0], TN == 2 ? res[p][e][TN - 1] : 0u);
     }
+    auto store_b16 = [&](uint32_t v, uint32_t off) __attribute__((always_inline)) { __builtin_amdgcn_raw_buffer_store_b16((uint16_t)v, ry, off, 0, 0); };
+    if constexpr (TN == 1) {
+#pragma unroll
+      for (int p = 0; p < PC; ++p)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) store_b16(as_u32(h[p][e]), offset(p0 + p, e, col));
+    } else {
+#pragma unroll
+      for (int p = 0; p < PC; ++p)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const uint32_t v = as_u32(h[p][e]);
+          if (shifted0 != (odd_n && (e & 1))) {
+            const uint32_t next = (uint32_t)__shfl_down((int)v, 1);
+            const bool whole = fr < 31 && n + 2 < N;
+            __builtin_amdgcn_raw_buffer_store_b32(v >> 16 | next << 16, ry, offset(p0 + p, e, whole ? col1 : kStreamOob), 0, 0);
+            store_b16(fr == 0 ? v : v >> 16, offset(p0 + p, e, fr == 0 ? col : whole ? kStreamOob : col1));
+            // (the first lane's second column where it has no whole pair)
+            if (n0 + cw * TN * 32 + 2 >= N) store_b16(v >> 16, offset(p0 + p, e, fr == 0 ? col1 : kStreamOob));
+          } else {
+            __builtin_amdgcn_raw_buffer_store_b32(v, ry, offset(p0 + p, e, n + 1 < N ? col : kStreamOob), 0, 0);
+            if (n0 + BN >= N) store_b16(v, offset(p0 + p, e, n + 1 == N ? col : kStreamOob));
+          }
+        }
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  });
 }
 
 namespace {
