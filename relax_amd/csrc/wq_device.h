@@ -34,6 +34,9 @@ __device__ __forceinline__ rsrc_t make_rsrc(const void* base, uint32_t bytes) {
 __device__ __forceinline__ u32x4 load_b128(rsrc_t r, uint32_t voff) {
   return __builtin_amdgcn_raw_buffer_load_b128(r, voff, 0, 0);
 }
+__device__ __forceinline__ u32x4 load_b128_once(rsrc_t r, uint32_t voff) {  // non-temporal: for lines nobody asks for twice
+  return __builtin_amdgcn_raw_buffer_load_b128(r, voff, 0, 2);
+}
 __device__ __forceinline__ u32x2 load_b64(rsrc_t r, uint32_t voff) {
   return __builtin_amdgcn_raw_buffer_load_b64(r, voff, 0, 0);
 }

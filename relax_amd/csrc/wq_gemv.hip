@@ -67,6 +67,30 @@ __device__ unsigned long long g_gemv_stamps[kStampLaunches * kStampWaves * kStam
 #define WQ_STAMP(i) ((void)0)
 #endif
 
+// Between the lanes of each pair (even, odd): the even lane's `odd_row` against the odd lane's `even_row`.  As assembly because
+// the compiler makes four instructions of what a select with a lane permutation in its first operand does in two.
+__device__ __forceinline__ void swap_pairs(u32x4& even_row, u32x4& odd_row) {
+  uint32_t e[4], o[4];
+  asm("s_mov_b64 vcc, %[even]\n\t"
+      "s_nop 1\n\t"
+      "v_cndmask_b32_dpp %[e0], %[y0], %[x0], vcc quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
+      "v_cndmask_b32_dpp %[e1], %[y1], %[x1], vcc quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
+      "v_cndmask_b32_dpp %[e2], %[y2], %[x2], vcc quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
+      "v_cndmask_b32_dpp %[e3], %[y3], %[x3], vcc quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
+      "s_not_b64 vcc, vcc\n\t"
+      "v_cndmask_b32_dpp %[o0], %[x0], %[y0], vcc quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
+      "v_cndmask_b32_dpp %[o1], %[x1], %[y1], vcc quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
+      "v_cndmask_b32_dpp %[o2], %[x2], %[y2], vcc quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
+      "v_cndmask_b32_dpp %[o3], %[x3], %[y3], vcc quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf"
+      : [e0] "=&v"(e[0]), [e1] "=&v"(e[1]), [e2] "=&v"(e[2]), [e3] "=&v"(e[3]), [o0] "=&v"(o[0]), [o1] "=&v"(o[1]), [o2] "=&v"(o[2]),
+        [o3] "=&v"(o[3])
+      : [x0] "v"(even_row[0]), [x1] "v"(even_row[1]), [x2] "v"(even_row[2]), [x3] "v"(even_row[3]), [y0] "v"(odd_row[0]),
+        [y1] "v"(odd_row[1]), [y2] "v"(odd_row[2]), [y3] "v"(odd_row[3]), [even] "s"(0x5555555555555555ull)
+      : "vcc", "scc");
+  even_row = u32x4{e[0], e[1], e[2], e[3]};
+  odd_row = u32x4{o[0], o[1], o[2], o[3]};
+}
+
 template <int D, int SPL>
 struct GemvBuf {
   u32x4 w[D];
@@ -97,10 +121,14 @@ struct GemvKernArgs {
   unsigned int* counters;
 };
 
+// READ: a lane's weights by requests of its own chunks; canonical weights by pairs of lanes, so that a request covers whole lines;
+// and whole lines (tile-major ones always are) by non-temporal requests.
+enum { kReadOwn, kReadPairs, kReadOnce };
+
 // ROUNDS: a workgroup has more tiles than its LDS has slots for.  The tiles are walked in rounds of half the slots (an even
 // number, so that a round ends with a trip of the stream); after a round one barrier, and the round's tiles are summed
 // and stored from one half of the slots while the next round fills the other, its first item already in flight.
-template <int BITS, int WAVES, int D, int SPL, bool TILED, int XS, bool KSPLIT, bool PHASES, bool ROUNDS>
+template <int BITS, int WAVES, int D, int SPL, bool TILED, int XS, bool KSPLIT, bool PHASES, bool ROUNDS, int READ>
 // PHASES: the launch walks K in more than one phase (activations beyond the LDS).  The host knows; as a template
 // flag it keeps the second phase description out of the build that runs the common launches, whose first memory
 // requests otherwise wait behind that bookkeeping (and behind the late kernel arguments, which the compiler
@@ -122,6 +150,9 @@ __global__ __launch_bounds__(WAVES * 64) __attribute__((amdgpu_waves_per_eu(2, 8
     int shift_and_zero_, int max_tiles_, int phase_chunks_, int ksplit_, int grid_, half_t* y_late, const Epilogue ep_late,
     float* partials_late, unsigned int* counters_late) {
   static_assert(!KSPLIT || !PHASES, "the cross-workgroup K split walks one window of K");
+  constexpr bool kPairs = READ >= kReadPairs && !TILED, kOnce = READ == kReadOnce;
+  static_assert(READ == kReadOwn || D == 2, "pairs of lanes share the two chunks a lane has in a super step");
+  auto load_weights = [](rsrc_t r, uint32_t off) { return kOnce ? load_b128_once(r, off) : load_b128(r, off); };
   static_assert(!ROUNDS || (!KSPLIT && !PHASES && XS == 0), "rounds of tiles: all of K in one phase");
   static_assert(XS == 0 || XS == 1 || XS == 2 || XS == 3 || XS == 4 || XS == 8 || XS == 16, "staging mode");
   constexpr bool ROWS = XS >= 4;
@@ -231,7 +262,7 @@ __global__ __launch_bounds__(WAVES * 64) __attribute__((amdgpu_waves_per_eu(2, 8
       ok = ok && (c.chunk_base + ss * 4 * D < nchunks);
       const uint32_t woff = ok ? item * (D * 1024u) + (uint32_t)lane * 16u : kOobOffset;
 #pragma unroll
-      for (int d = 0; d < D; ++d) b.w[d] = load_b128(rw, woff + d * 1024u);
+      for (int d = 0; d < D; ++d) b.w[d] = load_weights(rw, woff + d * 1024u);
       if constexpr (SPL == 1) b.sc[0] = load_b16(rs, ok ? (item * 16u + (uint32_t)col) * 2u : kOobOffset);
       else b.sc[0] = load_b32(rs, ok ? (item * 64u + (uint32_t)lane) * 4u : kOobOffset);
       return;
@@ -243,11 +274,22 @@ __global__ __launch_bounds__(WAVES * 64) __attribute__((amdgpu_waves_per_eu(2, 8
     // D > 1 is only launched when K is a multiple of 4*D chunks, so a lane's D
     // chunks are valid together; D == 1 checks its single chunk.
     ok = ok && (chunk0 < nchunks);
-    const uint32_t woff = ok ? (uint32_t)n * row_bytes + (uint32_t)chunk0 * 16u : kOobOffset;
     const uint32_t soff =
         ok ? ((uint32_t)n * groups_per_row + ((uint32_t)chunk0 >> group_shift_)) * 2u : kOobOffset;
+    if constexpr (kPairs) {
+      // Request d reads row d of a pair of rows, chunk kq * 2 + col % 2 of it: eight whole 128-byte lines.  What a pair of lanes
+      // then holds of each other's rows compute_super swaps.  Gated, the pair is a gate row and its up row.
+      const int r0 = tile * tile_rows + (col & ~1);
+      const bool live = i < my_tiles && chunk0 < nchunks;
+      const uint32_t first = (uint32_t)(gated ? r0 >> 1 : r0) * row_bytes + (uint32_t)(chunk0 + (col & 1)) * 16u;
+      const uint32_t second = first + (gated ? (uint32_t)(N >> 1) : 1u) * row_bytes;
+      b.w[0] = load_weights(rw, live && (col & ~1) < tile_rows && r0 < N ? first : kOobOffset);
+      b.w[1] = load_weights(rw, live && (col | 1) < tile_rows && r0 + 1 < N ? second : kOobOffset);
+    } else {
+      const uint32_t woff = ok ? (uint32_t)n * row_bytes + (uint32_t)chunk0 * 16u : kOobOffset;
 #pragma unroll
-    for (int d = 0; d < D; ++d) b.w[d] = load_b128(rw, woff + d * 16u);
+      for (int d = 0; d < D; ++d) b.w[d] = load_b128(rw, woff + d * 16u);
+    }
     if constexpr (SPL == 1) {
       b.sc[0] = load_b16(rs, soff);
     } else if constexpr (SPL == 2) {
@@ -269,7 +311,11 @@ __global__ __launch_bounds__(WAVES * 64) __attribute__((amdgpu_waves_per_eu(2, 8
   float4_t acc = float4_t{0.f, 0.f, 0.f, 0.f};
 
   // one super step of MFMAs on the staged activations at xp
-  auto compute_super = [&](const GemvBuf<D, SPL>& b, const half_t* xp) {
+  auto compute_super = [&](GemvBuf<D, SPL>& b, const half_t* xp) {
+    if constexpr (kPairs) {
+      // the even lane's chunk of the odd row and the odd lane's chunk of the even row change places
+      swap_pairs(b.w[0], b.w[1]);
+    }
     half8_t av[2][NJ];  // activations of chunk d+1 are read from LDS while chunk d is consumed
 #pragma unroll
     for (int j = 0; j < NJ; ++j) av[0][j] = *reinterpret_cast<const half8_t*>(xp + j * 8);
@@ -708,12 +754,14 @@ struct Plan {
 // them idle for a whole tile (5120 rows: 320 tiles on 256 CUs -- 64 walk two tiles, 192 one); shorter tiles even that
 // out (512 tiles of 10 rows: two each) at the price of load instructions whose lanes past the tile's rows request
 // nothing.  Cost of a choice: tiles per CU x (rows + 4) -- a tile costs its bytes plus about four rows' worth of
-// per-tile work -- and a shorter tile must win by an eighth.  Measured (us, 16 rows -> the rule's choice): int8
+// per-tile work -- and a shorter tile must win by a tenth (10240 x 8192 at batch 1, 14 rows instead of 16: int8 19.3 -> 17.4
+// us, int4 12.6 -> 11.2).  Measured (us, 16 rows -> the rule's choice): int8
 // 5120 x 5120 at 1 / 16 rows 8.80 -> 7.92 / 12.41 -> 11.22, 5120 x 13824 19.44 -> 16.68 / 26.14 -> 24.09, int4
 // 5120 x 5120 6.31 -> 5.98; what counts is the balance over CUs, not over workgroups: 12288 rows on two workgroups
 // per CU (768 tiles: two for one workgroup, one for the other, three per CU) lose with 12-row tiles (7.36 -> 8.28).
-// `forced` (8 .. 16) overrides the rule.
-inline int pick_tile_rows(int64_t n, int cap, int forced) {
+// `forced` (8 .. 16) overrides the rule.  (The K split's choice keeps an eighth, by which its measurements were taken and callers'
+// workspaces are sized.)
+inline int pick_tile_rows(int64_t n, int cap, int forced, int margin = 10) {
   if (forced >= 8 && forced <= 16) return forced;
   auto cost = [&](int tr) {
     const int64_t tiles = (n + tr - 1) / tr, grid = std::min<int64_t>(tiles, cap);
@@ -723,7 +771,7 @@ inline int pick_tile_rows(int64_t n, int cap, int forced) {
   int64_t best_cost = cost(16);
   for (int tr = 15; tr >= 8; --tr)
     if (cost(tr) < best_cost) best = tr, best_cost = cost(tr);
-  return best_cost * 8 <= cost(16) * 7 ? best : 16;
+  return best_cost * margin <= cost(16) * (margin - 1) ? best : 16;
 }
 
 // Chooses the grid (workgroups per CU), the tiles per workgroup and the K phase so
@@ -822,20 +870,41 @@ int launch_one(const Problem& p, int group_shift, const Plan& plan, int ksplit =
   float* const partials = reinterpret_cast<float*>(static_cast<char*>(workspace) + kSplitCounterBytes);
   // the builds of the kernel: by the way the activations are staged (the kernel's XS) and by whether K is walked in
   // several phases
-  auto go = [&](auto xs, auto phases) -> int {
+  auto go_read = [&](auto xs, auto phases, auto read) -> int {
     constexpr int XS = decltype(xs)::value;
     constexpr bool PHASES = decltype(phases)::value;
+    constexpr int READ = decltype(read)::value;
     static std::atomic<bool> lds_ok[kMaxDevices];
-    if (!ensure_dynamic_lds((const void*)wq_gemv_kernel<BITS, WAVES, D, SPL, TILED, XS, KSPLIT, PHASES, ROUNDS>, (int)kLdsPerWgMax,
+    if (!ensure_dynamic_lds((const void*)wq_gemv_kernel<BITS, WAVES, D, SPL, TILED, XS, KSPLIT, PHASES, ROUNDS, READ>, (int)kLdsPerWgMax,
                             lds_ok))
       return kFailed;
-    hipLaunchKernelGGL((wq_gemv_kernel<BITS, WAVES, D, SPL, TILED, XS, KSPLIT, PHASES, ROUNDS>), dim3(plan.grid), dim3(WAVES * 64),
+    hipLaunchKernelGGL((wq_gemv_kernel<BITS, WAVES, D, SPL, TILED, XS, KSPLIT, PHASES, ROUNDS, READ>), dim3(plan.grid), dim3(WAVES * 64),
                        plan.lds_bytes, p.stream, (const half_t*)p.x, (const uint32_t*)p.wq, (const half_t*)p.scales,
                        (int)p.m, (int)p.n, (int)p.k,
                        group_shift | (p.zero_point << 8) | (p.activation == kActGated ? 1 << 16 : 0) | (plan.tile_rows << 20),
                        plan.max_tiles, plan.phase_chunks, stamp_slot_or(ksplit, KSPLIT || ROUNDS), plan.grid, (half_t*)p.y, ep,
                        partials, counters);
     return kLaunched;
+  };
+  // How the weights are read (the kernel's READ).  Canonical int8 by pairs of lanes, whose requests cover whole lines (12288 x 4096
+  // at 2 rows 11.0 -> 9.9 us, 15360 x 5120 at 16 rows 19.8 -> 19.3), except matrices of up to 10 MB and super steps fewer than
+  // two a wavefront, launches that are mostly their start, and tiles of 8 .. 13 rows, whose vector work per byte is up to
+  // half as much again (5120 x 13824 at 4 rows 18.0 -> 19.0, 9472 x 3712 at 14 rows 11.6 -> 12.1).  int4, which has twice the vector work per byte, is level or behind.
+  // Matrices above 64 MB, a quarter of the last-level cache, in whole lines that are not kept: from memory int8 15360 x 5120 at
+  // 1 / 8 / 16 rows 16.0 / 17.7 / 19.7 -> 14.9 / 16.5 / 18.3, 76032 x 5120 at 3 rows 70 -> 63, int4 27648 x 5120 at 8 rows 19.2 -> 17.7,
+  // tile-major int8 15360 x 5120 at 8 rows 16.6 -> 15.5.  A smaller matrix may still be in that cache from its last use,
+  // which such requests give up (13184 x 2304 int8, three of them in turn: 7.9 -> 8.7 us).  Not int4 in rounds (152064 x 4096
+  // at 3 rows 76.2 -> 76.7).  With two requests to a line, a lane's own chunks, the second one misses: 15360 x 5120 21.7.
+  auto go = [&](auto xs, auto phases) -> int {
+    constexpr bool kForms = D == 2 && WAVES == 8 && !KSPLIT;
+    const int64_t bytes = p.n * p.k * BITS / 8;
+    if constexpr (kForms && !(ROUNDS && BITS == 4 && !TILED)) {
+      const bool narrow = plan.tile_rows < 14;
+      if (bytes > 64000000 && !narrow) return go_read(xs, phases, std::integral_constant<int, kReadOnce>{});
+      if constexpr (BITS == 8 && !TILED && !ROUNDS)
+        if (bytes > 10000000 && p.k >= 2048 && !narrow) return go_read(xs, phases, std::integral_constant<int, kReadPairs>{});
+    }
+    return go_read(xs, phases, std::integral_constant<int, kReadOwn>{});
   };
   using std::integral_constant;
   if constexpr (ROUNDS) {
@@ -1124,7 +1193,7 @@ bool choose_split(const Problem& p, int gs, SplitPlan* out) {
   // steps cost (rows + 4) / 20 of a 16-row one -- while its activations fit the LDS in one piece; the split's tiles
   // have 16 rows)
   const bool gated = p.activation == kActGated;
-  const int tr = (p.tiled || gated || (int64_t)p.m * p.k * 2 + 16384 > (int64_t)kLdsPerWgMax) ? 16 : pick_tile_rows(p.n, (int)cu, 0);
+  const int tr = (p.tiled || gated || (int64_t)p.m * p.k * 2 + 16384 > (int64_t)kLdsPerWgMax) ? 16 : pick_tile_rows(p.n, (int)cu, 0, 8);
   const int64_t tiles1 = (p.n + tr - 1) / tr;
   const int64_t path1 = ((tiles1 + std::min(tiles1, cu) - 1) / std::min(tiles1, cu)) * ((nsuper + kSplitWaves - 1) / kSplitWaves) * (tr + 4);
   int best = 1;
