@@ -408,6 +408,10 @@ int matmul_any_layout(const mi355x_wq_desc* desc, const void* x, const void* wq_
     const int rc = launch_gemv_split_static(p);
     if (rc != 0) return rc < 0 ? -1 : 0;
   }
+  if (m <= 16 && family == MI355X_WQ_KERNEL_AUTO) {
+    const int rc = launch_gemm_stream_decode(p);
+    if (rc != 0) return rc < 0 ? -1 : 0;
+  }
   // (tile-major weights: the same choice with crossovers of its own; the kernels that read the layout are the decode kernel,
   // the skinny kernel, the streamed GEMM and the direct-weight one, which needs K % 256 == 0)
   switch (family == MI355X_WQ_KERNEL_AUTO ? select_kernel(desc, m, tiled) : family) {

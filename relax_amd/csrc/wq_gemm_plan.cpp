@@ -202,4 +202,22 @@ GemmPlan plan_stream(const Problem& p, bool may_split) {
   return best;
 }
 
+// Up to 16 rows of canonical weights: where the streamed kernel's 32-row tiles, K split over workgroups, are ahead of the decode
+// kernel and the register-activation kernel.  Those have every CU walk all of K for its 16 columns, so each stages all of
+// the activations, in phases once they exceed the LDS; a split CU reads a part of them for more columns.  Lines by 840
+// timings (K 5120 - 13824, N 1024 - 16384, 4 - 16 rows, weights from memory; us, decode against streamed).  Row tiles of 16
+// between one and one and a quarter per CU, which divide worst: int8 5120 x 13824 at 6 / 16 rows 21.0 / 18.6 and 24.3 / 19.5,
+// 5120 x 8192 at 10 rows 14.5 / 13.6, int4 5120 x 11008 at 10 rows 17.3 / 14.3 (at 8: 13.6 / 14.3).  Up to one tile per CU: int8
+// 4096 x 11008 at 10 rows 18.2 / 15.0, 2048 x 13824 at 8 rows 15.4 / 12.3, int4 4096 x 13824 at 16 rows 16.3 / 14.4 (int8 4096 x
+// 8192 at 10 rows 11.5 / 13.7).  Up to two: int4 8192 x 11008 at 16 rows 20.2 / 18.5, int8 6144 x 13824 at 10 rows 24.6 / 23.3
+// (8192 x 9728 20.2 / 20.8).
+bool decode_streams(const Problem& p) {
+  if (p.m > 16 || p.tiled || p.k < 8192) return false;
+  const int64_t tiles = ceil_div(p.n, 16), cu = cu_count(), x = p.m * p.k;
+  if (tiles > cu && 4 * tiles <= 5 * cu) return x >= (p.bits == 8 ? 80000 : 96000);
+  if (tiles <= cu) return p.bits == 8 ? p.k >= 9728 && x >= 88000 : p.k >= 10752 && x >= 110000;
+  if (tiles <= 2 * cu) return p.bits == 8 ? p.k >= 13056 && x >= 138000 && 2 * tiles <= 3 * cu : p.k >= 10752 && x >= 110000;
+  return false;
+}
+
 }  // namespace wq

@@ -3,6 +3,7 @@
 
 #include <mutex>
 
+#include "../../include/mi355x_wq.h"
 #include "wq_internal.h"
 #include "wq_slots.h"
 
@@ -95,12 +96,12 @@ int64_t gemm_workspace_bytes(const Problem& p, bool skinny_family) {
   return plan.split > 1 && plan.us <= (skinny_family ? skinny_cost(p) : other_gemm_cost(p)) ? plan.bytes : 0;
 }
 
-int launch_gemm_stream_planned(const Problem& p, void* workspace, int64_t workspace_bytes, float other_us) {
-  if (!in_range(p)) return 0;
-  GemmPlan plan = plan_stream(p, p.m <= 256 || workspace != nullptr);
-  const bool slot = plan.split > 1 && plan.bytes > workspace_bytes;
-  if (slot && (p.m > 256 || capturing(p.stream))) plan = plan_stream(p, false);
-  if (other_us < plan.us) return 0;
+namespace {
+
+bool captured(const Problem& p) { return capturing(p.stream); }
+
+// `slot`: on a workspace of the library's
+int launch_plan(const Problem& p, const GemmPlan& plan, void* workspace, bool slot) {
   std::unique_lock<std::mutex> slot_lock;
   SplitSpace space{plan.split > 1 ? workspace : nullptr, nullptr, 0};
   if (plan.split > 1 && slot) space = plan.bytes <= kSlotBytes ? library_space(p.stream, plan.tiles, &slot_lock) : SplitSpace{};
@@ -111,6 +112,24 @@ int launch_gemm_stream_planned(const Problem& p, void* workspace, int64_t worksp
     return -1;
   }
   return 1;
+}
+
+}  // namespace
+
+int launch_gemm_stream_planned(const Problem& p, void* workspace, int64_t workspace_bytes, float other_us) {
+  if (!in_range(p)) return 0;
+  GemmPlan plan = plan_stream(p, p.m <= 256 || workspace != nullptr);
+  const bool slot = plan.split > 1 && plan.bytes > workspace_bytes;
+  if (slot && (p.m > 256 || captured(p))) plan = plan_stream(p, false);
+  if (other_us < plan.us) return 0;
+  return launch_plan(p, plan, workspace, slot);
+}
+
+int launch_gemm_stream_decode(const Problem& p) {
+  // (gelu onto its own residual stays with the kernels it is on)
+  if (!decode_streams(p) || !gemm_stream_applicable(p) || (p.activation == MI355X_WQ_ACT_GELU && p.residual == p.y)) return 0;
+  if (p.stream == hipStreamPerThread || captured(p)) return 0;
+  return launch_plan(p, plan_stream(p, true), nullptr, true);
 }
 
 }  // namespace wq

@@ -69,6 +69,10 @@ bool launch_gemm_stream(const Problem& p, int variant, int ksplit, const SplitSp
 template <int BITS>
 bool launch_gemm_stream_bits(const Problem& p, int variant, int ksplit, const SplitSpace& space);  // of that bit width
 int launch_gemm_stream_planned(const Problem& p, void* workspace, int64_t workspace_bytes, float other_us);
+// The same for up to 16 rows, where decode_streams says so; not under capture nor on hipStreamPerThread, where the library has no
+// workspace for it and the decode kernel is ahead of the unsplit form.
+int launch_gemm_stream_decode(const Problem& p);
+bool decode_streams(const Problem& p);
 // The workspace that a call of `p` from 17 rows on splits K on, 0 where it would not.
 int64_t gemm_workspace_bytes(const Problem& p, bool skinny_family);
 struct GemmPlan {

@@ -1,0 +1,66 @@
+"""Up to 16 rows on the streamed GEMM (long K on canonical weights): against the oracle on both sides of the rule's lines, with every
+tail, and where the call has to stay with the decode kernel -- under capture, on hipStreamPerThread, gelu in place."""
+import numpy as np
+import pytest
+
+from oracle import c_oracle, wq_oracle as O
+
+torch = pytest.importorskip("torch")
+pytestmark = pytest.mark.gpu
+
+from tests.test_gpu_parity import _dev, _fused_operands, assert_close  # noqa: E402
+
+# N at the edges of one tile of 16 per CU, of one and a quarter, of two; K and rows at the edges of the lines
+CASES = [(8, 6, 4097, 13824), (8, 5, 4112, 13824), (8, 10, 5120, 8192), (8, 16, 5121, 13824), (8, 16, 6145, 13824), (8, 9, 1000, 9856),
+         (8, 8, 4096, 11008), (4, 16, 4090, 11008), (4, 10, 4096, 11008), (4, 11, 8192, 10752), (4, 12, 8193, 10752), (4, 9, 4100, 11008)]
+
+
+@pytest.mark.parametrize("bits,m,n,k", CASES)
+def test_long_k_against_the_oracle(bits, m, n, k):
+    import relax_amd
+
+    x, wq, s, g = O.make_case(m + n, m, n, k, bits)
+    dx, dw, ds = _dev(x), _dev(wq), _dev(s)
+    bias, res = _fused_operands(m + n, m, n)
+    plain = relax_amd.wq_matmul(dx, dw, ds, bits, g).cpu().numpy()
+    rows = [0, m // 2, m - 1]
+    assert_close(plain[rows], c_oracle.wq_matmul(x[rows], wq, s, bits, g, nthreads=8), (bits, m, n, k), ulp_fraction=0.005)
+    again = relax_amd.wq_matmul(dx, dw, ds, bits, g).cpu().numpy()
+    assert np.array_equal(again.view(np.uint16), plain.view(np.uint16))
+    for tail in (dict(bias=bias, activation="relu", residual=res), dict(bias=bias, activation="gelu"), dict(residual=res)):
+        got = relax_amd.wq_matmul(dx, dw, ds, bits, g, **{a: _dev(b) if isinstance(b, np.ndarray) else b for a, b in tail.items()})
+        want = O.epilogue(plain, **tail)
+        assert (got.cpu().numpy().view(np.uint16) != want.view(np.uint16)).sum() <= (want.size // 1000 if tail.get("activation") == "gelu" else 0)
+
+
+def test_calls_that_stay_with_the_decode_kernel():
+    """They agree with the kernel family they name; a captured call replays to the same result."""
+    import relax_amd
+    from relax_amd import lib
+
+    bits, m, n, k = 8, 16, 5120, 13824
+    x, wq, s, g = O.make_case(5, m, n, k, bits)
+    dx, dw, ds = _dev(x), _dev(wq), _dev(s)
+    decode = relax_amd.wq_matmul(dx, dw, ds, bits, g, kernel=lib.KERNEL_GEMV)
+
+    class PerThread:
+        cuda_stream = 2
+
+    torch.cuda.synchronize()
+    per_thread = relax_amd.wq_matmul(dx, dw, ds, bits, g, stream=PerThread)
+    torch.cuda.synchronize()
+    assert torch.equal(per_thread.view(torch.int16), decode.view(torch.int16))
+    out, graph = torch.empty_like(decode), torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        relax_amd.wq_matmul(dx, dw, ds, bits, g, out=out)
+    for _ in range(3):
+        out.zero_()
+        graph.replay()
+        relax_amd.wq_matmul(dx, dw, ds, bits, g)
+        torch.cuda.synchronize()
+        assert torch.equal(out.view(torch.int16), decode.view(torch.int16))
+    res = _dev(_fused_operands(1, m, n)[1])
+    y = res.clone()
+    relax_amd.wq_matmul(dx, dw, ds, bits, g, activation="gelu", residual=y, out=y)
+    want = relax_amd.wq_matmul(dx, dw, ds, bits, g, activation="gelu", residual=res, kernel=lib.KERNEL_GEMV)
+    assert torch.equal(y.view(torch.int16), want.view(torch.int16))
