@@ -21,7 +21,12 @@ void set_error(const char* fmt, ...) {
   va_end(ap);
 }
 
+namespace {
+thread_local int call_device = -1;  // slot of the device of the call that this thread is in
+}
+
 int current_device_slot() {
+  if (call_device >= 0) return call_device;
   int dev = 0;
   if (hipGetDevice(&dev) != hipSuccess) {
     (void)hipGetLastError();
@@ -29,6 +34,15 @@ int current_device_slot() {
   }
   return dev >= 0 && dev < kMaxDevices ? dev : kMaxDevices - 1;
 }
+
+namespace {
+// For the length of a call the device is asked once: a plan and a launch need it ten times over, 0.05 us each.
+struct DeviceOfCall {
+  DeviceOfCall() : outer(call_device) { call_device = current_device_slot(); }
+  ~DeviceOfCall() { call_device = outer; }
+  int outer;
+};
+}  // namespace
 
 bool ensure_dynamic_lds(const void* kernel, int bytes, std::atomic<bool>* done) {
   const int slot = current_device_slot();
@@ -366,6 +380,7 @@ int matmul_any_layout(const mi355x_wq_desc* desc, const void* x, const void* wq_
     return -1;
   if (ep != nullptr && ep->bias != nullptr && !check_ptr(ep->bias, "bias", 2)) return -1;
   if (ep != nullptr && ep->residual != nullptr && !check_ptr(ep->residual, "residual", 2)) return -1;
+  const DeviceOfCall device;
   const int family = kernel & 0xFF, variant = (kernel >> 8) & 0xFFFF;
   Problem p{x, wq_, scales, y, m, desc->n, desc->k, desc->bits, desc->group, desc->zero_point,
             static_cast<hipStream_t>(stream)};

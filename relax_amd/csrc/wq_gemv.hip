@@ -763,15 +763,17 @@ struct Plan {
 // workspaces are sized.)
 inline int pick_tile_rows(int64_t n, int cap, int forced, int margin = 10) {
   if (forced >= 8 && forced <= 16) return forced;
-  auto cost = [&](int tr) {
-    const int64_t tiles = (n + tr - 1) / tr, grid = std::min<int64_t>(tiles, cap);
+  const uint32_t rows = (uint32_t)n, cus = (uint32_t)cap;
+  auto cost = [&](uint32_t tr) {
+    const uint32_t tiles = (rows + tr - 1) / tr, grid = std::min(tiles, cus);
     return ((tiles + grid - 1) / grid) * (tr + 4);
   };
   int best = 16;
-  int64_t best_cost = cost(16);
-  for (int tr = 15; tr >= 8; --tr)
-    if (cost(tr) < best_cost) best = tr, best_cost = cost(tr);
-  return best_cost * margin <= cost(16) * (margin - 1) ? best : 16;
+  uint32_t best_cost = cost(16);
+#pragma unroll
+  for (uint32_t tr = 15; tr >= 8; --tr)
+    if (const uint32_t c = cost(tr); c < best_cost) best = (int)tr, best_cost = c;
+  return best_cost * (uint32_t)margin <= cost(16) * (uint32_t)(margin - 1) ? best : 16;
 }
 
 // Chooses the grid (workgroups per CU), the tiles per workgroup and the K phase so
@@ -1092,7 +1094,8 @@ int launch_gemv(const Problem& p, int variant) {
     return -1;
   }
   int ok = kNotApplicable;
-  if (variant == 0 && gemv_applicable(p) && use_rounds_any(p)) {
+  // (rounds: from 12 tiles per CU on, or slots beyond the LDS, which are more than that)
+  if (variant == 0 && p.n > (int64_t)cu_count() * 16 * 8 && gemv_applicable(p) && use_rounds_any(p)) {
     ok = p.bits == 4 ? try_rounds<4>(p, gs, 1) : try_rounds<8>(p, gs, 1);
   } else if (variant == 0) {
     const int* order = default_order(p);
