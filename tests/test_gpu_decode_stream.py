@@ -1,5 +1,9 @@
 """Up to 16 rows on the streamed GEMM (long K on canonical weights): against the oracle on both sides of the rule's lines, with every
 tail, and where the call has to stay with the decode kernel -- under capture, on hipStreamPerThread, gelu in place."""
+import os
+import subprocess
+import sys
+
 import numpy as np
 import pytest
 
@@ -64,3 +68,33 @@ def test_calls_that_stay_with_the_decode_kernel():
     relax_amd.wq_matmul(dx, dw, ds, bits, g, activation="gelu", residual=y, out=y)
     want = relax_amd.wq_matmul(dx, dw, ds, bits, g, activation="gelu", residual=res, kernel=lib.KERNEL_GEMV)
     assert torch.equal(y.view(torch.int16), want.view(torch.int16))
+
+
+FIRST_LAUNCH_UNDER_CAPTURE = """
+import torch, relax_amd
+from relax_amd import lib
+from oracle import wq_oracle as O
+import numpy as np
+x, wq, s, g = O.make_case(5, 16, 5120, 13824, 8)
+dx, dw, ds = (torch.from_numpy(a.view(np.int32) if a.dtype == np.uint32 else a).cuda() for a in (x, wq, s))
+relax_amd.wq_matmul(dx, dw, ds, 8, g)
+torch.cuda.synchronize()
+out, graph = torch.empty((16, 5120), dtype=torch.float16, device="cuda"), torch.cuda.CUDAGraph()
+with torch.cuda.graph(graph):
+    relax_amd.wq_matmul(dx, dw, ds, 8, g, out=out)
+for _ in range(3):
+    out.zero_()
+    graph.replay()
+    torch.cuda.synchronize()
+    got = out.clone()
+    want = relax_amd.wq_matmul(dx, dw, ds, 8, g, kernel=lib.KERNEL_GEMV)
+    assert torch.equal(got.view(torch.int16), want.view(torch.int16))
+"""
+
+
+def test_one_eager_call_is_enough_before_a_capture():
+    """The eager call launches the streamed kernel, the captured one the decode kernel: its first launch in the process is the captured
+    one, so this needs a process of its own."""
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    r = subprocess.run([sys.executable, "-c", FIRST_LAUNCH_UNDER_CAPTURE], cwd=root, capture_output=True, text=True, timeout=100)
+    assert r.returncode == 0, r.stderr[-2000:]
