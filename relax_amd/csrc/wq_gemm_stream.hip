@@ -623,6 +623,12 @@ __global__ __launch_bounds__((CW * G + PROD) * 64, 1) void wq_gemm_stream_kernel
     const int r = row_in_tile(p, e);
     return r < rows && c != kStreamOob ? base + (uint32_t)(r - row_in_tile(0, 0)) * pitch + c : kStreamOob;
   };
+  // of row quad p, row e of the pairs.  (A column beyond N: kStreamOob and less than 2^31 on top stays out of range, so that
+  // only the row is compared.)
+  auto pair_offset = [&](int p, int e) __attribute__((always_inline)) {
+    const int r = row_in_tile(p, e);
+    return r < rows ? base + col + (uint32_t)(r - row_in_tile(0, 0)) * pitch : kStreamOob;
+  };
   auto tail = [&](half2_t (&h)[PC][4], half2_t b2) __attribute__((always_inline)) {
     if (ep.bias != nullptr) {
 #pragma unroll
@@ -659,7 +665,7 @@ __global__ __launch_bounds__((CW * G + PROD) * 64, 1) void wq_gemm_stream_kernel
 #pragma unroll
         for (int p = 0; p < PC; ++p)
 #pragma unroll
-          for (int e = 0; e < 4; ++e) res[p][e] = load_b32(rr, offset(p0 + p, e, col));
+          for (int e = 0; e < 4; ++e) res[p][e] = load_b32(rr, pair_offset(p0 + p, e));
 #pragma unroll
         for (int p = 0; p < PC; ++p)
 #pragma unroll
@@ -668,7 +674,7 @@ __global__ __launch_bounds__((CW * G + PROD) * 64, 1) void wq_gemm_stream_kernel
 #pragma unroll
       for (int p = 0; p < PC; ++p)
 #pragma unroll
-        for (int e = 0; e < 4; ++e) __builtin_amdgcn_raw_buffer_store_b32(as_u32(h[p][e]), ry, offset(p0 + p, e, col), 0, 0);
+        for (int e = 0; e < 4; ++e) __builtin_amdgcn_raw_buffer_store_b32(as_u32(h[p][e]), ry, pair_offset(p0 + p, e), 0, 0);
       __builtin_amdgcn_sched_barrier(0);
     });
     return;
