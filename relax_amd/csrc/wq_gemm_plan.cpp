@@ -220,4 +220,28 @@ bool decode_streams(const Problem& p) {
   return false;
 }
 
+// How the decode kernel reads its weights, by 23,000 timings (M 1 - 16, K 1536 - 14336, 4 - 256 MB, all group sizes and both layouts; means over
+// a class of problems against a lane's own chunks, "from memory" through 0.9 GB of matrices and "kept" where one or two stay in the
+// 256 MB last-level cache).
+//
+// Canonical int8 by pairs of lanes, whose requests cover whole lines: 10 - 20 MB from memory 0.92 - 0.97, above level, kept 0.96 - 1.0
+// (12288 x 4096 at 2 rows 11.0 -> 9.9 us).  Not matrices of up to 10 MB and super steps fewer than two a wavefront, launches that are
+// mostly their start, nor tiles of 8 .. 13 rows, whose vector work per byte is up to half as much again (5120 x 13824 at 4 rows
+// 18.0 -> 19.0, 9472 x 3712 at 14 rows 11.6 -> 12.1).  int4, which has twice the vector work per byte, is level or behind.
+//
+// Whole lines that are not kept, int8 above a quarter of that cache: canonical from memory 0.92 - 0.95 (15360 x 5120 at 1 / 8 / 16 rows
+// 15.8 / 17.7 / 19.9 -> 14.8 / 16.5 / 18.6, pairs 15.6 / 17.5 / 19.2), kept 0.98 - 1.03 up to 10 rows and 1.0 - 1.05 at 12 and 16 (the
+// same matrix 13.8 / 15.6 / 17.3 -> 14.4 / 16.0 / 18.0, pairs 13.3 / 15.1 / 16.7); tile-major from memory 0.91 - 0.94, kept 0.96 - 1.06.
+// The line stands for weights that come from memory: a matrix of 64 MB is found in the cache only by a program whose whole working set
+// is below 256 MB.  int4 above a third: tile-major from memory 0.93 - 0.98, kept 1.0 - 1.04; canonical, which pays for the swap of the pairs, at
+// 1 - 2 rows only -- from memory 0.92 - 0.97 (33792 x 5120 at 1 row 21.3 -> 19.1), kept 1.05 -- and not from 3 rows on: from memory 1.01 - 1.05
+// (33792 x 5120 at 16 rows 27.7 -> 28.9), kept 1.08 - 1.11 (25.1 -> 28.8).  Nor canonical int4 in rounds (152064 x 4096 at 3 rows 76.2 -> 76.7).
+int weight_reads(const Problem& p, int tile_rows, bool rounds) {
+  const int64_t bytes = p.n * p.k * p.bits / 8;
+  if (tile_rows < 14) return kReadOwn;
+  if (p.bits == 4) return bytes > 85000000 && (p.tiled || (p.m <= 2 && !rounds)) ? kReadOnce : kReadOwn;
+  if (bytes > 64000000) return kReadOnce;
+  return !p.tiled && !rounds && bytes > 10000000 && p.k >= 2048 ? kReadPairs : kReadOwn;
+}
+
 }  // namespace wq

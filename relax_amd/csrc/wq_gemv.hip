@@ -121,9 +121,8 @@ struct GemvKernArgs {
   unsigned int* counters;
 };
 
-// READ: a lane's weights by requests of its own chunks; canonical weights by pairs of lanes, so that a request covers whole lines;
-// and whole lines (tile-major ones always are) by non-temporal requests.
-enum { kReadOwn, kReadPairs, kReadOnce };
+// READ (wq_internal.h): a lane's weights by requests of its own chunks; canonical weights by pairs of lanes, so that a request covers
+// whole lines; and whole lines (tile-major ones always are) by non-temporal requests.
 
 // ROUNDS: a workgroup has more tiles than its LDS has slots for.  The tiles are walked in rounds of half the slots (an even
 // number, so that a round ends with a trip of the stream); after a round one barrier, and the round's tiles are summed
@@ -888,24 +887,15 @@ int launch_one(const Problem& p, int group_shift, const Plan& plan, int ksplit =
                        partials, counters);
     return kLaunched;
   };
-  // How the weights are read (the kernel's READ).  Canonical int8 by pairs of lanes, whose requests cover whole lines (12288 x 4096
-  // at 2 rows 11.0 -> 9.9 us, 15360 x 5120 at 16 rows 19.8 -> 19.3), except matrices of up to 10 MB and super steps fewer than
-  // two a wavefront, launches that are mostly their start, and tiles of 8 .. 13 rows, whose vector work per byte is up to
-  // half as much again (5120 x 13824 at 4 rows 18.0 -> 19.0, 9472 x 3712 at 14 rows 11.6 -> 12.1).  int4, which has twice the vector work per byte, is level or behind.
-  // Matrices above a quarter (int4: a third) of the 256 MB last-level cache in whole lines that are not kept: from memory int8 15360 x 5120 at
-  // 1 / 8 / 16 rows 16.0 / 17.7 / 19.7 -> 14.9 / 16.5 / 18.3, 76032 x 5120 at 3 rows 70 -> 63, int4 27648 x 5120 at 8 rows 19.2 -> 17.7,
-  // tile-major int8 15360 x 5120 at 8 rows 16.6 -> 15.5.  A smaller matrix may still be in that cache from its last use,
-  // which such requests give up (three of a kind in turn: int8 13184 x 2304 7.9 -> 8.7 us, 15360 x
-  // 5120 15.7 -> 16.1, int4 11904 x 12032 19.7 -> 23.1).  Not int4 in rounds (152064 x 4096
-  // at 3 rows 76.2 -> 76.7).  With two requests to a line, a lane's own chunks, the second one misses: 15360 x 5120 21.7.
+  // how the weights are read (the kernel's READ; the rule is weight_reads): the builds that it can choose
   auto go = [&](auto xs, auto phases) -> int {
     constexpr bool kForms = D == 2 && WAVES == 8 && !KSPLIT;
-    const int64_t bytes = p.n * p.k * BITS / 8;
-    if constexpr (kForms && !(ROUNDS && BITS == 4 && !TILED)) {
-      const bool narrow = plan.tile_rows < 14;
-      if (bytes > (BITS == 4 ? 85000000 : 64000000) && !narrow) return go_read(xs, phases, std::integral_constant<int, kReadOnce>{});
+    // (canonical int4 from 3 rows on, staged by columns, and in rounds: own chunks only)
+    if constexpr (kForms && !(BITS == 4 && !TILED && (ROUNDS || decltype(xs)::value >= 4))) {
+      const int read = weight_reads(p, plan.tile_rows, ROUNDS);
+      if (read == kReadOnce) return go_read(xs, phases, std::integral_constant<int, kReadOnce>{});
       if constexpr (BITS == 8 && !TILED && !ROUNDS)
-        if (bytes > 10000000 && p.k >= 2048 && !narrow) return go_read(xs, phases, std::integral_constant<int, kReadPairs>{});
+        if (read == kReadPairs) return go_read(xs, phases, std::integral_constant<int, kReadPairs>{});
     }
     return go_read(xs, phases, std::integral_constant<int, kReadOwn>{});
   };

@@ -33,6 +33,10 @@ constexpr int64_t kSplitCounterBytes = kSplitMaxTiles * 4;
 // Tuning variant: 0 = library default for the shape, >0 = explicit choice
 // (only reachable through mi355x_wq_matmul_ex; used by sweeps).
 int launch_gemv(const Problem& p, int variant);
+// How the decode kernel requests its weights: a lane its own chunks, pairs of lanes whole lines, whole lines non-temporally; and which
+// of them its default shape (eight wavefronts, two-chunk super steps) takes on tiles of so many rows, in rounds or not.
+enum { kReadOwn, kReadPairs, kReadOnce };
+int weight_reads(const Problem& p, int tile_rows, bool rounds);
 bool gemv_applicable(const Problem& p);  // M <= 16 and a default variant's LDS plan (slots + activations) fits
 // The decode kernel with its tiles in rounds, where the default takes that: 1 launched, 0 not its problem, -1 failure.
 int launch_gemv_rounds(const Problem& p);
