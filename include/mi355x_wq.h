@@ -74,8 +74,9 @@ enum {
  * capture uses none of the library's memory and, without a workspace of the caller's (mi355x_wq_matmul_ws), runs
  * unsplit: its float32 sums are added in another order than the eager call's, the same in every replay.
  * Up to 16 rows the same holds for canonical weights with long K (from 8192 on) and few row tiles per CU, where such a
- * split is ahead of the decode kernel; under capture and on hipStreamPerThread these run the decode kernel,
- * whose sums are in another order too. */
+ * split is ahead of the decode kernel: these calls have 24 workspaces of 4 MB of their own (96 MB more of each GPU, 24 KB of
+ * pinned host memory at the first call), and one that finds none, on a 25th busy stream, takes two to three times as
+ * long; under capture and on hipStreamPerThread these run the decode kernel, whose sums are in another order too. */
 MI355X_WQ_API int mi355x_wq_matmul(const mi355x_wq_desc* desc, const void* x, const void* wq, const void* scales,
                      void* y, int64_t m, void* stream);
 

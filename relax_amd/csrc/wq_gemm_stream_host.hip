@@ -24,9 +24,9 @@ namespace {
 // Workspaces of the library's own for calls of up to 256 rows that bring none (more rows fill the chip without a split).
 // The memory is part of the code object (zero at load, as the counters have to be).  A call that finds
 // no slot runs its windows one after the other, with the same result (kSerial in wq_gemm_stream.hip).
-constexpr int kSlots = 8;
 constexpr int64_t kSlotBytes = kSplitCounterBytes + (20ll << 20);  // (the largest plan: 288 windows of 128 x 128 float32)
 __device__ unsigned char stream_slots[kSlots][kSlotBytes];
+__device__ unsigned char decode_slots[kDecodeSlots][kDecodeSplitBytes];
 
 // Under capture nothing of the library's is used: a graph may be replayed beside anything.
 bool capturing(hipStream_t s) {
@@ -36,48 +36,57 @@ bool capturing(hipStream_t s) {
   return true;
 }
 
+template <int SLOTS, int64_t BYTES>
 struct Slots {
   std::mutex mutex;
-  SlotOwners<kSlots> owners;
+  SlotOwners<SLOTS> owners;
   char* base = nullptr;
-  uint32_t* done = nullptr;  // [kSlots][kSlotTiles], host memory that the kernels write
+  uint32_t* done = nullptr;  // [SLOTS][kSlotTiles], host memory that the kernels write
 };
 
-// The memory of a device's slots: the workspaces and, at the first call that needs one, 8 KB of pinned host memory.
-bool find_memory(Slots* o) {
+// The memory of a device's slots: the workspaces and, at the first call that needs one, 1 KB of pinned host memory for each.
+template <int SLOTS, int64_t BYTES>
+bool find_memory(Slots<SLOTS, BYTES>* o, const void* symbol) {
   if (o->done != nullptr) return true;
   void* base = nullptr;
   void* done = nullptr;
   // (another thread may be capturing, which an allocation must not end)
   hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
   const bool relaxed = hipThreadExchangeStreamCaptureMode(&mode) == hipSuccess;
-  const bool ok = relaxed && hipGetSymbolAddress(&base, HIP_SYMBOL(stream_slots)) == hipSuccess &&
-                  hipHostMalloc(&done, sizeof(uint32_t) * kSlots * kSlotTiles, hipHostMallocPortable | hipHostMallocMapped | hipHostMallocCoherent) == hipSuccess;
+  const bool ok = relaxed && hipGetSymbolAddress(&base, symbol) == hipSuccess &&
+                  hipHostMalloc(&done, sizeof(uint32_t) * SLOTS * kSlotTiles, hipHostMallocPortable | hipHostMallocMapped | hipHostMallocCoherent) == hipSuccess;
   if (relaxed) (void)hipThreadExchangeStreamCaptureMode(&mode);
   if (!ok) {
     (void)hipGetLastError();
     return false;
   }
-  memset(done, 0, sizeof(uint32_t) * kSlots * kSlotTiles);
+  memset(done, 0, sizeof(uint32_t) * SLOTS * kSlotTiles);
   o->base = static_cast<char*>(base);
   o->done = static_cast<uint32_t*>(done);
   return true;
 }
 
-// A workspace for one launch of `tiles` tiles on `s`; empty where there is none.  The caller passes `lock` in and keeps it until
-// its launch is in the stream: another thread's launch on the same stream must not come between the two.
-SplitSpace library_space(hipStream_t s, int64_t tiles, std::unique_lock<std::mutex>* lock) {
-  if (s == hipStreamPerThread || tiles > kSlotTiles) return {};  // (one handle for a stream in every thread)
-  static Slots slots[kMaxDevices];
-  Slots& o = slots[current_device_slot()];
-  *lock = std::unique_lock<std::mutex>(o.mutex);
-  if (!find_memory(&o)) return {};
-  Slot* const slot = o.owners.take(s);
+template <int SLOTS, int64_t BYTES>
+SplitSpace take_slot(Slots<SLOTS, BYTES>* o, const void* symbol, hipStream_t s, const GemmPlan& plan, std::unique_lock<std::mutex>* lock) {
+  if (plan.bytes > BYTES) return {};
+  *lock = std::unique_lock<std::mutex>(o->mutex);
+  if (!find_memory(o, symbol)) return {};
+  Slot* const slot = o->owners.take(s);
   if (slot == nullptr) return {};
-  const int64_t i = slot - o.owners.slot;
-  slot->done = o.done + i * kSlotTiles;
-  slot->tiles = (int)tiles;
-  return SplitSpace{o.base + i * kSlotBytes, o.done + i * kSlotTiles, ++slot->launch};
+  const int64_t i = slot - o->owners.slot;
+  slot->done = o->done + i * kSlotTiles;
+  slot->tiles = (int)plan.tiles;
+  return SplitSpace{o->base + i * BYTES, o->done + i * kSlotTiles, ++slot->launch};
+}
+
+// A workspace for one launch of a plan on `s`; empty where there is none.  The caller passes `lock` in and keeps it until
+// its launch is in the stream: another thread's launch on the same stream must not come between the two.
+SplitSpace library_space(hipStream_t s, const GemmPlan& plan, bool decode, std::unique_lock<std::mutex>* lock) {
+  if (s == hipStreamPerThread || plan.tiles > kSlotTiles) return {};  // (one handle for a stream in every thread)
+  static Slots<kSlots, kSlotBytes> slots[kMaxDevices];
+  static Slots<kDecodeSlots, kDecodeSplitBytes> small[kMaxDevices];
+  const int device = current_device_slot();
+  return decode ? take_slot(&small[device], HIP_SYMBOL(decode_slots), s, plan, lock) : take_slot(&slots[device], HIP_SYMBOL(stream_slots), s, plan, lock);
 }
 
 }  // namespace
@@ -104,7 +113,7 @@ bool captured(const Problem& p) { return capturing(p.stream); }
 int launch_plan(const Problem& p, const GemmPlan& plan, void* workspace, bool slot) {
   std::unique_lock<std::mutex> slot_lock;
   SplitSpace space{plan.split > 1 ? workspace : nullptr, nullptr, 0};
-  if (plan.split > 1 && slot) space = plan.bytes <= kSlotBytes ? library_space(p.stream, plan.tiles, &slot_lock) : SplitSpace{};
+  if (plan.split > 1 && slot) space = library_space(p.stream, plan, p.m <= 16, &slot_lock);
   if (!launch_gemm_stream(p, plan.variant, plan.split, space)) return -1;
   const hipError_t e = hipGetLastError();
   if (e != hipSuccess) {
@@ -129,7 +138,8 @@ int launch_gemm_stream_decode(const Problem& p) {
   // (gelu onto its own residual stays with the kernels it is on)
   if (!decode_streams(p) || !gemm_stream_applicable(p) || (p.activation == MI355X_WQ_ACT_GELU && p.residual == p.y)) return 0;
   if (p.stream == hipStreamPerThread || captured(p)) return 0;
-  return launch_plan(p, plan_stream(p, true), nullptr, true);
+  const GemmPlan plan = plan_stream(p, true);
+  return plan.bytes <= kDecodeSplitBytes ? launch_plan(p, plan, nullptr, true) : 0;
 }
 
 }  // namespace wq

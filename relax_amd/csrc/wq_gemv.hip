@@ -1277,11 +1277,11 @@ int launch_gemv_split(const Problem& p, void* workspace, int64_t workspace_bytes
 // object is loaded) and every launch returns its counters to zero, so consecutive calls need no
 // clearing; partial tiles are written before they are read.  All calls on one GPU share the array:
 // calls that overlap in time on one GPU (different streams, different threads) race.
-static __device__ __align__(256) unsigned char scratch[kSplitCounterBytes + 4 * 1024 * 1024];
+static __device__ __align__(256) unsigned char scratch[kDecodeSplitBytes];
 
 namespace {
 
-constexpr int64_t kStaticScratchBytes = kSplitCounterBytes + 4 * 1024 * 1024;
+constexpr int64_t kStaticScratchBytes = kDecodeSplitBytes;
 std::atomic<void*> g_scratch_ptr[kMaxDevices];
 
 // Device address of the current device's copy of `scratch`, or nullptr with the error set.

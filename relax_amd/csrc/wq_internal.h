@@ -29,6 +29,8 @@ struct Problem {
 // decode kernel: N <= 65536).
 constexpr int64_t kSplitMaxTiles = 4096;
 constexpr int64_t kSplitCounterBytes = kSplitMaxTiles * 4;
+// Counters and partial tiles of a call of up to 16 rows on memory of the library's.
+constexpr int64_t kDecodeSplitBytes = kSplitCounterBytes + 4 * 1024 * 1024;
 
 // Tuning variant: 0 = library default for the shape, >0 = explicit choice
 // (only reachable through mi355x_wq_matmul_ex; used by sweeps).

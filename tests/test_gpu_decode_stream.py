@@ -70,6 +70,24 @@ def test_calls_that_stay_with_the_decode_kernel():
     assert torch.equal(y.view(torch.int16), want.view(torch.int16))
 
 
+@pytest.mark.parametrize("streams", [9, 24, 30])
+def test_as_many_streams_as_slots_and_more(streams):
+    """Calls in flight on every stream at once: the bits of a call that is alone, which are the streamed kernel's, on all of them."""
+    import relax_amd
+    from relax_amd import lib
+
+    x, wq, s, g = O.make_case(6, 16, 1000, 9856, 8)
+    dx, dw, ds = _dev(x), _dev(wq), _dev(s)
+    alone = relax_amd.wq_matmul(dx, dw, ds, 8, g)
+    decode = relax_amd.wq_matmul(dx, dw, ds, 8, g, kernel=lib.KERNEL_GEMV)
+    assert not torch.equal(alone.view(torch.int16), decode.view(torch.int16)), "the case is meant to be one of the streamed kernel's"
+    handles = [torch.cuda.Stream() for _ in range(streams)]
+    torch.cuda.synchronize()
+    outs = [relax_amd.wq_matmul(dx, dw, ds, 8, g, stream=h, out=torch.empty_like(alone)) for _ in range(4) for h in handles]
+    torch.cuda.synchronize()
+    assert all(torch.equal(o.view(torch.int16), alone.view(torch.int16)) for o in outs)
+
+
 FIRST_LAUNCH_UNDER_CAPTURE = """
 import torch, relax_amd
 from relax_amd import lib

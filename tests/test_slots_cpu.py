@@ -54,6 +54,16 @@ int main() {
   CHECK(i == 0 && o.slot[0].launch == 0 && !o.slot[0].idle());
   finish(0, 0, 3);
   CHECK(o.slot[0].idle());
+  // calls of up to 16 rows: more streams than slots for larger calls, each busy, each with a slot
+  static SlotOwners<kDecodeSlots> decode;
+  static uint32_t never[kSlotTiles];
+  static_assert(kDecodeSlots >= 3 * kSlots, "as many as a program has streams");
+  for (long s = 0; s < kDecodeSlots; ++s) {
+    Slot* const slot = decode.take(at(1000 + s));
+    CHECK(slot == &decode.slot[s]);
+    slot->done = never, slot->launch = 1, slot->tiles = 80;
+  }
+  CHECK(decode.take(at(5000)) == nullptr);
   std::printf("ok\\n");
   return 0;
 }
