@@ -184,13 +184,16 @@ MI355X_WQ_API int mi355x_wq_matmul_tiled_ex(const mi355x_wq_desc* desc, const vo
  * whole rounds (5120 rows: 320 tiles on 256 CUs) or whose activations are large against one tile per CU,
  * the decode kernel splits K over two to four workgroups per tile; each writes a float32 partial tile
  * to the workspace, and the last to arrive adds them in the order of their K windows (the result does
- * not depend on the order of arrival), applies the epilogue and stores.  5120 x 13824 int8: 22 -> 20 us
- * at batch 1, 31 -> 23 us at 16 rows.  The reference's counterpart is CUTLASS split-K, whose workspace the generated host code
+ * not depend on the order of arrival), applies the epilogue and stores.  4096 x 11008 int8: 17.4 -> 13.8 us at 8 rows.
+ * Canonical weights with long K that this does not split and a call without a workspace splits for the streamed GEMM
+ * (mi355x_wq_matmul) are split so here as well, on the workspace and with the same bits, captured or not.  Where a call could have either,
+ * the workspace is the decode kernel's: int8 from half a row tile per CU to one and a quarter is up to a tenth faster without one
+ * (5120 x 13312 at 16 rows 21.1 us against 19.4), except under capture, where the call without runs unsplit (23.4).  The reference's counterpart is CUTLASS split-K, whose workspace the generated host code
  * allocates per call (python/tvm/contrib/cutlass/build.py:335, conv2d_operation.py:417-418); here the
  * caller owns it, so that nothing is allocated under a stream capture or in a serving loop.
  *
  * mi355x_wq_workspace_bytes: the size mi355x_wq_matmul_ws needs to split K for (desc, m, layout), whatever the tail --
- * 16 KB of arrival counters at the head, then a float32 partial tile per tile and K window (1 KB up to 16 rows), so one
+ * 16 KB of arrival counters at the head, then a float32 partial tile per tile and K window (1 KB in the decode kernel), so one
  * workspace sized for the largest projection serves projections of every shape; 0 if no tail's call would split on it
  * (then the call equals mi355x_wq_matmul_fused / _tiled and leaves the workspace alone), -1 on an invalid descriptor.
  *

@@ -216,7 +216,7 @@ int64_t call_workspace_bytes(const mi355x_wq_desc* d, int64_t m, bool tiled, int
   p.activation = activation;
   p.residual = residual ? d : nullptr;  // (whether, not where)
   const bool gated = activation == MI355X_WQ_ACT_SILU_MUL;
-  if (m <= 16) return gated ? 0 : gemv_split_workspace_bytes(p);
+  if (m <= 16) return gated ? 0 : decode_workspace_bytes(p);
   return gemm_workspace_bytes(p, !gated && select_kernel(d, m, tiled) == MI355X_WQ_KERNEL_SKINNY);
 }
 
@@ -414,17 +414,26 @@ int matmul_any_layout(const mi355x_wq_desc* desc, const void* x, const void* wq_
     const bool decode = family == MI355X_WQ_KERNEL_GEMV || (family == MI355X_WQ_KERNEL_AUTO && m <= 16 && gemv_applicable(p));
     return decode ? launch_gemv(p, variant) : launch_gemm(p, variant, workspace, workspace_bytes);
   }
-  if (workspace != nullptr && m <= 16) {
-    const int rc = launch_gemv_split(p, workspace, workspace_bytes);
-    if (rc != 0) return rc < 0 ? -1 : 0;
-  }
-  if (library_scratch) {
-    // the same split on the library's own device array: nothing is allocated, sizes beyond it are refused
-    const int rc = launch_gemv_split_static(p);
-    if (rc != 0) return rc < 0 ? -1 : 0;
-  }
   if (m <= 16 && family == MI355X_WQ_KERNEL_AUTO) {
-    const int rc = launch_gemm_stream_decode(p);
+    // K split over workgroups, by the decode kernel or the streamed one: on the caller's workspace, on the library's scratch array
+    // (nothing is allocated, sizes beyond it are refused), and without either by the latter alone on a slot
+    void* space = workspace;
+    int64_t space_bytes = workspace_bytes;
+    if (library_scratch) {
+      const int64_t need = decode_workspace_bytes(p);
+      space_bytes = need > 0 ? gemv_static_scratch_bytes() : 0;
+      if (need > space_bytes) {
+        set_error("the K split of this problem needs %lld bytes of scratch memory, the library's own array holds %lld: "
+                  "use mi355x_wq_matmul_ws with a caller workspace", (long long)need, (long long)space_bytes);
+        return -1;
+      }
+      space = need > 0 ? static_scratch_address() : nullptr;
+      if (need > 0 && space == nullptr) return -1;
+    }
+    int rc = 0;
+    if (space != nullptr) rc = launch_gemv_split(p, space, space_bytes);
+    if (space != nullptr && rc == 0) rc = launch_gemm_stream_decode(p, space, space_bytes);
+    if (rc == 0 && !library_scratch) rc = launch_gemm_stream_decode(p, nullptr, 0);
     if (rc != 0) return rc < 0 ? -1 : 0;
   }
   // (tile-major weights: the same choice with crossovers of its own; the kernels that read the layout are the decode kernel,

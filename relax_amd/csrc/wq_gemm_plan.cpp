@@ -212,12 +212,24 @@ GemmPlan plan_stream(const Problem& p, bool may_split) {
 // 8192 at 10 rows 11.5 / 13.7).  Up to two: int4 8192 x 11008 at 16 rows 20.2 / 18.5, int8 6144 x 13824 at 10 rows 24.6 / 23.3
 // (8192 x 9728 20.2 / 20.8).
 bool decode_streams(const Problem& p) {
-  if (p.m > 16 || p.tiled || p.k < 8192) return false;
+  if (p.m > 16 || p.tiled || p.k < 8192 || p.group < 32) return false;
   const int64_t tiles = ceil_div(p.n, 16), cu = cu_count(), x = p.m * p.k;
   if (tiles > cu && 4 * tiles <= 5 * cu) return x >= (p.bits == 8 ? 80000 : 96000);
   if (tiles <= cu) return p.bits == 8 ? p.k >= 9728 && x >= 88000 : p.k >= 10752 && x >= 110000;
   if (tiles <= 2 * cu) return p.bits == 8 ? p.k >= 13056 && x >= 138000 && 2 * tiles <= 3 * cu : p.k >= 10752 && x >= 110000;
   return false;
+}
+
+// That split as one of up to 16 rows has it on any memory: within the library's scratch array, which a call on it must not exceed.
+// `split` 1: the call is not the streamed kernel's.  (A workspace that the call brings, or the array, is the decode kernel's where that
+// splits K too.  Means over 850 problems of the rule above that have both, this split's time on a workspace against the decode kernel's: int8
+// up to a quarter of a tile per CU 1.11 - 1.20, a half 1.03 - 1.10, from there to one and a quarter 0.85 - 1.0 (5120 x 13312 at 12 / 16
+// rows 20.0 / 21.1 and 18.6 / 19.1 us), int4 1.02 - 1.20 up to half a tile and level above.  Where it is ahead callers' workspaces have no
+// room for it: its windows of 32 rows take up to twice the memory that they are sized for.)
+GemmPlan plan_decode_stream(const Problem& p) {
+  if (!decode_streams(p)) return {};
+  const GemmPlan plan = plan_stream(p, true);
+  return plan.bytes <= kDecodeSplitBytes ? plan : GemmPlan{};
 }
 
 // How the decode kernel reads its weights, by 23,000 timings (M 1 - 16, K 1536 - 14336, 4 - 256 MB, all group sizes and both layouts; means over

@@ -134,12 +134,26 @@ int launch_gemm_stream_planned(const Problem& p, void* workspace, int64_t worksp
   return launch_plan(p, plan, workspace, slot);
 }
 
-int launch_gemm_stream_decode(const Problem& p) {
-  // (gelu onto its own residual stays with the kernels it is on)
-  if (!decode_streams(p) || !gemm_stream_applicable(p) || (p.activation == MI355X_WQ_ACT_GELU && p.residual == p.y)) return 0;
-  if (p.stream == hipStreamPerThread || captured(p)) return 0;
-  const GemmPlan plan = plan_stream(p, true);
-  return plan.bytes <= kDecodeSplitBytes ? launch_plan(p, plan, nullptr, true) : 0;
+namespace {
+
+// (gelu onto its own residual stays with the kernels it is on)
+bool decode_applicable(const Problem& p) { return gemm_stream_applicable(p) && !(p.activation == MI355X_WQ_ACT_GELU && p.residual == p.y && p.y != nullptr); }
+
+}  // namespace
+
+int64_t decode_workspace_bytes(const Problem& p) {
+  const int64_t decode = gemv_split_workspace_bytes(p);
+  if (decode > 0 || !decode_applicable(p)) return decode;
+  const GemmPlan plan = plan_decode_stream(p);
+  return plan.split > 1 ? plan.bytes : 0;
+}
+
+int launch_gemm_stream_decode(const Problem& p, void* workspace, int64_t workspace_bytes) {
+  if (!decode_streams(p) || !decode_applicable(p)) return 0;
+  if (workspace == nullptr ? p.stream == hipStreamPerThread || captured(p) : gemv_split_workspace_bytes(p) > 0) return 0;
+  const GemmPlan plan = plan_decode_stream(p);
+  if (plan.split == 1 || (workspace != nullptr && plan.bytes > workspace_bytes)) return 0;
+  return launch_plan(p, plan, workspace, workspace == nullptr);
 }
 
 }  // namespace wq

@@ -1281,8 +1281,9 @@ static __device__ __align__(256) unsigned char scratch[kDecodeSplitBytes];
 
 namespace {
 
-constexpr int64_t kStaticScratchBytes = kDecodeSplitBytes;
 std::atomic<void*> g_scratch_ptr[kMaxDevices];
+
+}  // namespace
 
 // Device address of the current device's copy of `scratch`, or nullptr with the error set.
 void* static_scratch_address() {
@@ -1308,24 +1309,7 @@ void* static_scratch_address() {
   return ptr;
 }
 
-}  // namespace
-
-int64_t gemv_static_scratch_bytes() { return kStaticScratchBytes; }
-
-// 1 = launched with the K split on the library's scratch array, 0 = the split does not apply to `p`
-// (nothing launched), -1 = failure: the split would need more than the array holds, or a runtime error
-int launch_gemv_split_static(const Problem& p) {
-  const int64_t need = gemv_split_workspace_bytes(p);
-  if (need == 0) return 0;
-  if (need > kStaticScratchBytes) {
-    set_error("the K split of this problem needs %lld bytes of scratch memory, the library's own array holds %lld: "
-              "use mi355x_wq_matmul_ws with a caller workspace", (long long)need, (long long)kStaticScratchBytes);
-    return -1;
-  }
-  void* const ptr = static_scratch_address();
-  if (ptr == nullptr) return -1;
-  return launch_gemv_split(p, ptr, kStaticScratchBytes);
-}
+int64_t gemv_static_scratch_bytes() { return kDecodeSplitBytes; }
 
 }  // namespace wq
 

@@ -48,9 +48,9 @@ int launch_gemv_rounds(const Problem& p);
 // must be zero before the first use and are zero again when the kernel has finished.
 int64_t gemv_split_workspace_bytes(const Problem& p);
 int launch_gemv_split(const Problem& p, void* workspace, int64_t workspace_bytes);
-// The same split on the library's own file-scope device array (no caller workspace, no allocation):
-// 1 launched, 0 the split does not apply, -1 failure (also when the problem needs more than the array holds).
-int launch_gemv_split_static(const Problem& p);
+// The library's own file-scope device array for that split (no caller workspace, no allocation); nullptr with the error set
+// where it cannot be resolved.
+void* static_scratch_address();
 int64_t gemv_static_scratch_bytes();
 // (a workspace lets the streamed GEMM, where it is the default, split K)
 int launch_skinny(const Problem& p, int variant, void* workspace, int64_t workspace_bytes);
@@ -75,9 +75,12 @@ bool launch_gemm_stream(const Problem& p, int variant, int ksplit, const SplitSp
 template <int BITS>
 bool launch_gemm_stream_bits(const Problem& p, int variant, int ksplit, const SplitSpace& space);  // of that bit width
 int launch_gemm_stream_planned(const Problem& p, void* workspace, int64_t workspace_bytes, float other_us);
-// The same for up to 16 rows, where decode_streams says so; not under capture nor on hipStreamPerThread, where the library has no
-// workspace for it and the decode kernel is ahead of the unsplit form.
-int launch_gemm_stream_decode(const Problem& p);
+// The same for up to 16 rows, where decode_streams says so.  With a workspace: on that, where the decode kernel does not split K and it is
+// large enough.  Without: on a slot, but not under capture nor on hipStreamPerThread, where the library has none
+// for it and the decode kernel is ahead of the unsplit form.
+int launch_gemm_stream_decode(const Problem& p, void* workspace, int64_t workspace_bytes);
+// The workspace that a call of up to 16 rows splits K on, in the decode kernel or the streamed one; 0 where it would not.
+int64_t decode_workspace_bytes(const Problem& p);
 bool decode_streams(const Problem& p);
 // The workspace that a call of `p` from 17 rows on splits K on, 0 where it would not.
 int64_t gemm_workspace_bytes(const Problem& p, bool skinny_family);
@@ -87,6 +90,7 @@ struct GemmPlan {
   int64_t tiles = 0, bytes = 0;  // bytes of workspace
 };
 GemmPlan plan_stream(const Problem& p, bool may_split);
+GemmPlan plan_decode_stream(const Problem& p);
 float skinny_cost(const Problem& p);  // us by the cost model; out of reach where a kernel does not apply
 float other_gemm_cost(const Problem& p);  // of the kernels launch_gemm takes where not the streamed one
 bool gemm_direct_applicable(const Problem& p);  // K % 256 == 0, the standard group, operands below 1 GiB

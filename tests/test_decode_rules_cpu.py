@@ -18,6 +18,10 @@ static wq::Problem problem(int bits, int group, int64_t m, int64_t n, int64_t k,
   p.tiled = tiled != 0;
   return p;
 }
+extern "C" int64_t streams(int bits, int group, int64_t m, int64_t n, int64_t k) {
+  const wq::GemmPlan plan = wq::plan_decode_stream(problem(bits, group, m, n, k, 0));
+  return plan.split > 1 ? plan.bytes : 0;
+}
 extern "C" int reads(int bits, int64_t m, int64_t n, int64_t k, int tiled, int tile_rows, int rounds) {
   return wq::weight_reads(problem(bits, bits == 4 ? 32 : 128, m, n, k, tiled), tile_rows, rounds != 0);
 }
@@ -32,6 +36,7 @@ def rules(tmp_path_factory):
                     "-I" + CSRC, "-o", str(d / "rules.so"), str(d / "rules.cpp")], check=True)
     so = C.CDLL(str(d / "rules.so"))
     so.reads.argtypes = [C.c_int, C.c_int64, C.c_int64, C.c_int64, C.c_int, C.c_int, C.c_int]
+    so.streams.argtypes, so.streams.restype = [C.c_int, C.c_int, C.c_int64, C.c_int64, C.c_int64], C.c_int64
     return so
 
 
@@ -48,3 +53,65 @@ OWN, PAIRS, ONCE = 0, 1, 2
     (8, 4, 10240, 8192, 0, 14, 0, ONCE), (8, 3, 152064, 5120, 0, 16, 1, ONCE), (8, 3, 70000, 896, 0, 16, 1, OWN)])
 def test_how_the_decode_kernel_reads_its_weights(rules, bits, m, n, k, tiled, tile_rows, rounds, want):
     assert rules.reads(bits, m, n, k, tiled, tile_rows, rounds) == want
+
+
+# The calls of wq_capi.cpp with every launch replaced by a note of what it was asked for.
+CALLS = """
+#include <string>
+#include "%(csrc)s/wq_internal.h"
+#include "%(csrc)s/../../include/mi355x_wq.h"
+namespace wq {
+static std::string route;
+static int64_t need;
+static char array[16];
+static int note(const char* what, int rc) { route += what; return rc; }
+int launch_gemm_stream_decode(const Problem&, void* space, int64_t) {
+  return note(space == nullptr ? "slot " : space == array ? "stream:array " : "stream:workspace ", space == nullptr);
+}
+int launch_gemv_split(const Problem&, void* space, int64_t) { return note(space == array ? "split:array " : "split:workspace ", 0); }
+int64_t decode_workspace_bytes(const Problem&) { return need; }
+void* static_scratch_address() { return array; }
+int64_t gemv_static_scratch_bytes() { return kDecodeSplitBytes; }
+int64_t gemm_workspace_bytes(const Problem&, bool) { return 0; }
+bool gemv_applicable(const Problem& p) { return p.m <= 16; }
+int launch_gemv(const Problem&, int) { return note("decode ", 0); }
+int launch_skinny(const Problem&, int, void*, int64_t) { return note("skinny ", 0); }
+int launch_gemm(const Problem&, int, void*, int64_t) { return note("gemm ", 0); }
+int launch_dequant(const Problem&, void*) { return 0; }
+int launch_tile_weights(const Problem&, void*, void*, bool) { return 0; }
+bool tiled_layout_defined(int, int, int64_t) { return true; }
+}
+extern "C" const char* route(int form, int64_t m, int64_t need) {
+  static char x[64] __attribute__((aligned(16)));
+  const mi355x_wq_desc d{8, 128, 0, 0, 5120, 13824};
+  wq::route.clear();
+  wq::need = need;
+  const int rc = form == 0   ? mi355x_wq_matmul(&d, x, x, x, x, m, nullptr)
+                 : form == 1 ? mi355x_wq_matmul_ws(&d, x, x, x, nullptr, x, m, nullptr, 0, x, need)
+                             : mi355x_wq_matmul_static_ws(&d, x, x, x, nullptr, x, m, nullptr, 0);
+  if (rc != 0) wq::route += "refused";
+  return wq::route.c_str();
+}
+"""
+
+
+@pytest.fixture(scope="module")
+def route(tmp_path_factory):
+    d = tmp_path_factory.mktemp("calls")
+    (d / "calls.cpp").write_text(CALLS % dict(csrc=CSRC))
+    flags = ["-std=c++17", "-D__HIP_PLATFORM_AMD__", "-I/opt/rocm/include", "-I" + CSRC]
+    subprocess.run(["g++", "-shared", "-fPIC", *flags, "-o", str(d / "calls.so"), str(d / "calls.cpp"), os.path.join(CSRC, "wq_capi.cpp"),
+                    "-L/opt/rocm/lib", "-Wl,-rpath,/opt/rocm/lib", "-lamdhip64"], check=True)
+    so = C.CDLL(str(d / "calls.so"))
+    so.route.argtypes, so.route.restype = [C.c_int, C.c_int64, C.c_int64], C.c_char_p
+    return lambda form, m, need: so.route(("plain", "workspace", "array").index(form), m, need).decode().split()
+
+
+def test_the_scratch_array_call_never_asks_for_a_slot(route):
+    """A slot's first use allocates, which that entry point does not."""
+    assert route("plain", 16, 0) == ["slot"]
+    assert route("workspace", 16, 1 << 20) == ["split:workspace", "stream:workspace", "slot"]
+    assert route("array", 16, 1 << 20) == ["split:array", "stream:array", "decode"]
+    assert route("array", 16, 0) == ["decode"]
+    assert route("array", 16, (4 << 20) + 16385) == ["refused"]
+    assert route("array", 40, 0) == route("plain", 40, 0) == ["skinny"]

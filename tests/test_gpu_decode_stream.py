@@ -88,6 +88,56 @@ def test_as_many_streams_as_slots_and_more(streams):
     assert all(torch.equal(o.view(torch.int16), alone.view(torch.int16)) for o in outs)
 
 
+@pytest.mark.parametrize("bits,m,n,k,streamed", [(4, 16, 8191, 11008, True), (4, 10, 5120, 11008, True), (8, 16, 5760, 13824, True),
+                                                 (8, 16, 5120, 13824, False), (4, 12, 4096, 11008, False)])
+def test_on_a_workspace_and_on_the_scratch_array(bits, m, n, k, streamed):
+    """A workspace holds the decode kernel's split, and where that does not split the streamed one's: the results there have the eager
+    call's bits, captured and on hipStreamPerThread as well.  The library's scratch array is as good as a workspace."""
+    import relax_amd
+    from relax_amd import lib
+
+    x, wq, s, g = O.make_case(m + k, m, n, k, bits)
+    dx, dw, ds = _dev(x), _dev(wq), _dev(s)
+    res = _dev(_fused_operands(m, m, n)[1])
+    need = relax_amd.wq_workspace_bytes(bits, g, n, k, m)
+    assert 16384 < need <= lib.load().mi355x_wq_static_ws_bytes()
+    ws = relax_amd.wq_workspace(need)
+    rows = [0, m // 2, m - 1]
+    for tail in ({}, dict(residual=res)):
+        plain = relax_amd.wq_matmul(dx, dw, ds, bits, g, **tail)
+        on_ws = relax_amd.wq_matmul(dx, dw, ds, bits, g, workspace=ws, **tail)
+        torch.cuda.synchronize()
+        assert torch.equal(on_ws.view(torch.int16), plain.view(torch.int16)) == streamed
+        assert int(ws[:16384].view(torch.int32).abs().sum()) == 0
+
+        class PerThread:
+            cuda_stream = 2
+
+        outs = [relax_amd.wq_matmul(dx, dw, ds, bits, g, workspace=ws, stream=PerThread, **tail)]
+        torch.cuda.synchronize()
+        y = torch.empty_like(plain)
+        ep = lib.WqEpilogue(None, tail["residual"].data_ptr() if tail else None, lib.ACT_NONE, 0)
+        lib.check(lib.load().mi355x_wq_matmul_static_ws(lib.make_desc(bits, g, n, k), dx.data_ptr(), dw.data_ptr(), ds.data_ptr(), ep, y.data_ptr(),
+                                                        m, int(torch.cuda.current_stream().cuda_stream), 0))
+        torch.cuda.synchronize()
+        outs.append(y)
+        graph, out = torch.cuda.CUDAGraph(), torch.empty_like(plain)
+        with torch.cuda.graph(graph):
+            relax_amd.wq_matmul(dx, dw, ds, bits, g, workspace=ws, out=out, **tail)
+        for _ in range(3):
+            out.zero_()
+            graph.replay()
+            relax_amd.wq_matmul(dx, dw, ds, bits, g, **tail)
+            torch.cuda.synchronize()
+            outs.append(out.clone())
+        assert all(torch.equal(o.view(torch.int16), on_ws.view(torch.int16)) for o in outs)
+        if not tail:
+            assert_close(on_ws.cpu().numpy()[rows], c_oracle.wq_matmul(x[rows], wq, s, bits, g, nthreads=8), (bits, m, n, k), ulp_fraction=0.005)
+    # one that is too small: as without
+    small = relax_amd.wq_matmul(dx, dw, ds, bits, g, workspace=ws[:need - 16])
+    assert torch.equal(small.view(torch.int16), relax_amd.wq_matmul(dx, dw, ds, bits, g).view(torch.int16))
+
+
 FIRST_LAUNCH_UNDER_CAPTURE = """
 import torch, relax_amd
 from relax_amd import lib
