@@ -204,18 +204,20 @@ GemmPlan plan_stream(const Problem& p, bool may_split) {
 
 // Up to 16 rows of canonical weights: where the streamed kernel's 32-row tiles, K split over workgroups, are ahead of the decode
 // kernel and the register-activation kernel.  Those have every CU walk all of K for its 16 columns, so each stages all of
-// the activations, in phases once they exceed the LDS; a split CU reads a part of them for more columns.  Lines by 840
-// timings (K 5120 - 13824, N 1024 - 16384, 4 - 16 rows, weights from memory; us, decode against streamed).  Row tiles of 16
-// between one and one and a quarter per CU, which divide worst: int8 5120 x 13824 at 6 / 16 rows 21.0 / 18.6 and 24.3 / 19.5,
-// 5120 x 8192 at 10 rows 14.5 / 13.6, int4 5120 x 11008 at 10 rows 17.3 / 14.3 (at 8: 13.6 / 14.3).  Up to one tile per CU: int8
-// 4096 x 11008 at 10 rows 18.2 / 15.0, 2048 x 13824 at 8 rows 15.4 / 12.3, int4 4096 x 13824 at 16 rows 16.3 / 14.4 (int8 4096 x
-// 8192 at 10 rows 11.5 / 13.7).  Up to two: int4 8192 x 11008 at 16 rows 20.2 / 18.5, int8 6144 x 13824 at 10 rows 24.6 / 23.3
-// (8192 x 9728 20.2 / 20.8).
+// the activations, in phases once they exceed the LDS; a split CU reads a part of them for more columns.  The lines by 9,500 timings
+// (K 3072 - 60000, N 128 - 14000, 1 - 16 rows, all groups from 32 on, weights from memory; the streamed kernel's time against the other's, means).
+// Where the rule takes it: 0.79 on 726 problems of up to 17000 of K, 0.72 on 1859 others of K up to 60000 and near the lines; 2 % of these
+// are slower, by up to 9 %.  Activations (rows x K) from 4 - 10 % below a line to 10 % above it, by row tiles of 16 per CU:
+//   up to one, int8 88000: 0.88 / 0.84, from K 9728 (0.94 / 0.89; below 8000 1.07); int4 110000: 0.89 / 0.84, from 10752 (0.85 / 0.82);
+//   more, up to three windows of 64-column tiles on the CUs at once (N <= 5440 of 256), which divide worst among 16-row tiles, int8 80000:
+//   0.91 / 0.90, int4 96000: 0.92 / 0.88, from K 8192 (0.99 / 0.89); N 5136 - 5376 like 5120 (0.83 - 0.90), beyond 1.0 - 1.05 and so
+//   in the next class;
+//   up to two (int8: one and a half), int8 138000: 0.88 / 0.90 and 0.97 - 1.05 at less, from K 13056 (0.93); int4 110000: 1.0 / 0.95, from 10752.
 bool decode_streams(const Problem& p) {
   if (p.m > 16 || p.tiled || p.k < 8192 || p.group < 32) return false;
   const int64_t tiles = ceil_div(p.n, 16), cu = cu_count(), x = p.m * p.k;
-  if (tiles > cu && 4 * tiles <= 5 * cu) return x >= (p.bits == 8 ? 80000 : 96000);
   if (tiles <= cu) return p.bits == 8 ? p.k >= 9728 && x >= 88000 : p.k >= 10752 && x >= 110000;
+  if (3 * ceil_div(p.n, 64) <= cu) return x >= (p.bits == 8 ? 80000 : 96000);
   if (tiles <= 2 * cu) return p.bits == 8 ? p.k >= 13056 && x >= 138000 && 2 * tiles <= 3 * cu : p.k >= 10752 && x >= 110000;
   return false;
 }

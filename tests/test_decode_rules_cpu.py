@@ -55,6 +55,22 @@ def test_how_the_decode_kernel_reads_its_weights(rules, bits, m, n, k, tiled, ti
     assert rules.reads(bits, m, n, k, tiled, tile_rows, rounds) == want
 
 
+# (bits, group, M, N, K, streamed): on both sides of each line of decode_streams
+STREAMED = [
+    (8, 128, 8, 4096, 11008, 1), (8, 128, 8, 4096, 10880, 0), (8, 128, 16, 4096, 9728, 1), (8, 128, 16, 4096, 9600, 0), (8, 64, 10, 400, 9728, 1),
+    (4, 32, 10, 4096, 11008, 1), (4, 32, 9, 4096, 11008, 0), (4, 128, 16, 4096, 10752, 1), (4, 32, 16, 4096, 10496, 0),
+    (8, 128, 10, 5120, 8192, 1), (8, 128, 9, 5120, 8192, 0), (8, 128, 16, 5120, 8064, 0), (8, 128, 16, 4097, 8192, 1), (8, 32, 16, 5440, 8192, 1),
+    (8, 128, 16, 5441, 8192, 0), (8, 128, 16, 5441, 13824, 1), (8, 128, 9, 5441, 13824, 0), (8, 128, 16, 6144, 13056, 1), (8, 128, 16, 6145, 13824, 0),
+    (4, 64, 12, 5440, 8192, 1), (4, 32, 11, 5440, 8192, 0), (4, 32, 16, 5441, 8192, 0), (4, 32, 16, 8192, 10752, 1), (4, 32, 16, 8193, 10752, 0),
+    (8, 16, 16, 5120, 13824, 0), (8, 128, 17, 5120, 13824, 0), (8, 128, 1, 4096, 60032, 0), (8, 128, 2, 4096, 60032, 1)]
+
+
+@pytest.mark.parametrize("bits,group,m,n,k,streamed", STREAMED)
+def test_long_k_on_the_streamed_kernel(rules, bits, group, m, n, k, streamed):
+    got = rules.streams(bits, group, m, n, k)
+    assert (got > 0) == bool(streamed) and got <= 16384 + (4 << 20), got
+
+
 # The calls of wq_capi.cpp with every launch replaced by a note of what it was asked for.
 CALLS = """
 #include <string>
