@@ -21,9 +21,16 @@ constexpr float kNever = 1e30f;
 // (every call from 17 rows on plans, so the divisions are of 32 bits, which extents are within, and the device is asked once)
 int ceil_div(int64_t a, int b) { return (int)(((uint32_t)a + (uint32_t)b - 1u) / (uint32_t)b); }
 
-// One tile shape, in us: start + rounds of tiles * (tile start and end + 256-k steps * its loop alone on the chip + on odd N, whose
-// rows are stored one element at a time, the tail) + steps * tiles per CU * what a full chip adds, and with K split into windows
-// the exchange.
+// One tile shape, in us: start + rounds of tiles * (tile start and end + 256-k steps * its loop alone on the chip + on odd N
+// the tail) + steps * tiles per CU * what a full chip adds, and with K split into windows the exchange.
+//
+// The tail of odd N, timed on 5,000 random problems.  Streamed: rows that begin between two 4-byte boundaries; against the even N beside it,
+// 8.6 us a round in 128 x 256 tiles (with a residual 10.8), 4.15 (5.0) in 128 x 128, 20 (23) in 256 x 256, 2.0 (2.3) in 64 x 128 and nothing in
+// 64 x 64.  The other kernels store and read an element at a time: a plain call's 3 - 7 us a round (pipeline: none), with a
+// bias 10 - 20 and with a residual 14 - 31.  A call's kernel does not depend on its tail, so their terms here are a plain call's and a
+// third of what a bias adds.  Against always taking the fastest, calls of odd N lose 0.4 % (plain; tile-major 0.7), 0.4 (bias; 0.5), 0.5 (gelu;
+// 0.8) and 0.4 (residual; 1.8) on 2,100 problems that were not fitted to; before, with a plain call's alone and the streamed tail's of one
+// element at a time, 0.6 (0.6), 1.4 (1.9), 0.4 (0.9) and 1.8 (4.1).
 struct TileCost {
   int variant, bm, bn;
   float start, tile, loop, loaded, odd, split, window, spread;
@@ -31,13 +38,13 @@ struct TileCost {
 
 constexpr TileCost kStreamCost[2][2][7] = {
     {{  // int4, canonical
-         {kStream128x256, 128, 256, 0.00f, 5.47f, 2.244f, 1.157f, 11.03f, 0.f, 0.f, 0.f},
-         {kStream128x128, 128, 128, 0.00f, 5.68f, 1.212f, 0.494f, 3.53f, 4.12f, 1.383f, 0.31f},
-         {kStream256x256, 256, 256, 0.00f, 7.52f, 4.841f, 2.567f, 22.68f, 0.f, 0.f, 0.f},
-         {kStream64x128, 64, 128, 1.14f, 3.71f, 0.836f, 0.291f, 1.79f, 2.45f, 0.747f, 1.16f},
+         {kStream128x256, 128, 256, 0.00f, 5.47f, 2.244f, 1.157f, 8.60f, 0.f, 0.f, 0.f},
+         {kStream128x128, 128, 128, 0.00f, 5.68f, 1.212f, 0.494f, 4.15f, 4.12f, 1.383f, 0.31f},
+         {kStream256x256, 256, 256, 0.00f, 7.52f, 4.841f, 2.567f, 20.0f, 0.f, 0.f, 0.f},
+         {kStream64x128, 64, 128, 1.14f, 3.71f, 0.836f, 0.291f, 2.00f, 2.45f, 0.747f, 1.16f},
          {kStream64x64, 64, 64, 1.47f, 3.12f, 0.520f, 0.181f, 0.00f, 1.75f, 0.450f, 0.19f},
-         {kStream32x64, 32, 64, 1.10f, 2.44f, 0.459f, 0.065f, 0.02f, 1.75f, 0.275f, 0.24f},
-         {kStream32x128, 32, 128, 1.12f, 3.11f, 0.742f, 0.152f, 0.63f, 1.99f, 0.461f, 0.35f}},
+         {kStream32x64, 32, 64, 1.10f, 2.44f, 0.459f, 0.065f, 0.03f, 1.75f, 0.275f, 0.24f},
+         {kStream32x128, 32, 128, 1.12f, 3.11f, 0.742f, 0.152f, 0.52f, 1.99f, 0.461f, 0.35f}},
      {  // int4, tile-major
          {kStream128x256, 128, 256, 0.00f, 6.00f, 2.483f, 1.013f, 10.16f, 0.f, 0.f, 0.f},
          {kStream128x128, 128, 128, 0.29f, 5.37f, 1.339f, 0.471f, 3.49f, 3.97f, 1.275f, 0.65f},
@@ -47,13 +54,13 @@ constexpr TileCost kStreamCost[2][2][7] = {
          {kStream32x64, 32, 64, 1.45f, 2.23f, 0.490f, 0.069f, 0.15f, 1.62f, 0.246f, 0.36f},
          {kStream32x128, 32, 128, 1.21f, 3.22f, 0.786f, 0.108f, 0.63f, 1.96f, 0.473f, 0.22f}}},
     {{  // int8, canonical
-         {kStream128x256, 128, 256, 2.45f, 0.00f, 3.575f, 0.733f, 11.27f, 0.f, 0.f, 0.f},
-         {kStream128x128, 128, 128, 0.00f, 4.75f, 1.419f, 0.474f, 3.56f, 4.03f, 1.378f, 1.04f},
-         {kStream256x256, 256, 256, 0.00f, 7.50f, 5.039f, 1.840f, 23.68f, 0.f, 0.f, 0.f},
-         {kStream64x128, 64, 128, 1.79f, 1.69f, 1.201f, 0.192f, 2.09f, 2.61f, 0.798f, 1.83f},
+         {kStream128x256, 128, 256, 2.45f, 0.00f, 3.575f, 0.733f, 8.60f, 0.f, 0.f, 0.f},
+         {kStream128x128, 128, 128, 0.00f, 4.75f, 1.419f, 0.474f, 4.15f, 4.03f, 1.378f, 1.04f},
+         {kStream256x256, 256, 256, 0.00f, 7.50f, 5.039f, 1.840f, 20.0f, 0.f, 0.f, 0.f},
+         {kStream64x128, 64, 128, 1.79f, 1.69f, 1.201f, 0.192f, 2.00f, 2.61f, 0.798f, 1.83f},
          {kStream64x64, 64, 64, 1.79f, 2.47f, 0.608f, 0.161f, 0.00f, 1.87f, 0.479f, 0.57f},
          {kStream32x64, 32, 64, 1.43f, 2.01f, 0.519f, 0.063f, 0.03f, 1.74f, 0.324f, 0.47f},
-         {kStream32x128, 32, 128, 1.21f, 2.71f, 0.907f, 0.097f, 0.59f, 1.99f, 0.458f, 1.00f}},
+         {kStream32x128, 32, 128, 1.21f, 2.71f, 0.907f, 0.097f, 0.52f, 1.99f, 0.458f, 1.00f}},
      {  // int8, tile-major
          {kStream128x256, 128, 256, 1.75f, 3.44f, 3.984f, 0.646f, 10.07f, 0.f, 0.f, 0.f},
          {kStream128x128, 128, 128, 0.00f, 6.12f, 1.392f, 0.518f, 3.27f, 3.28f, 1.206f, 0.46f},
@@ -66,17 +73,17 @@ constexpr TileCost kStreamCost[2][2][7] = {
 
 // The direct-weight kernel's 128 x 256 (variant 2), 64 x 256 (4) and 64 x 128 (5) tiles in the same terms (from 65 rows on).
 constexpr TileCost kDirectCost[2][2][3] = {
-    {{{2, 128, 256, 0.36f, 9.29f, 2.13f, 1.23f, 6.12f}, {4, 64, 256, 1.52f, 4.53f, 1.58f, 0.79f, 3.67f}, {5, 64, 128, 2.30f, 5.61f, 0.91f, 0.44f, 3.47f}},
-     {{2, 128, 256, 0.56f, 9.34f, 2.10f, 1.10f, 5.74f}, {4, 64, 256, 1.27f, 5.18f, 1.46f, 0.62f, 3.19f}, {5, 64, 128, 1.63f, 6.66f, 0.82f, 0.34f, 3.11f}}},
-    {{{2, 128, 256, 1.98f, 5.53f, 3.45f, 0.58f, 6.75f}, {4, 64, 256, 2.76f, 3.40f, 1.91f, 0.60f, 3.53f}, {5, 64, 128, 2.42f, 5.91f, 1.05f, 0.35f, 3.19f}},
-     {{2, 128, 256, 0.00f, 9.64f, 2.40f, 0.93f, 5.85f}, {4, 64, 256, 3.18f, 2.34f, 1.92f, 0.62f, 3.40f}, {5, 64, 128, 2.70f, 4.59f, 1.11f, 0.33f, 3.70f}}},
+    {{{2, 128, 256, 0.36f, 9.29f, 2.13f, 1.23f, 10.62f}, {4, 64, 256, 1.52f, 4.53f, 1.58f, 0.79f, 6.37f}, {5, 64, 128, 2.30f, 5.61f, 0.91f, 0.44f, 6.17f}},
+     {{2, 128, 256, 0.56f, 9.34f, 2.10f, 1.10f, 10.24f}, {4, 64, 256, 1.27f, 5.18f, 1.46f, 0.62f, 5.89f}, {5, 64, 128, 1.63f, 6.66f, 0.82f, 0.34f, 5.81f}}},
+    {{{2, 128, 256, 1.98f, 5.53f, 3.45f, 0.58f, 11.25f}, {4, 64, 256, 2.76f, 3.40f, 1.91f, 0.60f, 6.23f}, {5, 64, 128, 2.42f, 5.91f, 1.05f, 0.35f, 5.89f}},
+     {{2, 128, 256, 0.00f, 9.64f, 2.40f, 0.93f, 10.35f}, {4, 64, 256, 3.18f, 2.34f, 1.92f, 0.62f, 6.10f}, {5, 64, 128, 2.70f, 4.59f, 1.11f, 0.33f, 6.40f}}},
 };
 
-// The LDS-staged pipeline's 256 x 128 and 128 x 128 tiles (canonical weights only; odd N hardly costs it anything: int8, group
-// 32, 1123 x 5165 x 1024 26.2 us against 33.0 streamed).
+// The LDS-staged pipeline's 256 x 128 and 128 x 128 tiles (canonical weights only; odd N hardly costs a plain call anything: int8, group
+// 32, 1123 x 5165 x 1024 25.0 us against 30.1 streamed).
 constexpr TileCost kPipeCost[2][2] = {
-    {{1, 256, 128, 1.45f, 4.48f, 3.43f, 1.12f, 0.18f}, {2, 128, 128, 0.63f, 3.18f, 2.65f, 0.65f, 0.27f}},
-    {{1, 256, 128, 0.36f, 5.60f, 3.80f, 0.97f, 0.12f}, {2, 128, 128, 1.68f, 2.30f, 2.85f, 0.77f, 0.25f}},
+    {{1, 256, 128, 1.45f, 4.48f, 3.43f, 1.12f, 2.68f}, {2, 128, 128, 0.63f, 3.18f, 2.65f, 0.65f, 3.27f}},
+    {{1, 256, 128, 0.36f, 5.60f, 3.80f, 0.97f, 2.62f}, {2, 128, 128, 1.68f, 2.30f, 2.85f, 0.77f, 3.25f}},
 };
 
 int layout_of(const Problem& p) { return p.tiled && p.choose_by_layout ? 1 : 0; }
