@@ -37,7 +37,9 @@ def test_rows_off_the_4_byte_grid(variant, m, n, shift):
     assert_close(plain, c_oracle.wq_matmul(x, wq, s, bits, g, nthreads=8), (variant, m, n))
     db, dr = at(bias, ob)[0], at(res, orr)[0]
     tails = [({}, {}), (dict(bias=db), dict(bias=bias)), (dict(residual=dr), dict(residual=res)),
-             (dict(bias=db, activation="relu", residual=dr), dict(bias=bias, activation="relu", residual=res))]
+             (dict(bias=db, activation="relu", residual=dr), dict(bias=bias, activation="relu", residual=res)),
+             (dict(bias=db, activation="gelu"), dict(bias=bias, activation="gelu")),
+             (dict(activation="gelu", residual=dr), dict(activation="gelu", residual=res))]
     for given, want in tails:
         y, flat = at(np.zeros((m, n), np.float16), oy)
         relax_amd.wq_matmul(dx, dw, ds, bits, g, out=y, **given, **kw)
