@@ -51,7 +51,8 @@ typedef struct mi355x_wq_desc {
 
 /* Kernel families; MI355X_WQ_KERNEL_AUTO picks by M and K.  From 17 rows on the default of the SKINNY and GEMM families is
  * the streamed GEMM (operands straight into LDS) wherever its cost model finds that the faster one, and up to 16 rows that
- * of SKINNY is the decode kernel where a vocabulary's tiles exceed its LDS slots; a forced family chooses as for
+ * of SKINNY is the decode kernel where a vocabulary's tiles exceed its LDS slots; up to 16 rows AUTO itself, and no family, may
+ * run the streamed GEMM too (mi355x_wq_matmul); a forced family chooses as for
  * canonical weights on either layout, so its results do not depend on the layout.  An explicit variant
  * (kernel | variant << 8) is the build it names. */
 enum {
@@ -102,9 +103,8 @@ enum {
    * with the float16 operation sequence of the CPU path -- nn.silu(x) = multiply(x, sigmoid(x))
    * (python/tvm/relax/transform/legalize_ops.py:506-510), sigmoid(x) = 1 / (1 + exp(-x))
    * (src/target/intrin_rule.cc:135-141), exp evaluated in float32 and rounded: five float16 roundings.
-   * Identical to the CPU result except where the last bit of the float32 exp differs between the two
-   * math libraries and survives the rounding to float16 (about one output in a few thousand, then a few
-   * float16 ulp).  The reference's counterpart is the activation member of its fused matmul patterns
+   * Every finite gate gives the result of a correctly rounded float32 exp; the CPU result can differ from it only where its math library's
+   * float32 exp is off in the last bit and that survives the rounding to float16.  The reference's counterpart is the activation member of its fused matmul patterns
    * (python/tvm/relax/dpl/pattern.py:1049-1095, python/tvm/contrib/cutlass/gen_tensor_op.py:377-380).
    * `y` is [M, N/2]; no bias, no residual, canonical weights, N even; M <= 16 runs the decode kernel,
    * larger M needs K % 256 == 0 with group 32 (int4) / 128 (int8). */
@@ -230,7 +230,8 @@ MI355X_WQ_API int64_t mi355x_wq_static_ws_bytes(void);
  * mi355x_wq_matmul would accept them. */
 MI355X_WQ_API int mi355x_wq_check(const mi355x_wq_desc* desc, int64_t m);
 
-/* The family whose default AUTO dispatch runs for `m` rows (MI355X_WQ_KERNEL_*; see there for what that may be), or -1. */
+/* The family whose default AUTO dispatch runs for `m` rows (MI355X_WQ_KERNEL_*; see there for what that may be), or -1.  Up to 16 rows on
+ * canonical weights with long K: the one that runs where the call is not split for the streamed GEMM (under capture, for one). */
 MI355X_WQ_API int mi355x_wq_select_kernel(const mi355x_wq_desc* desc, int64_t m);
 
 /* Thread-local description of the last failure on this thread ("" if none). */

@@ -161,7 +161,8 @@ constexpr int kActGelu = 3;
 // it, and erff, which evaluates both of its branches for a wavefront whose values fall into either, is sixty instructions of
 // it (int4 1024 x 10000 x 4224, bias and gelu: 128.6 -> 112.2 us, 105 with the bias alone).  This is x * P(x^2) with the first coefficient split
 // in two, the coefficients by a linear program that keeps every float16 input inside the rounding interval of its result: for
-// each of the 65536 the same float16 value as erff's, which is the correctly rounded one.
+// each that is not a NaN the same float16 value as erff's, which is the correctly rounded one.  (A NaN gives 1 or -1; gelu's last product is
+// with the NaN itself.)
 __device__ __forceinline__ half_t erf_f16(half_t h) {
   const float x = fminf(fabsf((float)h), 2.6f);  // (erf rounds to 1 from 2.5957 on)
   const float t = x * x;
@@ -198,7 +199,7 @@ __device__ __forceinline__ int gated_physical_row(int logical, int N) { return (
 // multiply(nn.silu(g), u) on float16 values, every operation rounded once as the CPU path executes them:
 // e = f16(exp(-g)), d = f16(1 + e), s = f16(1 / d), t = f16(g * s), y = f16(t * u).
 // exp and the quotient in float32 by one hardware instruction each (exp2 of g * -log2(e), rcp): rounded to float16 they are,
-// for each of the 65536 values of g and of d, the same as expf's and the division's, which took 40 instructions more (int4
+// for every finite g and every d, the same as expf's and the division's, which took 40 instructions more (int4
 // 2048 x 22016 x 4096: 362 -> 356 us).
 __device__ __forceinline__ half_t silu_mul(half_t g, half_t u) {
   const half_t e = (half_t)__builtin_amdgcn_exp2f((float)g * -1.4426950408889634f);

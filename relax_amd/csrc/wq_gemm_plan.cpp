@@ -1,4 +1,4 @@
-// Which kernel a call of 17 rows and more runs on: the streamed GEMM (wq_gemm_stream.hip) with which tile and how many windows
+// Which kernel a call runs on from 17 rows on (and, at the end of the file, two rules of the decode kernel up to 16): the streamed GEMM (wq_gemm_stream.hip) with which tile and how many windows
 // of K, the direct-weight GEMM (wq_gemm_direct.hip) or the register-activation kernel (wq_skinny.hip).  Host arithmetic only.
 //
 // Each kernel's time is a sum of terms of the problem's tiles, fitted per bit width and weight layout -- the layouts differ

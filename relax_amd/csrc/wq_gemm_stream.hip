@@ -1,4 +1,5 @@
-// MFMA GEMM whose operands stream through LDS: y[M,N] = x[M,K] @ dequant(Wq,S)^T, from 17 rows on.
+// MFMA GEMM whose operands stream through LDS: y[M,N] = x[M,K] @ dequant(Wq,S)^T, from 17 rows on and, with K split, for fewer rows
+// of long K (decode_streams in wq_gemm_plan.cpp).
 //
 // What bounds it: with 128 rows and more per tile the matrix pipes and, on random data, the board's power (the chip clocks
 // down); below that the vector instructions of the conversion (a weight is converted once per tile of rows: 8 per MFMA

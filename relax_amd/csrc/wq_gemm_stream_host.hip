@@ -93,8 +93,8 @@ SplitSpace library_space(hipStream_t s, const GemmPlan& plan, bool decode, std::
 
 namespace {
 
-// Up to 16 rows the decode kernel and the register-activation kernel read the weights faster.  With K below 1024 a launch is
-// mostly start-up and the kernels are level -- 600 x 15323 x 512: 38.2 us there, 36.3 - 40.9 here -- so those stay.
+// Up to 16 rows the decode kernel and the register-activation kernel read the weights faster, but for the long K that
+// launch_gemm_stream_decode takes.  With K below 1024 a launch is mostly start-up and the kernels are level -- 600 x 15323 x 512: 38.2 us there, 36.3 - 40.9 here -- so those stay.
 bool in_range(const Problem& p) { return p.m > 16 && p.k >= 1024 && gemm_stream_applicable(p); }
 
 }  // namespace
