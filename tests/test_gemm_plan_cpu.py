@@ -56,7 +56,9 @@ ABOVE_256_ROWS = [
     (4, 277, 13519, 9728, 1, "direct", 111.0, 124.2), (4, 768, 4096, 11008, 0, "stream", 104.1, 83.3), (4, 1906, 2640, 1280, 0, "stream", 28.5, 21.2),
     (8, 300, 2048, 1280, 0, "stream", 17.1, 8.3), (4, 300, 2048, 1280, 1, "stream", 15.3, 8.4),
     (8, 341, 29056, 1792, 1, "stream", 63.8, 57.5), (4, 467, 19584, 1792, 1, "stream", 58.0, 52.4),
-    (8, 512, 5120, 13824, 1, "stream", 134.7, 113.3), (4, 1024, 4096, 11008, 1, "stream", 105.8, 97.0)]
+    (8, 512, 5120, 13824, 1, "stream", 134.7, 113.3), (4, 1024, 4096, 11008, 1, "stream", 105.8, 97.0),
+    (4, 1273, 18827, 1280, 0, "stream", 105.3, 89.1), (4, 747, 7825, 1280, 0, "stream", 33.3, 29.4), (4, 1728, 8711, 3840, 0, "stream", 139.9, 126.6),
+    (4, 1158, 6239, 1280, 0, "stream", 35.9, 31.5), (8, 1124, 19983, 1280, 0, "stream", 108.9, 95.8)]
 
 
 @pytest.mark.parametrize("bits,m,n,k,tiled,faster,direct_us,stream_us", ABOVE_256_ROWS)
