@@ -215,11 +215,11 @@ GemmPlan plan_stream(const Problem& p, bool may_split) {
 // (K 3072 - 60000, N 128 - 14000, 1 - 16 rows, all groups from 32 on, weights from memory; the streamed kernel's time against the other's, means).
 // Where the rule takes it: 0.79 on 726 problems of up to 17000 of K, 0.72 on 1859 others of K up to 60000 and near the lines; 2 % of these
 // are slower, by up to 9 %.  Activations (rows x K) from 4 - 10 % below a line to 10 % above it, by row tiles of 16 per CU:
-//   up to one, int8 88000: 0.88 / 0.84, from K 9728 (0.94 / 0.89; below 8000 1.07); int4 110000: 0.89 / 0.84, from 10752 (0.85 / 0.82);
+//   up to one, int8 88000: 0.88 / 0.84, from K 9728 (0.87 - 0.94 / 0.90; below 7800 1.07); int4 110000: 0.89 / 0.84, from 10752 (0.85 / 0.79);
 //   more, up to three windows of 64-column tiles on the CUs at once (N <= 5440 of 256), which divide worst among 16-row tiles, int8 80000:
 //   0.91 / 0.90, int4 96000: 0.92 / 0.88, from K 8192 (0.99 / 0.89); N 5136 - 5376 like 5120 (0.83 - 0.90), beyond 1.0 - 1.05 and so
 //   in the next class;
-//   up to two (int8: one and a half), int8 138000: 0.88 / 0.90 and 0.97 - 1.05 at less, from K 13056 (0.93); int4 110000: 1.0 / 0.95, from 10752.
+//   up to two (int8: one and a half), int8 138000: 0.87 / 0.90 and 0.97 - 1.05 at less, from K 13056 (0.95 / 0.91); int4 110000: 1.0 / 0.95, from 10752.
 bool decode_streams(const Problem& p) {
   if (p.m > 16 || p.tiled || p.k < 8192 || p.group < 32) return false;
   const int64_t tiles = ceil_div(p.n, 16), cu = cu_count(), x = p.m * p.k;
