@@ -134,6 +134,68 @@ float skinny_cost(const Problem& p) {
   return c.by_tiles[r].start + steps * (c.by_tiles[r].step + c.by_tiles[r].rows * rb) + c.block * rb;
 }
 
+// The standard groups and whole steps of K: a request for weights covers a row's whole line, one for scales 16 bytes of them (int4), and
+// nothing is past a row's end.  (A workgroup's column tiles are within the matrix from its 128 columns on.)
+bool gemm_strip_applicable(const Problem& p) {
+  return p.m <= kStripMaxM && p.n >= 128 && p.n <= (4 << 20) && standard_group(p) && p.k % (1024 / p.bits) == 0;
+}
+
+int strip_row_blocks(int64_t m) {
+  const int slices = ceil_div(m, 64), blocks = ceil_div(ceil_div(m, slices), 8);
+  return blocks < 3 ? 3 : blocks == 7 ? 8 : blocks;
+}
+
+// The strip kernel's time: start; per round of workgroups what does not depend on K and what a block of eight rows adds to a
+// column tile; per stage of K (512 k: 64 for each of the eight wavefronts) and round column tiles and blocks, and what a full chip adds to
+// both; and, past eight stages, what the wavefronts' drifting apart costs.  Fitted to 2,070 timings of 1,385 problems (17 - 256 rows, N 512 - 28000, K 1024 -
+// 14000, weights and activations from memory) within 6 %.
+//
+// Why the line lies where these costs put it: a CU reads all of its rows' activations once per strip, so the kernel is ahead where
+// one round of workgroups covers the matrix and K is short, and behind where K is long: then K split over workgroups reads a part of them.
+// us before and now: int4 4096 x 4096 at 20 / 37 rows 8.1 / 11.4 -> 7.3 / 9.3, 12288 x 4096 12.4 / 15.5 -> 11.3 / 13.9; not 4096 x 11008 at
+// 37 rows (15.8, here 21.5).  Means over the 1,385, the call's time against its time without this kernel, weights from memory: 17 - 64 rows
+// int4 0.95 (tile-major 0.92), int8 0.97 (0.97), 65 - 256 rows 0.96 and 0.98; with weights in the last-level cache 0.93 (0.88), 0.95 (0.93),
+// 0.94 and 0.95; always taking the fastest would be 1 % better.
+namespace {
+struct StripCost {
+  float start, round, tiles, stage_tiles, stage_rows, loaded_tiles, loaded_rows, drift;
+};
+constexpr StripCost kStripCost[2][2] = {
+    {{1.721f, 1.020f, 0.095f, 0.137f, 0.062f, 0.112f, 0.032f, 0.133f},   // int4, canonical
+     {1.328f, 1.488f, 0.111f, 0.127f, 0.052f, 0.062f, 0.038f, 0.074f}},  // tile-major
+    {{1.376f, 1.163f, 0.066f, 0.145f, 0.091f, 0.226f, 0.010f, 0.200f},   // int8
+     {1.340f, 1.203f, 0.073f, 0.126f, 0.090f, 0.212f, 0.000f, 0.025f}},
+};
+}  // namespace
+
+GemmPlan plan_strip(const Problem& p) {
+  GemmPlan best;
+  best.us = best.both_us = kNever;
+  if (p.m <= 16 || !gemm_strip_applicable(p)) return best;
+  const int cu = cu_count(), blocks = strip_row_blocks(p.m), slices = ceil_div(p.m, blocks * 8), layout = layout_of(p);
+  const float rows = (float)blocks, stages = (float)p.k / 512.f;
+  for (int t = 1; t <= kStripMaxTiles; ++t) {
+    if (!strip_fits(p.bits, blocks, t)) break;
+    const int64_t groups = (int64_t)ceil_div(p.n, t * 16) * slices;
+    const float rounds = (float)((groups + cu - 1) / cu), full = (float)groups / (float)cu, tiles = (float)t;
+    auto cost = [&](const StripCost& c) {
+      const float drift = stages > 8.f ? (stages - 8.f) * c.drift : 0.f;
+      return c.start + rounds * (c.round + c.tiles * rows * tiles + stages * (c.stage_tiles * tiles + c.stage_rows * rows) + drift) +
+             stages * full * (c.loaded_tiles * tiles + c.loaded_rows * rows);
+    };
+    const float us = cost(kStripCost[p.bits == 8][layout]), both = us + cost(kStripCost[p.bits == 8][1 - layout]);
+    if (both < best.both_us) best = GemmPlan{t, 1, us, both, groups, 0};
+  }
+  return best;
+}
+
+// By both layouts' times together, as the streamed kernel's tile, so that the sums are the same on either.  Three per cent to spare, and
+// from eight stages of K on, where both kernels' times scatter most, two more for each: of the 1,385 problems one is more than 3 % slower.
+bool strip_ahead(const Problem& p, const GemmPlan& strip, const GemmPlan& stream) {
+  const float stages = (float)p.k / 512.f;
+  return strip.both_us < (0.97f - 0.02f * std::max(0.f, stages - 8.f)) * stream.both_us;
+}
+
 bool gemm_direct_applicable(const Problem& p) { return p.k % 256 == 0 && standard_group(p) && gemm_pipe_applicable(p); }
 
 // Columns of 128 x 256 tiles that fill whole rounds of the CUs where the rest, at most half a round, is worth 64-row tiles
@@ -187,7 +249,7 @@ float other_gemm_cost(const Problem& p) {
 // against each layout's own choice); `us` by the problem's layout.
 GemmPlan plan_stream(const Problem& p, bool may_split) {
   GemmPlan best;
-  float best_us = kNever;
+  best.both_us = kNever;
   const int layout = layout_of(p);
   const int cu = cu_count(), macros = ceil_div(p.k, 256);
   const bool odd = p.n % 2 != 0;
@@ -200,9 +262,8 @@ GemmPlan plan_stream(const Problem& p, bool may_split) {
       const int per = s == 1 ? macros : ceil_div(macros, s);
       if (s > 1 && (per < 2 || (s - 1) * per >= macros)) continue;  // (windows that would be empty are dropped)
       const float us = tile_cost(own, tiles * s, per, s, odd, cu), both = us + tile_cost(other, tiles * s, per, s, odd, cu);
-      if (both < best_us) {
-        best_us = both;
-        best = GemmPlan{own.variant, s, us, tiles, s > 1 ? kSplitCounterBytes + tiles * s * own.bm * own.bn * 4 : 0};
+      if (both < best.both_us) {
+        best = GemmPlan{own.variant, s, us, both, tiles, s > 1 ? kSplitCounterBytes + tiles * s * own.bm * own.bn * 4 : 0};
       }
     }
   }

@@ -1,6 +1,7 @@
 // Host side of the streamed GEMM (wq_gemm_stream.hip): the planned launch and the library's own workspaces.
 #include <string.h>
 
+#include <algorithm>
 #include <mutex>
 
 #include "../../include/mi355x_wq.h"
@@ -12,6 +13,11 @@ namespace wq {
 bool launch_gemm_stream(const Problem& p, int variant, int ksplit, const SplitSpace& space) {
   if (!gemm_stream_applicable(p)) return false;
   return p.bits == 4 ? launch_gemm_stream_bits<4>(p, variant, ksplit, space) : launch_gemm_stream_bits<8>(p, variant, ksplit, space);
+}
+
+bool launch_gemm_strip(const Problem& p, int tiles) {
+  if (!gemm_strip_applicable(p)) return false;
+  return p.bits == 4 ? launch_gemm_strip_bits<4>(p, tiles) : launch_gemm_strip_bits<8>(p, tiles);
 }
 
 bool gemm_stream_applicable(const Problem& p) {
@@ -109,18 +115,22 @@ namespace {
 
 bool captured(const Problem& p) { return capturing(p.stream); }
 
+int launched(bool ok, const char* which) {
+  if (!ok) return -1;
+  const hipError_t e = hipGetLastError();
+  if (e != hipSuccess) {
+    set_error("gemm kernel (%s) launch failed: %s", which, hipGetErrorString(e));
+    return -1;
+  }
+  return 1;
+}
+
 // `slot`: on a workspace of the library's
 int launch_plan(const Problem& p, const GemmPlan& plan, void* workspace, bool slot) {
   std::unique_lock<std::mutex> slot_lock;
   SplitSpace space{plan.split > 1 ? workspace : nullptr, nullptr, 0};
   if (plan.split > 1 && slot) space = library_space(p.stream, plan, p.m <= 16, &slot_lock);
-  if (!launch_gemm_stream(p, plan.variant, plan.split, space)) return -1;
-  const hipError_t e = hipGetLastError();
-  if (e != hipSuccess) {
-    set_error("gemm kernel (streamed operands) launch failed: %s", hipGetErrorString(e));
-    return -1;
-  }
-  return 1;
+  return launched(launch_gemm_stream(p, plan.variant, plan.split, space), "streamed operands");
 }
 
 }  // namespace
@@ -130,7 +140,10 @@ int launch_gemm_stream_planned(const Problem& p, void* workspace, int64_t worksp
   GemmPlan plan = plan_stream(p, p.m <= 256 || workspace != nullptr);
   const bool slot = plan.split > 1 && plan.bytes > workspace_bytes;
   if (slot && (p.m > 256 || captured(p))) plan = plan_stream(p, false);
-  if (other_us < plan.us) return 0;
+  const GemmPlan strip = plan_strip(p);
+  const bool ahead = strip_ahead(p, strip, plan);
+  if (other_us < (ahead ? std::min(strip.us, plan.us) : plan.us)) return 0;
+  if (ahead) return launched(launch_gemm_strip(p, strip.variant), "strip");
   return launch_plan(p, plan, workspace, slot);
 }
 

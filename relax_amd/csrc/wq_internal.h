@@ -84,13 +84,28 @@ int64_t decode_workspace_bytes(const Problem& p);
 bool decode_streams(const Problem& p);
 // The workspace that a call of `p` from 17 rows on splits K on, 0 where it would not.
 int64_t gemm_workspace_bytes(const Problem& p, bool skinny_family);
+// The strip kernel (wq_gemm_strip.hip): where it applies, the blocks of eight rows in a slice of rows, whether a wavefront's share of the
+// LDS holds its rings (and its partial sums) for so many column tiles of 16, and an explicit launch with that many.
+constexpr int64_t kStripMaxM = 256;
+constexpr int kStripWaves = 8, kStripMaxTiles = 4;
+constexpr int strip_ring_bytes(int bits, int row_blocks, int tiles) { return row_blocks * 2048 + tiles * 2048 + (bits == 4 ? 1024 : 256); }
+constexpr bool strip_fits(int bits, int row_blocks, int tiles) {
+  return strip_ring_bytes(bits, row_blocks, tiles) * kStripWaves <= 160 * 1024 && (row_blocks + 1) / 2 * tiles * 1024 * kStripWaves <= 160 * 1024;
+}
+bool gemm_strip_applicable(const Problem& p);
+int strip_row_blocks(int64_t m);
+bool launch_gemm_strip(const Problem& p, int tiles);
+template <int BITS>
+bool launch_gemm_strip_bits(const Problem& p, int tiles);  // of that bit width
 struct GemmPlan {
   int variant = 0, split = 1;  // tile, windows of K
-  float us = 0.f;
+  float us = 0.f, both_us = 0.f;  // on the problem's layout, on both together
   int64_t tiles = 0, bytes = 0;  // bytes of workspace
 };
 GemmPlan plan_stream(const Problem& p, bool may_split);
 GemmPlan plan_decode_stream(const Problem& p);
+GemmPlan plan_strip(const Problem& p);  // `variant`: its column tiles, 0 where it does not apply (`us` is out of reach then)
+bool strip_ahead(const Problem& p, const GemmPlan& strip, const GemmPlan& stream);
 float skinny_cost(const Problem& p);  // us by the cost model; out of reach where a kernel does not apply
 float other_gemm_cost(const Problem& p);  // of the kernels launch_gemm takes where not the streamed one
 bool gemm_direct_applicable(const Problem& p);  // K % 256 == 0, the standard group, operands below 1 GiB

@@ -1,0 +1,66 @@
+"""Where the strip kernel is taken from 17 rows on (wq_gemm_plan.cpp), compiled as host code and asked on problems that were timed on an
+MI355X without and with it; and what has to hold whatever the times: both layouts choose alike, and a build exists for the choice."""
+import ctypes as C
+import os
+import subprocess
+
+import pytest
+
+CSRC = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "relax_amd", "csrc")
+
+WRAPPER = """
+#include "%s/wq_gemm_plan.cpp"
+namespace wq {
+int cu_count() { return 256; }
+bool gemm_pipe_applicable(const Problem& p) { return p.k %% 64 == 0; }
+}
+extern "C" int ask(int bits, int group, int64_t m, int64_t n, int64_t k, int tiled) {
+  wq::Problem p{nullptr, nullptr, nullptr, nullptr, m, n, k, bits, group, 0, nullptr};
+  p.tiled = tiled != 0;
+  const wq::GemmPlan strip = wq::plan_strip(p);
+  const bool ahead = wq::strip_ahead(p, strip, wq::plan_stream(p, true));
+  if (ahead && (strip.variant < 1 || strip.variant > 4 || !wq::strip_fits(bits, wq::strip_row_blocks(m), strip.variant))) return -1;
+  return ahead ? strip.variant : 0;
+}
+"""
+
+
+@pytest.fixture(scope="module")
+def ask(tmp_path_factory):
+    d = tmp_path_factory.mktemp("strip")
+    (d / "plan.cpp").write_text(WRAPPER % CSRC)
+    subprocess.run(["g++", "-std=c++17", "-shared", "-fPIC", "-Wall", "-Werror", "-D__HIP_PLATFORM_AMD__", "-I/opt/rocm/include",
+                    "-I" + CSRC, "-o", str(d / "plan.so"), str(d / "plan.cpp")], check=True)
+    f = C.CDLL(str(d / "plan.so")).ask
+    f.argtypes = [C.c_int, C.c_int, C.c_int64, C.c_int64, C.c_int64, C.c_int]
+    return f
+
+
+# (bits, M, N, K, column tiles, us of the strip kernel, us of the call without it); 0: not taken
+TIMED = [(4, 37, 4096, 4096, 1, 9.3, 11.4), (4, 20, 4096, 4096, 1, 7.3, 8.1), (4, 37, 12288, 4096, 3, 13.9, 15.5), (4, 20, 12288, 4096, 3, 11.3, 12.4),
+         (4, 37, 4096, 11008, 0, 21.5, 15.8), (4, 64, 22016, 4096, 0, 58.7, 22.6), (8, 37, 5120, 13824, 0, 37.6, 23.1), (8, 37, 27648, 5120, 0, 42.2, 39.4)]
+
+
+@pytest.mark.parametrize("bits,m,n,k,tiles,strip_us,other_us", TIMED)
+def test_the_faster_one_is_taken(ask, bits, m, n, k, tiles, strip_us, other_us):
+    assert (strip_us < other_us) == (tiles > 0)
+    for tiled in (0, 1):
+        assert ask(bits, 32 if bits == 4 else 128, m, n, k, tiled) == tiles
+
+
+def test_both_layouts_choose_alike_and_the_build_is_there(ask):
+    taken = 0
+    for bits, step in ((4, 256), (8, 128)):
+        for m in (17, 24, 25, 33, 40, 41, 49, 56, 57, 64, 65, 72, 100, 129, 191, 256):
+            for n in (128, 130, 1024, 2304, 4096, 5121, 8192, 12288, 16384, 22528):
+                for k in (1024, 1024 + step, 2816, 4096, 8192, 13824):
+                    got = [ask(bits, 32 if bits == 4 else 128, m, n, k, tiled) for tiled in (0, 1)]
+                    assert got[0] == got[1] >= 0, (bits, m, n, k)
+                    taken += got[0] > 0
+    assert taken > 300
+
+
+@pytest.mark.parametrize("bits,group,m,n,k", [(4, 32, 16, 4096, 4096), (4, 32, 257, 1024, 1024), (4, 32, 37, 127, 4096), (4, 32, 37, 4096, 4096 + 128),
+                                              (4, 64, 37, 4096, 4096), (8, 128, 37, 2048, 2048 + 64), (8, 32, 37, 2048, 2048)])
+def test_not_where_it_does_not_apply(ask, bits, group, m, n, k):
+    assert ask(bits, group, m, n, k, 0) == 0
