@@ -51,6 +51,23 @@ __device__ __forceinline__ void static_for_s(F&& f) {
     static_for_s<B + 1, E>(f);
   }
 }
+
+// One request of 64 lanes from a buffer straight into LDS: lane l's 16 bytes land at lds + 16 l (its two bytes, zero
+// extended, at lds + 4 l); a lane whose offset is out of range writes zeros.  Written as assembly because the
+// compiler would order every LDS read behind every such request in flight; the kernel orders them itself.  The
+// destination is an operand in m0, which is the compiler's to write (a wait state apart from the request).  It does not see the wait
+// states that a request needs behind a vector instruction which writes its scalar operands, so `lds`, `r` and `soff` have to be computed by
+// scalar instructions alone (a branch on the way, or a call in the argument, and it refuses or moves one over right in front).
+__device__ __forceinline__ void dma_b128(uint32_t lds, uint32_t voff, rsrc_t r, uint32_t soff) {
+  asm volatile("s_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds" ::"{m0}"(lds), "v"(voff), "s"(r), "s"(soff) : "memory");
+}
+__device__ __forceinline__ void dma_u16(uint32_t lds, uint32_t voff, rsrc_t r, uint32_t soff) {
+  asm volatile("s_nop 0\n\tbuffer_load_ushort %1, %2, %3 offen lds" ::"{m0}"(lds), "v"(voff), "s"(r), "s"(soff) : "memory");
+}
+template <int N>
+__device__ __forceinline__ void wait_dma() {
+  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
+}
 }  // namespace
 
 template <int BITS, int TM, int TN, int CW, int G, int PROD, int KA, int KM, int NM>

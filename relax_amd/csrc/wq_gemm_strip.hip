@@ -33,6 +33,20 @@ __device__ __forceinline__ void static_for_p(F&& f) {
     static_for_p<B + 1, E>(f);
   }
 }
+
+// Requests straight into LDS and the wait for them, as in the streamed GEMM.  The compiler does not see the wait states that a request
+// needs behind a vector instruction which writes its scalar operands, so `lds`, `r` and `soff` have to be computed by scalar instructions
+// alone (a branch on the way, and it refuses or moves one over right in front).
+__device__ __forceinline__ void dma_b128(uint32_t lds, uint32_t voff, rsrc_t r, uint32_t soff) {
+  asm volatile("s_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds" ::"{m0}"(lds), "v"(voff), "s"(r), "s"(soff) : "memory");
+}
+[[maybe_unused]] __device__ __forceinline__ void dma_u16(uint32_t lds, uint32_t voff, rsrc_t r, uint32_t soff) {
+  asm volatile("s_nop 0\n\tbuffer_load_ushort %1, %2, %3 offen lds" ::"{m0}"(lds), "v"(voff), "s"(r), "s"(soff) : "memory");
+}
+template <int N>
+__device__ __forceinline__ void wait_dma() {
+  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
+}
 }  // namespace
 
 // R8 blocks of 8 rows, T tiles of 16 columns.

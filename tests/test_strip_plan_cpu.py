@@ -64,3 +64,12 @@ def test_both_layouts_choose_alike_and_the_build_is_there(ask):
                                               (4, 64, 37, 4096, 4096), (8, 128, 37, 2048, 2048 + 64), (8, 32, 37, 2048, 2048)])
 def test_not_where_it_does_not_apply(ask, bits, group, m, n, k):
     assert ask(bits, group, m, n, k, 0) == 0
+
+
+def test_requests_into_lds_take_m0_as_an_operand():
+    import re
+
+    asm = re.findall(r"asm volatile\((.*?)\);", open(os.path.join(CSRC, "wq_gemm_strip.hip")).read(), re.S)
+    requests = [a for a in asm if "offen lds" in a]
+    assert len(requests) == 2 and all('::"{m0}"(lds)' in a for a in requests)
+    assert not any(re.search(r"\bm0\b", a.split("::")[0]) for a in asm)
