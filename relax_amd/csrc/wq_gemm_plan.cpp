@@ -36,7 +36,9 @@ struct TileCost {
   float start, tile, loop, loaded, odd, split, window, spread;
 };
 
-constexpr TileCost kStreamCost[2][2][7] = {
+// (The tiles of 96 columns, fitted to 1,700 timings of up to 256 rows, are the fastest on 16400 - 24576 columns, where 64-column tiles are more than
+// a round and 128-column ones much less: 17 - 64 rows 0.82 - 0.93 of the time there.  K is not split in them.)
+constexpr TileCost kStreamCost[2][2][9] = {
     {{  // int4, canonical
          {kStream128x256, 128, 256, 0.00f, 5.47f, 2.244f, 1.157f, 8.60f, 0.f, 0.f, 0.f},
          {kStream128x128, 128, 128, 0.00f, 5.68f, 1.212f, 0.494f, 4.15f, 4.12f, 1.383f, 0.31f},
@@ -44,7 +46,9 @@ constexpr TileCost kStreamCost[2][2][7] = {
          {kStream64x128, 64, 128, 1.14f, 3.71f, 0.836f, 0.291f, 2.00f, 2.45f, 0.747f, 1.16f},
          {kStream64x64, 64, 64, 1.47f, 3.12f, 0.520f, 0.181f, 0.00f, 1.75f, 0.450f, 0.19f},
          {kStream32x64, 32, 64, 1.10f, 2.44f, 0.459f, 0.065f, 0.03f, 1.75f, 0.275f, 0.24f},
-         {kStream32x128, 32, 128, 1.12f, 3.11f, 0.742f, 0.152f, 0.52f, 1.99f, 0.461f, 0.35f}},
+         {kStream32x128, 32, 128, 1.12f, 3.11f, 0.742f, 0.152f, 0.52f, 1.99f, 0.461f, 0.35f},
+         {kStream64x96, 64, 96, 0.00f, 5.00f, 0.650f, 0.338f, 0.00f, 0.f, 0.f, 0.f},
+         {kStream32x96, 32, 96, 1.18f, 3.16f, 0.584f, 0.146f, 0.03f, 0.f, 0.f, 0.f}},
      {  // int4, tile-major
          {kStream128x256, 128, 256, 0.00f, 6.00f, 2.483f, 1.013f, 10.16f, 0.f, 0.f, 0.f},
          {kStream128x128, 128, 128, 0.29f, 5.37f, 1.339f, 0.471f, 3.49f, 3.97f, 1.275f, 0.65f},
@@ -52,7 +56,9 @@ constexpr TileCost kStreamCost[2][2][7] = {
          {kStream64x128, 64, 128, 1.11f, 3.78f, 0.902f, 0.262f, 1.90f, 2.52f, 0.802f, 0.53f},
          {kStream64x64, 64, 64, 1.53f, 2.96f, 0.577f, 0.176f, 0.00f, 1.86f, 0.453f, 0.06f},
          {kStream32x64, 32, 64, 1.45f, 2.23f, 0.490f, 0.069f, 0.15f, 1.62f, 0.246f, 0.36f},
-         {kStream32x128, 32, 128, 1.21f, 3.22f, 0.786f, 0.108f, 0.63f, 1.96f, 0.473f, 0.22f}}},
+         {kStream32x128, 32, 128, 1.21f, 3.22f, 0.786f, 0.108f, 0.63f, 1.96f, 0.473f, 0.22f},
+         {kStream64x96, 64, 96, 1.65f, 3.01f, 0.774f, 0.284f, 0.00f, 0.f, 0.f, 0.f},
+         {kStream32x96, 32, 96, 2.12f, 2.40f, 0.608f, 0.170f, 0.03f, 0.f, 0.f, 0.f}}},
     {{  // int8, canonical
          {kStream128x256, 128, 256, 2.45f, 0.00f, 3.575f, 0.733f, 8.60f, 0.f, 0.f, 0.f},
          {kStream128x128, 128, 128, 0.00f, 4.75f, 1.419f, 0.474f, 4.15f, 4.03f, 1.378f, 1.04f},
@@ -60,7 +66,9 @@ constexpr TileCost kStreamCost[2][2][7] = {
          {kStream64x128, 64, 128, 1.79f, 1.69f, 1.201f, 0.192f, 2.00f, 2.61f, 0.798f, 1.83f},
          {kStream64x64, 64, 64, 1.79f, 2.47f, 0.608f, 0.161f, 0.00f, 1.87f, 0.479f, 0.57f},
          {kStream32x64, 32, 64, 1.43f, 2.01f, 0.519f, 0.063f, 0.03f, 1.74f, 0.324f, 0.47f},
-         {kStream32x128, 32, 128, 1.21f, 2.71f, 0.907f, 0.097f, 0.52f, 1.99f, 0.458f, 1.00f}},
+         {kStream32x128, 32, 128, 1.21f, 2.71f, 0.907f, 0.097f, 0.52f, 1.99f, 0.458f, 1.00f},
+         {kStream64x96, 64, 96, 0.31f, 4.29f, 0.754f, 0.692f, 0.00f, 0.f, 0.f, 0.f},
+         {kStream32x96, 32, 96, 1.68f, 2.64f, 0.582f, 0.289f, 0.03f, 0.f, 0.f, 0.f}},
      {  // int8, tile-major
          {kStream128x256, 128, 256, 1.75f, 3.44f, 3.984f, 0.646f, 10.07f, 0.f, 0.f, 0.f},
          {kStream128x128, 128, 128, 0.00f, 6.12f, 1.392f, 0.518f, 3.27f, 3.28f, 1.206f, 0.46f},
@@ -68,7 +76,9 @@ constexpr TileCost kStreamCost[2][2][7] = {
          {kStream64x128, 64, 128, 1.65f, 3.14f, 1.186f, 0.223f, 1.87f, 2.27f, 0.609f, 1.04f},
          {kStream64x64, 64, 64, 1.91f, 2.95f, 0.698f, 0.191f, 0.00f, 1.70f, 0.422f, 0.19f},
          {kStream32x64, 32, 64, 1.52f, 2.32f, 0.625f, 0.047f, 0.01f, 1.54f, 0.288f, 0.44f},
-         {kStream32x128, 32, 128, 1.90f, 2.67f, 1.236f, 0.000f, 0.59f, 1.32f, 0.402f, 1.29f}}},
+         {kStream32x128, 32, 128, 1.90f, 2.67f, 1.236f, 0.000f, 0.59f, 1.32f, 0.402f, 1.29f},
+         {kStream64x96, 64, 96, 1.06f, 3.78f, 1.129f, 0.376f, 0.00f, 0.f, 0.f, 0.f},
+         {kStream32x96, 32, 96, 1.23f, 3.34f, 0.825f, 0.138f, 0.03f, 0.f, 0.f, 0.f}}},
 };
 
 // The direct-weight kernel's 128 x 256 (variant 2), 64 x 256 (4) and 64 x 128 (5) tiles in the same terms (from 65 rows on).
@@ -253,7 +263,7 @@ GemmPlan plan_stream(const Problem& p, bool may_split) {
   const int layout = layout_of(p);
   const int cu = cu_count(), macros = ceil_div(p.k, 256);
   const bool odd = p.n % 2 != 0;
-  for (int i = 0; i < 7; ++i) {
+  for (int i = 0; i < 9; ++i) {
     const TileCost &own = kStreamCost[p.bits == 8][layout][i], &other = kStreamCost[p.bits == 8][1 - layout][i];
     const int64_t tiles = (int64_t)ceil_div(p.m, own.bm) * ceil_div(p.n, own.bn);
     // a window has at least two steps of 256 k; up to an eighth more windows than CUs

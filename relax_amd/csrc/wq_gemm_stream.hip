@@ -30,8 +30,9 @@
 // 27648 x 5120 at 99 71.7 -> 65.3, 5120 x 5120 at 256 29.5 -> 25.7.  int4 64 x 128 has enough in flight and gains from two K
 // groups instead of four (half of the exchange at the end): 12288 x 4096 at 37 rows 20.2 -> 18.7.  32-row tiles for up to 32
 // rows (half of the MFMAs and of the activation traffic; a remainder of up to 32 rows as well): int4 12288 x 4096 at 20 rows
-// 14.0 -> 11.8, 22016 x 4096 21.1 -> 17.8, int8 27648 x 5120 at 32 rows 41.5 -> 32.7 us.  Level or behind: deeper rings elsewhere,
-// reading fragments two slices ahead from LDS, one column wave, not requesting rows past M.
+// 14.0 -> 11.8, 22016 x 4096 21.1 -> 17.8, int8 27648 x 5120 at 32 rows 41.5 -> 32.7 us.  96 columns for
+// matrices of more than one round of 64-column tiles and far less than one of 128-column tiles: int4 22016 x 4096 at 20 / 37
+// rows (230 tiles, not 172) 18.7 / 22.5 -> 17.8 / 21.4, 18243 x 4352 at 59 0.85 of the time.  Level or behind: deeper rings elsewhere, reading fragments two slices ahead from LDS, one column wave, not requesting rows past M.
 #include <algorithm>
 #include <atomic>
 #include <type_traits>
@@ -801,6 +802,8 @@ bool launch_gemm_stream_bits(const Problem& p, int variant, int ksplit, const Sp
       WQ_STREAM(kStream64x64, kAllBuilds, 2, 1, 2, 4, 4, 128, 256, 3)
       WQ_STREAM(kStream32x64, kAllBuilds, 1, 1, 2, 4, 4, 128, 256, 3)
       WQ_STREAM(kStream32x128, kAllBuilds, 1, 2, 2, 4, 4, 128, 256, 3)
+      WQ_STREAM(kStream64x96, kWholeOnly, 2, 1, 3, 4, 4, 128, 256, 3)
+      WQ_STREAM(kStream32x96, kWholeOnly, 1, 1, 3, 4, 4, 128, 256, 3)
     }
   } else {
     switch (variant) {
@@ -811,6 +814,8 @@ bool launch_gemm_stream_bits(const Problem& p, int variant, int ksplit, const Sp
       WQ_STREAM(kStream64x64, kAllBuilds, 2, 1, 2, 4, 4, 128, 256, 3)
       WQ_STREAM(kStream32x64, kAllBuilds, 1, 1, 2, 4, 4, 128, 256, 3)
       WQ_STREAM(kStream32x128, kAllBuilds, 1, 2, 2, 4, 4, 128, 256, 3)
+      WQ_STREAM(kStream64x96, kWholeOnly, 2, 1, 3, 4, 4, 128, 256, 3)
+      WQ_STREAM(kStream32x96, kWholeOnly, 1, 1, 3, 4, 4, 128, 256, 3)
     }
   }
   return false;

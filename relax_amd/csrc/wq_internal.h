@@ -61,7 +61,7 @@ bool launch_gemm_pipe(const Problem& p, int group_shift, int variant);
 // The streamed GEMM (wq_gemm_stream.hip): its tiles, an explicit launch, and the one its cost model picks (wq_gemm_plan.cpp)
 // -- K split over workgroups where `workspace` has room for that and it pays -- unless another kernel's time on the problem,
 // `other_us`, is less.  1 launched, 0 not its problem, -1 failure.
-enum { kStream128x256 = 1, kStream128x128, kStream256x256, kStream64x128, kStream64x64, kStream32x64, kStream32x128 };
+enum { kStream128x256 = 1, kStream128x128, kStream256x256, kStream64x128, kStream64x64, kStream32x64, kStream32x128, kStream64x96, kStream32x96 };
 bool gemm_stream_applicable(const Problem& p);
 // A workspace for K in windows over workgroups: the caller's, or one of the library's own, whose launches are numbered and
 // write their number to `done[tile]`, in host memory, when a tile's partial sums have been read.
