@@ -71,7 +71,9 @@ __device__ __forceinline__ void wait_dma() {
 }
 }  // namespace
 
-template <int BITS, int TM, int TN, int CW, int G, int PROD, int KA, int KM, int NM>
+// SV: scales come 16 bytes of a row at a time, eight groups, and only where a macro step begins such a piece or a window; the other
+// macro steps send the same number of requests, out of range, into a place nobody reads.
+template <int BITS, int TM, int TN, int CW, int G, int PROD, int KA, int KM, int NM, bool SV>
 struct StreamShape {
   static constexpr int kBM = TM * 32, kBN = CW * TN * 32, kWaves = CW * G, kThreads = (kWaves + PROD) * 64;
   static constexpr int kIssuers = PROD > 0 ? PROD : kWaves;  // wavefronts that send requests
@@ -82,13 +84,14 @@ struct StreamShape {
   static constexpr int kARow = KA * 2;                 // bytes of an activation row per stage
   static constexpr int kWRow = kKM * BITS / 8;         // packed bytes of a weight row per macro step
   static constexpr int kSub = kKM / 32;                // scales of a row per macro step (one dword per 32 k)
-  static constexpr int kABytes = kBM * kARow, kWBytes = kBN * kWRow, kSBytes = kBN * kSub * 4;
-  static constexpr int kQA = kABytes / 1024, kQW = kWBytes / 1024, kQS = kSBytes / 256;  // requests
+  static constexpr int kSRow = SV ? 16 : kSub * 4;     // bytes of a row's scales in LDS
+  static constexpr int kABytes = kBM * kARow, kWBytes = kBN * kWRow, kSBytes = SV ? (kBN * 16 + 1023) / 1024 * 1024 : kBN * kSRow;
+  static constexpr int kQA = kABytes / 1024, kQW = kWBytes / 1024, kQS = kSBytes / (SV ? 1024 : 256);  // requests
   static constexpr int kNA = kQA / kIssuers;                                    // ... of one of them
   static constexpr int kNW = (kQW + kIssuers - 1) / kIssuers;
   static constexpr int kNS = (kQS + kIssuers - 1) / kIssuers;
   static constexpr int kNWS = kNW + kNS;
-  static constexpr bool kDummy = kQW % kIssuers != 0 || kQS % kIssuers != 0;
+  static constexpr bool kDummy = SV || kQW % kIssuers != 0 || kQS % kIssuers != 0;
   static constexpr int kLdsMax = 160 * 1024 - (kDummy ? 1024 : 0);
   static constexpr int kMacros = NM;                      // macro steps in the ring
   static constexpr int kRoom = (kLdsMax - kMacros * (kWBytes + kSBytes)) / kABytes;
@@ -124,11 +127,12 @@ struct StreamShape {
 __device__ __forceinline__ int stream_swizzle(int row, int chunks) { return (row / (16 / chunks)) % chunks; }
 
 // The requests of one wavefront: request q of an operand fills 1 KB of its LDS area (64 dwords for scales).
-template <class C, int BITS, int TN, bool TILED>
+template <class C, int BITS, int TN, bool TILED, bool SV>
 struct StreamRequests {
   static constexpr int R = C::kIssuers;
   uint32_t av[C::kNA], wv[C::kNW], sv[C::kNS];
-  int a_k, w_k, s_sub, me, k_end, group_log2;
+  int a_k, w_k, s_sub, me, k_begin, k_end, group_log2;
+  int s_place = 0, s_fill = 0;  // SV: place in the ring of the last piece of scales, and whether this macro step begins one
   uint32_t lds0;
   rsrc_t rx, rw, rs;
 
@@ -172,10 +176,11 @@ struct StreamRequests {
         }
       }
     }
-    s_sub = lane % C::kSub;
+    s_sub = SV ? 0 : lane % C::kSub;
+    constexpr int SPR = SV ? 1 : C::kSub;  // lanes of a request that ask for a row's scales
 #pragma unroll
     for (int i = 0; i < C::kNS; ++i) {
-      const int r = (me + i * R) * (64 / C::kSub) + lane / C::kSub;
+      const int r = (me + i * R) * (64 / SPR) + lane / SPR;
       const int n = n0 + matrix_row(r);
       if (r >= C::kBN || n >= N) sv[i] = kStreamOob;
       else if constexpr (TILED && BITS == 4) sv[i] = ((uint32_t)n >> 4) * (row_bytes / 128u) * 256u + (((uint32_t)s_sub >> 1) * 16u + ((uint32_t)n & 15u)) * 4u + ((uint32_t)s_sub & 1u) * 2u;
@@ -192,12 +197,22 @@ struct StreamRequests {
   }
   // request P of the weights and scales of the macro step from k0 on, into place `ring` of their rings
   template <int P>
-  __device__ __forceinline__ void issue_ws(int k0, uint32_t ring) const {
+  __device__ __forceinline__ void issue_ws(int k0, uint32_t ring) {
     if constexpr (P < C::kNW) {
       const int q = me + P * R;
       const bool mine = C::kQW % R == 0 || q < C::kQW;
       const uint32_t byte = k0 < k_end ? (uint32_t)k0 * BITS / 8u : 0u, off = TILED ? (byte >> 7) * 2048u + ((byte >> 5) & 3u) * 256u : byte;
       dma_b128(lds0 + (mine ? C::kWBase + ring * C::kWBytes + (uint32_t)q * 1024u : (uint32_t)C::kDummyBase), k0 + w_k < k_end ? wv[P] : kStreamOob, rw, off);
+    } else if constexpr (SV) {
+      constexpr int i = P - C::kNW;
+      const int q = me + i * R;
+      if constexpr (i == 0) {
+        s_fill = k0 < k_end && (k0 == k_begin || (k0 & ((8 << group_log2) - 1)) == 0);
+        if (k0 == k_begin) s_place = 0;
+        else if (s_fill) s_place = s_place + 1 == C::kMacros ? 0 : s_place + 1;
+      }
+      dma_b128(lds0 + (s_fill && q < C::kQS ? C::kSBase + (uint32_t)s_place * C::kSBytes + (uint32_t)q * 1024u : (uint32_t)C::kDummyBase),
+               s_fill ? sv[i] : kStreamOob, rs, s_fill ? (uint32_t)(k0 >> (group_log2 + 3)) * 16u : 0u);
     } else {
       constexpr int i = P - C::kNW;
       const int q = me + i * R;
@@ -210,7 +225,7 @@ struct StreamRequests {
   }
   // What stages -(kStages - 1) .. -1 would have issued, in their order; weights due before that first.
   template <int SPM, int KA, int KM>
-  __device__ __forceinline__ void prologue(int k_begin) const {
+  __device__ __forceinline__ void prologue() {
     auto issue_macro = [&](auto mm) __attribute__((always_inline)) {
       static_for_s<0, C::kNWS>([&](auto piece) __attribute__((always_inline)) { issue_ws<decltype(piece)::value>(k_begin + decltype(mm)::value * KM, decltype(mm)::value); });
     };
@@ -230,12 +245,13 @@ struct StreamRequests {
 // workgroup -- slower, but without a workspace and with the sums in the same order, bit for bit.
 enum { kWhole, kSplit, kSerial };
 
-template <int BITS, int TM, int TN, int CW, int G, int PROD, int KA, int KM, int NM, bool TILED, int MODE>
+template <int BITS, int TM, int TN, int CW, int G, int PROD, int KA, int KM, int NM, bool TILED, int MODE, bool SV>
 __global__ __launch_bounds__((CW * G + PROD) * 64, 1) void wq_gemm_stream_kernel(
     const half_t* __restrict__ x, const uint32_t* __restrict__ wq, const half_t* __restrict__ scales, int M, int N, int K,
     int shift_and_zero, int tiles_m, int tiles_n, int ksplit, half_t* y, const Epilogue ep, float* partials,
     unsigned int* counters, uint32_t* done, uint32_t launch) {
-  using C = StreamShape<BITS, TM, TN, CW, G, PROD, KA, KM, NM>;
+  using C = StreamShape<BITS, TM, TN, CW, G, PROD, KA, KM, NM, SV>;
+  static_assert(!(TILED && SV), "tile-major scales lie as they are read");
   constexpr int BM = C::kBM, BN = C::kBN, WAVES = C::kWaves, SPM = C::kSPM, NS = C::kSlices;
   const int group_log2 = shift_and_zero & 0xFF, zero_point = (shift_and_zero >> 8) & 0xFF;  // group = 1 << group_log2 >= 32
   const bool gated = (shift_and_zero >> 16) & 1;
@@ -268,7 +284,8 @@ __global__ __launch_bounds__((CW * G + PROD) * 64, 1) void wq_gemm_stream_kernel
   constexpr int kExchangeBarriers = G == 1 ? 0 : 2 * ((G + C::kTargets - 1) / C::kTargets);
 
   using std::integral_constant;
-  StreamRequests<C, BITS, TN, TILED> req;
+  StreamRequests<C, BITS, TN, TILED, SV> req;
+  req.k_begin = k_begin;
   req.k_end = k_end;
   req.group_log2 = group_log2;
   req.lds0 = lds0;
@@ -284,7 +301,7 @@ __global__ __launch_bounds__((CW * G + PROD) * 64, 1) void wq_gemm_stream_kernel
       __builtin_amdgcn_s_setprio(2);
       req.init(wave - WAVES, lane, m0, n0, M, N, K, gated);
       for (;;) {
-        req.template prologue<SPM, KA, KM>(k_begin);
+        req.template prologue<SPM, KA, KM>();
         __builtin_amdgcn_s_barrier();
         asm volatile("" ::: "memory");
         uint32_t abuf = (C::kStages - 1) * C::kABytes, ring = C::kMacros - 1;
@@ -307,7 +324,7 @@ __global__ __launch_bounds__((CW * G + PROD) * 64, 1) void wq_gemm_stream_kernel
         if constexpr (MODE == kSerial) {
           if (++ks == S) return;
           for (int i = 0; i < kExchangeBarriers + 1; ++i) __builtin_amdgcn_s_barrier();
-          k_begin = ks * per_window * KM;
+          req.k_begin = k_begin = ks * per_window * KM;
           req.k_end = k_end = min(k_begin + per_window * KM, K);
         } else {
           return;
@@ -316,7 +333,7 @@ __global__ __launch_bounds__((CW * G + PROD) * 64, 1) void wq_gemm_stream_kernel
     }
   } else {
     req.init(wave, lane, m0, n0, M, N, K, gated);
-    req.template prologue<SPM, KA, KM>(k_begin);
+    req.template prologue<SPM, KA, KM>();
   }
 
   // ---- LDS reads of this lane: KL contiguous k of a stage, from (grp * kKG + fh * KL) on ------------------------
@@ -333,7 +350,7 @@ __global__ __launch_bounds__((CW * G + PROD) * 64, 1) void wq_gemm_stream_kernel
       const int byte = (t * KA + kl0) * BITS / 8 + v * 16;
       w_rd[t][v] = C::kWBase + (uint32_t)wrow * C::kWRow + (uint32_t)(((byte / 16) ^ stream_swizzle(wrow, C::kWRow / 16)) << 4) + (byte & 15);
     }
-    s_rd[t] = C::kSBase + (uint32_t)(wrow * C::kSub + (t * KA + kl0) / 32) * 4u;
+    s_rd[t] = C::kSBase + (uint32_t)(wrow * C::kSRow) + (SV ? (uint32_t)((t * KA + kl0) >> group_log2) * 2u : (uint32_t)((t * KA + kl0) / 32) * 4u);
   }
 
   const Q4Consts qc = make_q4_consts(zero_point);
@@ -352,10 +369,11 @@ __global__ __launch_bounds__((CW * G + PROD) * 64, 1) void wq_gemm_stream_kernel
     half_t s[TN];
   };
   Words words[2];
-  auto read_words = [&](Words& d, uint32_t ring, auto tt) __attribute__((always_inline)) {
+  // (`soff`: the macro step's scales)
+  auto read_words = [&](Words& d, uint32_t ring, uint32_t soff, auto tt) __attribute__((always_inline)) {
     constexpr int t = decltype(tt)::value;
     const unsigned char* const wb = smem + ring * C::kWBytes;
-    const unsigned char* const sb = smem + ring * C::kSBytes;
+    const unsigned char* const sb = smem + soff;
 #pragma unroll
     for (int j = 0; j < TN; ++j) {
       if constexpr (WB >= 16) {
@@ -371,7 +389,7 @@ __global__ __launch_bounds__((CW * G + PROD) * 64, 1) void wq_gemm_stream_kernel
       } else {
         d.w[j][0] = *reinterpret_cast<const uint32_t*>(wb + w_rd[t][0] + j * 32 * C::kWRow);
       }
-      d.s[j] = *reinterpret_cast<const half_t*>(sb + s_rd[t] + j * 32 * C::kSub * 4);
+      d.s[j] = *reinterpret_cast<const half_t*>(sb + s_rd[t] + j * 32 * C::kSRow);
     }
   };
   // Weight pair PR (of four) of a lane's eight k of slice KK, column tile J, in two halves: integers with the float16
@@ -405,8 +423,11 @@ __global__ __launch_bounds__((CW * G + PROD) * 64, 1) void wq_gemm_stream_kernel
         for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.f;
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
-    read_words(words[0], 0, integral_constant<int, 0>{});
-    if constexpr (NS == 1) read_words(words[1], 0, integral_constant<int, 1>{});
+    // (SV: the group of a k0, which its macro step begins or lies within, is the sum of k0's and of the lane's own)
+    auto in_piece = [&](int k0) __attribute__((always_inline)) { return (uint32_t)((k0 >> group_log2) & 7) * 2u; };
+    uint32_t s_base = 0, s_off = SV ? in_piece(k_begin) : 0;
+    read_words(words[0], 0, s_off, integral_constant<int, 0>{});
+    if constexpr (NS == 1) read_words(words[1], 0, s_off, integral_constant<int, 1>{});
 #pragma unroll
     for (int i = 0; i < TM; ++i) a[0][i] = *reinterpret_cast<const half8_t*>(smem + a_rd[0] + i * 32 * C::kARow);
     static_for_s<0, PAIRS>([&](auto q) __attribute__((always_inline)) {
@@ -419,6 +440,11 @@ __global__ __launch_bounds__((CW * G + PROD) * 64, 1) void wq_gemm_stream_kernel
     uint32_t abuf = 0, abuf_issue = (C::kStages - 1) * C::kABytes, ring = 0;
     for (int k0 = k_begin; k0 < k_end; k0 += KM) {
       const uint32_t ring_next = ring + 1 == C::kMacros ? 0 : ring + 1, ring_issue = ring == 0 ? C::kMacros - 1 : ring - 1;
+      uint32_t s_next = ring_next * C::kSBytes;
+      if constexpr (SV) {
+        if (((k0 + KM) & ((8 << group_log2) - 1)) == 0) s_base = s_base + C::kSBytes == C::kMacros * C::kSBytes ? 0 : s_base + C::kSBytes;
+        s_next = s_base + in_piece(k0 + KM);
+      }
       static_for_s<0, SPM>([&](auto tc) __attribute__((always_inline)) {
         constexpr int t = decltype(tc)::value;
         const uint32_t abuf_next = abuf + C::kABytes == C::kStages * C::kABytes ? 0 : abuf + C::kABytes;
@@ -437,7 +463,7 @@ __global__ __launch_bounds__((CW * G + PROD) * 64, 1) void wq_gemm_stream_kernel
                 a[q & 1][i], __builtin_bit_cast(half8_t, *reinterpret_cast<const u32x4*>(b[q & 1][j])), acc[i][j], 0, 0, 0);
             if constexpr (s < TM)
               a[(q + 1) & 1][s] = *reinterpret_cast<const half8_t*>(smem + (kk1 == 0 ? abuf_next : abuf) + a_rd[kk1] + s * 32 * C::kARow);
-            if constexpr (s == 0 && kk2 == 0) read_words(words[t2 & 1], t2 >= SPM ? ring_next : ring, integral_constant<int, t2 % SPM>{});
+            if constexpr (s == 0 && kk2 == 0) read_words(words[t2 & 1], t2 >= SPM ? ring_next : ring, t2 >= SPM ? s_next : s_off, integral_constant<int, t2 % SPM>{});
             if constexpr (PROD == 0) {
               // requests of later stages, evenly over the slots: weights and scales first
               constexpr int slot = kk * SLOTS + s, WS = t == 0 ? C::kNWS : 0, ALL = WS + C::kNA;
@@ -464,6 +490,7 @@ __global__ __launch_bounds__((CW * G + PROD) * 64, 1) void wq_gemm_stream_kernel
         abuf = abuf_next;
       });
       ring = ring_next;
+      s_off = s_next;
     }
     if constexpr (PROD == 0) wait_dma<0>();
     __builtin_amdgcn_s_barrier();  // the last requests (all out of range) have landed
@@ -743,12 +770,12 @@ __global__ __launch_bounds__((CW * G + PROD) * 64, 1) void wq_gemm_stream_kernel
 
 namespace {
 
-template <int BITS, int TM, int TN, int CW, int G, int PROD, int KA, int KM, int NM, bool TILED, int MODE>
+template <int BITS, int TM, int TN, int CW, int G, int PROD, int KA, int KM, int NM, bool TILED, int MODE, bool SV>
 bool launch_stream(const Problem& p, int ksplit, const SplitSpace& space) {
-  using C = StreamShape<BITS, TM, TN, CW, G, PROD, KA, KM, NM>;
+  using C = StreamShape<BITS, TM, TN, CW, G, PROD, KA, KM, NM, SV>;
   const int tiles_m = (int)((p.m + C::kBM - 1) / C::kBM), tiles_n = (int)((p.n + C::kBN - 1) / C::kBN);
   static std::atomic<bool> lds_ok[kMaxDevices];
-  const auto kernel = wq_gemm_stream_kernel<BITS, TM, TN, CW, G, PROD, KA, KM, NM, TILED, MODE>;
+  const auto kernel = wq_gemm_stream_kernel<BITS, TM, TN, CW, G, PROD, KA, KM, NM, TILED, MODE, SV>;
   if (!ensure_dynamic_lds((const void*)kernel, C::kLds, lds_ok)) return false;
   int group_log2 = 0;
   while ((1 << group_log2) < p.group) ++group_log2;
@@ -765,19 +792,32 @@ bool launch_stream(const Problem& p, int ksplit, const SplitSpace& space) {
 // accumulators would not fit the registers.
 enum { kWholeOnly, kWholeAndSplit, kAllBuilds, kSerialOnly };
 
+// Scales in pieces of eight groups: their rows have to be whole 4-byte words (an even number of groups), and no macro step may reach
+// past a row's end, where the next row's scales, not zeros, would follow.  Where a piece lasts for more than one macro step the rows'
+// lines are asked for that much less often: a scale request touches as many lines as one for eight times the weights, and the L1
+// has room for 32 KB of lines in flight.  us, with two bytes a request and with pieces: int8 99 x 15360 x 5120 / 27648 x 5120 39.0 / 52.6 ->
+// 35.8 / 47.9, 256 x 15360 x 5120 / 5120 x 13824 51.0 / 53.2 -> 47.7 / 48.7; means over 140 problems: int8 17 - 64 rows 0.94, 65 - 256 0.95, above
+// 0.97 (groups of 32 and 64 0.96 - 0.98), int4 groups of 64 and 128 0.95 - 1.0.  Where it does not -- int4 groups of 32 in macro steps of 256 -- the
+// lines are as many and the times level, 0.9 - 1.1.
+bool scale_pieces(const Problem& p, int macro_step) { return !p.tiled && p.k % 256 == 0 && (p.k / p.group) % 2 == 0 && 8 * p.group > macro_step; }
+
+template <int BITS, int MODE, int... SHAPE>
+bool launch_stream_mode(const Problem& p, int ksplit, const SplitSpace& ws) {
+  if (p.tiled) return launch_stream<BITS, SHAPE..., true, MODE, false>(p, ksplit, ws);
+  constexpr int shape[] = {SHAPE...};
+  return scale_pieces(p, shape[6]) ? launch_stream<BITS, SHAPE..., false, MODE, true>(p, ksplit, ws) : launch_stream<BITS, SHAPE..., false, MODE, false>(p, ksplit, ws);
+}
+
 template <int BITS, int BUILDS, int... SHAPE>
 bool launch_stream_any(const Problem& p, int ksplit, const SplitSpace& ws) {
   if constexpr (BUILDS == kWholeAndSplit || BUILDS == kAllBuilds) {
-    if (ksplit > 1 && ws.base != nullptr)
-      return p.tiled ? launch_stream<BITS, SHAPE..., true, kSplit>(p, ksplit, ws) : launch_stream<BITS, SHAPE..., false, kSplit>(p, ksplit, ws);
+    if (ksplit > 1 && ws.base != nullptr) return launch_stream_mode<BITS, kSplit, SHAPE...>(p, ksplit, ws);
   }
   if constexpr (BUILDS == kAllBuilds || BUILDS == kSerialOnly) {
-    if (ksplit > 1)
-      return p.tiled ? launch_stream<BITS, SHAPE..., true, kSerial>(p, ksplit, ws) : launch_stream<BITS, SHAPE..., false, kSerial>(p, ksplit, ws);
+    if (ksplit > 1) return launch_stream_mode<BITS, kSerial, SHAPE...>(p, ksplit, ws);
   }
   if constexpr (BUILDS != kSerialOnly) {
-    if (ksplit == 1)
-      return p.tiled ? launch_stream<BITS, SHAPE..., true, kWhole>(p, 1, ws) : launch_stream<BITS, SHAPE..., false, kWhole>(p, 1, ws);
+    if (ksplit == 1) return launch_stream_mode<BITS, kWhole, SHAPE...>(p, 1, ws);
   }
   return false;
 }
