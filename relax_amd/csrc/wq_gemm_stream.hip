@@ -798,8 +798,11 @@ enum { kWholeOnly, kWholeAndSplit, kAllBuilds, kSerialOnly };
 // has room for 32 KB of lines in flight.  us, with two bytes a request and with pieces: int8 99 x 15360 x 5120 / 27648 x 5120 39.0 / 52.6 ->
 // 35.8 / 47.9, 256 x 15360 x 5120 / 5120 x 13824 51.0 / 53.2 -> 47.7 / 48.7; means over 140 problems: int8 17 - 64 rows 0.94, 65 - 256 0.95, above
 // 0.97 (groups of 32 and 64 0.96 - 0.98), int4 groups of 64 and 128 0.95 - 1.0.  Where it does not -- int4 groups of 32 in macro steps of 256 -- the
-// lines are as many and the times level, 0.9 - 1.1.
-bool scale_pieces(const Problem& p, int macro_step) { return !p.tiled && p.k % 256 == 0 && (p.k / p.group) % 2 == 0 && 8 * p.group > macro_step; }
+// lines are as many and a seventh of the requests goes: above 1024 rows 0.985 (18 problems; a 4096 / 11008 layer at 2048 rows 787 -> 777),
+// 513 - 1024 0.995, below level with single problems 5 - 7 % behind, which so stay.
+bool scale_pieces(const Problem& p, int macro_step) {
+  return !p.tiled && p.k % 256 == 0 && (p.k / p.group) % 2 == 0 && (8 * p.group > macro_step || p.m > 512);
+}
 
 template <int BITS, int MODE, int... SHAPE>
 bool launch_stream_mode(const Problem& p, int ksplit, const SplitSpace& ws) {

@@ -15,7 +15,8 @@ from tests.test_gpu_parity import _dev, assert_close  # noqa: E402
 
 @pytest.mark.parametrize("variant", [31, 32, 33, 34, 35, 36, 37, 38, 39])
 @pytest.mark.parametrize("bits,m,n,k,group", [(8, 20, 67, 256, 128), (8, 65, 130, 2304, 128), (8, 33, 97, 1280, 32), (8, 33, 97, 1536, 256), (8, 20, 40, 1280, 256),
-                                              (4, 40, 129, 2816, 128), (4, 20, 70, 1536, 64), (4, 33, 65, 1280, 128), (4, 17, 60, 768, 256)])
+                                              (4, 40, 129, 2816, 128), (4, 20, 70, 1536, 64), (4, 33, 65, 1280, 128), (4, 17, 60, 768, 256),
+                                              (4, 515, 130, 768, 32), (4, 600, 66, 1280, 32)])
 def test_pieces_at_their_edges(variant, bits, m, n, k, group):
     stream.test_every_tile_shape_at_its_edges(variant, bits, m, n, k, group)
 
