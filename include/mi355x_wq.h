@@ -196,6 +196,8 @@ MI355X_WQ_API int mi355x_wq_matmul_tiled_ex(const mi355x_wq_desc* desc, const vo
  * 16 KB of arrival counters at the head, then a float32 partial tile per tile and K window (1 KB in the decode kernel), so one
  * workspace sized for the largest projection serves projections of every shape; 0 if no tail's call would split on it
  * (then the call equals mi355x_wq_matmul_fused / _tiled and leaves the workspace alone), -1 on an invalid descriptor.
+ * A call of 17 - 256 rows that one round of column strips serves best (17 x 4096 x 4096 int4) needs none and leaves it alone; the size is
+ * then the one that it would split on otherwise.
  *
  * From 17 rows on the same call splits K for the streamed GEMM where its tiles leave CUs idle (e.g. 99 rows x 5120 columns: 40
  * tiles of 128 x 128): two to eight workgroups per tile, each on a window of at least 512 of K, 8 to 64 KB of float32

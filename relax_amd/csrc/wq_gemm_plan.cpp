@@ -144,10 +144,10 @@ float skinny_cost(const Problem& p) {
   return c.by_tiles[r].start + steps * (c.by_tiles[r].step + c.by_tiles[r].rows * rb) + c.block * rb;
 }
 
-// The standard groups and whole steps of K: a request for weights covers a row's whole line, one for scales 16 bytes of them (int4), and
-// nothing is past a row's end.  (A workgroup's column tiles are within the matrix from its 128 columns on.)
+// The standard groups and whole steps of K: a request for weights covers a row's whole line, one for scales 16 bytes of a row that begins
+// on a 4-byte word, and no step is past a row's end.  (A workgroup's column tiles are within the matrix from its 128 columns on.)
 bool gemm_strip_applicable(const Problem& p) {
-  return p.m <= kStripMaxM && p.n >= 128 && p.n <= (4 << 20) && standard_group(p) && p.k % (1024 / p.bits) == 0;
+  return p.m <= kStripMaxM && p.n >= 128 && p.n <= (4 << 20) && standard_group(p) && p.k % 256 == 0;
 }
 
 int strip_row_blocks(int64_t m) {
@@ -185,7 +185,7 @@ GemmPlan plan_strip(const Problem& p) {
   const int cu = cu_count(), blocks = strip_row_blocks(p.m), slices = ceil_div(p.m, blocks * 8), layout = layout_of(p);
   const float rows = (float)blocks, stages = (float)p.k / 512.f;
   for (int t = 1; t <= kStripMaxTiles; ++t) {
-    if (!strip_fits(p.bits, blocks, t)) break;
+    if (!strip_fits(blocks, t)) break;
     const int64_t groups = (int64_t)ceil_div(p.n, t * 16) * slices;
     const float rounds = (float)((groups + cu - 1) / cu), full = (float)groups / (float)cu, tiles = (float)t;
     auto cost = [&](const StripCost& c) {

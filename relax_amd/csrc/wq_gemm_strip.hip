@@ -14,7 +14,8 @@
 // T column tiles.  MFMAs are 16 x 16 x 32, so that 37 rows pay for 48 and not for 64.  The partial sums meet in LDS, in the order of the wavefronts.
 //
 // Measured against the kernels it takes over from, us, weights from memory: int4 4096 x 4096 at 20 / 37 rows 8.1 / 11.4 -> 7.3 / 9.3, 12288 x 4096
-// 12.4 / 15.5 -> 11.3 / 13.9 (with the weights in the last-level cache 4096 x 4096 8.0 / 10.9 -> 6.4 / 7.9).
+// 12.4 / 15.5 -> 11.3 / 13.9 (with the weights in the last-level cache 4096 x 4096 8.0 / 10.9 -> 6.4 / 7.9).  int8 by pieces of scales, which with two
+// bytes a step were half of the lines that weights and scales touch: 0.94 of the time on 406 timings of 131 problems.
 #include <algorithm>
 #include <atomic>
 #include <type_traits>
@@ -49,18 +50,20 @@ __device__ __forceinline__ void wait_dma() {
 }
 }  // namespace
 
-// R8 blocks of 8 rows, T tiles of 16 columns.
-template <int BITS, int R8, int T>
+// R8 blocks of 8 rows, T tiles of 16 columns.  Scales are asked for with every step's weights, but for int8 on canonical weights, whose
+// rows have one of two bytes a step and a line to be touched for it: 16 bytes, eight steps, at a time.
+template <int BITS, int R8, int T, bool TILED>
 struct StripShape {
+  static constexpr bool kPieces = BITS == 8 && !TILED;
   static constexpr int MB = (R8 + 1) / 2;                         // MFMA row blocks
   static constexpr int kStep = 1024 / BITS;                       // k of a row's 128-byte line of weights
   static constexpr int kSPS = kStep / 64;                         // stages (64 k, 128 bytes of an activation row) per step
-  static constexpr int kNA = R8, kNWS = 2 * T + 1;                // requests a stage / step
-  static constexpr int kABytes = R8 * 1024, kSBase = T * 2048, kWBytes = kSBase + (BITS == 4 ? 1024 : 256);
+  static constexpr int kNA = R8, kNWS = 2 * T + (kPieces ? 0 : 1);                // requests a stage / step
+  static constexpr int kABytes = R8 * 1024, kSBase = T * 2048, kWBytes = kSBase + 1024;
   static constexpr int kWBase = 2 * kABytes;                      // two stages of activations in the ring
   static constexpr int kWaveBytes = std::max(kWBase + kWBytes, MB * T * 1024);  // (a wavefront's partial sums at the end)
   static constexpr int kLds = kStripWaves * kWaveBytes;
-  static_assert(kWBase + kWBytes == strip_ring_bytes(BITS, R8, T) && kLds <= 160 * 1024, "shape");
+  static_assert(kWBase + kWBytes == strip_ring_bytes(R8, T) && kLds <= 160 * 1024, "shape");
   // Weights and scales of the next step are requested in a step's first stage (int8) or its first two (int4), ahead of the
   // stage's activations.
   static constexpr int kWsStages = kSPS / 2;
@@ -72,7 +75,7 @@ template <int BITS, int R8, int T, bool TILED>
 __global__ __launch_bounds__(kStripWaves * 64, 1) void wq_gemm_strip_kernel(
     const half_t* __restrict__ x, const uint32_t* __restrict__ wq, const half_t* __restrict__ scales, int M, int N, int K,
     int zero_and_gated, half_t* y, const Epilogue ep) {
-  using C = StripShape<BITS, R8, T>;
+  using C = StripShape<BITS, R8, T, TILED>;
   using std::integral_constant;
   constexpr int MB = C::MB, SPS = C::kSPS, UNITS = 2 * T;
   const int zero_point = zero_and_gated & 0xFF, gated = (zero_and_gated >> 8) & 1;
@@ -126,10 +129,19 @@ __global__ __launch_bounds__(kStripWaves * 64, 1) void wq_gemm_strip_kernel(
     } else if constexpr (BITS == 4) {
       dma_b128(ring0 + C::kWBase + C::kSBase, in ? sv : kOobOffset, rs, in ? (TILED ? (uint32_t)k0 : (uint32_t)k0 / 16u) : 0u);
     } else {
-      dma_u16(ring0 + C::kWBase + C::kSBase, in ? sv : kOobOffset, rs, in ? (TILED ? (uint32_t)k0 / 4u : (uint32_t)k0 / 64u) : 0u);
+      dma_u16(ring0 + C::kWBase + C::kSBase, in ? sv : kOobOffset, rs, in ? (uint32_t)k0 / 4u : 0u);
     }
   };
   // the first step's, and what the stages before the first would have issued, in their order
+  // (int8, canonical: eight scales of every row from an even group on, 4-byte words)
+  int s_first = 0;
+  auto issue_piece = [&](int k0) __attribute__((always_inline)) {
+    s_first = (k0 >> 7) & ~1;
+    dma_b128(ring0 + C::kWBase + C::kSBase, sv, rs, (uint32_t)s_first * 2u);
+  };
+  if constexpr (C::kPieces) {
+    if (count > 0) issue_piece(k_begin);
+  }
   static_for_p<0, C::kNWS>([&](auto pc) __attribute__((always_inline)) { issue_ws(pc, k_begin); });
   static_for_p<0, 2>([&](auto tc) __attribute__((always_inline)) {
     static_for_p<0, C::kNA>([&](auto pc) __attribute__((always_inline)) { issue_a(pc, k_begin + decltype(tc)::value * 64, decltype(tc)::value * C::kABytes); });
@@ -166,7 +178,7 @@ __global__ __launch_bounds__(kStripWaves * 64, 1) void wq_gemm_strip_kernel(
     const int chunk = BITS == 4 ? h * 2 + (kq >> 1) : h * 4 + kq, inner = BITS == 4 ? (kq & 1) * 8 : 0;
     w_rd[h] = (TILED ? (chunk & 1) * 1024 + ((chunk >> 1) * 16 + col) * 16 : col * 128 + ((chunk ^ ((col >> 1) & 7)) << 4)) + inner;
   }
-  const uint32_t s_rd = C::kSBase + (BITS == 4 && !TILED ? col * 16 : col * 4);
+  const uint32_t s_rd = C::kSBase + (TILED ? col * 4 : col * 16);
   const uint32_t s_shift = BITS == 4 ? (kq >> 1) * 16 : 0;
 
   const Q4Consts qc = make_q4_consts(zero_point);
@@ -186,7 +198,7 @@ __global__ __launch_bounds__(kStripWaves * 64, 1) void wq_gemm_strip_kernel(
 #pragma unroll
       for (int i = 0; i < MB; ++i) a[h][j][i] = *reinterpret_cast<const half8_t*>(my + h * C::kABytes + a_rd[j] + i * 2048);
   };
-  auto read_step = [&]() __attribute__((always_inline)) {
+  auto read_step = [&](int k0) __attribute__((always_inline)) {
     const unsigned char* const wb = my + C::kWBase;
 #pragma unroll
     for (int j = 0; j < T; ++j) {
@@ -209,7 +221,7 @@ __global__ __launch_bounds__(kStripWaves * 64, 1) void wq_gemm_strip_kernel(
 #pragma unroll
         for (int e = 0; e < 4; ++e) sc[j][e] = q[e];
       } else {
-        sc[j][0] = *reinterpret_cast<const uint16_t*>(wb + s_rd + j * 64);
+        sc[j][0] = *reinterpret_cast<const uint16_t*>(C::kPieces ? wb + s_rd + j * 256 + ((k0 >> 7) - s_first) * 2 : wb + s_rd + j * 64);
       }
     }
   };
@@ -227,7 +239,7 @@ __global__ __launch_bounds__(kStripWaves * 64, 1) void wq_gemm_strip_kernel(
   };
 
   wait_dma<C::kNA>();
-  read_step();
+  read_step(k_begin);
   read_a(integral_constant<int, 0>{});
   static_for_p<0, 4>([&](auto pc) __attribute__((always_inline)) { b[0][decltype(pc)::value] = convert(integral_constant<int, 0>{}, integral_constant<int, 0>{}, pc); });
   asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
@@ -236,6 +248,10 @@ __global__ __launch_bounds__(kStripWaves * 64, 1) void wq_gemm_strip_kernel(
   // ---- K loop (program order is issue order: sched_barrier after every MFMA).  A stage multiplies what has been read, sends the
   // requests of later ones over its MFMAs, and before its last unit waits for and reads the next stage's operands.
   for (int k0 = k_begin; k0 < k_end; k0 += C::kStep) {
+    if constexpr (C::kPieces) {
+      // (not among the requests that are counted: where it is sent, the first wait is for it as well)
+      if (k0 + C::kStep < k_end && ((k0 + C::kStep) >> 7) - s_first > 7) issue_piece(k0 + C::kStep);
+    }
     static_for_p<0, SPS>([&](auto hc) __attribute__((always_inline)) {
       constexpr int h = decltype(hc)::value, h1 = (h + 1) % SPS;
       static_for_p<0, UNITS>([&](auto qc_) __attribute__((always_inline)) {
@@ -243,7 +259,7 @@ __global__ __launch_bounds__(kStripWaves * 64, 1) void wq_gemm_strip_kernel(
         if constexpr (q == UNITS - 1) {
           wait_dma<C::requests(h)>();
           read_a(integral_constant<int, (h + 1) & 1>{});
-          if constexpr (h1 == 0) read_step();
+          if constexpr (h1 == 0) read_step(k0 + C::kStep);
           __builtin_amdgcn_sched_barrier(0);
         }
         static_for_p<0, MB>([&](auto ic) __attribute__((always_inline)) {
@@ -334,7 +350,7 @@ namespace {
 
 template <int BITS, int R8, int T, bool TILED>
 bool launch_strip(const Problem& p) {
-  using C = StripShape<BITS, R8, T>;
+  using C = StripShape<BITS, R8, T, TILED>;
   static std::atomic<bool> lds_ok[kMaxDevices];
   const auto kernel = wq_gemm_strip_kernel<BITS, R8, T, TILED>;
   if (!ensure_dynamic_lds((const void*)kernel, C::kLds, lds_ok)) return false;
@@ -348,7 +364,7 @@ bool launch_strip(const Problem& p) {
 
 template <int BITS, int R8, int T>
 bool launch_strip_layout(const Problem& p) {
-  if constexpr (strip_fits(BITS, R8, T)) return p.tiled ? launch_strip<BITS, R8, T, true>(p) : launch_strip<BITS, R8, T, false>(p);
+  if constexpr (strip_fits(R8, T)) return p.tiled ? launch_strip<BITS, R8, T, true>(p) : launch_strip<BITS, R8, T, false>(p);
   return false;
 }
 

@@ -88,9 +88,9 @@ int64_t gemm_workspace_bytes(const Problem& p, bool skinny_family);
 // LDS holds its rings (and its partial sums) for so many column tiles of 16, and an explicit launch with that many.
 constexpr int64_t kStripMaxM = 256;
 constexpr int kStripWaves = 8, kStripMaxTiles = 4;
-constexpr int strip_ring_bytes(int bits, int row_blocks, int tiles) { return row_blocks * 2048 + tiles * 2048 + (bits == 4 ? 1024 : 256); }
-constexpr bool strip_fits(int bits, int row_blocks, int tiles) {
-  return strip_ring_bytes(bits, row_blocks, tiles) * kStripWaves <= 160 * 1024 && (row_blocks + 1) / 2 * tiles * 1024 * kStripWaves <= 160 * 1024;
+constexpr int strip_ring_bytes(int row_blocks, int tiles) { return row_blocks * 2048 + tiles * 2048 + 1024; }
+constexpr bool strip_fits(int row_blocks, int tiles) {
+  return strip_ring_bytes(row_blocks, tiles) * kStripWaves <= 160 * 1024 && (row_blocks + 1) / 2 * tiles * 1024 * kStripWaves <= 160 * 1024;
 }
 bool gemm_strip_applicable(const Problem& p);
 int strip_row_blocks(int64_t m);

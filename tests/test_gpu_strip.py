@@ -18,15 +18,15 @@ def fits(bits, m, variant):
     slices = -(-m // 64)
     blocks = max(3, -(-(-(-m // slices)) // 8))
     blocks = 8 if blocks == 7 else blocks
-    return 8 * (blocks * 2048 + (variant - 40) * 2048 + (1024 if bits == 4 else 256)) <= 160 * 1024
+    return 8 * (blocks * 2048 + (variant - 40) * 2048 + 1024) <= 160 * 1024
 
 
 @pytest.mark.parametrize("variant", VARIANTS)
 @pytest.mark.parametrize("bits,m,n,k", [
     (4, 1, 128, 256), (4, 17, 129, 2048), (4, 24, 257, 2304), (4, 25, 130, 1024), (4, 33, 191, 4096), (4, 40, 2001, 1280), (4, 41, 144, 2560),
     (4, 49, 300, 512), (4, 64, 128, 4352), (4, 65, 258, 2304), (4, 129, 200, 1024), (4, 256, 136, 1280),
-    (8, 2, 131, 128), (8, 17, 128, 1152), (8, 32, 515, 1280), (8, 37, 190, 2048), (8, 48, 1001, 896), (8, 57, 128, 3200), (8, 72, 250, 1024),
-    (8, 200, 128, 1152)])
+    (8, 2, 131, 256), (8, 17, 128, 1280), (8, 32, 515, 2304), (8, 37, 190, 2048), (8, 48, 1001, 768), (8, 57, 128, 3328), (8, 72, 250, 1024),
+    (8, 200, 128, 1280)])
 def test_every_build_at_its_edges(variant, bits, m, n, k):
     import relax_amd
 
@@ -52,7 +52,22 @@ def test_every_build_at_its_edges(variant, bits, m, n, k):
         assert np.array_equal(run(dx, wt, st, bits, g, variant, tiled_n=n).view(np.uint16), plain.view(np.uint16)), "tile-major"
 
 
-@pytest.mark.parametrize("bits,m,n,k,variant", [(4, 37, 200, 2304, 43), (4, 70, 144, 1024, 41), (8, 20, 130, 1152, 44)])
+@pytest.mark.parametrize("variant", VARIANTS)
+@pytest.mark.parametrize("k", [8448, 8704, 16640])
+def test_int8_scales_past_a_wavefronts_first_piece(variant, k):
+    """A wavefront's share of K is more than the eight steps of a piece of scales: the bits of the tile-major build, which asks for them
+    step by step (and the oracle, at the bound of the other calls of long K)."""
+    import relax_amd
+
+    x, wq, s, g = O.make_case(k, 33, 160, k, 8)
+    dx, dw, ds = _dev(x), _dev(wq), _dev(s)
+    plain = run(dx, dw, ds, 8, g, variant)
+    wt, st = relax_amd.wq_tile_weights(dw, ds, 8, g)
+    assert np.array_equal(run(dx, wt, st, 8, g, variant, tiled_n=160).view(np.uint16), plain.view(np.uint16))
+    assert_close(plain, c_oracle.wq_matmul(x, wq, s, 8, g, nthreads=8), (variant, k), ulp_fraction=0.005)
+
+
+@pytest.mark.parametrize("bits,m,n,k,variant", [(4, 37, 200, 2304, 43), (4, 70, 144, 1024, 41), (8, 20, 130, 1280, 44)])
 def test_what_is_not_finite_stays_in_its_row_and_column(bits, m, n, k, variant):
     """Rows and columns meet in LDS rows, fragments and slices: an infinite or NaN activation changes its row only, an infinite or NaN
     scale its column only, and the outputs past the end keep what they held."""

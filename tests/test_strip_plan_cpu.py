@@ -19,7 +19,7 @@ extern "C" int ask(int bits, int group, int64_t m, int64_t n, int64_t k, int til
   p.tiled = tiled != 0;
   const wq::GemmPlan strip = wq::plan_strip(p);
   const bool ahead = wq::strip_ahead(p, strip, wq::plan_stream(p, true));
-  if (ahead && (strip.variant < 1 || strip.variant > 4 || !wq::strip_fits(bits, wq::strip_row_blocks(m), strip.variant))) return -1;
+  if (ahead && (strip.variant < 1 || strip.variant > 4 || !wq::strip_fits(wq::strip_row_blocks(m), strip.variant))) return -1;
   return ahead ? strip.variant : 0;
 }
 """
@@ -50,10 +50,10 @@ def test_the_faster_one_is_taken(ask, bits, m, n, k, tiles, strip_us, other_us):
 
 def test_both_layouts_choose_alike_and_the_build_is_there(ask):
     taken = 0
-    for bits, step in ((4, 256), (8, 128)):
+    for bits in (4, 8):
         for m in (17, 24, 25, 33, 40, 41, 49, 56, 57, 64, 65, 72, 100, 129, 191, 256):
             for n in (128, 130, 1024, 2304, 4096, 5121, 8192, 12288, 16384, 22528):
-                for k in (1024, 1024 + step, 2816, 4096, 8192, 13824):
+                for k in (1024, 1024 + 256, 2816, 4096, 8192, 13824):
                     got = [ask(bits, 32 if bits == 4 else 128, m, n, k, tiled) for tiled in (0, 1)]
                     assert got[0] == got[1] >= 0, (bits, m, n, k)
                     taken += got[0] > 0
@@ -61,7 +61,7 @@ def test_both_layouts_choose_alike_and_the_build_is_there(ask):
 
 
 @pytest.mark.parametrize("bits,group,m,n,k", [(4, 32, 16, 4096, 4096), (4, 32, 257, 1024, 1024), (4, 32, 37, 127, 4096), (4, 32, 37, 4096, 4096 + 128),
-                                              (4, 64, 37, 4096, 4096), (8, 128, 37, 2048, 2048 + 64), (8, 32, 37, 2048, 2048)])
+                                              (4, 64, 37, 4096, 4096), (8, 128, 37, 2048, 2048 + 128), (8, 32, 37, 2048, 2048)])
 def test_not_where_it_does_not_apply(ask, bits, group, m, n, k):
     assert ask(bits, group, m, n, k, 0) == 0
 
