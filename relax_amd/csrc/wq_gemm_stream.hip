@@ -32,7 +32,8 @@
 // rows (half of the MFMAs and of the activation traffic; a remainder of up to 32 rows as well): int4 12288 x 4096 at 20 rows
 // 14.0 -> 11.8, 22016 x 4096 21.1 -> 17.8, int8 27648 x 5120 at 32 rows 41.5 -> 32.7 us.  96 columns for
 // matrices of more than one round of 64-column tiles and far less than one of 128-column tiles: int4 22016 x 4096 at 20 / 37
-// rows (230 tiles, not 172) 18.7 / 22.5 -> 17.8 / 21.4, 18243 x 4352 at 59 0.85 of the time.  Level or behind: deeper rings elsewhere, reading fragments two slices ahead from LDS, one column wave, not requesting rows past M.
+// rows (230 tiles, not 172) 18.7 / 22.5 -> 17.8 / 21.4, 18243 x 4352 at 59 0.85 of the time.  Level or behind: deeper rings
+// elsewhere, reading fragments two slices ahead from LDS, one column wave, not requesting rows past M.
 #include <algorithm>
 #include <atomic>
 #include <type_traits>
@@ -799,7 +800,8 @@ enum { kWholeOnly, kWholeAndSplit, kAllBuilds, kSerialOnly };
 // 35.8 / 47.9, 256 x 15360 x 5120 / 5120 x 13824 51.0 / 53.2 -> 47.7 / 48.7; means over 140 problems: int8 17 - 64 rows 0.94, 65 - 256 0.95, above
 // 0.97 (groups of 32 and 64 0.96 - 0.98), int4 groups of 64 and 128 0.95 - 1.0.  Where it does not -- int4 groups of 32 in macro steps of 256 -- the
 // lines are as many and a seventh of the requests goes, which pays where 128 x 256 tiles fill the chip and its power is the limit (a
-// 4096 / 11008 layer at 2048 rows 747.6 -> 737.6), and not where a launch waits for few tiles' requests (333 x 3712 x 4608 22.2 -> 24.0, 1183 x 1536 x 12288 58.3 -> 60.7).
+// 4096 / 11008 layer at 2048 rows 747.6 -> 737.6), and not where a launch waits for few tiles' requests (333 x 3712 x 4608 22.2 ->
+// 24.0, 1183 x 1536 x 12288 58.3 -> 60.7).
 bool scale_pieces(const Problem& p, int rows, int columns, int macro_step) {
   if (p.tiled || p.k % 256 != 0 || (p.k / p.group) % 2 != 0) return false;
   const int64_t tiles = (p.m + rows - 1) / rows * ((p.n + columns - 1) / columns);
