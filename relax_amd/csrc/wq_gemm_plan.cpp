@@ -155,26 +155,27 @@ int strip_row_blocks(int64_t m) {
   return blocks < 3 ? 3 : blocks == 7 ? 8 : blocks;
 }
 
-// The strip kernel's time: start; per round of workgroups what does not depend on K and what a block of eight rows adds to a
-// column tile; per stage of K (512 k: 64 for each of the eight wavefronts) and round column tiles and blocks, and what a full chip adds to
-// both; and, past eight stages, what the wavefronts' drifting apart costs.  Fitted to 2,070 timings of 1,385 problems (17 - 256 rows, N 512 - 28000, K 1024 -
-// 14000, weights and activations from memory) within 6 %.
+// The strip kernel's time for one round of workgroups: start; what a block of eight rows adds, and the exchange of the sums of more than one column
+// tile; per 512 of K what it costs by itself and per MFMA block of 16 rows and column tile; the same on the busiest SIMD, whose two
+// wavefronts have a quarter of the steps of K between them, rounded up to a whole one, per block of rows and column tile (3840 x 1280 int4 at 57 rows has
+// five steps and takes 6.3 us, with four 5.4, with eight 6.5); per megabyte of weights; and, past 4096 of K, the wavefronts' drifting apart.
+// Fitted to 9,500 timings of 6,800 problems (17 - 256 rows, N 512 - 28000, K 1024 - 11000, weights from memory) within 4.4 %, and two per cent
+// below them: the other kernels' tables lie between their times with weights from memory and with weights in the last-level cache.
 //
 // Why the line lies where these costs put it: a CU reads all of its rows' activations once per strip, so the kernel is ahead where
 // one round of workgroups covers the matrix and K is short, and behind where K is long: then K split over workgroups reads a part of them.
 // us before and now: int4 4096 x 4096 at 20 / 37 rows 8.1 / 11.4 -> 7.3 / 9.3, 12288 x 4096 12.4 / 15.5 -> 11.3 / 13.9; not 4096 x 11008 at
-// 37 rows (15.8, here 21.5).  Means over the 1,385, the call's time against its time without this kernel, weights from memory: 17 - 64 rows
-// int4 0.95 (tile-major 0.92), int8 0.97 (0.97), 65 - 256 rows 0.96 and 0.98; with weights in the last-level cache 0.93 (0.88), 0.95 (0.93),
-// 0.94 and 0.95; always taking the fastest would be 1 % better.
+// 37 rows (15.8, here 21.5), nor more than a round.  Four column tiles in slices of rows are too few strips that read the weights twice
+// (int8 7424 x 3072 at 70 rows 14.0 us, 64 x 64 streamed tiles 12.6).
 namespace {
 struct StripCost {
-  float start, round, tiles, stage_tiles, stage_rows, loaded_tiles, loaded_rows, drift;
+  float start, rows, exchange, stage, stage_mfma, busy_rows, busy_tiles, megabyte, drift;
 };
 constexpr StripCost kStripCost[2][2] = {
-    {{1.721f, 1.020f, 0.095f, 0.137f, 0.062f, 0.112f, 0.032f, 0.133f},   // int4, canonical
-     {1.328f, 1.488f, 0.111f, 0.127f, 0.052f, 0.062f, 0.038f, 0.074f}},  // tile-major
-    {{1.376f, 1.163f, 0.066f, 0.145f, 0.091f, 0.226f, 0.010f, 0.200f},   // int8
-     {1.340f, 1.203f, 0.073f, 0.126f, 0.090f, 0.212f, 0.000f, 0.025f}},
+    {{1.976f, 0.152f, 0.142f, 0.259f, 0.027f, 0.051f, 0.043f, 0.102f, 0.087f},   // int4, canonical
+     {2.369f, 0.122f, 0.159f, 0.118f, 0.025f, 0.057f, 0.037f, 0.100f, 0.011f}},  // tile-major
+    {{2.279f, 0.161f, 0.087f, 0.180f, 0.032f, 0.057f, 0.067f, 0.071f, 0.030f},   // int8
+     {2.177f, 0.174f, 0.087f, 0.193f, 0.029f, 0.052f, 0.066f, 0.079f, 0.000f}},
 };
 }  // namespace
 
@@ -183,15 +184,16 @@ GemmPlan plan_strip(const Problem& p) {
   best.us = best.both_us = kNever;
   if (p.m <= 16 || !gemm_strip_applicable(p)) return best;
   const int cu = cu_count(), blocks = strip_row_blocks(p.m), slices = ceil_div(p.m, blocks * 8), layout = layout_of(p);
-  const float rows = (float)blocks, stages = (float)p.k / 512.f;
-  for (int t = 1; t <= kStripMaxTiles; ++t) {
-    if (!strip_fits(blocks, t)) break;
-    const int64_t groups = (int64_t)ceil_div(p.n, t * 16) * slices;
-    const float rounds = (float)((groups + cu - 1) / cu), full = (float)groups / (float)cu, tiles = (float)t;
+  const int step = 1024 / p.bits, steps = ceil_div(p.k, step), most = slices > 1 ? 3 : kStripMaxTiles;
+  const float rows = (float)blocks, mfma_rows = (float)((blocks + 1) / 2), stages = (float)p.k / 512.f, past = std::max(0.f, stages - 8.f);
+  const float busy = (float)((steps + 3) / 4 * step) / 128.f, megabytes = (float)(p.n * p.k) * (float)p.bits / 8e6f;
+  for (int t = 1; t <= most && strip_fits(blocks, t); ++t) {
+    const int groups = ceil_div(p.n, t * 16) * slices;
+    if (groups > cu) continue;
+    const float tiles = (float)t;
     auto cost = [&](const StripCost& c) {
-      const float drift = stages > 8.f ? (stages - 8.f) * c.drift : 0.f;
-      return c.start + rounds * (c.round + c.tiles * rows * tiles + stages * (c.stage_tiles * tiles + c.stage_rows * rows) + drift) +
-             stages * full * (c.loaded_tiles * tiles + c.loaded_rows * rows);
+      return c.start + c.rows * rows + c.exchange * tiles * (tiles - 1.f) + stages * (c.stage + c.stage_mfma * mfma_rows * tiles) +
+             busy * (c.busy_rows * rows + c.busy_tiles * tiles) + c.megabyte * megabytes + c.drift * past;
     };
     const float us = cost(kStripCost[p.bits == 8][layout]), both = us + cost(kStripCost[p.bits == 8][1 - layout]);
     if (both < best.both_us) best = GemmPlan{t, 1, us, both, groups, 0};
@@ -199,11 +201,12 @@ GemmPlan plan_strip(const Problem& p) {
   return best;
 }
 
-// By both layouts' times together, as the streamed kernel's tile, so that the sums are the same on either.  Three per cent to spare, and
-// from eight stages of K on, where both kernels' times scatter most, two more for each: of the 1,385 problems one is more than 3 % slower.
+// By both layouts' times together, as the streamed kernel's tile, so that the sums are the same on either.  Four per cent to spare, and
+// from 4096 of K on, where both kernels' times scatter most, half a per cent more for every 512.  Of 6,834
+// problems (those of the fit) it takes 2,178; the call's time against its time without this kernel, means over all of them: weights from memory 0.955, in the
+// last-level cache 0.934; 46 and 12 are more than 5 % slower.  Always taking the fastest would be 0.6 % better with weights from memory.
 bool strip_ahead(const Problem& p, const GemmPlan& strip, const GemmPlan& stream) {
-  const float stages = (float)p.k / 512.f;
-  return strip.both_us < (0.97f - 0.02f * std::max(0.f, stages - 8.f)) * stream.both_us;
+  return strip.both_us < (0.96f - 0.005f * std::max(0.f, (float)p.k / 512.f - 8.f)) * stream.both_us;
 }
 
 bool gemm_direct_applicable(const Problem& p) { return p.k % 256 == 0 && standard_group(p) && gemm_pipe_applicable(p); }
