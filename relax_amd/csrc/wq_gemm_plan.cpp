@@ -286,6 +286,24 @@ GemmPlan plan_stream(const Problem& p, bool may_split) {
   return best;
 }
 
+// The streamed kernel's scales in pieces of eight groups: their rows have to be whole 4-byte words (an even number of groups), and no macro step may reach
+// past a row's end, where the next row's scales, not zeros, would follow.  Where a piece lasts for more than one macro step the rows'
+// lines are asked for that much less often: a scale request touches as many lines as one for eight times the weights, and the L1
+// has room for 32 KB of lines in flight.  us, with two bytes a request and with pieces: int8 99 x 15360 x 5120 / 27648 x 5120 39.0 / 52.6 ->
+// 35.8 / 47.9, 256 x 15360 x 5120 / 5120 x 13824 51.0 / 53.2 -> 47.7 / 48.7; means over 2,300 problems, weights from memory and in the last-level
+// cache: int8 64 x 128 tiles 0.94 / 1.01, 128 x 128 0.98 / 0.99, int4 groups of 64 and 128 0.97 - 0.99 from 64 x 128 on, 64 x 64 tiles of either 0.99 / 1.0.
+// Not on 32 x 64 tiles, whose rows of scales are one request for four wavefronts that all send one: int4 groups of 64 and 128 1.03 / 1.03
+// (20 x 2304 x 5632 8.8 -> 9.2 us), int8 up to 40 MB 1.0 / 1.015; above, where memory is the limit, int8 0.97 / 1.0 (20 x 14592 x 5632, 0.95), and so those have them.
+// Where a piece does not last -- int4 groups of 32 in macro steps of 256 -- the lines are as many and seven of 32 requests go, which pays where
+// 128 x 256 tiles fill the chip and its power is the limit (a 4096 / 11008 layer at 2048 rows 747.6 -> 737.6; 192 - 255 tiles of 256 CUs 0.988 / 0.985
+// on 96 problems, more 0.985), and not where a launch waits for few tiles' requests (333 x 3712 x 4608 22.2 -> 24.0, 1183 x 1536 x 12288 58.3 -> 60.7).
+bool stream_scale_pieces(const Problem& p, int rows, int columns, int macro_step) {
+  if (!stream_pieces_built(p.bits, rows, columns) || p.tiled || p.k % 256 != 0 || (p.k / p.group) % 2 != 0) return false;
+  if (rows == 32 && columns == 64 && p.n * p.k <= 40000000) return false;
+  const int64_t tiles = (int64_t)ceil_div(p.m, rows) * ceil_div(p.n, columns);
+  return 8 * p.group > macro_step || (columns == 256 && 4 * tiles >= 3 * cu_count());
+}
+
 // Up to 16 rows of canonical weights: where the streamed kernel's 32-row tiles, K split over workgroups, are ahead of the decode
 // kernel and the register-activation kernel.  Those have every CU walk all of K for its 16 columns, so each stages all of
 // the activations, in phases once they exceed the LDS; a split CU reads a part of them for more columns.  The lines by 9,500 timings

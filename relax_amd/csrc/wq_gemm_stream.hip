@@ -793,26 +793,14 @@ bool launch_stream(const Problem& p, int ksplit, const SplitSpace& space) {
 // accumulators would not fit the registers.
 enum { kWholeOnly, kWholeAndSplit, kAllBuilds, kSerialOnly };
 
-// Scales in pieces of eight groups: their rows have to be whole 4-byte words (an even number of groups), and no macro step may reach
-// past a row's end, where the next row's scales, not zeros, would follow.  Where a piece lasts for more than one macro step the rows'
-// lines are asked for that much less often: a scale request touches as many lines as one for eight times the weights, and the L1
-// has room for 32 KB of lines in flight.  us, with two bytes a request and with pieces: int8 99 x 15360 x 5120 / 27648 x 5120 39.0 / 52.6 ->
-// 35.8 / 47.9, 256 x 15360 x 5120 / 5120 x 13824 51.0 / 53.2 -> 47.7 / 48.7; means over 140 problems: int8 17 - 64 rows 0.94, 65 - 256 0.95, above
-// 0.97 (groups of 32 and 64 0.96 - 0.98), int4 groups of 64 and 128 0.95 - 1.0.  Where it does not -- int4 groups of 32 in macro steps of 256 -- the
-// lines are as many and a seventh of the requests goes, which pays where 128 x 256 tiles fill the chip and its power is the limit (a
-// 4096 / 11008 layer at 2048 rows 747.6 -> 737.6), and not where a launch waits for few tiles' requests (333 x 3712 x 4608 22.2 ->
-// 24.0, 1183 x 1536 x 12288 58.3 -> 60.7).
-bool scale_pieces(const Problem& p, int rows, int columns, int macro_step) {
-  if (p.tiled || p.k % 256 != 0 || (p.k / p.group) % 2 != 0) return false;
-  const int64_t tiles = (p.m + rows - 1) / rows * ((p.n + columns - 1) / columns);
-  return 8 * p.group > macro_step || (columns == 256 && 4 * tiles >= 3 * cu_count());
-}
-
 template <int BITS, int MODE, int... SHAPE>
 bool launch_stream_mode(const Problem& p, int ksplit, const SplitSpace& ws) {
   if (p.tiled) return launch_stream<BITS, SHAPE..., true, MODE, false>(p, ksplit, ws);
-  constexpr int shape[] = {SHAPE...};
-  return scale_pieces(p, shape[0] * 32, shape[1] * shape[2] * 32, shape[6]) ? launch_stream<BITS, SHAPE..., false, MODE, true>(p, ksplit, ws) : launch_stream<BITS, SHAPE..., false, MODE, false>(p, ksplit, ws);
+  constexpr int shape[] = {SHAPE...}, rows = shape[0] * 32, columns = shape[1] * shape[2] * 32;
+  if constexpr (stream_pieces_built(BITS, rows, columns)) {
+    if (stream_scale_pieces(p, rows, columns, shape[6])) return launch_stream<BITS, SHAPE..., false, MODE, true>(p, ksplit, ws);
+  }
+  return launch_stream<BITS, SHAPE..., false, MODE, false>(p, ksplit, ws);
 }
 
 template <int BITS, int BUILDS, int... SHAPE>

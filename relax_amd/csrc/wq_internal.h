@@ -63,6 +63,9 @@ bool launch_gemm_pipe(const Problem& p, int group_shift, int variant);
 // `other_us`, is less.  1 launched, 0 not its problem, -1 failure.
 enum { kStream128x256 = 1, kStream128x128, kStream256x256, kStream64x128, kStream64x64, kStream32x64, kStream32x128, kStream64x96, kStream32x96 };
 bool gemm_stream_applicable(const Problem& p);
+// Whether a tile of so many rows and columns, `macro_step` of K at a time, asks for `p`'s scales in pieces; and the tiles that have a build for it.
+constexpr bool stream_pieces_built(int bits, int rows, int columns) { return bits == 8 || rows > 32 || columns > 64; }
+bool stream_scale_pieces(const Problem& p, int rows, int columns, int macro_step);
 // A workspace for K in windows over workgroups: the caller's, or one of the library's own, whose launches are numbered and
 // write their number to `done[tile]`, in host memory, when a tile's partial sums have been read.
 struct SplitSpace {

@@ -17,6 +17,9 @@ bool gemm_pipe_applicable(const Problem& p) { return p.k %% 64 == 0; }
 extern "C" int64_t plan_bytes(int bits, int group, int64_t m, int64_t n, int64_t k) {
   return wq::plan_stream(wq::Problem{nullptr, nullptr, nullptr, nullptr, m, n, k, bits, group, 0, nullptr}, true).bytes;
 }
+extern "C" int pieces(int bits, int group, int64_t m, int64_t n, int64_t k, int rows, int columns, int macro_step) {
+  return wq::stream_scale_pieces(wq::Problem{nullptr, nullptr, nullptr, nullptr, m, n, k, bits, group, 0, nullptr}, rows, columns, macro_step);
+}
 extern "C" int ask(int bits, int group, int64_t m, int64_t n, int64_t k, int tiled, int may_split, float* us) {
   wq::Problem p{nullptr, nullptr, nullptr, nullptr, m, n, k, bits, group, 0, nullptr};
   p.tiled = tiled != 0;
@@ -42,7 +45,8 @@ def ask(tmp_path_factory):
         us = (C.c_float * 3)()
         r = f(bits, group or (32 if bits == 4 else 128), m, n, k, tiled, may_split, us)
         return r & 0xFF, r >> 8, dict(zip(("stream", "other", "skinny"), us))
-    call.plan_bytes = so.plan_bytes
+    so.pieces.argtypes = [C.c_int, C.c_int] + [C.c_int64] * 3 + [C.c_int] * 3
+    call.plan_bytes, call.pieces = so.plan_bytes, so.pieces
     return call
 
 
@@ -132,3 +136,20 @@ def test_the_workspace_query_is_the_size_of_the_split_that_runs(ask):
                             assert got == need > 16384, (bits, group, m, n, k, tiled)
                             split += 1
     assert split > 300
+
+
+# (bits, group, M, N, K, tile, macro step of it, us with two bytes a scale request, us in pieces of eight groups)
+SCALE_PIECES = [(4, 64, 20, 2304, 5632, 32, 64, 256, 8.8, 9.2), (4, 128, 95, 1545, 9728, 32, 64, 256, 11.9, 12.5), (8, 128, 87, 4608, 1536, 32, 64, 256, 6.17, 6.38),
+                (8, 128, 20, 14592, 5632, 32, 64, 256, 21.4, 20.3),
+                (8, 128, 99, 15360, 5120, 128, 128, 128, 39.0, 35.8), (8, 128, 99, 27648, 5120, 128, 128, 128, 52.6, 47.9),
+                (4, 32, 333, 3712, 4608, 128, 256, 256, 22.2, 24.0), (4, 32, 2048, 22016, 4096, 128, 256, 256, 364.0, 358.0)]
+
+
+@pytest.mark.parametrize("bits,group,m,n,k,rows,columns,macro_step,plain_us,pieces_us", SCALE_PIECES)
+def test_scale_pieces_where_they_were_the_faster(ask, bits, group, m, n, k, rows, columns, macro_step, plain_us, pieces_us):
+    assert bool(ask.pieces(bits, group, m, n, k, rows, columns, macro_step)) == (pieces_us < plain_us)
+
+
+@pytest.mark.parametrize("bits,group,k", [(8, 128, 1152), (4, 64, 4160), (8, 256, 256)])
+def test_no_scale_pieces_past_a_rows_end_or_off_the_word_grid(ask, bits, group, k):
+    assert not ask.pieces(bits, group, 4096, 4096, k, 128, 128, 128)
