@@ -370,11 +370,11 @@ __global__ __launch_bounds__((CW * G + PROD) * 64, 1) void wq_gemm_stream_kernel
     half_t s[TN];
   };
   Words words[2];
-  // (`soff`: the macro step's scales)
-  auto read_words = [&](Words& d, uint32_t ring, uint32_t soff, auto tt) __attribute__((always_inline)) {
+  // (`piece`: where the macro step's scales are if they come in pieces; else by its place in the ring, as its weights)
+  auto read_words = [&](Words& d, uint32_t ring, uint32_t piece, auto tt) __attribute__((always_inline)) {
     constexpr int t = decltype(tt)::value;
     const unsigned char* const wb = smem + ring * C::kWBytes;
-    const unsigned char* const sb = smem + soff;
+    const unsigned char* const sb = smem + (SV ? piece : ring * C::kSBytes);
 #pragma unroll
     for (int j = 0; j < TN; ++j) {
       if constexpr (WB >= 16) {
@@ -441,7 +441,7 @@ __global__ __launch_bounds__((CW * G + PROD) * 64, 1) void wq_gemm_stream_kernel
     uint32_t abuf = 0, abuf_issue = (C::kStages - 1) * C::kABytes, ring = 0;
     for (int k0 = k_begin; k0 < k_end; k0 += KM) {
       const uint32_t ring_next = ring + 1 == C::kMacros ? 0 : ring + 1, ring_issue = ring == 0 ? C::kMacros - 1 : ring - 1;
-      uint32_t s_next = ring_next * C::kSBytes;
+      uint32_t s_next = 0;
       if constexpr (SV) {
         if (((k0 + KM) & ((8 << group_log2) - 1)) == 0) s_base = s_base + C::kSBytes == C::kMacros * C::kSBytes ? 0 : s_base + C::kSBytes;
         s_next = s_base + in_piece(k0 + KM);
