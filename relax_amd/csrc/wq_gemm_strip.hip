@@ -37,7 +37,8 @@ __device__ __forceinline__ void static_for_p(F&& f) {
 
 // Requests straight into LDS and the wait for them, as in the streamed GEMM.  The compiler does not see the wait states that a request
 // needs behind a vector instruction which writes its scalar operands, so `lds`, `r` and `soff` have to be computed by scalar instructions
-// alone (a branch on the way, and it refuses or moves one over right in front).
+// alone (a branch on the way, and it refuses or moves one over right in front).  The built objects are read for that
+// (tests/test_lds_requests_cpu.py): five wait states in every request instead cost 1 - 3 %.
 __device__ __forceinline__ void dma_b128(uint32_t lds, uint32_t voff, rsrc_t r, uint32_t soff) {
   asm volatile("s_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds" ::"{m0}"(lds), "v"(voff), "s"(r), "s"(soff) : "memory");
 }
