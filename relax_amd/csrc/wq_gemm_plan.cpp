@@ -209,6 +209,13 @@ bool strip_ahead(const Problem& p, const GemmPlan& strip, const GemmPlan& stream
   return strip.both_us < (0.96f - 0.005f * std::max(0.f, (float)p.k / 512.f - 8.f)) * stream.both_us;
 }
 
+// The layouts' joint choice of the two, unless the other kernel is faster than what that would run.
+StreamedChoice choose_streamed(const Problem& p, const GemmPlan& strip, const GemmPlan& stream, float other_us) {
+  const bool ahead = strip_ahead(p, strip, stream);
+  if (other_us < (ahead ? strip.us : stream.us)) return kOtherKernel;
+  return ahead ? kStrips : kStreamedTiles;
+}
+
 bool gemm_direct_applicable(const Problem& p) { return p.k % 256 == 0 && standard_group(p) && gemm_pipe_applicable(p); }
 
 // Columns of 128 x 256 tiles that fill whole rounds of the CUs where the rest, at most half a round, is worth 64-row tiles

@@ -1,7 +1,6 @@
 // Host side of the streamed GEMM (wq_gemm_stream.hip): the planned launch and the library's own workspaces.
 #include <string.h>
 
-#include <algorithm>
 #include <mutex>
 
 #include "../../include/mi355x_wq.h"
@@ -141,10 +140,11 @@ int launch_gemm_stream_planned(const Problem& p, void* workspace, int64_t worksp
   const bool slot = plan.split > 1 && plan.bytes > workspace_bytes;
   if (slot && (p.m > 256 || captured(p))) plan = plan_stream(p, false);
   const GemmPlan strip = plan_strip(p);
-  const bool ahead = strip_ahead(p, strip, plan);
-  if (other_us < (ahead ? std::min(strip.us, plan.us) : plan.us)) return 0;
-  if (ahead) return launched(launch_gemm_strip(p, strip.variant), "strip");
-  return launch_plan(p, plan, workspace, slot);
+  switch (choose_streamed(p, strip, plan, other_us)) {
+    case kOtherKernel: return 0;
+    case kStrips: return launched(launch_gemm_strip(p, strip.variant), "strip");
+    default: return launch_plan(p, plan, workspace, slot);
+  }
 }
 
 namespace {

@@ -22,6 +22,13 @@ extern "C" int ask(int bits, int group, int64_t m, int64_t n, int64_t k, int til
   if (ahead && (strip.variant < 1 || strip.variant > 4 || !wq::strip_fits(wq::strip_row_blocks(m), strip.variant))) return -1;
   return ahead ? strip.variant : 0;
 }
+extern "C" int chosen(int bits, int group, int64_t m, int64_t n, int64_t k, int tiled, float other_us, float* us) {
+  wq::Problem p{nullptr, nullptr, nullptr, nullptr, m, n, k, bits, group, 0, nullptr};
+  p.tiled = tiled != 0;
+  const wq::GemmPlan strip = wq::plan_strip(p), stream = wq::plan_stream(p, true);
+  us[0] = other_us > 0.f ? other_us : wq::skinny_cost(p), us[1] = stream.us, us[2] = strip.us;
+  return wq::choose_streamed(p, strip, stream, us[0]);
+}
 """
 
 
@@ -31,8 +38,11 @@ def ask(tmp_path_factory):
     (d / "plan.cpp").write_text(WRAPPER % CSRC)
     subprocess.run(["g++", "-std=c++17", "-shared", "-fPIC", "-Wall", "-Werror", "-D__HIP_PLATFORM_AMD__", "-I/opt/rocm/include",
                     "-I" + CSRC, "-o", str(d / "plan.so"), str(d / "plan.cpp")], check=True)
-    f = C.CDLL(str(d / "plan.so")).ask
+    so = C.CDLL(str(d / "plan.so"))
+    f = so.ask
     f.argtypes = [C.c_int, C.c_int, C.c_int64, C.c_int64, C.c_int64, C.c_int]
+    so.chosen.argtypes = f.argtypes + [C.c_float, C.POINTER(C.c_float)]
+    f.chosen = so.chosen
     return f
 
 
@@ -66,6 +76,17 @@ def test_both_layouts_choose_alike_and_the_build_is_there(ask):
                                               (4, 64, 37, 4096, 4096), (8, 128, 37, 2048, 2048 + 128), (8, 32, 37, 2048, 2048)])
 def test_not_where_it_does_not_apply(ask, bits, group, m, n, k):
     assert ask(bits, group, m, n, k, 0) == 0
+
+
+@pytest.mark.parametrize("bits,m,n,k,other_us", [(4, 29, 3840, 5120, 0.0), (4, 26, 3840, 5120, 0.0), (4, 37, 4096, 4096, 8.0), (4, 37, 4096, 4096, 8.6), (8, 128, 1024, 2048, 0.0)])
+def test_the_other_kernel_is_compared_with_what_would_run(ask, bits, m, n, k, other_us):
+    """No kernel runs that is called slower than the other one, also where the strips are ahead of the streamed tiles on both
+    layouts together and behind them on this one."""
+    for tiled in (0, 1):
+        us = (C.c_float * 3)()
+        choice = ask.chosen(bits, 32 if bits == 4 else 128, m, n, k, tiled, other_us, us)
+        assert choice == 0 or us[choice] <= us[0], (choice, list(us))
+        assert (choice == 2) == (ask(bits, 32 if bits == 4 else 128, m, n, k, tiled) > 0 and us[2] <= us[0])
 
 
 def test_requests_into_lds_take_m0_as_an_operand():
