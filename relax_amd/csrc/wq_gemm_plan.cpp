@@ -179,26 +179,24 @@ constexpr StripCost kStripCost[2][2] = {
 };
 }  // namespace
 
+// (every column tile costs something: the fewest with which one round covers the matrix)
 GemmPlan plan_strip(const Problem& p) {
-  GemmPlan best;
-  best.us = best.both_us = kNever;
-  if (p.m <= 16 || !gemm_strip_applicable(p)) return best;
-  const int cu = cu_count(), blocks = strip_row_blocks(p.m), slices = ceil_div(p.m, blocks * 8), layout = layout_of(p);
-  const int step = 1024 / p.bits, steps = ceil_div(p.k, step), most = slices > 1 ? 3 : kStripMaxTiles;
-  const float rows = (float)blocks, mfma_rows = (float)((blocks + 1) / 2), stages = (float)p.k / 512.f, past = std::max(0.f, stages - 8.f);
-  const float busy = (float)((steps + 3) / 4 * step) / 128.f, megabytes = (float)(p.n * p.k) * (float)p.bits / 8e6f;
-  for (int t = 1; t <= most && strip_fits(blocks, t); ++t) {
-    const int groups = ceil_div(p.n, t * 16) * slices;
-    if (groups > cu) continue;
-    const float tiles = (float)t;
-    auto cost = [&](const StripCost& c) {
-      return c.start + c.rows * rows + c.exchange * tiles * (tiles - 1.f) + stages * (c.stage + c.stage_mfma * mfma_rows * tiles) +
-             busy * (c.busy_rows * rows + c.busy_tiles * tiles) + c.megabyte * megabytes + c.drift * past;
-    };
-    const float us = cost(kStripCost[p.bits == 8][layout]), both = us + cost(kStripCost[p.bits == 8][1 - layout]);
-    if (both < best.both_us) best = GemmPlan{t, 1, us, both, groups, 0};
-  }
-  return best;
+  GemmPlan none;
+  none.us = none.both_us = kNever;
+  if (p.m <= 16 || !gemm_strip_applicable(p)) return none;
+  const int blocks = strip_row_blocks(p.m), slices = ceil_div(p.m, blocks * 8), columns = ceil_div(p.n, 16), strips = cu_count() / slices;
+  const int t = strips > 0 ? ceil_div(columns, strips) : kStripMaxTiles + 1;
+  if (t > (slices > 1 ? 3 : kStripMaxTiles) || !strip_fits(blocks, t)) return none;
+  const int shift = p.bits == 4 ? 8 : 7, steps = (int)(p.k >> shift);
+  const float rows = (float)blocks, tiles = (float)t, mfma = (float)((blocks + 1) / 2) * tiles, stages = (float)p.k / 512.f;
+  const float busy = (float)((steps + 3) >> 2 << shift) / 128.f, megabytes = (float)(p.n * p.k) * (float)p.bits / 8e6f, past = std::max(0.f, stages - 8.f);
+  auto cost = [&](const StripCost& c) {
+    return c.start + c.rows * rows + c.exchange * tiles * (tiles - 1.f) + stages * (c.stage + c.stage_mfma * mfma) + busy * (c.busy_rows * rows + c.busy_tiles * tiles) +
+           c.megabyte * megabytes + c.drift * past;
+  };
+  const int layout = layout_of(p);
+  const float us = cost(kStripCost[p.bits == 8][layout]);
+  return GemmPlan{t, 1, us, us + cost(kStripCost[p.bits == 8][1 - layout]), (int64_t)ceil_div(p.n, t * 16) * slices, 0};
 }
 
 // By both layouts' times together, as the streamed kernel's tile, so that the sums are the same on either.  Four per cent to spare, and
@@ -275,7 +273,8 @@ GemmPlan plan_stream(const Problem& p, bool may_split) {
   const bool odd = p.n % 2 != 0;
   for (int i = 0; i < 9; ++i) {
     const TileCost &own = kStreamCost[p.bits == 8][layout][i], &other = kStreamCost[p.bits == 8][1 - layout][i];
-    const int64_t tiles = (int64_t)ceil_div(p.m, own.bm) * ceil_div(p.n, own.bn);
+    // (heights and widths are powers of two but for 96 columns: no division by what only the table knows)
+    const int64_t tiles = (int64_t)((p.m + own.bm - 1) >> __builtin_ctz(own.bm)) * (own.bn == 96 ? ceil_div(p.n, 96) : (int)((p.n + own.bn - 1) >> __builtin_ctz(own.bn)));
     // (96 columns above 64 rows, in several row tiles, only by a clear margin: 141 x 7680 x 1536 int4, 240 of them for 180 tiles of 64 x 128, was
     // called 3 % faster and took a layer of such projections 68.9 -> 70.3 us; where it is called 6 % faster it mostly is, 0.86 - 0.91)
     const float spare = own.bn == 96 && p.m > 64 ? 1.05f : 1.f;
