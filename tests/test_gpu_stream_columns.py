@@ -7,6 +7,7 @@ torch = pytest.importorskip("torch")
 pytestmark = pytest.mark.gpu
 
 from tests import test_gpu_stream as stream  # noqa: E402
+from tests import test_gpu_stream_tail as stream_tail  # noqa: E402
 from tests.test_gpu_parity import _dev, assert_close  # noqa: E402
 
 
@@ -16,6 +17,12 @@ from tests.test_gpu_parity import _dev, assert_close  # noqa: E402
     (8, 2, 3, 128, 128), (8, 64, 193, 384, 128), (8, 31, 96, 704, 64), (8, 100, 130, 160, 32), (8, 40, 575, 1280, 128)])
 def test_at_the_edges(variant, bits, m, n, k, group):
     stream.test_every_tile_shape_at_its_edges(variant, bits, m, n, k, group)
+
+
+@pytest.mark.parametrize("variant", [38, 39])
+@pytest.mark.parametrize("m,n,shift", [(37, 1, (1, 0, 0)), (33, 95, (1, 1, 0)), (64, 97, (0, 1, 1)), (70, 193, (1, 1, 0)), (31, 96, (1, 0, 0))])
+def test_rows_off_the_4_byte_grid_and_in_place(variant, m, n, shift):
+    stream_tail.test_rows_off_the_4_byte_grid(variant, m, n, shift)
 
 
 @pytest.mark.parametrize("m,variant", [(37, 38), (20, 39)])

@@ -20,12 +20,13 @@ def test_pieces_at_their_edges(variant, bits, m, n, k, group):
     stream.test_every_tile_shape_at_its_edges(variant, bits, m, n, k, group)
 
 
-@pytest.mark.parametrize("variant", [31, 33])
-def test_pieces_of_one_macro_step(variant):
-    """Enough tiles of 256 columns to fill the chip: the bits of the tile-major layout, and of a smaller call, which has no pieces there."""
+@pytest.mark.parametrize("variant,k", [(31, 512), (31, 1280), (31, 2816), (33, 512), (33, 2816)])
+def test_pieces_of_one_macro_step(variant, k):
+    """Enough tiles of 256 columns to fill the chip: the bits of the tile-major layout, which has no pieces, and of a smaller call, which has
+    none on 128 x 256 tiles (31).  There a piece is one macro step, and from 1280 of K on its place in the ring of two has been used before; on 256 x 256 tiles (33) it is two."""
     import relax_amd
 
-    m, n, k = 1030, 6146, 512
+    m, n = 1030, 6146
     x, wq, s, g = O.make_case(5, m, n, k, 4)
     dx, dw, ds = _dev(x), _dev(wq), _dev(s)
     plain = stream.run(dx, dw, ds, 4, g, variant)
@@ -56,7 +57,9 @@ def test_windows_that_begin_within_a_piece(bits, m, n, k, group):
     torch.cuda.synchronize()
     need = relax_amd.wq_workspace_bytes(bits, g, n, k, m)
     assert need > 16384, "the case is meant to split"
-    on_ws = relax_amd.wq_matmul(dx, dw, ds, bits, g, workspace=relax_amd.wq_workspace(need))
+    ws = relax_amd.wq_workspace(need)
+    on_ws = relax_amd.wq_matmul(dx, dw, ds, bits, g, workspace=ws)
+    assert int(ws.count_nonzero()) > 0, "the split ran on the workspace"
     rows = [0, m // 2, m - 1]
     assert_close(on_ws.cpu().numpy()[rows], c_oracle.wq_matmul(x[rows], wq, s, bits, g, nthreads=8), (bits, m, n, k), ulp_fraction=0.005)
     assert torch.equal(relax_amd.wq_matmul(dx, dw, ds, bits, g).view(torch.int16), on_ws.view(torch.int16))

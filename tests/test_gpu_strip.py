@@ -87,6 +87,24 @@ def test_what_is_not_finite_stays_in_its_row_and_column(bits, m, n, k, variant):
     assert np.array_equal(guarded[32:32 + m * n].view(m, n).cpu().numpy().view(np.uint16), plain)
 
 
+@pytest.mark.parametrize("variant,bits,m,n,k", [(v, *c) for c in ((4, 20, 145, 1280), (4, 70, 262, 512), (8, 33, 131, 1024), (8, 130, 128, 768))
+                                                for v in VARIANTS if fits(c[0], c[1], v)])
+def test_the_residual_in_the_output_buffer(variant, bits, m, n, k):
+    """The residual is read before the K loop, by the lane that writes the element."""
+    import relax_amd
+
+    x, wq, s, g = O.make_case(3000 + m + n, m, n, k, bits)
+    dx, dw, ds = _dev(x), _dev(wq), _dev(s)
+    bias, res = _fused_operands(m + n, m, n)
+    layouts = [(dw, ds, {}), (*relax_amd.wq_tile_weights(dw, ds, bits, g), dict(tiled_n=n))]
+    for w_, s_, kw in layouts:
+        plain = run(dx, w_, s_, bits, g, variant, **kw)
+        for tail, want in (({}, {}), (dict(bias=_dev(bias), activation="relu"), dict(bias=bias, activation="relu"))):
+            y = _dev(res)
+            run(dx, w_, s_, bits, g, variant, out=y, residual=y, **tail, **kw)
+            assert np.array_equal(y.cpu().numpy().view(np.uint16), O.epilogue(plain, residual=res, **want).view(np.uint16)), (variant, list(kw), list(tail))
+
+
 @pytest.mark.parametrize("bits,m,n,k", [(4, 37, 4096, 4096), (4, 20, 8064, 2048), (8, 128, 1024, 2048)])
 def test_default_calls_that_take_it(bits, m, n, k):
     """The same bits with a workspace, on other streams, and from every replay of a graph."""

@@ -69,7 +69,7 @@ GEMV_CASES = [(4, 1, 48, 256), (4, 3, 100, 512), (4, 16, 72, 1024), (4, 8, 4096,
               (8, 16, 5120, 13824), (8, 7, 333, 1280)]
 SKINNY_CASES = [(4, 17, 136, 768), (4, 64, 200, 1280), (4, 40, 4096, 4096), (4, 16, 4096, 4096), (4, 24, 12288, 4096),
                 (8, 33, 300, 2304), (8, 48, 5120, 5120), (4, 20, 6200, 512), (4, 30, 16400, 256),
-                (4, 20, 5120, 512), (4, 1, 152064, 256), (4, 40, 16400, 256), (8, 30, 16400, 256)]  # every tile-major skinny variant
+                (4, 20, 5120, 512), (4, 1, 152064, 256), (4, 40, 16400, 256), (8, 30, 16400, 256)]  # (defaults of the family: strips take some; each tile-major build by its variant below)
 GEMM_CASES = [(4, 70, 136, 768), (4, 300, 521, 1024), (4, 2048, 4096, 4096), (4, 48, 12288, 4096), (4, 24, 22016, 4096),
               (8, 129, 72, 256), (8, 513, 260, 1024), (8, 256, 5120, 5120)]
 
@@ -92,6 +92,30 @@ def test_matmul_on_tile_major_weights_is_bit_identical_to_canonical(bits, m, n, 
     torch.cuda.synchronize()
     if m * n * k <= 3e9:
         assert_close(y_tiled.cpu().numpy(), c_oracle.wq_matmul(x, wq, s, bits, g, nthreads=16), (bits, m, n, k))
+
+
+@pytest.mark.parametrize("bits", [4, 8])
+@pytest.mark.parametrize("m", [16, 17, 40, 64, 100])
+def test_every_tile_major_build_of_the_register_activation_kernel(bits, m):
+    """The bits of the same build on canonical weights, whatever the family's default is."""
+    import relax_amd
+    from relax_amd import lib
+
+    n, k = 200, 1280
+    x, wq, s, g = O.make_case(90 + m, m, n, k, bits)
+    wt, st = _tiled(wq, s, bits, g)
+    dx, dw, ds = _dev(x), _dev(wq), _dev(s)
+    want, ran = c_oracle.wq_matmul(x, wq, s, bits, g, nthreads=8), []
+    for variant in list(range(1, 12)) + list(range(21, 32)):
+        try:
+            tiled = relax_amd.wq_matmul(dx, wt, st, bits, g, tiled_n=n, kernel=lib.KERNEL_SKINNY, variant=variant).cpu().numpy()
+        except lib.WqError:
+            continue
+        canonical = relax_amd.wq_matmul(dx, dw, ds, bits, g, kernel=lib.KERNEL_SKINNY, variant=variant).cpu().numpy()
+        assert np.array_equal(tiled.view(np.uint16), canonical.view(np.uint16)), variant
+        assert_close(tiled, want, (bits, m, variant))
+        ran.append(variant)
+    assert len(ran) >= 6, ran
 
 
 @pytest.mark.parametrize("bits,m,n,k", [(4, 4, 200, 1024), (8, 16, 72, 384), (4, 130, 520, 1280), (8, 70, 300, 1024)])
