@@ -164,8 +164,8 @@ int strip_row_blocks(int64_t m) {
 //
 // Why the line lies where these costs put it: a CU reads all of its rows' activations once per strip, so the kernel is ahead where
 // one round of workgroups covers the matrix and K is short, and behind where K is long: then K split over workgroups reads a part of them.
-// us before and now: int4 4096 x 4096 at 20 / 37 rows 8.1 / 11.4 -> 7.3 / 9.3, 12288 x 4096 12.4 / 15.5 -> 11.3 / 13.9; not 4096 x 11008 at
-// 37 rows (15.8, here 21.5), nor more than a round.  Four column tiles in slices of rows are too few strips that read the weights twice
+// us before and now: int4 4096 x 4096 at 20 / 37 rows 8.1 / 10.5 -> 7.3 / 9.1, 12288 x 4096 12.1 / 14.5 -> 11.3 / 13.7; not 4096 x 11008 at
+// 37 rows (15.3, here 20.9), nor more than a round.  Four column tiles in slices of rows are too few strips that read the weights twice
 // (int8 7424 x 3072 at 70 rows 14.0 us, 64 x 64 streamed tiles 12.6).
 namespace {
 struct StripCost {
@@ -295,8 +295,8 @@ GemmPlan plan_stream(const Problem& p, bool may_split) {
 // The streamed kernel's scales in pieces of eight groups: their rows have to be whole 4-byte words (an even number of groups), and no macro step may reach
 // past a row's end, where the next row's scales, not zeros, would follow.  Where a piece lasts for more than one macro step the rows'
 // lines are asked for that much less often: a scale request touches as many lines as one for eight times the weights, and the L1
-// has room for 32 KB of lines in flight.  us, with two bytes a request and with pieces: int8 99 x 15360 x 5120 / 27648 x 5120 39.0 / 52.6 ->
-// 35.8 / 47.9, 256 x 15360 x 5120 / 5120 x 13824 51.0 / 53.2 -> 47.7 / 48.7; means over 2,300 problems, weights from memory and in the last-level
+// has room for 32 KB of lines in flight.  us, with two bytes a request and with pieces: int8 99 x 27648 x 5120 47.6 -> 45.9,
+// 256 x 15360 x 5120 / 5120 x 13824 47.0 / 49.6 -> 46.1 / 48.5; means over 2,300 problems, weights from memory and in the last-level
 // cache: int8 64 x 128 tiles 0.94 / 1.01, 128 x 128 0.98 / 0.99, int4 groups of 64 and 128 0.97 - 0.99 from 64 x 128 on, 64 x 64 tiles of either 0.99 / 1.0.
 // Not on 32 x 64 tiles, whose rows of scales are one request for four wavefronts that all send one: int4 groups of 64 and 128 1.03 / 1.03
 // (20 x 2304 x 5632 8.8 -> 9.2 us), int8 up to 40 MB 1.0 / 1.015; above, where memory is the limit, int8 0.97 / 1.0 (20 x 14592 x 5632, 0.95), and so those have them.

@@ -1,11 +1,11 @@
 // MFMA kernel for a batch's rows (17 - 256): y[M,N] = x[M,K] @ dequant(Wq,S)^T.
 //
-// What bounds it: the CU's vector L1, which returns what all of its wavefronts ask for in order and holds 32 KB in flight: weights
-// come through it at what memory gives a CU (25 KB/us), activations at what L2 does (90 - 100 KB/us), one after the other.  (12288 x 4096 int4 at
-// 37 rows, three column tiles: 13.0 us; without the requests for activations 9.8, without those for weights 8.9, without conversion and
-// MFMAs 10.8; an empty launch of this shape 4.5.)  Deeper rings, wavefronts of their own for the weights' requests and another order of K in each workgroup
-// are level; more steps of weights in the
-// rings are 1 - 4 % behind, 64-byte pieces of a weight row instead of its whole lines 5 - 10 %.
+// What bounds it, by requests sent out of range (12288 x 4096 int4 at 37 rows, three column tiles, launches back to back; us, weights from memory /
+// in the last-level cache): 13.7 / 10.7; without the activations 12.0 / 9.8, without the weights 9.7 / 9.6, without either 9.1 / 9.0, without the
+// K loop 3.8 / 3.9.  So it is start, exchange and tail, then the wavefronts' own chain of requests, LDS reads, conversion and MFMAs (5.2), and
+// then the CU's vector L1, which returns what all of its wavefronts ask for in order and holds 32 KB in flight: weights at what memory gives a CU
+// (25 KB/us), activations behind them.  Deeper rings, wavefronts of their own for the weights' requests and another order of K in each workgroup
+// are level; more steps of weights in the rings are 1 - 4 % behind, 64-byte pieces of a weight row instead of its whole lines 5 - 10 %.
 //
 // A workgroup owns all rows (above 64: a slice of them) of a strip of T column tiles of 16, so that one round of workgroups
 // covers the matrix and every CU has the same share of it: 12288 columns are 256 strips of 48, where 64-column tiles are 192.  Its eight
@@ -13,8 +13,8 @@
 // waits for its own requests only, without a barrier in the loop; each weight is converted once and each fragment read once, for
 // T column tiles.  MFMAs are 16 x 16 x 32, so that 37 rows pay for 48 and not for 64.  The partial sums meet in LDS, in the order of the wavefronts.
 //
-// Measured against the kernels it takes over from, us, weights from memory: int4 4096 x 4096 at 20 / 37 rows 8.1 / 11.4 -> 7.3 / 9.3, 12288 x 4096
-// 12.4 / 15.5 -> 11.3 / 13.9 (with the weights in the last-level cache 4096 x 4096 8.0 / 10.9 -> 6.4 / 7.9).  int8 by pieces of scales, which with two
+// Measured against the kernels it takes over from, us, weights from memory: int4 4096 x 4096 at 20 / 37 rows 8.1 / 10.5 -> 7.3 / 9.1, 12288 x 4096
+// 12.1 / 14.5 -> 11.3 / 13.7 (with the weights in the last-level cache 4096 x 4096 6.7 / 10.2 -> 5.3 / 6.6).  int8 by pieces of scales, which with two
 // bytes a step were half of the lines that weights and scales touch: 0.94 of the time on 406 timings of 131 problems.
 #include <algorithm>
 #include <atomic>

@@ -85,7 +85,8 @@ int launch_gemm_stream_decode(const Problem& p, void* workspace, int64_t workspa
 // The workspace that a call of up to 16 rows splits K on, in the decode kernel or the streamed one; 0 where it would not.
 int64_t decode_workspace_bytes(const Problem& p);
 bool decode_streams(const Problem& p);
-// The workspace that a call of `p` from 17 rows on splits K on, 0 where it would not.
+// The workspace that a call of `p` from 17 rows on splits K on, 0 where it would not.  (A call that the strips take leaves it alone: then
+// the size is that of the streamed plan, as it is for a call on either kernel.)
 int64_t gemm_workspace_bytes(const Problem& p, bool skinny_family);
 // The strip kernel (wq_gemm_strip.hip): where it applies, the blocks of eight rows in a slice of rows, whether a wavefront's share of the
 // LDS holds its rings (and its partial sums) for so many column tiles of 16, and an explicit launch with that many.

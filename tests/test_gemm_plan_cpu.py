@@ -141,7 +141,7 @@ def test_the_workspace_query_is_the_size_of_the_split_that_runs(ask):
 # (bits, group, M, N, K, tile, macro step of it, us with two bytes a scale request, us in pieces of eight groups)
 SCALE_PIECES = [(4, 64, 20, 2304, 5632, 32, 64, 256, 8.8, 9.2), (4, 128, 95, 1545, 9728, 32, 64, 256, 11.9, 12.5), (8, 128, 87, 4608, 1536, 32, 64, 256, 6.17, 6.38),
                 (8, 128, 20, 14592, 5632, 32, 64, 256, 21.4, 20.3),
-                (8, 128, 99, 15360, 5120, 128, 128, 128, 39.0, 35.8), (8, 128, 99, 27648, 5120, 128, 128, 128, 52.6, 47.9),
+                (8, 128, 256, 15360, 5120, 128, 128, 128, 47.0, 46.1), (8, 128, 99, 27648, 5120, 128, 128, 128, 47.6, 45.9),
                 (4, 32, 333, 3712, 4608, 128, 256, 256, 22.2, 24.0), (4, 32, 2048, 22016, 4096, 128, 256, 256, 364.0, 358.0)]
 
 
