@@ -199,12 +199,15 @@ GemmPlan plan_strip(const Problem& p) {
   return GemmPlan{t, 1, us, us + cost(kStripCost[p.bits == 8][1 - layout]), (int64_t)ceil_div(p.n, t * 16) * slices, 0};
 }
 
-// By both layouts' times together, as the streamed kernel's tile, so that the sums are the same on either.  Four per cent to spare, and
-// from 4096 of K on, where both kernels' times scatter most, half a per cent more for every 512.  Of 6,834
-// problems (those of the fit) it takes 2,178; the call's time against its time without this kernel, means over all of them: weights from memory 0.955, in the
-// last-level cache 0.934; 46 and 12 are more than 5 % slower.  Always taking the fastest would be 0.6 % better with weights from memory.
+// By both layouts' times together, as the streamed kernel's tile, so that the sums are the same on either.  Four per cent to spare, none
+// against K split over workgroups, and from 4096 of K on, where both kernels' times scatter most, half a per cent more for every 512.  The lines by what
+// lies on either side, strips against what runs otherwise, weights from memory / in the last-level cache, whose gain a split's exchange does not have:
+// against a split up to 4 % below the line 0.98 / 0.82, 4 % above it 1.0 / 0.82 (295 problems); against whole K up to 4 % below 0.94 / 0.88, above 0.99 / 0.94 (239).
+// Of 6,834 problems (those of the fit) it takes a third; the call's time against its time without this kernel, means over all of them: 0.955 / 0.930; 83 / 13
+// are more than 5 % slower, 11 in the mean of both.
 bool strip_ahead(const Problem& p, const GemmPlan& strip, const GemmPlan& stream) {
-  return strip.both_us < (0.96f - 0.005f * std::max(0.f, (float)p.k / 512.f - 8.f)) * stream.both_us;
+  const float level = stream.split > 1 ? 1.f : 0.96f;
+  return strip.both_us < (level - 0.005f * std::max(0.f, (float)p.k / 512.f - 8.f)) * stream.both_us;
 }
 
 // The layouts' joint choice of the two, unless the other kernel is faster than what that would run.
