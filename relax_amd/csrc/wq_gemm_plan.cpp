@@ -210,9 +210,11 @@ bool strip_ahead(const Problem& p, const GemmPlan& strip, const GemmPlan& stream
   return strip.both_us < (level - 0.005f * std::max(0.f, (float)p.k / 512.f - 8.f)) * stream.both_us;
 }
 
-// The layouts' joint choice of the two, unless the other kernel is faster than what that would run.
-StreamedChoice choose_streamed(const Problem& p, const GemmPlan& strip, const GemmPlan& stream, float other_us) {
-  const bool ahead = strip_ahead(p, strip, stream);
+// The layouts' joint choice of the two, unless the other kernel is faster than what that would run.  `kept`: the strips are ahead of the split
+// that the call has no memory for under capture.  They run there as well, with the eager call's bits: they are faster than the
+// unsplit tiles then, if by less than these are given elsewhere (25 x 8544 x 5632 int4, a split in three called 2 % faster than none).
+StreamedChoice choose_streamed(const Problem& p, const GemmPlan& strip, const GemmPlan& stream, float other_us, bool kept) {
+  const bool ahead = kept || strip_ahead(p, strip, stream);
   if (other_us < (ahead ? strip.us : stream.us)) return kOtherKernel;
   return ahead ? kStrips : kStreamedTiles;
 }

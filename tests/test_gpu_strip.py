@@ -105,7 +105,7 @@ def test_the_residual_in_the_output_buffer(variant, bits, m, n, k):
             assert np.array_equal(y.cpu().numpy().view(np.uint16), O.epilogue(plain, residual=res, **want).view(np.uint16)), (variant, list(kw), list(tail))
 
 
-@pytest.mark.parametrize("bits,m,n,k", [(4, 37, 4096, 4096), (4, 20, 8064, 2048), (8, 128, 1024, 2048)])
+@pytest.mark.parametrize("bits,m,n,k", [(4, 37, 4096, 4096), (4, 20, 8064, 2048), (8, 128, 1024, 2048), (4, 25, 8544, 5632)])
 def test_default_calls_that_take_it(bits, m, n, k):
     """The same bits with a workspace, on other streams, and from every replay of a graph."""
     import relax_amd
