@@ -199,22 +199,21 @@ GemmPlan plan_strip(const Problem& p) {
   return GemmPlan{t, 1, us, us + cost(kStripCost[p.bits == 8][1 - layout]), (int64_t)ceil_div(p.n, t * 16) * slices, 0};
 }
 
-// By both layouts' times together, as the streamed kernel's tile, so that the sums are the same on either.  Four per cent to spare, none
-// against K split over workgroups, and from 4096 of K on, where both kernels' times scatter most, half a per cent more for every 512.  The lines by what
-// lies on either side, strips against what runs otherwise, weights from memory / in the last-level cache, whose gain a split's exchange does not have:
-// against a split up to 4 % below the line 0.98 / 0.82, 4 % above it 1.0 / 0.82 (295 problems); against whole K up to 4 % below 0.94 / 0.88, above 0.99 / 0.94 (239).
-// Of 6,834 problems (those of the fit) it takes a third; the call's time against its time without this kernel, means over all of them: 0.955 / 0.930; 83 / 13
-// are more than 5 % slower, 11 in the mean of both.
+// By both layouts' times together, as the streamed kernel's tile, so that the sums are the same on either.  Level cost up to 32 rows, 4 % to
+// spare up to 64 and 7 % above: every strip reads all of its rows, so the more rows, the more it loses where they come from another XCD's
+// kernel or from memory and not from its own L2.  The lines by 720 problems around them, strips against what runs otherwise, canonical weights from
+// memory, activations in L2 / from memory: 17 - 32 rows up to 4 % below the line 0.95 / 0.94, above it 1.00 / 0.98; 33 - 64 rows 0.97 / 0.99 and 1.02 / 1.03;
+// more rows 0.94 / 1.03 and 0.99 / 1.05 (tile-major 0.86 / 0.91 and 0.90 / 0.96; with the weights in the last-level cache, whose gain K split
+// over workgroups does not have, 0.76 - 0.86).  From 4096 of K on, where both kernels' times scatter most, half a per cent more for every 512.
 bool strip_ahead(const Problem& p, const GemmPlan& strip, const GemmPlan& stream) {
-  const float level = stream.split > 1 ? 1.f : 0.96f;
+  const float level = p.m <= 32 ? 1.f : p.m <= 64 ? 0.96f : 0.93f;
   return strip.both_us < (level - 0.005f * std::max(0.f, (float)p.k / 512.f - 8.f)) * stream.both_us;
 }
 
-// The layouts' joint choice of the two, unless the other kernel is faster than what that would run.  `kept`: the strips are ahead of the split
-// that the call has no memory for under capture.  They run there as well, with the eager call's bits: they are faster than the
-// unsplit tiles then, if by less than these are given elsewhere (25 x 8544 x 5632 int4, a split in three called 2 % faster than none).
-StreamedChoice choose_streamed(const Problem& p, const GemmPlan& strip, const GemmPlan& stream, float other_us, bool kept) {
-  const bool ahead = kept || strip_ahead(p, strip, stream);
+// The layouts' joint choice of the two, unless the other kernel is faster than what that would run.  (What is ahead of a split is ahead of the slower whole
+// K as well, so a captured call without memory for the split runs the strips that the eager one does.)
+StreamedChoice choose_streamed(const Problem& p, const GemmPlan& strip, const GemmPlan& stream, float other_us) {
+  const bool ahead = strip_ahead(p, strip, stream);
   if (other_us < (ahead ? strip.us : stream.us)) return kOtherKernel;
   return ahead ? kStrips : kStreamedTiles;
 }

@@ -138,13 +138,9 @@ int launch_gemm_stream_planned(const Problem& p, void* workspace, int64_t worksp
   if (!in_range(p)) return 0;
   GemmPlan plan = plan_stream(p, p.m <= 256 || workspace != nullptr);
   const bool slot = plan.split > 1 && plan.bytes > workspace_bytes;
+  if (slot && (p.m > 256 || captured(p))) plan = plan_stream(p, false);
   const GemmPlan strip = plan_strip(p);
-  bool kept = false;
-  if (slot && (p.m > 256 || captured(p))) {
-    kept = strip_ahead(p, strip, plan);
-    plan = plan_stream(p, false);
-  }
-  switch (choose_streamed(p, strip, plan, other_us, kept)) {
+  switch (choose_streamed(p, strip, plan, other_us)) {
     case kOtherKernel: return 0;
     case kStrips: return launched(launch_gemm_strip(p, strip.variant), "strip");
     default: return launch_plan(p, plan, workspace, slot);

@@ -112,7 +112,7 @@ GemmPlan plan_strip(const Problem& p);  // `variant`: its column tiles, 0 where 
 bool strip_ahead(const Problem& p, const GemmPlan& strip, const GemmPlan& stream);
 // What a call of 17 rows on runs, where the kernel that its family would run instead takes `other_us`.
 enum StreamedChoice { kOtherKernel, kStreamedTiles, kStrips };
-StreamedChoice choose_streamed(const Problem& p, const GemmPlan& strip, const GemmPlan& stream, float other_us, bool kept = false);
+StreamedChoice choose_streamed(const Problem& p, const GemmPlan& strip, const GemmPlan& stream, float other_us);
 float skinny_cost(const Problem& p);  // us by the cost model; out of reach where a kernel does not apply
 float other_gemm_cost(const Problem& p);  // of the kernels launch_gemm takes where not the streamed one
 bool gemm_direct_applicable(const Problem& p);  // K % 256 == 0, the standard group, operands below 1 GiB

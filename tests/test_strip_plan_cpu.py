@@ -32,8 +32,7 @@ extern "C" int chosen(int bits, int group, int64_t m, int64_t n, int64_t k, int 
 extern "C" int captured(int bits, int group, int64_t m, int64_t n, int64_t k, int tiled) {
   wq::Problem p{nullptr, nullptr, nullptr, nullptr, m, n, k, bits, group, 0, nullptr};
   p.tiled = tiled != 0;
-  const wq::GemmPlan strip = wq::plan_strip(p), stream = wq::plan_stream(p, true), whole = wq::plan_stream(p, false);
-  return wq::choose_streamed(p, strip, whole, wq::skinny_cost(p), wq::strip_ahead(p, strip, stream));
+  return wq::choose_streamed(p, wq::plan_strip(p), wq::plan_stream(p, false), wq::skinny_cost(p));
 }
 """
 
