@@ -283,13 +283,13 @@ GemmPlan plan_stream(const Problem& p, bool may_split) {
     // called 3 % faster and took a layer of such projections 68.9 -> 70.3 us; where it is called 6 % faster it mostly is, 0.86 - 0.91)
     const float spare = own.bn == 96 && p.m > 64 ? 1.05f : 1.f;
     // a window has at least two steps of 256 k; up to an eighth more windows than CUs
-    const int most = may_split && own.split > 0.f && 2 * tiles <= cu + cu / 8 ? std::min({8, (cu + cu / 8) / (int)tiles, macros}) : 1;
+    const int most = may_split && own.split > 0.f && 2 * tiles <= cu + cu / 8 && tiles <= kSplitMaxTiles / kStreamCounterWords ? std::min({kMaxWindows, (cu + cu / 8) / (int)tiles, macros}) : 1;
     for (int s = 1; s <= most; ++s) {
       const int per = s == 1 ? macros : ceil_div(macros, s);
       if (s > 1 && (per < 2 || (s - 1) * per >= macros)) continue;  // (windows that would be empty are dropped)
       const float us = tile_cost(own, tiles * s, per, s, odd, cu), both = spare * (us + tile_cost(other, tiles * s, per, s, odd, cu));
       if (both < best.both_us) {
-        best = GemmPlan{own.variant, s, us, both, tiles, s > 1 ? kSplitCounterBytes + tiles * s * own.bm * own.bn * 4 : 0};
+        best = GemmPlan{own.variant, s, us, both, tiles, s > 1 ? kSplitCounterBytes + tiles * s * own.bm * own.bn * 4 : 0, stream_split_shares(own.bm, own.bn)};
       }
     }
   }

@@ -103,8 +103,12 @@ struct StreamShape {
   static constexpr int kPG = TM * 4 / G;
   static constexpr int kXPerTarget = (G - 1) * CW * kPG * TN * 1024;              // LDS bytes a target group receives
   static constexpr int kTargets = G == 1 ? 1 : (160 * 1024 / kXPerTarget < G ? 160 * 1024 / kXPerTarget : G);  // per phase
-  static constexpr int kLds = std::max(kDummyBase + (kDummy ? 1024 : 0), kTargets * kXPerTarget);
-  static_assert(kQA % kIssuers == 0 && kSlices >= 1 && kStages >= 3 && TM * 4 % G == 0 && kSPM % 2 == 0 && CW * G % 4 == 0, "shape");
+  // ... and so do the requests' wavefronts where they are whole groups that the row quads divide by: kFG groups finish kFPG quads each
+  static constexpr bool kHelp = PROD > 0 && PROD % CW == 0 && TM * 4 % (G + PROD / CW) == 0;
+  static constexpr int kFG = kHelp ? G + PROD / CW : G, kFPG = TM * 4 / kFG;
+  static constexpr int kHelpLds = kHelp ? (G * (G - 1) + (kFG - G) * G) * CW * kFPG * TN * 1024 : 0;
+  static constexpr int kLds = std::max({kDummyBase + (kDummy ? 1024 : 0), kTargets * kXPerTarget, kHelpLds});
+  static_assert(kQA % kIssuers == 0 && kSlices >= 1 && kStages >= 3 && TM * 4 % G == 0 && kSPM % 2 == 0 && CW * G % 4 == 0 && kLds <= 160 * 1024, "shape");
 
   // Requests that may still be in flight at the top of stage t (of a macro step), where the activations of stage t + 1 and
   // the weights of stage t + kAhead have to be there.  Stage u issues the activations of stage u + kStages - 1, and a macro
@@ -255,6 +259,14 @@ __global__ __launch_bounds__((CW * G + PROD) * 64, 1) void wq_gemm_stream_kernel
   using C = StreamShape<BITS, TM, TN, CW, G, PROD, KA, KM, NM, SV>;
   static_assert(!(TILED && SV), "tile-major scales lie as they are read");
   constexpr int BM = C::kBM, BN = C::kBN, WAVES = C::kWaves, SPM = C::kSPM, NS = C::kSlices;
+  // The wavefronts that finish the tile.  One wavefront a SIMD is what the K loop has for 128 rows, and alone it is slow at the tail's chain of
+  // conversions, loads and stores, so the requests' wavefronts take their share of the row quads through LDS (us): int4 333 x 10001 x 4224
+  // with bias and gelu 42.8 -> 40.5, plain 333 x 10000 37.9 -> 37.0, 512 x 12288 on 128 x 256 tiles 55.9 -> 55.1; on 64 x 128 tiles, unsplit, 2 % behind.
+  // (The windows of kSerial keep them busy to the end.)
+  constexpr bool HELP = C::kHelp && MODE != kSerial && (TM > 2 || MODE == kSplit);
+  constexpr int PG = HELP ? C::kFPG : C::kPG, FINISHERS = HELP ? WAVES + PROD : WAVES;
+  constexpr bool SCATTER = MODE == kSplit && stream_split_shares(BM, BN);  // a split's windows share the finishing
+  static_assert(!SCATTER || HELP, "the builds it was measured on");
   const int group_log2 = shift_and_zero & 0xFF, zero_point = (shift_and_zero >> 8) & 0xFF;  // group = 1 << group_log2 >= 32
   const bool gated = (shift_and_zero >> 16) & 1;
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
@@ -284,6 +296,13 @@ __global__ __launch_bounds__((CW * G + PROD) * 64, 1) void wq_gemm_stream_kernel
   int k_begin = ks * per_window * KM, k_end = min(k_begin + per_window * KM, K);
   // (barriers of the exchange between the K groups at a window's end)
   constexpr int kExchangeBarriers = G == 1 ? 0 : 2 * ((G + C::kTargets - 1) / C::kTargets);
+
+  float4_t fin[PG][TN], total[MODE == kSerial ? PG : 1][TN];
+  // HELP: where quad p of target group t from group g is in LDS, `lane`s apart
+  auto handed = [&](int t, int g) __attribute__((always_inline)) {
+    const int place = t < G ? t * (G - 1) + (g < t ? g : g - 1) : G * (G - 1) + (t - G) * G + g;
+    return reinterpret_cast<float4_t*>(smem) + (place * CW + cw) * PG * TN * 64 + lane;
+  };
 
   using std::integral_constant;
   StreamRequests<C, BITS, TN, TILED, SV> req;
@@ -328,9 +347,24 @@ __global__ __launch_bounds__((CW * G + PROD) * 64, 1) void wq_gemm_stream_kernel
           for (int i = 0; i < kExchangeBarriers + 1; ++i) __builtin_amdgcn_s_barrier();
           req.k_begin = k_begin = ks * per_window * KM;
           req.k_end = k_end = min(k_begin + per_window * KM, K);
-        } else {
+        } else if constexpr (!HELP) {
           return;
+        } else {
+          break;
         }
+      }
+      if constexpr (HELP) {
+        // the share of the row quads of a group that has no sums of its own
+        __builtin_amdgcn_s_setprio(0);
+        __syncthreads();
+#pragma unroll
+        for (int p = 0; p < PG; ++p)
+#pragma unroll
+          for (int j = 0; j < TN; ++j) {
+            fin[p][j] = handed(grp, 0)[(p * TN + j) * 64];
+#pragma unroll
+            for (int g = 1; g < G; ++g) fin[p][j] += handed(grp, g)[(p * TN + j) * 64];
+          }
       }
     }
   } else {
@@ -338,186 +372,176 @@ __global__ __launch_bounds__((CW * G + PROD) * 64, 1) void wq_gemm_stream_kernel
     req.template prologue<SPM, KA, KM>();
   }
 
-  // ---- LDS reads of this lane: KL contiguous k of a stage, from (grp * kKG + fh * KL) on ------------------------
-  constexpr int KL = C::kKG / 2, WB = KL * BITS / 8, WL = WB > 16 ? WB / 16 : 1, WORDS = WB / 4;
-  const int kl0 = grp * C::kKG + fh * KL;
-  uint32_t a_rd[NS], w_rd[SPM][WL], s_rd[SPM];
+  if (!HELP || wave < WAVES) {
+    // ---- LDS reads of this lane: KL contiguous k of a stage, from (grp * kKG + fh * KL) on ------------------------
+    constexpr int KL = C::kKG / 2, WB = KL * BITS / 8, WL = WB > 16 ? WB / 16 : 1, WORDS = WB / 4;
+    const int kl0 = grp * C::kKG + fh * KL;
+    uint32_t a_rd[NS], w_rd[SPM][WL], s_rd[SPM];
 #pragma unroll
-  for (int kk = 0; kk < NS; ++kk) a_rd[kk] = (uint32_t)fr * C::kARow + (uint32_t)(((kl0 / 8 + kk) ^ stream_swizzle(fr, C::kARow / 16)) << 4);
-  const int wrow = cw * TN * 32 + fr;  // + 32 j
+    for (int kk = 0; kk < NS; ++kk) a_rd[kk] = (uint32_t)fr * C::kARow + (uint32_t)(((kl0 / 8 + kk) ^ stream_swizzle(fr, C::kARow / 16)) << 4);
+    const int wrow = cw * TN * 32 + fr;  // + 32 j
 #pragma unroll
-  for (int t = 0; t < SPM; ++t) {
+    for (int t = 0; t < SPM; ++t) {
 #pragma unroll
-    for (int v = 0; v < WL; ++v) {
-      const int byte = (t * KA + kl0) * BITS / 8 + v * 16;
-      w_rd[t][v] = C::kWBase + (uint32_t)wrow * C::kWRow + (uint32_t)(((byte / 16) ^ stream_swizzle(wrow, C::kWRow / 16)) << 4) + (byte & 15);
-    }
-    s_rd[t] = C::kSBase + (uint32_t)(wrow * C::kSRow) + (SV ? (uint32_t)((t * KA + kl0) >> group_log2) * 2u : (uint32_t)((t * KA + kl0) / 32) * 4u);
-  }
-
-  const Q4Consts qc = make_q4_consts(zero_point);
-  float16_t acc[TM][TN];
-  constexpr int PG = C::kPG;
-  float4_t fin[PG][TN], total[MODE == kSerial ? PG : 1][TN];
-  if constexpr (MODE == kSerial) {
-#pragma unroll
-    for (int p = 0; p < PG; ++p)
-#pragma unroll
-      for (int j = 0; j < TN; ++j) total[p][j] = float4_t{0.f, 0.f, 0.f, 0.f};
-  }
-
-  struct Words {
-    uint32_t w[TN][WORDS];
-    half_t s[TN];
-  };
-  Words words[2];
-  // (`piece`: where the macro step's scales are if they come in pieces; else by its place in the ring, as its weights)
-  auto read_words = [&](Words& d, uint32_t ring, uint32_t piece, auto tt) __attribute__((always_inline)) {
-    constexpr int t = decltype(tt)::value;
-    const unsigned char* const wb = smem + ring * C::kWBytes;
-    const unsigned char* const sb = smem + (SV ? piece : ring * C::kSBytes);
-#pragma unroll
-    for (int j = 0; j < TN; ++j) {
-      if constexpr (WB >= 16) {
-#pragma unroll
-        for (int v = 0; v < WL; ++v) {
-          const u32x4 q = *reinterpret_cast<const u32x4*>(wb + w_rd[t][v] + j * 32 * C::kWRow);
-#pragma unroll
-          for (int e = 0; e < 4; ++e) d.w[j][v * 4 + e] = q[e];
-        }
-      } else if constexpr (WB == 8) {
-        const u32x2 q = *reinterpret_cast<const u32x2*>(wb + w_rd[t][0] + j * 32 * C::kWRow);
-        d.w[j][0] = q[0], d.w[j][1] = q[1];
-      } else {
-        d.w[j][0] = *reinterpret_cast<const uint32_t*>(wb + w_rd[t][0] + j * 32 * C::kWRow);
+      for (int v = 0; v < WL; ++v) {
+        const int byte = (t * KA + kl0) * BITS / 8 + v * 16;
+        w_rd[t][v] = C::kWBase + (uint32_t)wrow * C::kWRow + (uint32_t)(((byte / 16) ^ stream_swizzle(wrow, C::kWRow / 16)) << 4) + (byte & 15);
       }
-      d.s[j] = *reinterpret_cast<const half_t*>(sb + s_rd[t] + j * 32 * C::kSRow);
+      s_rd[t] = C::kSBase + (uint32_t)(wrow * C::kSRow) + (SV ? (uint32_t)((t * KA + kl0) >> group_log2) * 2u : (uint32_t)((t * KA + kl0) / 32) * 4u);
     }
-  };
-  // Weight pair PR (of four) of a lane's eight k of slice KK, column tile J, in two halves: integers with the float16
-  // exponent bits in place, then the exact subtraction and the one rounding of the product with the scale.
-  auto convert_front = [&](const Words& d, auto kk, auto jj, auto pp) __attribute__((always_inline)) -> uint32_t {
-    constexpr int KK = decltype(kk)::value, J = decltype(jj)::value, PR = decltype(pp)::value;
-    if constexpr (BITS == 4) {
-      const uint32_t t = __builtin_amdgcn_perm(0u, d.w[J][KK], 0x0c000c00u | PR | (PR << 16));
-      return (t & 0x00F0000Fu) | qc.magic;
-    } else {
-      return cvt_i8_lo<PR % 2 * 2>(d.w[J][2 * KK + PR / 2]);
-    }
-  };
-  auto convert_back = [&](const Words& d, uint32_t f, auto kk, auto jj, auto pp) __attribute__((always_inline)) -> uint32_t {
-    constexpr int KK = decltype(kk)::value, J = decltype(jj)::value, PR = decltype(pp)::value;
-    if constexpr (BITS == 4) return as_u32(__builtin_elementwise_fma(as_h2(f), qc.mix_mul, -qc.mix_sub) * bcast_h2(d.s[J]));
-    else return as_u32(as_h2(cvt_i8_hi<PR % 2 * 2 + 1>(f, d.w[J][2 * KK + PR / 2])) * bcast_h2(d.s[J]));
-  };
-  half8_t a[2][TM];
-  uint32_t b[2][TN][4];
-  constexpr int SLOTS = TM * TN, PAIRS = TN * 4;  // MFMAs and weight pairs of a slice
 
-  // ---- K loop (program order is issue order: sched_barrier after every MFMA).  Slice q is multiplied while the A fragments of slice q + 1 are read and its weights converted; packed
-  // words and scales are read a slice before their conversion begins.
-  for (;;) {  // (a single window but for kSerial)
-#pragma unroll
-    for (int i = 0; i < TM; ++i)
-#pragma unroll
-      for (int j = 0; j < TN; ++j)
-#pragma unroll
-        for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.f;
-    __builtin_amdgcn_s_barrier();
-    asm volatile("" ::: "memory");
-    // (SV: the group of a k0, which its macro step begins or lies within, is the sum of k0's and of the lane's own)
-    auto in_piece = [&](int k0) __attribute__((always_inline)) { return (uint32_t)((k0 >> group_log2) & 7) * 2u; };
-    uint32_t s_base = 0, s_off = SV ? in_piece(k_begin) : 0;
-    read_words(words[0], 0, s_off, integral_constant<int, 0>{});
-    if constexpr (NS == 1) read_words(words[1], 0, s_off, integral_constant<int, 1>{});
-#pragma unroll
-    for (int i = 0; i < TM; ++i) a[0][i] = *reinterpret_cast<const half8_t*>(smem + a_rd[0] + i * 32 * C::kARow);
-    static_for_s<0, PAIRS>([&](auto q) __attribute__((always_inline)) {
-      constexpr int j = decltype(q)::value / 4, pr = decltype(q)::value % 4;
-      integral_constant<int, 0> kk;
-      integral_constant<int, j> jj;
-      integral_constant<int, pr> pp;
-      b[0][j][pr] = convert_back(words[0], convert_front(words[0], kk, jj, pp), kk, jj, pp);
-    });
-    uint32_t abuf = 0, abuf_issue = (C::kStages - 1) * C::kABytes, ring = 0;
-    for (int k0 = k_begin; k0 < k_end; k0 += KM) {
-      const uint32_t ring_next = ring + 1 == C::kMacros ? 0 : ring + 1, ring_issue = ring == 0 ? C::kMacros - 1 : ring - 1;
-      uint32_t s_next = 0;
-      if constexpr (SV) {
-        if (((k0 + KM) & ((8 << group_log2) - 1)) == 0) s_base = s_base + C::kSBytes == C::kMacros * C::kSBytes ? 0 : s_base + C::kSBytes;
-        s_next = s_base + in_piece(k0 + KM);
-      }
-      static_for_s<0, SPM>([&](auto tc) __attribute__((always_inline)) {
-        constexpr int t = decltype(tc)::value;
-        const uint32_t abuf_next = abuf + C::kABytes == C::kStages * C::kABytes ? 0 : abuf + C::kABytes;
-        if constexpr (PROD == 0) wait_dma<C::in_flight(t)>();  // (otherwise the producers have waited)
-        __builtin_amdgcn_sched_barrier(0);
-        __builtin_amdgcn_s_barrier();
-        asm volatile("" ::: "memory");
-        static_for_s<0, NS>([&](auto kkc) __attribute__((always_inline)) {
-          constexpr int kk = decltype(kkc)::value, q = t * NS + kk;         // slice of the macro step
-          constexpr int t1 = (q + 1) / NS, kk1 = (q + 1) % NS;              // the next slice, being converted
-          constexpr int t2 = (q + 2) / NS, kk2 = (q + 2) % NS;              // the one after it
-          uint32_t front[PAIRS];
-          static_for_s<0, SLOTS>([&](auto sc) __attribute__((always_inline)) {
-            constexpr int s = decltype(sc)::value, i = s / TN, j = s % TN;
-            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(
-                a[q & 1][i], __builtin_bit_cast(half8_t, *reinterpret_cast<const u32x4*>(b[q & 1][j])), acc[i][j], 0, 0, 0);
-            if constexpr (s < TM)
-              a[(q + 1) & 1][s] = *reinterpret_cast<const half8_t*>(smem + (kk1 == 0 ? abuf_next : abuf) + a_rd[kk1] + s * 32 * C::kARow);
-            if constexpr (s == 0 && kk2 == 0) read_words(words[t2 & 1], t2 >= SPM ? ring_next : ring, t2 >= SPM ? s_next : s_off, integral_constant<int, t2 % SPM>{});
-            if constexpr (PROD == 0) {
-              // requests of later stages, evenly over the slots: weights and scales first
-              constexpr int slot = kk * SLOTS + s, WS = t == 0 ? C::kNWS : 0, ALL = WS + C::kNA;
-              constexpr int P0 = slot * ALL / (NS * SLOTS), P1 = (slot + 1) * ALL / (NS * SLOTS);
-              static_for_s<P0, P1>([&](auto pc) __attribute__((always_inline)) {
-                constexpr int P = decltype(pc)::value;
-                if constexpr (P < WS) req.template issue_ws<P>(k0 + (C::kMacros - 1) * KM, ring_issue);
-                else req.template issue_a<P - WS>(k0 + (t + C::kStages - 1) * KA, abuf_issue);
-              });
-            }
-            constexpr int F0 = s * PAIRS / SLOTS, F1 = (s + 1) * PAIRS / SLOTS, B0 = s == 0 ? 0 : (s - 1) * PAIRS / SLOTS, B1 = s + 1 == SLOTS ? PAIRS : F0;
-            static_for_s<F0, F1>([&](auto qc_) __attribute__((always_inline)) {
-              constexpr int p = decltype(qc_)::value;
-              front[p] = convert_front(words[t1 & 1], integral_constant<int, kk1>{}, integral_constant<int, p / 4>{}, integral_constant<int, p % 4>{});
-            });
-            static_for_s<B0, B1>([&](auto qc_) __attribute__((always_inline)) {
-              constexpr int p = decltype(qc_)::value;
-              b[(q + 1) & 1][p / 4][p % 4] = convert_back(words[t1 & 1], front[p], integral_constant<int, kk1>{}, integral_constant<int, p / 4>{}, integral_constant<int, p % 4>{});
-            });
-            __builtin_amdgcn_sched_barrier(0);
-          });
-        });
-        abuf_issue = abuf;
-        abuf = abuf_next;
-      });
-      ring = ring_next;
-      s_off = s_next;
-    }
-    if constexpr (PROD == 0) wait_dma<0>();
-    __builtin_amdgcn_s_barrier();  // the last requests (all out of range) have landed
-    asm volatile("" ::: "memory");
-
-    // ---- K groups: every group hands its partial sums of the other groups' row quads over through LDS ----------------
-    auto part = [&](int pair, int j) __attribute__((always_inline)) {
-      const float16_t& c = acc[pair / 4][j];
-      const int v = pair % 4 * 4;
-      return float4_t{c[v], c[v + 1], c[v + 2], c[v + 3]};
-    };
-    if constexpr (G == 1) {
+    const Q4Consts qc = make_q4_consts(zero_point);
+    float16_t acc[TM][TN];
+    if constexpr (MODE == kSerial) {
 #pragma unroll
       for (int p = 0; p < PG; ++p)
 #pragma unroll
-        for (int j = 0; j < TN; ++j) fin[p][j] = part(p, j);
-    } else {
-      static_for_s<0, (G + C::kTargets - 1) / C::kTargets>([&](auto phase) __attribute__((always_inline)) {
-        constexpr int T0 = decltype(phase)::value * C::kTargets, T1 = T0 + C::kTargets < G ? T0 + C::kTargets : G;
-        __syncthreads();
-        static_for_s<T0, T1>([&](auto tt) __attribute__((always_inline)) {
+        for (int j = 0; j < TN; ++j) total[p][j] = float4_t{0.f, 0.f, 0.f, 0.f};
+    }
+
+    struct Words {
+      uint32_t w[TN][WORDS];
+      half_t s[TN];
+    };
+    Words words[2];
+    // (`piece`: where the macro step's scales are if they come in pieces; else by its place in the ring, as its weights)
+    auto read_words = [&](Words& d, uint32_t ring, uint32_t piece, auto tt) __attribute__((always_inline)) {
+      constexpr int t = decltype(tt)::value;
+      const unsigned char* const wb = smem + ring * C::kWBytes;
+      const unsigned char* const sb = smem + (SV ? piece : ring * C::kSBytes);
+#pragma unroll
+      for (int j = 0; j < TN; ++j) {
+        if constexpr (WB >= 16) {
+#pragma unroll
+          for (int v = 0; v < WL; ++v) {
+            const u32x4 q = *reinterpret_cast<const u32x4*>(wb + w_rd[t][v] + j * 32 * C::kWRow);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) d.w[j][v * 4 + e] = q[e];
+          }
+        } else if constexpr (WB == 8) {
+          const u32x2 q = *reinterpret_cast<const u32x2*>(wb + w_rd[t][0] + j * 32 * C::kWRow);
+          d.w[j][0] = q[0], d.w[j][1] = q[1];
+        } else {
+          d.w[j][0] = *reinterpret_cast<const uint32_t*>(wb + w_rd[t][0] + j * 32 * C::kWRow);
+        }
+        d.s[j] = *reinterpret_cast<const half_t*>(sb + s_rd[t] + j * 32 * C::kSRow);
+      }
+    };
+    // Weight pair PR (of four) of a lane's eight k of slice KK, column tile J, in two halves: integers with the float16
+    // exponent bits in place, then the exact subtraction and the one rounding of the product with the scale.
+    auto convert_front = [&](const Words& d, auto kk, auto jj, auto pp) __attribute__((always_inline)) -> uint32_t {
+      constexpr int KK = decltype(kk)::value, J = decltype(jj)::value, PR = decltype(pp)::value;
+      if constexpr (BITS == 4) {
+        const uint32_t t = __builtin_amdgcn_perm(0u, d.w[J][KK], 0x0c000c00u | PR | (PR << 16));
+        return (t & 0x00F0000Fu) | qc.magic;
+      } else {
+        return cvt_i8_lo<PR % 2 * 2>(d.w[J][2 * KK + PR / 2]);
+      }
+    };
+    auto convert_back = [&](const Words& d, uint32_t f, auto kk, auto jj, auto pp) __attribute__((always_inline)) -> uint32_t {
+      constexpr int KK = decltype(kk)::value, J = decltype(jj)::value, PR = decltype(pp)::value;
+      if constexpr (BITS == 4) return as_u32(__builtin_elementwise_fma(as_h2(f), qc.mix_mul, -qc.mix_sub) * bcast_h2(d.s[J]));
+      else return as_u32(as_h2(cvt_i8_hi<PR % 2 * 2 + 1>(f, d.w[J][2 * KK + PR / 2])) * bcast_h2(d.s[J]));
+    };
+    half8_t a[2][TM];
+    uint32_t b[2][TN][4];
+    constexpr int SLOTS = TM * TN, PAIRS = TN * 4;  // MFMAs and weight pairs of a slice
+
+    // ---- K loop (program order is issue order: sched_barrier after every MFMA).  Slice q is multiplied while the A fragments of slice q + 1 are read and its weights converted; packed
+    // words and scales are read a slice before their conversion begins.
+    for (;;) {  // (a single window but for kSerial)
+#pragma unroll
+      for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j)
+#pragma unroll
+          for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.f;
+      __builtin_amdgcn_s_barrier();
+      asm volatile("" ::: "memory");
+      // (SV: the group of a k0, which its macro step begins or lies within, is the sum of k0's and of the lane's own)
+      auto in_piece = [&](int k0) __attribute__((always_inline)) { return (uint32_t)((k0 >> group_log2) & 7) * 2u; };
+      uint32_t s_base = 0, s_off = SV ? in_piece(k_begin) : 0;
+      read_words(words[0], 0, s_off, integral_constant<int, 0>{});
+      if constexpr (NS == 1) read_words(words[1], 0, s_off, integral_constant<int, 1>{});
+#pragma unroll
+      for (int i = 0; i < TM; ++i) a[0][i] = *reinterpret_cast<const half8_t*>(smem + a_rd[0] + i * 32 * C::kARow);
+      static_for_s<0, PAIRS>([&](auto q) __attribute__((always_inline)) {
+        constexpr int j = decltype(q)::value / 4, pr = decltype(q)::value % 4;
+        integral_constant<int, 0> kk;
+        integral_constant<int, j> jj;
+        integral_constant<int, pr> pp;
+        b[0][j][pr] = convert_back(words[0], convert_front(words[0], kk, jj, pp), kk, jj, pp);
+      });
+      uint32_t abuf = 0, abuf_issue = (C::kStages - 1) * C::kABytes, ring = 0;
+      for (int k0 = k_begin; k0 < k_end; k0 += KM) {
+        const uint32_t ring_next = ring + 1 == C::kMacros ? 0 : ring + 1, ring_issue = ring == 0 ? C::kMacros - 1 : ring - 1;
+        uint32_t s_next = 0;
+        if constexpr (SV) {
+          if (((k0 + KM) & ((8 << group_log2) - 1)) == 0) s_base = s_base + C::kSBytes == C::kMacros * C::kSBytes ? 0 : s_base + C::kSBytes;
+          s_next = s_base + in_piece(k0 + KM);
+        }
+        static_for_s<0, SPM>([&](auto tc) __attribute__((always_inline)) {
+          constexpr int t = decltype(tc)::value;
+          const uint32_t abuf_next = abuf + C::kABytes == C::kStages * C::kABytes ? 0 : abuf + C::kABytes;
+          if constexpr (PROD == 0) wait_dma<C::in_flight(t)>();  // (otherwise the producers have waited)
+          __builtin_amdgcn_sched_barrier(0);
+          __builtin_amdgcn_s_barrier();
+          asm volatile("" ::: "memory");
+          static_for_s<0, NS>([&](auto kkc) __attribute__((always_inline)) {
+            constexpr int kk = decltype(kkc)::value, q = t * NS + kk;         // slice of the macro step
+            constexpr int t1 = (q + 1) / NS, kk1 = (q + 1) % NS;              // the next slice, being converted
+            constexpr int t2 = (q + 2) / NS, kk2 = (q + 2) % NS;              // the one after it
+            uint32_t front[PAIRS];
+            static_for_s<0, SLOTS>([&](auto sc) __attribute__((always_inline)) {
+              constexpr int s = decltype(sc)::value, i = s / TN, j = s % TN;
+              acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(
+                  a[q & 1][i], __builtin_bit_cast(half8_t, *reinterpret_cast<const u32x4*>(b[q & 1][j])), acc[i][j], 0, 0, 0);
+              if constexpr (s < TM)
+                a[(q + 1) & 1][s] = *reinterpret_cast<const half8_t*>(smem + (kk1 == 0 ? abuf_next : abuf) + a_rd[kk1] + s * 32 * C::kARow);
+              if constexpr (s == 0 && kk2 == 0) read_words(words[t2 & 1], t2 >= SPM ? ring_next : ring, t2 >= SPM ? s_next : s_off, integral_constant<int, t2 % SPM>{});
+              if constexpr (PROD == 0) {
+                // requests of later stages, evenly over the slots: weights and scales first
+                constexpr int slot = kk * SLOTS + s, WS = t == 0 ? C::kNWS : 0, ALL = WS + C::kNA;
+                constexpr int P0 = slot * ALL / (NS * SLOTS), P1 = (slot + 1) * ALL / (NS * SLOTS);
+                static_for_s<P0, P1>([&](auto pc) __attribute__((always_inline)) {
+                  constexpr int P = decltype(pc)::value;
+                  if constexpr (P < WS) req.template issue_ws<P>(k0 + (C::kMacros - 1) * KM, ring_issue);
+                  else req.template issue_a<P - WS>(k0 + (t + C::kStages - 1) * KA, abuf_issue);
+                });
+              }
+              constexpr int F0 = s * PAIRS / SLOTS, F1 = (s + 1) * PAIRS / SLOTS, B0 = s == 0 ? 0 : (s - 1) * PAIRS / SLOTS, B1 = s + 1 == SLOTS ? PAIRS : F0;
+              static_for_s<F0, F1>([&](auto qc_) __attribute__((always_inline)) {
+                constexpr int p = decltype(qc_)::value;
+                front[p] = convert_front(words[t1 & 1], integral_constant<int, kk1>{}, integral_constant<int, p / 4>{}, integral_constant<int, p % 4>{});
+              });
+              static_for_s<B0, B1>([&](auto qc_) __attribute__((always_inline)) {
+                constexpr int p = decltype(qc_)::value;
+                b[(q + 1) & 1][p / 4][p % 4] = convert_back(words[t1 & 1], front[p], integral_constant<int, kk1>{}, integral_constant<int, p / 4>{}, integral_constant<int, p % 4>{});
+              });
+              __builtin_amdgcn_sched_barrier(0);
+            });
+          });
+          abuf_issue = abuf;
+          abuf = abuf_next;
+        });
+        ring = ring_next;
+        s_off = s_next;
+      }
+      if constexpr (PROD == 0) wait_dma<0>();
+      __builtin_amdgcn_s_barrier();  // the last requests (all out of range) have landed
+      asm volatile("" ::: "memory");
+
+      // ---- K groups: every group hands its partial sums of the other groups' row quads over through LDS ----------------
+      auto part = [&](int pair, int j) __attribute__((always_inline)) {
+        const float16_t& c = acc[pair / 4][j];
+        const int v = pair % 4 * 4;
+        return float4_t{c[v], c[v + 1], c[v + 2], c[v + 3]};
+      };
+      if constexpr (HELP) {
+        static_for_s<0, C::kFG>([&](auto tt) __attribute__((always_inline)) {
           constexpr int t = decltype(tt)::value;
-          if (grp != t) {
-            const int src = grp < t ? grp : grp - 1;
-            float4_t* const dst = reinterpret_cast<float4_t*>(smem) + (((t - T0) * (G - 1) + src) * CW + cw) * PG * TN * 64 + lane;
+          if (t >= G || grp != t) {
+            float4_t* const dst = handed(t, grp);
 #pragma unroll
             for (int p = 0; p < PG; ++p)
 #pragma unroll
@@ -525,100 +549,220 @@ __global__ __launch_bounds__((CW * G + PROD) * 64, 1) void wq_gemm_stream_kernel
           }
         });
         __syncthreads();
-        static_for_s<T0, T1>([&](auto tt) __attribute__((always_inline)) {
+        static_for_s<0, G>([&](auto tt) __attribute__((always_inline)) {
           constexpr int t = decltype(tt)::value;
           if (grp == t) {
-            const float4_t* const sp = reinterpret_cast<const float4_t*>(smem) + ((t - T0) * (G - 1) * CW + cw) * PG * TN * 64 + lane;
 #pragma unroll
             for (int p = 0; p < PG; ++p)
 #pragma unroll
               for (int j = 0; j < TN; ++j) {
-                // (in the order of the groups, whichever of them adds: an output does not depend on its place in the tile)
-                float4_t f = t == 0 ? part(p, j) : sp[(p * TN + j) * 64];
+                fin[p][j] = t == 0 ? part(p, j) : handed(t, 0)[(p * TN + j) * 64];
 #pragma unroll
-                for (int g = 1; g < G; ++g) f += g == t ? part(t * PG + p, j) : sp[((g < t ? g : g - 1) * CW * PG * TN + p * TN + j) * 64];
-                fin[p][j] = f;
+                for (int g = 1; g < G; ++g) fin[p][j] += g == t ? part(t * PG + p, j) : handed(t, g)[(p * TN + j) * 64];
               }
           }
         });
-      });
-    }
+      } else if constexpr (G == 1) {
+#pragma unroll
+        for (int p = 0; p < PG; ++p)
+#pragma unroll
+          for (int j = 0; j < TN; ++j) fin[p][j] = part(p, j);
+      } else {
+        static_for_s<0, (G + C::kTargets - 1) / C::kTargets>([&](auto phase) __attribute__((always_inline)) {
+          constexpr int T0 = decltype(phase)::value * C::kTargets, T1 = T0 + C::kTargets < G ? T0 + C::kTargets : G;
+          __syncthreads();
+          static_for_s<T0, T1>([&](auto tt) __attribute__((always_inline)) {
+            constexpr int t = decltype(tt)::value;
+            if (grp != t) {
+              const int src = grp < t ? grp : grp - 1;
+              float4_t* const dst = reinterpret_cast<float4_t*>(smem) + (((t - T0) * (G - 1) + src) * CW + cw) * PG * TN * 64 + lane;
+#pragma unroll
+              for (int p = 0; p < PG; ++p)
+#pragma unroll
+                for (int j = 0; j < TN; ++j) dst[(p * TN + j) * 64] = part(t * PG + p, j);
+            }
+          });
+          __syncthreads();
+          static_for_s<T0, T1>([&](auto tt) __attribute__((always_inline)) {
+            constexpr int t = decltype(tt)::value;
+            if (grp == t) {
+              const float4_t* const sp = reinterpret_cast<const float4_t*>(smem) + ((t - T0) * (G - 1) * CW + cw) * PG * TN * 64 + lane;
+#pragma unroll
+              for (int p = 0; p < PG; ++p)
+#pragma unroll
+                for (int j = 0; j < TN; ++j) {
+                  // (in the order of the groups, whichever of them adds: an output does not depend on its place in the tile)
+                  float4_t f = t == 0 ? part(p, j) : sp[(p * TN + j) * 64];
+#pragma unroll
+                  for (int g = 1; g < G; ++g) f += g == t ? part(t * PG + p, j) : sp[((g < t ? g : g - 1) * CW * PG * TN + p * TN + j) * 64];
+                  fin[p][j] = f;
+                }
+            }
+          });
+        });
+      }
 
+      if constexpr (MODE == kSerial) {
+#pragma unroll
+        for (int p = 0; p < PG; ++p)
+#pragma unroll
+          for (int j = 0; j < TN; ++j) total[p][j] += fin[p][j];
+        if (++ks == S) break;
+        __syncthreads();  // (the exchange has been read: the requests of the next window may land)
+        k_begin = ks * per_window * KM, k_end = min(k_begin + per_window * KM, K);
+      } else {
+        break;
+      }
+    }
     if constexpr (MODE == kSerial) {
 #pragma unroll
       for (int p = 0; p < PG; ++p)
 #pragma unroll
-        for (int j = 0; j < TN; ++j) total[p][j] += fin[p][j];
-      if (++ks == S) break;
-      __syncthreads();  // (the exchange has been read: the requests of the next window may land)
-      k_begin = ks * per_window * KM, k_end = min(k_begin + per_window * KM, K);
-    } else {
-      break;
+        for (int j = 0; j < TN; ++j) fin[p][j] = total[p][j];
     }
-  }
-  if constexpr (MODE == kSerial) {
-#pragma unroll
-    for (int p = 0; p < PG; ++p)
-#pragma unroll
-      for (int j = 0; j < TN; ++j) fin[p][j] = total[p][j];
   }
 
+  uint32_t owned = ~0u;  // the wavefront's row quads that are this workgroup's to store
   if constexpr (MODE == kSplit) {
-    // K split over workgroups: float32 partial tiles through the workspace, added in window order by the last to arrive.
-    // Partials and counters are only touched by accesses performed at the memory side of the L2s (sc1).
+    // K split over workgroups: float32 partial tiles through the workspace, every output's sum in window order by one workgroup.  Partials and
+    // counters are only touched by accesses performed at the memory side of the L2s (sc1).  A tile's counter has 64 bytes to
+    // itself, as atomics to one line are performed one after the other (int4 20 x 4096 x 11008 in four 12.35 -> 12.05 us).
     constexpr uint32_t kWaveBytes = PG * TN * 1024u;
-    const rsrc_t rp = make_rsrc(reinterpret_cast<char*>(partials) + (size_t)tile_lin * S * WAVES * kWaveBytes, (uint32_t)S * WAVES * kWaveBytes);
+    const rsrc_t rp = make_rsrc(reinterpret_cast<char*>(partials) + (size_t)tile_lin * S * FINISHERS * kWaveBytes, (uint32_t)S * FINISHERS * kWaveBytes);
+    const int counter = tile_lin * kStreamCounterWords;
+    uint32_t* const word = reinterpret_cast<uint32_t*>(smem);
+    auto live = [&](int p) __attribute__((always_inline)) { return (grp * PG + p) * 8 < M - m0; };  // (quads that begin past M are nobody's)
+    auto place = [&](int q, int p, int j) __attribute__((always_inline)) { return (uint32_t)(q * FINISHERS + wave) * kWaveBytes + (p * TN + j) * 1024u; };
+    if constexpr (SCATTER) {
+      // Window w's workgroup finishes part w, every S-th quad: it writes the other parts, counts itself in, waits for the others, and reads its
+      // part of theirs.  Bound by trips to memory: written, counted, seen, read.  Against the last to arrive finishing the whole tile, with
+      // every workgroup writing all of its own (us): int8 256 x 5120 x 5120 in three 26.2 -> 24.6, 256 x 5120 x 13824 in three 51.9 -> 49.2, 99 x 5120 x
+      // 13824 in six 34.0 -> 30.6, int4 149 x 5760 x 6656 in two 28.7 -> 27.9; 64 x 128 tiles 0.99.
+      //
+      // Nobody waits for long: a workgroup whose fellows are not in after kLooks looks at the counter resigns -- it writes its own part
+      // too and leaves it to the last to arrive, whom the counter tells.  The counter: arrivals, a bit for each window that has resigned, parts
+      // accounted for (with all of them it returns to zero).  All of that are adds, so of a resigning workgroup and the last to
+      // arrive exactly one learns of the other.
+      constexpr int kLooks = 8;
+      auto part_of = [&](int w) __attribute__((always_inline)) {
+        uint32_t quads = 0;
+        int owner = wave * PG % S;
 #pragma unroll
-    for (int p = 0; p < PG; ++p)
+        for (int p = 0; p < PG; ++p) {
+          quads |= owner == w ? 1u << p : 0u;
+          owner = owner + 1 == S ? 0 : owner + 1;
+        }
+        return quads;
+      };
+      auto write_quads = [&](uint32_t quads) __attribute__((always_inline)) {
 #pragma unroll
-      for (int j = 0; j < TN; ++j)
-        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, fin[p][j]), rp, (uint32_t)(ks * WAVES + wave) * kWaveBytes + (p * TN + j) * 1024u + lane * 16u, 0, 0x10);
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    __syncthreads();
-    int* const last = reinterpret_cast<int*>(smem);
-    if (threadIdx.x == 0)
-      *last = __hip_atomic_fetch_add(&counters[tile_lin], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == (unsigned)(S - 1);
-    __syncthreads();
-    if (!*last) return;
-    if (threadIdx.x == 0) __hip_atomic_store(&counters[tile_lin], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    // (the last to arrive has its own window in registers: half of the reads of a split in two.  int8 99 x 15360 x 5120 33.8 -> 32.8 us,
-    // 256 x 5120 x 5120 29.3 -> 28.2)
-    constexpr int PS = PG < 4 ? PG : 4, WIN = PS * TN <= 4 ? 4 : 2;  // row quads summed at a time, windows in flight
-    static_for_s<0, PG / PS>([&](auto portion) __attribute__((always_inline)) {
-      constexpr int p0 = decltype(portion)::value * PS;
-      float4_t sum[PS][TN];
+        for (int p = 0; p < PG; ++p)
+          if ((quads >> p & 1u) != 0 && live(p)) {
 #pragma unroll
-      for (int p = 0; p < PS; ++p)
-#pragma unroll
-        for (int j = 0; j < TN; ++j) sum[p][j] = float4_t{0.f, 0.f, 0.f, 0.f};
-      for (int q = 0; q < S; q += WIN) {
-        u32x4 win[WIN][PS][TN];
-#pragma unroll
-        for (int w = 0; w < WIN; ++w)
-#pragma unroll
-          for (int p = 0; p < PS; ++p)
-#pragma unroll
-            for (int j = 0; j < TN; ++j)
-              win[w][p][j] = __builtin_amdgcn_raw_buffer_load_b128(
-                  rp, (q + w < S && q + w != ks ? (uint32_t)((q + w) * WAVES + wave) * kWaveBytes : kStreamOob) + ((p0 + p) * TN + j) * 1024u + lane * 16u, 0, 0x10);
-#pragma unroll
-        for (int w = 0; w < WIN; ++w)
-#pragma unroll
-          for (int p = 0; p < PS; ++p)
-#pragma unroll
-            for (int j = 0; j < TN; ++j) sum[p][j] += q + w == ks ? fin[p0 + p][j] : __builtin_bit_cast(float4_t, win[w][p][j]);
+            for (int j = 0; j < TN; ++j) __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, fin[p][j]), rp, place(ks, p, j) + lane * 16u, 0, 0x10);
+          }
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        __syncthreads();
+      };
+      auto all_in = [&](uint32_t v) __attribute__((always_inline)) { return (v & 0xFFu) == (uint32_t)S; };
+      const uint32_t own = part_of(ks), own_bit = 1u << ks;
+      write_quads(~own);
+      if (threadIdx.x == 0) {
+        uint32_t v = __hip_atomic_fetch_add(&counters[counter], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1u;
+        const uint32_t left = all_in(v) ? v >> 8 & 0xFFu : 0u;
+        for (int i = 0; i < kLooks && !all_in(v); ++i) v = __hip_atomic_fetch_add(&counters[counter], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        *word = all_in(v) ? own_bit | left : 0u;
       }
+      __syncthreads();
+      uint32_t parts = __builtin_amdgcn_readfirstlane(*word);
+      if (parts == 0) {
+        write_quads(own);
+        if (threadIdx.x == 0) *word = all_in(__hip_atomic_fetch_add(&counters[counter], 0x100u << ks, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) ? own_bit : 0u;
+        __syncthreads();
+        parts = __builtin_amdgcn_readfirstlane(*word);
+      }
+      if (threadIdx.x == 0 && parts != 0) {
+        const uint32_t here = (uint32_t)__builtin_popcount(parts) << 16;
+        if ((__hip_atomic_fetch_add(&counters[counter], here, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + here) >> 16 == (uint32_t)S)
+          __hip_atomic_store(&counters[counter], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      }
+      owned = 0;
+      for (uint32_t todo = parts; todo != 0; todo &= todo - 1) owned |= part_of(__builtin_ctz(todo));
 #pragma unroll
-      for (int p = 0; p < PS; ++p)
+      for (int p = 0; p < PG; ++p)
+        if ((owned >> p & 1u) != 0 && live(p)) {
+          u32x4 win[kMaxWindows][TN];
 #pragma unroll
-        for (int j = 0; j < TN; ++j) fin[p0 + p][j] = sum[p][j];
-    });
-    if (done != nullptr) {
-      // (a workspace of the library's: once every wavefront has read and the counter is back at zero, the host may know)
+          for (int q = 0; q < kMaxWindows; ++q)
+            if (q < S && q != ks) {
+#pragma unroll
+              for (int j = 0; j < TN; ++j) win[q][j] = __builtin_amdgcn_raw_buffer_load_b128(rp, place(q, p, j) + lane * 16u, 0, 0x10);
+            }
+          float4_t sum[TN];
+#pragma unroll
+          for (int j = 0; j < TN; ++j) sum[j] = float4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+          for (int q = 0; q < kMaxWindows; ++q)
+            if (q < S) {
+#pragma unroll
+              for (int j = 0; j < TN; ++j) sum[j] += q == ks ? fin[p][j] : __builtin_bit_cast(float4_t, win[q][j]);
+            }
+#pragma unroll
+          for (int j = 0; j < TN; ++j) fin[p][j] = sum[j];
+        }
+    } else {
+      // The last to arrive finishes the tile, its own window still in registers: no trip to see the others arrive, which is worth more than
+      // sharing the reads where a tile has few of them (64 x 64 and 32 rows: shared 0.3 - 0.6 us slower).
+#pragma unroll
+      for (int p = 0; p < PG; ++p)
+#pragma unroll
+        for (int j = 0; j < TN; ++j)
+          __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, fin[p][j]), rp, (live(p) ? place(ks, p, j) : kStreamOob) + lane * 16u, 0, 0x10);
       asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
       __syncthreads();
-      if (threadIdx.x == 0) __hip_atomic_store(&done[tile_lin], launch, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+      if (threadIdx.x == 0)
+        *word = __hip_atomic_fetch_add(&counters[counter], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == (unsigned)(S - 1);
+      __syncthreads();
+      if (*word == 0) return;
+      if (threadIdx.x == 0) __hip_atomic_store(&counters[counter], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      constexpr int PS = PG < 4 ? PG : 4, WIN = PS * TN <= 4 ? 4 : 2;  // row quads summed at a time, windows in flight
+      static_for_s<0, PG / PS>([&](auto portion) __attribute__((always_inline)) {
+        constexpr int p0 = decltype(portion)::value * PS;
+        float4_t sum[PS][TN];
+#pragma unroll
+        for (int p = 0; p < PS; ++p)
+#pragma unroll
+          for (int j = 0; j < TN; ++j) sum[p][j] = float4_t{0.f, 0.f, 0.f, 0.f};
+        for (int q = 0; q < S; q += WIN) {
+          u32x4 win[WIN][PS][TN];
+#pragma unroll
+          for (int w = 0; w < WIN; ++w)
+#pragma unroll
+            for (int p = 0; p < PS; ++p)
+#pragma unroll
+              for (int j = 0; j < TN; ++j)
+                win[w][p][j] = __builtin_amdgcn_raw_buffer_load_b128(rp, (q + w < S && q + w != ks && live(p0 + p) ? place(q + w, p0 + p, j) : kStreamOob) + lane * 16u, 0, 0x10);
+#pragma unroll
+          for (int w = 0; w < WIN; ++w)
+#pragma unroll
+            for (int p = 0; p < PS; ++p)
+#pragma unroll
+              for (int j = 0; j < TN; ++j) sum[p][j] += q + w == ks ? fin[p0 + p][j] : __builtin_bit_cast(float4_t, win[w][p][j]);
+        }
+#pragma unroll
+        for (int p = 0; p < PS; ++p)
+#pragma unroll
+          for (int j = 0; j < TN; ++j) fin[p0 + p][j] = sum[p][j];
+      });
     }
+    if (done != nullptr) {
+      // (a workspace of the library's: once every wavefront has read, and the counter, if it was this workgroup's to return, is back at
+      // zero, the host may know)
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      __syncthreads();
+      if (threadIdx.x == 0) __hip_atomic_store(&done[SCATTER ? tile_lin * S + ks : tile_lin], launch, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    }
+    if (SCATTER && owned == 0) return;
   }
 
   // ---- epilogue: lane holds columns n .. n + TN - 1, rows 8 (pair % 4) + 4 fh + e of row block pair / 4.  The tail's shape
@@ -639,7 +783,7 @@ __global__ __launch_bounds__((CW * G + PROD) * 64, 1) void wq_gemm_stream_kernel
         float up = fin[p][TN - 1][e];
         if constexpr (TN == 1) up = __shfl_down(up, 1);
         const half_t h = silu_mul((half_t)fin[p][0][e], (half_t)up);
-        __builtin_amdgcn_raw_buffer_store_b16(__builtin_bit_cast(uint16_t, h), ry, r < (uint32_t)rows && col != kStreamOob ? r * (uint32_t)half_n * 2u + col : kStreamOob, 0, 0);
+        __builtin_amdgcn_raw_buffer_store_b16(__builtin_bit_cast(uint16_t, h), ry, r < (uint32_t)rows && (owned >> p & 1u) != 0 && col != kStreamOob ? r * (uint32_t)half_n * 2u + col : kStreamOob, 0, 0);
       }
     return;
   }
@@ -654,13 +798,13 @@ __global__ __launch_bounds__((CW * G + PROD) * 64, 1) void wq_gemm_stream_kernel
   // of row quad p, row e, column offset c; p = 0, e = 0 is `base`
   auto offset = [&](int p, int e, uint32_t c) __attribute__((always_inline)) {
     const int r = row_in_tile(p, e);
-    return r < rows && c != kStreamOob ? base + (uint32_t)(r - row_in_tile(0, 0)) * pitch + c : kStreamOob;
+    return r < rows && (owned >> p & 1u) != 0 && c != kStreamOob ? base + (uint32_t)(r - row_in_tile(0, 0)) * pitch + c : kStreamOob;
   };
   // of row quad p, row e of the pairs.  (A column beyond N: kStreamOob and less than 2^31 on top stays out of range, so that
   // only the row is compared.)
   auto pair_offset = [&](int p, int e) __attribute__((always_inline)) {
     const int r = row_in_tile(p, e);
-    return r < rows ? base + col + (uint32_t)(r - row_in_tile(0, 0)) * pitch : kStreamOob;
+    return r < rows && (owned >> p & 1u) != 0 ? base + col + (uint32_t)(r - row_in_tile(0, 0)) * pitch : kStreamOob;
   };
   auto tail = [&](half2_t (&h)[PC][4], half2_t b2) __attribute__((always_inline)) {
     if (ep.bias != nullptr) {

@@ -71,6 +71,9 @@ bool find_memory(Slots<SLOTS, BYTES>* o, const void* symbol) {
   return true;
 }
 
+// how many of a slot's `done` a launch writes
+int launch_marks(const GemmPlan& plan) { return (int)plan.tiles * (plan.shares ? plan.split : 1); }
+
 template <int SLOTS, int64_t BYTES>
 SplitSpace take_slot(Slots<SLOTS, BYTES>* o, const void* symbol, hipStream_t s, const GemmPlan& plan, std::unique_lock<std::mutex>* lock) {
   if (plan.bytes > BYTES) return {};
@@ -80,14 +83,14 @@ SplitSpace take_slot(Slots<SLOTS, BYTES>* o, const void* symbol, hipStream_t s, 
   if (slot == nullptr) return {};
   const int64_t i = slot - o->owners.slot;
   slot->done = o->done + i * kSlotTiles;
-  slot->tiles = (int)plan.tiles;
+  slot->tiles = launch_marks(plan);
   return SplitSpace{o->base + i * BYTES, o->done + i * kSlotTiles, ++slot->launch};
 }
 
 // A workspace for one launch of a plan on `s`; empty where there is none.  The caller passes `lock` in and keeps it until
 // its launch is in the stream: another thread's launch on the same stream must not come between the two.
 SplitSpace library_space(hipStream_t s, const GemmPlan& plan, bool decode, std::unique_lock<std::mutex>* lock) {
-  if (s == hipStreamPerThread || plan.tiles > kSlotTiles) return {};  // (one handle for a stream in every thread)
+  if (s == hipStreamPerThread || launch_marks(plan) > kSlotTiles) return {};  // (one handle for a stream in every thread)
   static Slots<kSlots, kSlotBytes> slots[kMaxDevices];
   static Slots<kDecodeSlots, kDecodeSplitBytes> small[kMaxDevices];
   const int device = current_device_slot();

@@ -29,6 +29,7 @@ struct Problem {
 // decode kernel: N <= 65536).
 constexpr int64_t kSplitMaxTiles = 4096;
 constexpr int64_t kSplitCounterBytes = kSplitMaxTiles * 4;
+constexpr int kStreamCounterWords = 16;  // of the streamed GEMM's split, a tile
 // Counters and partial tiles of a call of up to 16 rows on memory of the library's.
 constexpr int64_t kDecodeSplitBytes = kSplitCounterBytes + 4 * 1024 * 1024;
 
@@ -64,10 +65,14 @@ bool launch_gemm_pipe(const Problem& p, int group_shift, int variant);
 enum { kStream128x256 = 1, kStream128x128, kStream256x256, kStream64x128, kStream64x64, kStream32x64, kStream32x128, kStream64x96, kStream32x96 };
 bool gemm_stream_applicable(const Problem& p);
 // Whether a tile of so many rows and columns, `macro_step` of K at a time, asks for `p`'s scales in pieces; and the tiles that have a build for it.
+// Whether the windows of such a tile split over workgroups share the finishing of it; else the last to arrive does that.
+constexpr bool stream_split_shares(int rows, int columns) { return rows >= 64 && columns == 128; }
+constexpr int kMaxWindows = 8;
 constexpr bool stream_pieces_built(int bits, int rows, int columns) { return bits == 8 || rows > 32 || columns > 64; }
 bool stream_scale_pieces(const Problem& p, int rows, int columns, int macro_step);
 // A workspace for K in windows over workgroups: the caller's, or one of the library's own, whose launches are numbered and
-// write their number to `done[tile]`, in host memory, when a tile's partial sums have been read.
+// write their number to `done`, in host memory, for every workgroup (where those share the finishing of a tile, else tile) whose share of the
+// partial sums has been read.
 struct SplitSpace {
   void* base = nullptr;
   uint32_t* done = nullptr;
@@ -105,6 +110,7 @@ struct GemmPlan {
   int variant = 0, split = 1;  // tile, windows of K
   float us = 0.f, both_us = 0.f;  // on the problem's layout, on both together
   int64_t tiles = 0, bytes = 0;  // bytes of workspace
+  bool shares = false;  // stream_split_shares
 };
 GemmPlan plan_stream(const Problem& p, bool may_split);
 GemmPlan plan_decode_stream(const Problem& p);

@@ -6,15 +6,15 @@
 
 namespace wq {
 
-constexpr int kSlotTiles = 256;  // tiles of a launch that splits K over workgroups: at most half of 9/8 times the CUs
+constexpr int kSlotTiles = 512;  // what a launch that splits K over workgroups marks: its tiles or its workgroups, at most 9/8 times the CUs
 
 // Workspaces of a device.  Calls of up to 16 rows, whose launches are short and which a program may have on many streams at once, have
 // small ones of their own: without a slot such a call takes 2.2 times as long as on the decode kernel (1.6 - 2.9 times in eight of
 // ten of 726 problems), with one 0.79 times.
 constexpr int kSlots = 8, kDecodeSlots = 24;
 
-// One workspace: the stream that launches on it, and for every tile the number of the launch that has read its partial
-// sums last, written by the kernel into host memory.
+// One workspace: the stream that launches on it, and for every tile (workgroup, where those share the finishing of one: `tiles` of them)
+// the number of the launch that has read its partial sums last, written by the kernel into host memory.
 struct Slot {
   hipStream_t stream = nullptr;
   const volatile uint32_t* done = nullptr;
