@@ -38,11 +38,13 @@ struct TileCost {
 
 // (The tiles of 96 columns, fitted to 1,700 timings of up to 256 rows, are the fastest on 16400 - 24576 columns, where 64-column tiles are more than
 // a round and 128-column ones much less: 17 - 64 rows 0.82 - 0.93 of the time there.  K is not split in them.)
+// (int8 128 x 256 and int4 256 x 256: refitted with their rings of 32-k stages, 320 timings of 130 - 2048 rows, within 3 - 4.5 %; the choice among the three
+// largest tiles by these is within 0.2 % of the fastest.)
 constexpr TileCost kStreamCost[2][2][9] = {
     {{  // int4, canonical
          {kStream128x256, 128, 256, 0.00f, 5.47f, 2.244f, 1.157f, 8.60f, 0.f, 0.f, 0.f},
          {kStream128x128, 128, 128, 0.00f, 5.68f, 1.212f, 0.494f, 4.15f, 4.12f, 1.383f, 0.31f},
-         {kStream256x256, 256, 256, 0.00f, 7.52f, 4.841f, 2.567f, 20.0f, 0.f, 0.f, 0.f},
+         {kStream256x256, 256, 256, 0.00f, 10.36f, 4.505f, 1.704f, 20.0f, 0.f, 0.f, 0.f},
          {kStream64x128, 64, 128, 1.14f, 3.71f, 0.836f, 0.291f, 2.00f, 2.45f, 0.747f, 1.16f},
          {kStream64x64, 64, 64, 1.47f, 3.12f, 0.520f, 0.181f, 0.00f, 1.75f, 0.450f, 0.19f},
          {kStream32x64, 32, 64, 1.10f, 2.44f, 0.459f, 0.065f, 0.03f, 1.75f, 0.275f, 0.24f},
@@ -52,7 +54,7 @@ constexpr TileCost kStreamCost[2][2][9] = {
      {  // int4, tile-major
          {kStream128x256, 128, 256, 0.00f, 6.00f, 2.483f, 1.013f, 10.16f, 0.f, 0.f, 0.f},
          {kStream128x128, 128, 128, 0.29f, 5.37f, 1.339f, 0.471f, 3.49f, 3.97f, 1.275f, 0.65f},
-         {kStream256x256, 256, 256, 0.00f, 8.65f, 4.752f, 2.505f, 20.05f, 0.f, 0.f, 0.f},
+         {kStream256x256, 256, 256, 0.00f, 11.85f, 4.305f, 1.617f, 20.05f, 0.f, 0.f, 0.f},
          {kStream64x128, 64, 128, 1.11f, 3.78f, 0.902f, 0.262f, 1.90f, 2.52f, 0.802f, 0.53f},
          {kStream64x64, 64, 64, 1.53f, 2.96f, 0.577f, 0.176f, 0.00f, 1.86f, 0.453f, 0.06f},
          {kStream32x64, 32, 64, 1.45f, 2.23f, 0.490f, 0.069f, 0.15f, 1.62f, 0.246f, 0.36f},
@@ -60,7 +62,7 @@ constexpr TileCost kStreamCost[2][2][9] = {
          {kStream64x96, 64, 96, 1.65f, 3.01f, 0.774f, 0.284f, 0.00f, 0.f, 0.f, 0.f},
          {kStream32x96, 32, 96, 2.12f, 2.40f, 0.608f, 0.170f, 0.03f, 0.f, 0.f, 0.f}}},
     {{  // int8, canonical
-         {kStream128x256, 128, 256, 2.45f, 0.00f, 3.575f, 0.733f, 8.60f, 0.f, 0.f, 0.f},
+         {kStream128x256, 128, 256, 1.29f, 5.25f, 2.456f, 1.368f, 8.60f, 0.f, 0.f, 0.f},
          {kStream128x128, 128, 128, 0.00f, 4.75f, 1.419f, 0.474f, 4.15f, 4.03f, 1.378f, 1.04f},
          {kStream256x256, 256, 256, 0.00f, 7.50f, 5.039f, 1.840f, 20.0f, 0.f, 0.f, 0.f},
          {kStream64x128, 64, 128, 1.79f, 1.69f, 1.201f, 0.192f, 2.00f, 2.61f, 0.798f, 1.83f},
@@ -70,7 +72,7 @@ constexpr TileCost kStreamCost[2][2][9] = {
          {kStream64x96, 64, 96, 0.31f, 4.29f, 0.754f, 0.692f, 0.00f, 0.f, 0.f, 0.f},
          {kStream32x96, 32, 96, 1.68f, 2.64f, 0.582f, 0.289f, 0.03f, 0.f, 0.f, 0.f}},
      {  // int8, tile-major
-         {kStream128x256, 128, 256, 1.75f, 3.44f, 3.984f, 0.646f, 10.07f, 0.f, 0.f, 0.f},
+         {kStream128x256, 128, 256, 0.91f, 5.22f, 3.007f, 0.881f, 10.07f, 0.f, 0.f, 0.f},
          {kStream128x128, 128, 128, 0.00f, 6.12f, 1.392f, 0.518f, 3.27f, 3.28f, 1.206f, 0.46f},
          {kStream256x256, 256, 256, 0.00f, 9.99f, 4.983f, 1.781f, 25.92f, 0.f, 0.f, 0.f},
          {kStream64x128, 64, 128, 1.65f, 3.14f, 1.186f, 0.223f, 1.87f, 2.27f, 0.609f, 1.04f},

@@ -28,7 +28,11 @@
 // Rings: what a tile has in flight decides below 128 rows.  int8 64 x 128 with 128-byte weight rows has 32 KB a macro step, and
 // two of them leave one ahead: with 64-byte rows, four macro steps and two K groups 15360 x 5120 at 128 rows 37.9 -> 35.2 us,
 // 27648 x 5120 at 99 71.7 -> 65.3, 5120 x 5120 at 256 29.5 -> 25.7.  int4 64 x 128 has enough in flight and gains from two K
-// groups instead of four (half of the exchange at the end): 12288 x 4096 at 37 rows 20.2 -> 18.7.  32-row tiles for up to 32
+// groups instead of four (half of the exchange at the end): 12288 x 4096 at 37 rows 20.2 -> 18.7.  The tiles of 256 columns whose ring had
+// room for three stages of 64 k of activations, two ahead of the MFMAs, waited for them; stages of 32 k, six of them in less memory: int8 128 x 256
+// 256 x 15360 x 5120 84 -> 69 us (256 x 27648 x 5120 takes it now, one round for two of 128 x 128: 88 -> 79), int4 256 x 256 512 x 6144 x 4096 108 -> 87
+// (2048 x 22016 x 4096 338 -> 329, on 128 x 256 tiles 335).  256 x 128 tiles, which convert a weight half as often, are behind (int8 256 x 7680 x 5120 82 us
+// against 67): twice the activations of a row's weights go through the L1.  32-row tiles for up to 32
 // rows (half of the MFMAs and of the activation traffic; a remainder of up to 32 rows as well): int4 12288 x 4096 at 20 rows
 // 14.0 -> 11.8, 22016 x 4096 21.1 -> 17.8, int8 27648 x 5120 at 32 rows 41.5 -> 32.7 us.  96 columns for
 // matrices of more than one round of 64-column tiles and far less than one of 128-column tiles: int4 22016 x 4096 at 20 / 37
@@ -977,7 +981,7 @@ bool launch_gemm_stream_bits(const Problem& p, int variant, int ksplit, const Sp
     switch (variant) {
       WQ_STREAM(kStream128x256, kWholeOnly, 4, 2, 4, 1, 4, 64, 256, 2)
       WQ_STREAM(kStream128x128, kWholeAndSplit, 4, 2, 2, 2, 4, 64, 256, 2)
-      WQ_STREAM(kStream256x256, kWholeOnly, 8, 2, 4, 1, 0, 64, 128, 3)
+      WQ_STREAM(kStream256x256, kWholeOnly, 8, 2, 4, 1, 0, 32, 128, 3)
       WQ_STREAM(kStream64x128, kAllBuilds, 2, 2, 2, 2, 4, 128, 256, 3)
       WQ_STREAM(kStream64x64, kAllBuilds, 2, 1, 2, 4, 4, 128, 256, 3)
       WQ_STREAM(kStream32x64, kAllBuilds, 1, 1, 2, 4, 4, 128, 256, 3)
@@ -987,7 +991,7 @@ bool launch_gemm_stream_bits(const Problem& p, int variant, int ksplit, const Sp
     }
   } else {
     switch (variant) {
-      WQ_STREAM(kStream128x256, kWholeOnly, 4, 2, 4, 1, 4, 64, 128, 3)
+      WQ_STREAM(kStream128x256, kWholeOnly, 4, 2, 4, 1, 4, 32, 128, 3)
       WQ_STREAM(kStream128x128, kWholeAndSplit, 4, 2, 2, 2, 4, 64, 128, 3)
       WQ_STREAM(kStream256x256, kWholeOnly, 8, 2, 4, 1, 0, 32, 128, 2)
       WQ_STREAM(kStream64x128, kAllBuilds, 2, 2, 2, 2, 4, 64, 128, 4)
