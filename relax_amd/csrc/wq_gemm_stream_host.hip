@@ -26,7 +26,9 @@ bool gemm_stream_applicable(const Problem& p) {
 
 namespace {
 
-// Workspaces of the library's own for calls of up to 256 rows that bring none (more rows fill the chip without a split).
+// Workspaces of the library's own for calls that bring none.  From 257 rows on too, wherever at most half of the CUs would have a tile: int4 512 x 4096 x 11008
+// 59.6 -> 52.5 us, int8 300 x 5120 x 13824 / 5120 x 5120 70.0 -> 59.6 / 30.3 -> 27.4; 40 problems of 257 - 1400 rows 0.87 of the unsplit time (0.62 - 1.0,
+// one of 10 us 1.07).
 // The memory is part of the code object (zero at load, as the counters have to be).  A call that finds
 // no slot runs its windows one after the other, with the same result (kSerial in wq_gemm_stream.hip).
 constexpr int64_t kSlotBytes = kSplitCounterBytes + (20ll << 20);  // (the largest plan: 288 windows of 128 x 128 float32)
@@ -139,9 +141,10 @@ int launch_plan(const Problem& p, const GemmPlan& plan, void* workspace, bool sl
 
 int launch_gemm_stream_planned(const Problem& p, void* workspace, int64_t workspace_bytes, float other_us) {
   if (!in_range(p)) return 0;
-  GemmPlan plan = plan_stream(p, p.m <= 256 || workspace != nullptr);
+  GemmPlan plan = plan_stream(p, true);
   const bool slot = plan.split > 1 && plan.bytes > workspace_bytes;
-  if (slot && (p.m > 256 || captured(p))) plan = plan_stream(p, false);
+  // (hipStreamPerThread never has a slot: many rows, whose windows one after the other would take the longest, are not split there)
+  if (slot && (captured(p) || (p.m > 256 && p.stream == hipStreamPerThread))) plan = plan_stream(p, false);
   const GemmPlan strip = plan_strip(p);
   switch (choose_streamed(p, strip, plan, other_us)) {
     case kOtherKernel: return 0;

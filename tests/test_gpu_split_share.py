@@ -57,3 +57,38 @@ def test_workgroups_that_come_late():
             outs.append((i % 3, relax_amd.wq_matmul(*operands[i % 3], stream=stream, out=torch.empty_like(alone[i % 3]))))
     torch.cuda.synchronize()
     assert all(torch.equal(y.view(torch.int16), alone[i].view(torch.int16)) for i, y in outs)
+
+
+@pytest.mark.parametrize("bits,m,n,k", [(4, 512, 4096, 11008), (8, 300, 5120, 13824), (8, 257, 1001, 9216), (4, 1024, 2048, 8192), (4, 385, 640, 12800)])
+def test_more_than_256_rows_split_on_the_librarys_memory(bits, m, n, k):
+    """Without a workspace the bits of the split on one; captured, and on hipStreamPerThread, the unsplit call's."""
+    import relax_amd
+
+    x, wq, s, g = O.make_case(m + n, m, n, k, bits)
+    dx, dw, ds = _dev(x), _dev(wq), _dev(s)
+    res = _dev(_fused_operands(m + n, m, n)[1])
+    need = relax_amd.wq_workspace_bytes(bits, g, n, k, m)
+    assert need > 16384, "the case is meant to split"
+    space = relax_amd.wq_workspace(need)
+    rows = [0, m // 2, m - 1]
+    want = c_oracle.wq_matmul(x[rows], wq, s, bits, g, nthreads=8)
+    for tail in ({}, dict(residual=res)):
+        split = relax_amd.wq_matmul(dx, dw, ds, bits, g, workspace=space, **tail)
+        for stream in (None, torch.cuda.Stream()):
+            torch.cuda.synchronize()
+            y = relax_amd.wq_matmul(dx, dw, ds, bits, g, stream=stream, **tail)
+            torch.cuda.synchronize()
+            assert torch.equal(y.view(torch.int16), split.view(torch.int16)), list(tail)
+        whole = relax_amd.wq_matmul(dx, dw, ds, bits, g, stream=PerThread, **tail)
+        torch.cuda.synchronize()
+        captured, graph = torch.empty_like(whole), torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            relax_amd.wq_matmul(dx, dw, ds, bits, g, out=captured, **tail)
+        for _ in range(3):
+            captured.zero_()
+            graph.replay()
+            torch.cuda.synchronize()
+            assert torch.equal(captured.view(torch.int16), whole.view(torch.int16)), list(tail)
+        if not tail:
+            assert_close(split.cpu().numpy()[rows], want, (bits, m, n, k), ulp_fraction=0.005)
+            assert_close(whole.cpu().numpy()[rows], want, (bits, m, n, k), ulp_fraction=0.005)
