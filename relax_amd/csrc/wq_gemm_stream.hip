@@ -301,6 +301,7 @@ __global__ __launch_bounds__((CW * G + PROD) * 64, 1) void wq_gemm_stream_kernel
   // (barriers of the exchange between the K groups at a window's end)
   constexpr int kExchangeBarriers = G == 1 ? 0 : 2 * ((G + C::kTargets - 1) / C::kTargets);
 
+  float16_t acc[TM][TN];
   float4_t fin[PG][TN], total[MODE == kSerial ? PG : 1][TN];
   // HELP: where quad p of target group t from group g is in LDS, `lane`s apart
   auto handed = [&](int t, int g) __attribute__((always_inline)) {
@@ -395,7 +396,6 @@ __global__ __launch_bounds__((CW * G + PROD) * 64, 1) void wq_gemm_stream_kernel
     }
 
     const Q4Consts qc = make_q4_consts(zero_point);
-    float16_t acc[TM][TN];
     if constexpr (MODE == kSerial) {
 #pragma unroll
       for (int p = 0; p < PG; ++p)
