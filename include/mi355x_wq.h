@@ -68,14 +68,14 @@ enum {
  * (pointer/shape extraction, launch on the current stream, no host sync).
  *
  * Calls of 17 rows and more whose tiles leave half of the CUs idle split K over workgroups on one of eight workspaces of 20 MB per GPU
- * that are part of the library's code object (160 MB of each GPU while the library is loaded; the first such call allocates 8 KB
+ * that are part of the library's code object (160 MB of each GPU while the library is loaded; the first such call allocates 16 KB
  * of pinned host memory, the others nothing).  One belongs to a stream and passes to another once its owner's last launch
  * on it has ended, also if the owner is gone; a call that finds none (a ninth busy stream, hipStreamPerThread) adds up the same windows one after the other in each workgroup, which takes up to three times as
  * long.  The result has the same bits on every stream, whatever other threads and streams do (up to 16 rows and from 257 on: on every stream but hipStreamPerThread, where the latter run unsplit).  A call under stream
  * capture uses none of the library's memory and, without a workspace of the caller's (mi355x_wq_matmul_ws), runs
  * unsplit: its float32 sums are added in another order than the eager call's, the same in every replay.
  * Up to 16 rows the same holds for canonical weights with long K (from 8192 on) and few row tiles per CU, where such a
- * split is ahead of the decode kernel: these calls have 24 workspaces of 4 MB of their own (96 MB more of each GPU, 24 KB of
+ * split is ahead of the decode kernel: these calls have 24 workspaces of 4 MB of their own (96 MB more of each GPU, 48 KB of
  * pinned host memory at the first call), and one that finds none, on a 25th busy stream, takes two to three times as
  * long; under capture and on hipStreamPerThread these run the decode kernel, whose sums are in another order too. */
 MI355X_WQ_API int mi355x_wq_matmul(const mi355x_wq_desc* desc, const void* x, const void* wq, const void* scales,
