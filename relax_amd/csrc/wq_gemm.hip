@@ -296,7 +296,9 @@ int launch_gemm_any(const Problem& p, int variant, bool direct_ok) {
     return -1;
   }
   if (variant >= 31) {
-    if (!(variant > 40 ? launch_gemm_strip(p, variant - 40) : launch_gemm_stream(p, variant - 30, 1, SplitSpace{}))) {
+    if (!(variant == 50  ? launch_gemm_stream_unwatched(p)
+          : variant > 40 ? launch_gemm_strip(p, variant - 40)
+                         : launch_gemm_stream(p, variant - 30, 1, SplitSpace{}))) {
       set_error("gemm kernel: streamed variant %d does not apply to M=%lld N=%lld K=%lld group=%d", variant, (long long)p.m,
                 (long long)p.n, (long long)p.k, p.group);
       return -1;

@@ -44,6 +44,7 @@
 
 #include "wq_device.h"
 #include "wq_internal.h"
+#include "wq_split_share.h"
 
 namespace wq {
 
@@ -259,7 +260,7 @@ template <int BITS, int TM, int TN, int CW, int G, int PROD, int KA, int KM, int
 __global__ __launch_bounds__((CW * G + PROD) * 64, 1) void wq_gemm_stream_kernel(
     const half_t* __restrict__ x, const uint32_t* __restrict__ wq, const half_t* __restrict__ scales, int M, int N, int K,
     int shift_and_zero, int tiles_m, int tiles_n, int ksplit, half_t* y, const Epilogue ep, float* partials,
-    unsigned int* counters, uint32_t* done, uint32_t launch) {
+    unsigned int* counters, uint32_t* done, uint32_t launch, int looks) {
   using C = StreamShape<BITS, TM, TN, CW, G, PROD, KA, KM, NM, SV>;
   static_assert(!(TILED && SV), "tile-major scales lie as they are read");
   constexpr int BM = C::kBM, BN = C::kBN, WAVES = C::kWaves, SPM = C::kSPM, NS = C::kSlices;
@@ -643,11 +644,9 @@ __global__ __launch_bounds__((CW * G + PROD) * 64, 1) void wq_gemm_stream_kernel
       // every workgroup writing all of its own (us): int8 256 x 5120 x 5120 in three 26.2 -> 24.6, 256 x 5120 x 13824 in three 51.9 -> 49.2, 99 x 5120 x
       // 13824 in six 34.0 -> 30.6, int4 149 x 5760 x 6656 in two 28.7 -> 27.9; 64 x 128 tiles 0.99.
       //
-      // Nobody waits for long: a workgroup whose fellows are not in after kLooks looks at the counter resigns -- it writes its own part
-      // too and leaves it to the last to arrive, whom the counter tells.  The counter: arrivals, a bit for each window that has resigned, parts
-      // accounted for (with all of them it returns to zero).  All of that are adds, so of a resigning workgroup and the last to
-      // arrive exactly one learns of the other.
-      constexpr int kLooks = 8;
+      // Nobody waits for long: a workgroup whose fellows are not in after `looks` looks at the counter resigns (wq_split_share.h).  Every access to the
+      // counter but its return to zero is an add, so that all of them are in one order.  The addend is one that the compiler does not see: it would
+      // make an add of zero a load, with which fourteen shapes take 1 % longer (int8 99 x 5120 x 13824 31.3 -> 31.8 us).
       auto part_of = [&](int w) __attribute__((always_inline)) {
         uint32_t quads = 0;
         int owner = wave * PG % S;
@@ -658,7 +657,9 @@ __global__ __launch_bounds__((CW * G + PROD) * 64, 1) void wq_gemm_stream_kernel
         }
         return quads;
       };
-      auto write_quads = [&](uint32_t quads) __attribute__((always_inline)) {
+      const uint32_t own = part_of(ks);
+      auto write_parts = [&](uint32_t parts) __attribute__((always_inline)) {
+        const uint32_t quads = (parts >> ks & 1u) != 0 ? own : ~own;
 #pragma unroll
         for (int p = 0; p < PG; ++p)
           if ((quads >> p & 1u) != 0 && live(p)) {
@@ -668,30 +669,19 @@ __global__ __launch_bounds__((CW * G + PROD) * 64, 1) void wq_gemm_stream_kernel
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         __syncthreads();
       };
-      auto all_in = [&](uint32_t v) __attribute__((always_inline)) { return (v & 0xFFu) == (uint32_t)S; };
-      const uint32_t own = part_of(ks), own_bit = 1u << ks;
-      write_quads(~own);
-      if (threadIdx.x == 0) {
-        uint32_t v = __hip_atomic_fetch_add(&counters[counter], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1u;
-        const uint32_t left = all_in(v) ? v >> 8 & 0xFFu : 0u;
-        uint32_t nothing = 0;
-        asm volatile("" : "+v"(nothing));  // (an addend that the compiler sees to be zero makes the look a load: fourteen shapes 1 % slower, int8 99 x 5120 x 13824 31.3 -> 31.8 us)
-        for (int i = 0; i < kLooks && !all_in(v); ++i) v = __hip_atomic_fetch_add(&counters[counter], nothing, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        *word = all_in(v) ? own_bit | left : 0u;
-      }
-      __syncthreads();
-      uint32_t parts = __builtin_amdgcn_readfirstlane(*word);
-      if (parts == 0) {
-        write_quads(own);
-        if (threadIdx.x == 0) *word = all_in(__hip_atomic_fetch_add(&counters[counter], 0x100u << ks, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) ? own_bit : 0u;
+      auto add = [&](uint32_t by) __attribute__((always_inline)) {
+        asm volatile("" : "+v"(by));
+        return __hip_atomic_fetch_add(&counters[counter], by, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      };
+      auto one = [&](auto&& f) __attribute__((always_inline)) {
+        if (threadIdx.x == 0) *word = f();
         __syncthreads();
-        parts = __builtin_amdgcn_readfirstlane(*word);
-      }
-      if (threadIdx.x == 0 && parts != 0) {
-        const uint32_t here = (uint32_t)__builtin_popcount(parts) << 16;
-        if ((__hip_atomic_fetch_add(&counters[counter], here, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + here) >> 16 == (uint32_t)S)
-          __hip_atomic_store(&counters[counter], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      }
+        return (uint32_t)__builtin_amdgcn_readfirstlane(*word);
+      };
+      auto zero = [&](auto&& if_last) __attribute__((always_inline)) {
+        if (threadIdx.x == 0 && if_last()) __hip_atomic_store(&counters[counter], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      };
+      const uint32_t parts = split_parts(S, ks, looks, write_parts, one, add, zero);
       owned = 0;
       for (uint32_t todo = parts; todo != 0; todo &= todo - 1) owned |= part_of(__builtin_ctz(todo));
 #pragma unroll
@@ -942,7 +932,7 @@ bool launch_stream(const Problem& p, int ksplit, const SplitSpace& space) {
   hipLaunchKernelGGL(kernel, dim3(tiles_m * tiles_n * (MODE == kSplit ? ksplit : 1)), dim3(C::kThreads), C::kLds, p.stream,
                      (const half_t*)p.x, (const uint32_t*)p.wq, (const half_t*)p.scales, (int)p.m, (int)p.n, (int)p.k,
                      group_log2 | (p.zero_point << 8) | (p.activation == kActGated ? 1 << 16 : 0), tiles_m, tiles_n, ksplit,
-                     (half_t*)p.y, Epilogue{(const half_t*)p.bias, (const half_t*)p.residual, p.activation}, partials, counters, space.done, space.launch);
+                     (half_t*)p.y, Epilogue{(const half_t*)p.bias, (const half_t*)p.residual, p.activation}, partials, counters, space.done, space.launch, space.looks);
   return true;
 }
 

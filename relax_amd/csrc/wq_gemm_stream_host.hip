@@ -153,6 +153,15 @@ int launch_gemm_stream_planned(const Problem& p, void* workspace, int64_t worksp
   }
 }
 
+bool launch_gemm_stream_unwatched(const Problem& p) {
+  const GemmPlan plan = in_range(p) && !captured(p) ? plan_stream(p, true) : GemmPlan{};
+  if (plan.split == 1 || !plan.shares || strip_ahead(p, plan_strip(p), plan)) return false;
+  std::unique_lock<std::mutex> slot_lock;
+  SplitSpace space = library_space(p.stream, plan, false, &slot_lock);
+  space.looks = 0;
+  return space.base != nullptr && launch_gemm_stream(p, plan.variant, plan.split, space);
+}
+
 namespace {
 
 // (gelu onto its own residual stays with the kernels it is on)

@@ -68,6 +68,7 @@ bool gemm_stream_applicable(const Problem& p);
 // Whether the windows of such a tile split over workgroups share the finishing of it; else the last to arrive does that.
 constexpr bool stream_split_shares(int rows, int columns) { return rows >= 64 && columns == 128; }
 constexpr int kMaxWindows = 8;
+constexpr int kSplitLooks = 8;  // looks of such a workgroup at its tile's counter before it gives its fellows up (a trip to memory of about 1 us each)
 constexpr bool stream_pieces_built(int bits, int rows, int columns) { return bits == 8 || rows > 32 || columns > 64; }
 bool stream_scale_pieces(const Problem& p, int rows, int columns, int macro_step);
 // A workspace for K in windows over workgroups: the caller's, or one of the library's own, whose launches are numbered and
@@ -77,13 +78,17 @@ struct SplitSpace {
   void* base = nullptr;
   uint32_t* done = nullptr;
   uint32_t launch = 0;
+  int looks = kSplitLooks;  // (tests: 0, as if every workgroup's fellows came late)
 };
 // (K in `ksplit` windows: over workgroups on a workspace, without one one after the other, with the same result)
 bool launch_gemm_stream(const Problem& p, int variant, int ksplit, const SplitSpace& space);
 template <int BITS>
 bool launch_gemm_stream_bits(const Problem& p, int variant, int ksplit, const SplitSpace& space);  // of that bit width
 int launch_gemm_stream_planned(const Problem& p, void* workspace, int64_t workspace_bytes, float other_us);
-// The same for up to 16 rows, where decode_streams says so.  With a workspace: on that, where the decode kernel does not split K and it is
+// (tests) The planned split on the library's memory, no workgroup of which looks whether its fellows are in: all but a tile's last to arrive
+// resign.  False where the call runs strips, the plan does not split, its windows do not share the finishing, or there is no memory for it.
+bool launch_gemm_stream_unwatched(const Problem& p);
+// launch_gemm_stream_planned for up to 16 rows, where decode_streams says so.  With a workspace: on that, where the decode kernel does not split K and it is
 // large enough.  Without: on a slot, but not under capture nor on hipStreamPerThread, where the library has none
 // for it and the decode kernel is ahead of the unsplit form.
 int launch_gemm_stream_decode(const Problem& p, void* workspace, int64_t workspace_bytes);

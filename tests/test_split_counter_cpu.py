@@ -34,3 +34,135 @@ def test_every_access_to_the_counter_but_its_return_to_zero_is_an_add(name, tmp_
         accesses = [i.split()[0] for i in code if re.match(r"(global|flat)_", i)]
         assert sorted(accesses) == ["global_atomic_add"] * 4 + ["global_store_dword"] * 2, (kernel, accesses)
         assert all("sc0" in i for i in code if i.startswith("global_atomic_add")), kernel
+
+
+PROGRAM = """
+#include <cstdio>
+#include <cstdlib>
+#include <random>
+#include <set>
+#include <vector>
+#include "%s/wq_split_share.h"
+using namespace wq;
+#define CHECK(c) do { if (!(c)) { std::printf("line %%d: %%s (%%d windows, %%d looks)\\n", __LINE__, #c, windows, looks); std::exit(1); } } while (0)
+
+static int windows, looks;
+
+// What is shared, and of every workgroup what its accesses to memory so far have returned.
+struct State {
+  uint32_t counter = 0, returned = 0, finished = 0, shared = 0, written[8] = {};
+  std::vector<uint32_t> seen[8];
+  bool ended[8] = {};
+};
+
+struct Stop {};
+
+// Workgroup w from its beginning again, what it did before answered from `seen`, up to and with one more access to memory.
+static void step(State& s, int w) {
+  size_t at = 0;
+  bool moved = false;
+  auto access = [&](auto&& f) -> uint32_t {
+    if (at < s.seen[w].size()) return s.seen[w][at++];
+    if (moved) throw Stop{};
+    moved = true;
+    s.seen[w].push_back(f());
+    return s.seen[w][at++];
+  };
+  try {
+    const uint32_t parts = split_parts(
+        windows, w, looks, [&](uint32_t p) { access([&] { return s.written[w] |= p & ((1u << windows) - 1); }); }, [&](auto&& f) { return f(); },
+        [&](uint32_t by) {
+          return access([&] {
+            CHECK(!s.returned);  // nobody touches the counter once it is back at zero
+            const uint32_t before = s.counter;
+            s.counter += by;
+            return before;
+          });
+        },
+        [&](auto&& if_last) { if (if_last()) access([&] { return s.counter = 0, ++s.returned; }); });
+    access([&] {
+      CHECK(!(parts & s.finished));  // no part by two workgroups
+      for (int v = 0; v < windows; ++v) CHECK(v == w || (s.written[v] & parts) == parts);  // nor read before it was written
+      s.finished |= parts;
+      if (parts & ~(1u << w)) s.shared |= 1;  // somebody finished another's part
+      if (parts == 0) s.shared |= 2;          // somebody left his own
+      return 0u;
+    });
+    s.ended[w] = true;
+  } catch (Stop) {
+  }
+}
+
+static bool over(const State& s) {
+  for (int w = 0; w < windows; ++w)
+    if (!s.ended[w]) return false;
+  CHECK(s.finished == (1u << windows) - 1 && s.counter == 0 && s.returned == 1);
+  return true;
+}
+
+static std::set<std::vector<uint32_t>> been;
+static uint32_t ends, shared;
+
+static void every_order(const State& s) {
+  std::vector<uint32_t> key{s.counter, s.returned, s.finished, s.shared};
+  for (int w = 0; w < windows; ++w) {
+    key.push_back(s.written[w]), key.push_back(0xFFFFFFFFu);
+    key.insert(key.end(), s.seen[w].begin(), s.seen[w].end());
+  }
+  if (!been.insert(key).second) return;
+  if (over(s)) {
+    ++ends, shared |= s.shared;
+    return;
+  }
+  for (int w = 0; w < windows; ++w)
+    if (!s.ended[w]) {
+      State next = s;
+      step(next, w);
+      every_order(next);
+    }
+}
+
+int main(int argc, char** argv) {
+  windows = std::atoi(argv[1]), looks = std::atoi(argv[2]);
+  if (argc == 3) {
+    every_order(State{});
+    std::printf("%%u ends, shared %%u\\n", ends, shared);
+    return 0;
+  }
+  std::mt19937 rng(windows);
+  for (int run = 0; run < 3000; ++run) {
+    State s;
+    const uint32_t late = rng() %% 100;
+    while (!over(s)) {
+      int w = rng() %% 100 < late ? 0 : rng() %% windows;
+      while (s.ended[w]) w = (w + 1) %% windows;
+      step(s, w);
+    }
+    ++ends, shared |= s.shared;
+  }
+  std::printf("%%u ends, shared %%u\\n", ends, shared);
+  return 0;
+}
+"""
+
+
+@pytest.fixture(scope="module")
+def orders(tmp_path_factory):
+    d = tmp_path_factory.mktemp("orders")
+    (d / "orders.cpp").write_text(PROGRAM % CSRC)
+    subprocess.run(["g++", "-std=c++17", "-O2", "-Wall", "-Werror", "-Wno-attributes", "-o", str(d / "orders"), str(d / "orders.cpp")], check=True)
+    return lambda *args: subprocess.run([str(d / "orders")] + [str(a) for a in args], stdout=subprocess.PIPE, text=True)
+
+
+@pytest.mark.parametrize("windows,looks", [(2, 0), (2, 1), (2, 2), (2, 8), (3, 0), (3, 1), (3, 2), (4, 0)])
+def test_every_part_is_finished_once_in_every_order_of_the_kernels_own_steps(orders, windows, looks):
+    """wq_split_share.h, which the kernel runs, one access to memory at a time."""
+    r = orders(windows, looks)
+    assert r.returncode == 0 and r.stdout.endswith("shared 3\n"), r.stdout
+
+
+@pytest.mark.parametrize("windows", [3, 5, 8])
+@pytest.mark.parametrize("looks", [0, 2, 8])
+def test_every_part_is_finished_once_in_random_orders_of_the_kernels_own_steps(orders, windows, looks):
+    r = orders(windows, looks, "random")
+    assert r.returncode == 0 and r.stdout == "3000 ends, shared 3\n", r.stdout
