@@ -67,11 +67,12 @@ enum {
  * DLTensor* out)`: python/tvm/contrib/cutlass/gemm_operation.py:265-303
  * (pointer/shape extraction, launch on the current stream, no host sync).
  *
- * Calls of 17 rows and more whose tiles leave half of the CUs idle split K over workgroups on one of eight workspaces of 20 MB per GPU
- * that are part of the library's code object (160 MB of each GPU while the library is loaded; the first such call allocates 16 KB
- * of pinned host memory, the others nothing).  One belongs to a stream and passes to another once its owner's last launch
- * on it has ended, also if the owner is gone; a call that finds none (a ninth busy stream, hipStreamPerThread) adds up the same windows one after the other in each workgroup, which takes up to three times as
- * long.  The result has the same bits on every stream, whatever other threads and streams do (up to 16 rows and from 257 on: on every stream but hipStreamPerThread, where the latter run unsplit).  A call under stream
+ * Calls of 17 rows and more whose tiles leave CUs idle (up to 9/16 as many tiles as CUs; from 257 rows on only where that is clearly ahead) split K over
+ * workgroups on one of eight workspaces of 20 MB per GPU that are part of the library's code object (160 MB of each GPU while the library is loaded;
+ * the first such call allocates 16 KB of pinned host memory, the others nothing).  One belongs to a stream and passes to another once its owner's last launch
+ * on it has ended, also if the owner is gone; a call that finds none (a ninth busy stream, hipStreamPerThread) adds up the same windows one after the other in each workgroup.
+ * Where the GPU is idle otherwise that takes up to three times as long as the split, and from 257 rows on 1.4 times as long as an unsplit call (75 problems, 1.0 - 2.1;
+ * with twelve streams busy 0.97).  The result has the same bits on every stream, whatever other threads and streams do (up to 16 rows and from 257 on: on every stream but hipStreamPerThread, where the latter run unsplit).  A call under stream
  * capture uses none of the library's memory and, without a workspace of the caller's (mi355x_wq_matmul_ws), runs
  * unsplit: its float32 sums are added in another order than the eager call's, the same in every replay.
  * Up to 16 rows the same holds for canonical weights with long K (from 8192 on) and few row tiles per CU, where such a

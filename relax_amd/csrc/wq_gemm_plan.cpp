@@ -289,13 +289,24 @@ GemmPlan plan_stream(const Problem& p, bool may_split) {
     for (int s = 1; s <= most; ++s) {
       const int per = s == 1 ? macros : ceil_div(macros, s);
       if (s > 1 && (per < 2 || (s - 1) * per >= macros)) continue;  // (windows that would be empty are dropped)
-      const float us = tile_cost(own, tiles * s, per, s, odd, cu), both = spare * (us + tile_cost(other, tiles * s, per, s, odd, cu));
+      const float us = tile_cost(own, tiles * s, per, s, odd, cu), other_us = tile_cost(other, tiles * s, per, s, odd, cu), both = spare * (us + other_us);
       if (both < best.both_us) {
-        best = GemmPlan{own.variant, s, us, both, tiles, s > 1 ? kSplitCounterBytes + tiles * s * own.bm * own.bn * 4 : 0, stream_split_shares(own.bm, own.bn)};
+        best = GemmPlan{own.variant, s, us, both, tiles, s > 1 ? kSplitCounterBytes + tiles * s * own.bm * own.bn * 4 : 0, stream_split_shares(own.bm, own.bn), other_us};
       }
     }
   }
   return best;
+}
+
+// Whether a call of more than 256 rows that brings no workspace splits on the library's.  Level cost is not enough: the split's costs scatter most where
+// little is gained, the call without memory for it takes up to twice as long (wq_gemm_stream_host.hip), and captured it runs whole with other bits.  Ahead by 3 % and
+// 1 us on both layouts (so that their sums are the same), or calls of 29 us and more, where the costs call the split 5 % dearer than it is.
+// By 170 problems of 257 - 1456 rows for which plan_stream splits, weights from memory: the 130 taken 0.875 of the time whole (four are 2 - 3 % slower),
+// the 40 left would be 1.012 (0.88 - 1.11); 150 others: 124 at 0.863 (none slower), 26 that would be 1.028 (up to 1.15).
+bool split_clearly_ahead(const GemmPlan& split, const GemmPlan& whole) {
+  if (std::min(whole.us, whole.other_us) >= 29.f) return true;
+  auto ahead = [](float a, float b) { return a <= 0.97f * b && a + 1.f <= b; };
+  return ahead(split.us, whole.us) && ahead(split.other_us, whole.other_us);
 }
 
 // The streamed kernel's scales in pieces of eight groups: their rows have to be whole 4-byte words (an even number of groups), and no macro step may reach

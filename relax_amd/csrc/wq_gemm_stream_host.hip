@@ -26,11 +26,12 @@ bool gemm_stream_applicable(const Problem& p) {
 
 namespace {
 
-// Workspaces of the library's own for calls that bring none.  From 257 rows on too, wherever at most half of the CUs would have a tile: int4 512 x 4096 x 11008
-// 59.6 -> 52.5 us, int8 300 x 5120 x 13824 / 5120 x 5120 70.0 -> 59.6 / 30.3 -> 27.4; 40 problems of 257 - 1400 rows 0.87 of the unsplit time (0.62 - 1.0,
-// one of 10 us 1.07).
+// Workspaces of the library's own for calls that bring none; from 257 rows on where split_clearly_ahead says so.
 // The memory is part of the code object (zero at load, as the counters have to be).  A call that finds
-// no slot runs its windows one after the other, with the same result (kSerial in wq_gemm_stream.hip).
+// no slot runs its windows one after the other, with the same result (kSerial in wq_gemm_stream.hip).  What that costs where the chip is idle otherwise (us: split,
+// in turn, whole): int8 99 x 5120 x 13824 31.7, 73.5, 43.1, 300 x 5120 x 13824 59.7, 70.0, 73.1, 259 x 1096 x 11520 18.8, 57.2, 22.5; 75 problems
+// of more than 256 rows 1.38 times the unsplit call (1.0 - 2.1).  With twelve streams at work, which is when a slot is missing, these take 0.97 of the
+// unsplit calls' time (0.73 - 1.16).  Unsplit instead, the bits of a result would depend on what other streams do.
 constexpr int64_t kSlotBytes = kSplitCounterBytes + (20ll << 20);  // (the largest plan: 288 windows of 128 x 128 float32)
 __device__ unsigned char stream_slots[kSlots][kSlotBytes];
 __device__ unsigned char decode_slots[kDecodeSlots][kDecodeSplitBytes];
@@ -51,7 +52,7 @@ struct Slots {
   uint32_t* done = nullptr;  // [SLOTS][kSlotTiles], host memory that the kernels write
 };
 
-// The memory of a device's slots: the workspaces and, at the first call that needs one, 1 KB of pinned host memory for each.
+// The memory of a device's slots: the workspaces and, at the first call that needs one, 2 KB of pinned host memory for each.
 template <int SLOTS, int64_t BYTES>
 bool find_memory(Slots<SLOTS, BYTES>* o, const void* symbol) {
   if (o->done != nullptr) return true;
@@ -139,12 +140,25 @@ int launch_plan(const Problem& p, const GemmPlan& plan, void* workspace, bool sl
 
 }  // namespace
 
+namespace {
+
+// The streamed plan of a call that brings so much workspace; `slot`: its split is to run on one of the library's.
+GemmPlan plan_call(const Problem& p, int64_t workspace_bytes, bool* slot) {
+  const GemmPlan plan = plan_stream(p, true);
+  *slot = plan.split > 1 && plan.bytes > workspace_bytes;
+  if (!*slot || !(p.m > 256 || captured(p))) return plan;
+  // (hipStreamPerThread never has a slot: many rows are not split there)
+  const GemmPlan whole = plan_stream(p, false);
+  *slot = p.stream != hipStreamPerThread && split_clearly_ahead(plan, whole) && !captured(p);
+  return *slot ? plan : whole;
+}
+
+}  // namespace
+
 int launch_gemm_stream_planned(const Problem& p, void* workspace, int64_t workspace_bytes, float other_us) {
   if (!in_range(p)) return 0;
-  GemmPlan plan = plan_stream(p, true);
-  const bool slot = plan.split > 1 && plan.bytes > workspace_bytes;
-  // (hipStreamPerThread never has a slot: many rows, whose windows one after the other would take the longest, are not split there)
-  if (slot && (captured(p) || (p.m > 256 && p.stream == hipStreamPerThread))) plan = plan_stream(p, false);
+  bool slot;
+  const GemmPlan plan = plan_call(p, workspace_bytes, &slot);
   const GemmPlan strip = plan_strip(p);
   switch (choose_streamed(p, strip, plan, other_us)) {
     case kOtherKernel: return 0;
@@ -154,8 +168,9 @@ int launch_gemm_stream_planned(const Problem& p, void* workspace, int64_t worksp
 }
 
 bool launch_gemm_stream_unwatched(const Problem& p) {
-  const GemmPlan plan = in_range(p) && !captured(p) ? plan_stream(p, true) : GemmPlan{};
-  if (plan.split == 1 || !plan.shares || strip_ahead(p, plan_strip(p), plan)) return false;
+  bool slot = false;
+  const GemmPlan plan = in_range(p) ? plan_call(p, 0, &slot) : GemmPlan{};
+  if (!slot || !plan.shares || strip_ahead(p, plan_strip(p), plan)) return false;
   std::unique_lock<std::mutex> slot_lock;
   SplitSpace space = library_space(p.stream, plan, false, &slot_lock);
   space.looks = 0;

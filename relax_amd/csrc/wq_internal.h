@@ -116,8 +116,10 @@ struct GemmPlan {
   float us = 0.f, both_us = 0.f;  // on the problem's layout, on both together
   int64_t tiles = 0, bytes = 0;  // bytes of workspace
   bool shares = false;  // stream_split_shares
+  float other_us = 0.f;  // on the other layout
 };
 GemmPlan plan_stream(const Problem& p, bool may_split);
+bool split_clearly_ahead(const GemmPlan& split, const GemmPlan& whole);
 GemmPlan plan_decode_stream(const Problem& p);
 GemmPlan plan_strip(const Problem& p);  // `variant`: its column tiles, 0 where it does not apply (`us` is out of reach then)
 bool strip_ahead(const Problem& p, const GemmPlan& strip, const GemmPlan& stream);
