@@ -38,13 +38,13 @@ struct TileCost {
 
 // (The tiles of 96 columns, fitted to 1,700 timings of up to 256 rows, are the fastest on 16400 - 24576 columns, where 64-column tiles are more than
 // a round and 128-column ones much less: 17 - 64 rows 0.82 - 0.93 of the time there.  K is not split in them.)
-// (int8 128 x 256 and int4 256 x 256: refitted with their rings of 32-k stages, 320 timings of 130 - 2048 rows, within 3 - 4.5 %; the choice among the three
-// largest tiles by these is within 0.2 % of the fastest.)
+// (int8 128 x 256: refitted with its ring of 32-k stages, 320 timings of 130 - 2048 rows, within 3 %.  int4 256 x 256 likewise, with scales in pieces where they
+// run, by 1,300 timings of 321 problems of 129 - 2048 rows, odd N among them: so that it is to its neighbour 128 x 256 as measured.)
 constexpr TileCost kStreamCost[2][2][9] = {
     {{  // int4, canonical
          {kStream128x256, 128, 256, 0.00f, 5.47f, 2.244f, 1.157f, 8.60f, 0.f, 0.f, 0.f},
          {kStream128x128, 128, 128, 0.00f, 5.68f, 1.212f, 0.494f, 4.15f, 4.12f, 1.383f, 0.31f},
-         {kStream256x256, 256, 256, 0.00f, 10.36f, 4.505f, 1.704f, 20.0f, 0.f, 0.f, 0.f},
+         {kStream256x256, 256, 256, 0.00f, 8.60f, 4.459f, 2.142f, 31.2f, 0.f, 0.f, 0.f},
          {kStream64x128, 64, 128, 1.14f, 3.71f, 0.836f, 0.291f, 2.00f, 2.45f, 0.747f, 1.16f},
          {kStream64x64, 64, 64, 1.47f, 3.12f, 0.520f, 0.181f, 0.00f, 1.75f, 0.450f, 0.19f},
          {kStream32x64, 32, 64, 1.10f, 2.44f, 0.459f, 0.065f, 0.03f, 1.75f, 0.275f, 0.24f},
@@ -54,7 +54,7 @@ constexpr TileCost kStreamCost[2][2][9] = {
      {  // int4, tile-major
          {kStream128x256, 128, 256, 0.00f, 6.00f, 2.483f, 1.013f, 10.16f, 0.f, 0.f, 0.f},
          {kStream128x128, 128, 128, 0.29f, 5.37f, 1.339f, 0.471f, 3.49f, 3.97f, 1.275f, 0.65f},
-         {kStream256x256, 256, 256, 0.00f, 11.85f, 4.305f, 1.617f, 20.05f, 0.f, 0.f, 0.f},
+         {kStream256x256, 256, 256, 0.00f, 9.69f, 4.270f, 2.057f, 33.8f, 0.f, 0.f, 0.f},
          {kStream64x128, 64, 128, 1.11f, 3.78f, 0.902f, 0.262f, 1.90f, 2.52f, 0.802f, 0.53f},
          {kStream64x64, 64, 64, 1.53f, 2.96f, 0.577f, 0.176f, 0.00f, 1.86f, 0.453f, 0.06f},
          {kStream32x64, 32, 64, 1.45f, 2.23f, 0.490f, 0.069f, 0.15f, 1.62f, 0.246f, 0.36f},
@@ -283,7 +283,10 @@ GemmPlan plan_stream(const Problem& p, bool may_split) {
     const int64_t tiles = (int64_t)((p.m + own.bm - 1) >> __builtin_ctz(own.bm)) * (own.bn == 96 ? ceil_div(p.n, 96) : (int)((p.n + own.bn - 1) >> __builtin_ctz(own.bn)));
     // (96 columns above 64 rows, in several row tiles, only by a clear margin: 141 x 7680 x 1536 int4, 240 of them for 180 tiles of 64 x 128, was
     // called 3 % faster and took a layer of such projections 68.9 -> 70.3 us; where it is called 6 % faster it mostly is, 0.86 - 0.91)
-    const float spare = own.bn == 96 && p.m > 64 ? 1.05f : 1.f;
+    // (int4 in 256 x 256 tiles by as clear a margin: ahead mostly on tile-major weights, 2048 x 22016 x 4096 335.8 -> 327.5 canonical and 346 -> 324, and behind
+    // canonically where a round is not full or N odd -- at level cost 1087 x 12288 x 3840 had become 101 -> 107, 1945 x 6461 x 3072 89 -> 105.  Of the 321
+    // problems its costs are by none is more than 1.2 % slower than with the costs before the shorter stages; of 91 that level cost moved to it 51 stay, at 0.998 and 0.970)
+    const float spare = own.bn == 96 && p.m > 64 ? 1.05f : own.bm == 256 && p.bits == 4 ? 1.07f : 1.f;
     // a window has at least two steps of 256 k; up to an eighth more windows than CUs
     const int most = may_split && own.split > 0.f && 2 * tiles <= cu + cu / 8 && tiles <= kSplitMaxTiles / kStreamCounterWords ? std::min({kMaxWindows, (cu + cu / 8) / (int)tiles, macros}) : 1;
     for (int s = 1; s <= most; ++s) {
