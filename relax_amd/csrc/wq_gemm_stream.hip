@@ -28,10 +28,10 @@
 // Rings: what a tile has in flight decides below 128 rows.  int8 64 x 128 with 128-byte weight rows has 32 KB a macro step, and
 // two of them leave one ahead: with 64-byte rows, four macro steps and two K groups 15360 x 5120 at 128 rows 37.9 -> 35.2 us,
 // 27648 x 5120 at 99 71.7 -> 65.3, 5120 x 5120 at 256 29.5 -> 25.7.  int4 64 x 128 has enough in flight and gains from two K
-// groups instead of four (half of the exchange at the end): 12288 x 4096 at 37 rows 20.2 -> 18.7.  The tiles of 256 columns whose ring had
-// room for three stages of 64 k of activations, two ahead of the MFMAs, waited for them; stages of 32 k, six of them in less memory: int8 128 x 256
-// 256 x 15360 x 5120 84 -> 69 us (256 x 27648 x 5120 takes it now, one round for two of 128 x 128: 88 -> 79), int4 256 x 256 512 x 6144 x 4096 108 -> 87
-// (2048 x 22016 x 4096 338 -> 329, on 128 x 256 tiles 335).  256 x 128 tiles, which convert a weight half as often, are behind (int8 256 x 7680 x 5120 82 us
+// groups instead of four (half of the exchange at the end): 12288 x 4096 at 37 rows 20.2 -> 18.7.  Two of the tiles of 256
+// columns, int8 128 x 256 and int4 256 x 256, whose ring had three stages of 64 k of activations, waited for them; six stages of 32 k in the same memory are 160 k
+// ahead of the MFMAs and not 128: int8 128 x 256 256 x 15360 x 5120 84 -> 69 us (256 x 27648 x 5120 takes it now, one round for two of 128 x 128: 88 -> 79),
+// int4 256 x 256 512 x 6144 x 4096 108 -> 87 (2048 x 22016 x 4096 338 -> 328, on 128 x 256 tiles 336).  256 x 128 tiles, which convert a weight half as often, are behind (int8 256 x 7680 x 5120 82 us
 // against 67): twice the activations of a row's weights go through the L1.  32-row tiles for up to 32
 // rows (half of the MFMAs and of the activation traffic; a remainder of up to 32 rows as well): int4 12288 x 4096 at 20 rows
 // 14.0 -> 11.8, 22016 x 4096 21.1 -> 17.8, int8 27648 x 5120 at 32 rows 41.5 -> 32.7 us.  96 columns for
@@ -641,8 +641,8 @@ __global__ __launch_bounds__((CW * G + PROD) * 64, 1) void wq_gemm_stream_kernel
     if constexpr (SCATTER) {
       // Window w's workgroup finishes part w, every S-th quad: it writes the other parts, counts itself in, waits for the others, and reads its
       // part of theirs.  Bound by trips to memory: written, counted, seen, read.  Against the last to arrive finishing the whole tile, with
-      // every workgroup writing all of its own (us): int8 256 x 5120 x 5120 in three 26.2 -> 24.6, 256 x 5120 x 13824 in three 51.9 -> 49.2, 99 x 5120 x
-      // 13824 in six 34.0 -> 30.6, int4 149 x 5760 x 6656 in two 28.7 -> 27.9; 64 x 128 tiles 0.99.
+      // every workgroup writing all of its own (us): int8 256 x 5120 x 5120 in three 27.9 -> 25.9, 256 x 5120 x 13824 in three 49.7 -> 47.2, 99 x 5120 x
+      // 13824 in six 34.7 -> 31.3, int4 256 x 4096 x 11008 in two 35.4 -> 32.5, 149 x 5760 x 6656 in two level at 27.7; 64 x 128 tiles 0.99.
       //
       // Nobody waits for long: a workgroup whose fellows are not in after `looks` looks at the counter resigns (wq_split_share.h).  Every access to the
       // counter but its return to zero is an add, so that all of them are in one order.  The addend is one that the compiler does not see: it would

@@ -64,11 +64,11 @@ bool launch_gemm_pipe(const Problem& p, int group_shift, int variant);
 // `other_us`, is less.  1 launched, 0 not its problem, -1 failure.
 enum { kStream128x256 = 1, kStream128x128, kStream256x256, kStream64x128, kStream64x64, kStream32x64, kStream32x128, kStream64x96, kStream32x96 };
 bool gemm_stream_applicable(const Problem& p);
-// Whether a tile of so many rows and columns, `macro_step` of K at a time, asks for `p`'s scales in pieces; and the tiles that have a build for it.
 // Whether the windows of such a tile split over workgroups share the finishing of it; else the last to arrive does that.
 constexpr bool stream_split_shares(int rows, int columns) { return rows >= 64 && columns == 128; }
 constexpr int kMaxWindows = 8;
 constexpr int kSplitLooks = 8;  // looks of such a workgroup at its tile's counter before it gives its fellows up (a trip to memory of about 1 us each)
+// Whether a tile of so many rows and columns, `macro_step` of K at a time, asks for `p`'s scales in pieces; and the tiles that have a build for it.
 constexpr bool stream_pieces_built(int bits, int rows, int columns) { return bits == 8 || rows > 32 || columns > 64; }
 bool stream_scale_pieces(const Problem& p, int rows, int columns, int macro_step);
 // A workspace for K in windows over workgroups: the caller's, or one of the library's own, whose launches are numbered and
